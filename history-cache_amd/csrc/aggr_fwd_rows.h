@@ -1,0 +1,674 @@
+// History-aware CSR gather-reduce, forward.
+//
+// One wavefront owns one destination row.  The row's neighbour ids are staged
+// 64 at a time with one coalesced load (one id per lane); each id is then
+// broadcast with v_readlane so the neighbour row's base address is
+// wave-uniform and the 64 lanes read one contiguous span of the row with
+// vector loads (as wide as the row length and the pointers' alignment allow).
+// Up to UNROLL neighbour rows are in flight per wave before the first add; the
+// adds run in CSR order in fp32.  Rows of up to 256 edges are therefore summed in
+// exactly the order a sequential CPU loop would use; longer rows (mean and
+// single-head weights) are summed as four contiguous quarters combined left to
+// right -- a fixed order, so results stay bit-reproducible.
+//
+// What bounds it: the bulk of a block is bound by the memory system (5 - 6 TB/s of random rows once the chip is
+// full), the rest by its longest rows, which are therefore shared out slice by slice (seg_list.h).  Measured on
+// MI355X, before (rows of four waves, widths off a multiple of 64 element by element) and after: 3 M edges x 256
+// bf16 with a row of 14 000 edges 1.42 -> 0.30 ms; 600 k edges x 100 fp32 0.64 -> 0.055 ms; 20 M edges x 256 fp32
+// over 20 GB 4.21 -> 4.22 ms (its long rows are short beside the launch).
+//
+// Semantics follow the reference kernels gen_fwd_history_v2,
+// gen_fwd_history_v2_edge_value and gen_fwd_history_v2_edge_value_multi_head
+// (/root/reference/src/cpp/src/history_aggr.cu:7-125); offsets are 64-bit
+// (the reference truncates neighbour ids and offsets to 32-bit int, :19,34-35).
+#pragma once
+
+#include "hc_common.h"
+#include "seg_list.h"
+
+#include <type_traits>
+
+// Rows with more edges than this are summed as four quarters (mean, single-head weights).
+// The CPU checker applies the same rule; the header documents it.
+constexpr int64_t HC_LONG_ROW_EDGES = 256;
+// Rows of several heads are never split into quarters; those above this many edges are summed slice by
+// slice on several compute units (each slice strictly in CSR order).
+constexpr int64_t FWD_HEAD_SLICE_EDGES = 128;
+
+// Wave-cooperative copy of one row of a history buffer into an fp32 output row.
+template <typename TH>
+__device__ __forceinline__ void copy_row_typed(const TH *__restrict__ src, float *__restrict__ dst,
+                                               int64_t F, int lane) {
+  constexpr int V = 4;
+  const bool vec_ok = (F % V == 0) && ((reinterpret_cast<uintptr_t>(src) % (sizeof(TH) * V)) == 0) &&
+                      ((reinterpret_cast<uintptr_t>(dst) % 16) == 0);
+  if (vec_ok) {
+    for (int64_t c = (int64_t)lane * V; c < F; c += HC_WAVE * V) {
+      float v[V];
+      hc_vec<TH, V>::load(src + c, v);
+      *reinterpret_cast<float4 *>(dst + c) = make_float4(v[0], v[1], v[2], v[3]);
+    }
+  } else {
+    for (int64_t c = lane; c < F; c += HC_WAVE) dst[c] = hc_to_f32<TH>(src[c]);
+  }
+}
+
+__device__ __forceinline__ void copy_row_any(const void *hbuf, int hist_dtype, int64_t elem_off,
+                                             float *dst, int64_t F, int lane) {
+  if (hist_dtype == HC_F32) {
+    copy_row_typed<float>(static_cast<const float *>(hbuf) + elem_off, dst, F, lane);
+  } else if (hist_dtype == HC_F16) {
+    copy_row_typed<__half>(static_cast<const __half *>(hbuf) + elem_off, dst, F, lane);
+  } else {
+    copy_row_typed<__hip_bfloat16>(static_cast<const __hip_bfloat16 *>(hbuf) + elem_off, dst, F, lane);
+  }
+}
+
+// WMODE 0: acc += row.  WMODE 1: acc = fma(row, edge_value[edge], acc).  WMODE 2: the row holds
+// n_head heads side by side and every head has its own weight, edge_value[edge, head]; a lane's VEC
+// elements of a chunk lie inside one head, whose weight the lane loads itself.
+constexpr int W_NONE = 0, W_EDGE = 1, W_EDGE_HEAD = 2;
+
+struct FwdArgs {
+  const int64_t *ptr, *idx;
+  const void *vin;
+  const int64_t *hmap;
+  const void *hbuf;
+  int hist_dtype;
+  int64_t hsize;
+  const uint32_t *src_bits;   // per-source substitution, nullable: one bit per source, "has an entry"
+  const float *ev;
+  int n_head;
+  float *vout;
+  int64_t R, F;
+  int slots;                  // F / VEC
+  bool small_matrix;          // vin holds less than 4 GiB
+  int64_t split_above;        // rows with more edges are summed as four quarters (0: never)
+  int64_t slice_above;        // rows with more edges belong to the front blocks, when there are any (0: none)
+  SegList near, far;          // whole-row and slice-wise tasks of the front blocks
+  int n_tiles;                // tiles of the lists; 0: every front block looks the rows through itself
+  int64_t tile;
+  int front;                  // blocks at the start of the grid that work through the lists
+};
+
+// Rows above this many edges are shared out slice by slice; up to it a long row is one block's task.  On large
+// blocks a row may take one compute unit 1/32 of the launch's time (a row of E / 8192 edges) without harm, and
+// whole rows move more bytes per load.
+__device__ __forceinline__ int64_t fwd_far_above(const FwdArgs &a, int64_t total) {
+  const int64_t t = total / 8192;
+  return a.split_above > 0 && t > a.slice_above ? t : a.slice_above;
+}
+
+// Address of the neighbour row that edge `e` reads (and its weight).
+// Per-source substitution: a source whose bit is clear never touches the map, which costs a whole cache line
+// per lookup.  TH is the element type of the history table; when it differs from T the address carries a tag
+// in its lowest bit (rows are at least 2-byte aligned) and the load of a neighbour row picks the element type
+// from it -- the branch is wave-uniform, as the row address is.
+template <typename T, typename TH, bool SRC>
+__device__ __forceinline__ int64_t fwd_row_address(const FwdArgs &a, int64_t id) {
+  int64_t addr = reinterpret_cast<int64_t>(static_cast<const T *>(a.vin) + id * a.F);
+  if constexpr (SRC) {
+    const bool maybe = a.src_bits == nullptr || ((a.src_bits[id >> 5] >> (id & 31)) & 1u) != 0u;
+    if (maybe) {
+      const int64_t slot = a.hmap[id];
+      if (slot != -1)
+        addr = reinterpret_cast<int64_t>(static_cast<const TH *>(a.hbuf) + slot * a.hsize) |
+               (std::is_same<T, TH>::value ? 0 : 1);
+    }
+  }
+  return addr;
+}
+
+// Columns of a lane: chunk k holds elements off[k] .. off[k] + VEC - 1; lanes behind the row's end read
+// the last slot again (no extra line) and store nothing.
+template <int VEC, int CHUNKS>
+struct FwdCols {
+  uint32_t off[CHUNKS];
+  bool on[CHUNKS];
+  int hd[CHUNKS];
+  __device__ __forceinline__ FwdCols(const FwdArgs &a, int tile, int lane, bool heads) {
+#pragma unroll
+    for (int k = 0; k < CHUNKS; ++k) {
+      const int slot = (tile * CHUNKS + k) * HC_WAVE + lane;
+      on[k] = slot < a.slots;
+      off[k] = (uint32_t)(on[k] ? slot : a.slots - 1) * VEC;
+      hd[k] = heads ? (int)(off[k] / (uint32_t)(a.F / a.n_head)) : 0;
+    }
+  }
+};
+
+// Sum of the neighbour rows of edges [begin, end), added to acc in edge order by the calling wave.
+// SRC (per-source substitution): neighbour rows and ids are loaded with the non-temporal hint.  Every edge
+// also looks its source up in the map, and the map (not the rows, which are too many to be reused) is what
+// is worth keeping in the caches.
+template <typename T, typename TH, int VEC, int CHUNKS, int UNROLL, bool SRC, int WMODE>
+__device__ __forceinline__ void fwd_accumulate(const FwdArgs &a, const FwdCols<VEC, CHUNKS> &col, int64_t begin,
+                                               int64_t end, int lane, float (&acc)[CHUNKS][VEC]) {
+  constexpr bool MIXED = SRC && !std::is_same<T, TH>::value;
+  for (int64_t base = begin; base < end; base += HC_WAVE) {
+    const int64_t left = end - base;
+    const int n = left < HC_WAVE ? (int)left : HC_WAVE;
+    // Stage: lane l resolves the address of neighbour base+l.
+    int64_t my_addr = 0;
+    float my_w = 0.0f;
+    if (lane < n) {
+      const int64_t id = SRC ? __builtin_nontemporal_load(a.idx + base + lane) : a.idx[base + lane];
+      my_addr = fwd_row_address<T, TH, SRC>(a, id);
+      if constexpr (WMODE == W_EDGE) my_w = a.ev[base + lane];
+    }
+    for (int j = 0; j < n; j += UNROLL) {
+      typename hc_piece<T, VEC>::raw_t v[UNROLL][CHUNKS];
+      float vm[MIXED ? UNROLL : 1][CHUNKS][VEC];
+      float wh[WMODE == W_EDGE_HEAD ? UNROLL : 1][CHUNKS];
+#pragma unroll
+      for (int u = 0; u < UNROLL; ++u) {
+        if (j + u < n) {
+          const int64_t p = hc_readlane64(my_addr, j + u);
+          if constexpr (MIXED) {
+            if ((p & 1) != 0) {      // a row of the history table, in its own element type
+              typename hc_piece<TH, VEC>::raw_t h[CHUNKS];
+#pragma unroll
+              for (int k = 0; k < CHUNKS; ++k) h[k] = hc_piece<TH, VEC>::template load<true>(p - 1, col.off[k] * (uint32_t)sizeof(TH));
+#pragma unroll
+              for (int k = 0; k < CHUNKS; ++k)
+#pragma unroll
+                for (int i = 0; i < VEC; ++i) vm[u][k][i] = hc_piece<TH, VEC>::widen(h[k], i);
+            } else {
+#pragma unroll
+              for (int k = 0; k < CHUNKS; ++k) v[0][k] = hc_piece<T, VEC>::template load<true>(p, col.off[k] * (uint32_t)sizeof(T));
+#pragma unroll
+              for (int k = 0; k < CHUNKS; ++k)
+#pragma unroll
+                for (int i = 0; i < VEC; ++i) vm[u][k][i] = hc_piece<T, VEC>::widen(v[0][k], i);
+            }
+          } else {
+#pragma unroll
+            for (int k = 0; k < CHUNKS; ++k) {
+              v[u][k] = hc_piece<T, VEC>::template load<SRC>(p, col.off[k] * (uint32_t)sizeof(T));
+              if constexpr (WMODE == W_EDGE_HEAD) wh[u][k] = a.ev[(base + j + u) * a.n_head + col.hd[k]];
+            }
+          }
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < UNROLL; ++u) {
+        if (j + u < n) {
+          const float w1 = WMODE == W_EDGE ? hc_readlane_f(my_w, j + u) : 0.0f;
+#pragma unroll
+          for (int k = 0; k < CHUNKS; ++k)
+#pragma unroll
+            for (int i = 0; i < VEC; ++i) {
+              float x;
+              if constexpr (MIXED) x = vm[u][k][i];
+              else x = hc_piece<T, VEC>::widen(v[u][k], i);
+              if constexpr (WMODE == W_NONE) acc[k][i] += x;
+              else acc[k][i] = __fmaf_rn(x, WMODE == W_EDGE_HEAD ? wh[u][k] : w1, acc[k][i]);
+            }
+        }
+      }
+    }
+  }
+}
+
+// SV adjacent columns per lane of edges [begin, end), summed in edge order with D to 2 D rows in flight: the loads of
+// a group of D rows are issued before the adds of the group in front of it, and the ids of the next 64 edges
+// before the rows of these.  (Straight-line code over whole stages of 64 edges: only then can a wave wait for
+// the older group alone.  A wave on its own is bound by the latency of its groups: 20 000 edges of 64 fp32
+// columns took 390 us with eight rows in flight and one wait for all of them.)
+// W_EDGE: the weight of edge e is ev[e * ev_stride] (rows of several heads whose slice lies in one head).
+// BUF: the matrix is smaller than 4 GiB and its rows are addressed by 32-bit offsets (a wave on its own issues
+// one instruction in four cycles: with 64-bit row addresses the eleven instructions per edge took 23 ns).
+template <typename T, typename TH, int SV, bool SRC, int WMODE, int D, bool BUF>
+__device__ __forceinline__ void fwd_slice_sum(const FwdArgs &a, uint32_t c, int64_t begin, int64_t end, int lane,
+                                              const float *__restrict__ ev, int64_t ev_stride, float (&acc)[SV]) {
+  static_assert(!BUF || !SRC, "the substituted rows lie in another matrix");
+  constexpr int G = HC_WAVE / D;
+  constexpr bool MIXED = SRC && !std::is_same<T, TH>::value;
+  typedef typename hc_piece<T, SV>::raw_t raw_t;
+  const int hd = WMODE == W_EDGE_HEAD ? (int)(c / (uint32_t)(a.F / a.n_head)) : 0;
+#pragma unroll
+  for (int i = 0; i < SV; ++i) acc[i] = 0.0f;
+  if (begin >= end) return;
+  const hc_buffer buf = hc_make_buffer(a.vin);
+  const uint32_t row_bytes = (uint32_t)a.F * (uint32_t)sizeof(T);
+  const auto address = [&](int64_t id) -> int64_t {
+    if constexpr (BUF) return (int64_t)((uint32_t)id * row_bytes);
+    else return fwd_row_address<T, TH, SRC>(a, id);
+  };
+  const auto load = [&](raw_t (&x)[D], float (&w)[D], int64_t addr, int64_t base, int g, int last) {
+    uint32_t off[D];
+    if constexpr (BUF) {
+#pragma unroll
+      for (int u = 0; u < D; ++u) {
+        const int j = g * D + u;
+        off[u] = (uint32_t)__builtin_amdgcn_readlane((int)addr, j < last ? j : last);
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < D; ++u) {
+      int j = g * D + u;
+      j = j < last ? j : last;                                 // behind the end: the last row again, not added
+      if constexpr (BUF) {
+        x[u] = hc_buffer_load<raw_t>(buf, c * (uint32_t)sizeof(T), off[u]);
+      } else {
+        const int64_t p = hc_readlane64(addr, j);
+        if constexpr (MIXED) {
+          static_assert(!MIXED || SV == 1, "a table of another element type beside fp32 rows");
+          if ((p & 1) != 0) w[u] = hc_piece<TH, 1>::widen(hc_piece<TH, 1>::template load<true>(p - 1, c * (uint32_t)sizeof(TH)), 0);
+          else w[u] = hc_piece<T, 1>::widen(hc_piece<T, 1>::template load<true>(p, c * (uint32_t)sizeof(T)), 0);
+        } else {
+          x[u] = hc_piece<T, SV>::template load<SRC>(p, c * (uint32_t)sizeof(T));
+        }
+      }
+      if constexpr (WMODE == W_EDGE_HEAD) w[u] = ev[(base + j) * a.n_head + hd];
+    }
+  };
+  const auto add1 = [&](const raw_t &x, float w, float my_w, int j) {
+    const float w1 = WMODE == W_EDGE ? hc_readlane_f(my_w, j) : w;
+#pragma unroll
+    for (int i = 0; i < SV; ++i) {
+      if constexpr (MIXED) acc[i] += w;
+      else if constexpr (WMODE == W_NONE) acc[i] += hc_piece<T, SV>::widen(x, i);
+      else acc[i] = __fmaf_rn(hc_piece<T, SV>::widen(x, i), w1, acc[i]);
+    }
+  };
+  raw_t x[2][D];
+  float w[2][D];
+  int64_t e = begin + lane < end ? begin + lane : end - 1;
+  int64_t addr = address(a.idx[e]);
+  float my_w = WMODE == W_EDGE ? ev[e * ev_stride] : 0.0f;
+  int last = end - begin < HC_WAVE ? (int)(end - begin) - 1 : HC_WAVE - 1;
+  load(x[0], w[0], addr, begin, 0, last);
+  int64_t base = begin;
+  for (; base + HC_WAVE <= end; base += HC_WAVE) {
+    const int64_t next = base + HC_WAVE;
+    e = next + lane < end ? next + lane : end - 1;
+    const int64_t next_id = a.idx[e];
+    const float next_w = WMODE == W_EDGE ? ev[e * ev_stride] : 0.0f;
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+      if (g + 1 < G) {
+        load(x[(g + 1) & 1], w[(g + 1) & 1], addr, base, g + 1, HC_WAVE - 1);
+      } else {
+        addr = address(next_id);
+        last = end - next < HC_WAVE ? (int)(end - next) - 1 : HC_WAVE - 1;
+        last = last < 0 ? 0 : last;
+        load(x[0], w[0], addr, next < end ? next : end - 1, 0, last);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int u = 0; u < D; ++u) add1(x[g & 1][u], w[g & 1][u], my_w, g * D + u);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    my_w = next_w;
+  }
+  // the last, partial stage: its first group is on its way
+  const int n = (int)(end - base);
+  for (int g = 0; g * D < n; ++g) {
+    if (g > 0) load(x[0], w[0], addr, base, g, n - 1);
+#pragma unroll
+    for (int u = 0; u < D; ++u)
+      if (g * D + u < n) add1(x[0][u], w[0][u], my_w, g * D + u);
+  }
+}
+
+template <typename T, typename TH, int SV, bool SRC, int WMODE, int D>
+__device__ __forceinline__ void fwd_slice_any(const FwdArgs &a, uint32_t c, int64_t begin, int64_t end, int lane,
+                                              const float *__restrict__ ev, int64_t ev_stride, float (&acc)[SV]) {
+  if constexpr (!SRC) {
+    if (a.small_matrix) {
+      fwd_slice_sum<T, TH, SV, SRC, WMODE, D, true>(a, c, begin, end, lane, ev, ev_stride, acc);
+      return;
+    }
+  }
+  fwd_slice_sum<T, TH, SV, SRC, WMODE, D, false>(a, c, begin, end, lane, ev, ev_stride, acc);
+}
+
+// A block owns four consecutive destination rows, one per wave.  Rows of up to 256 edges are summed by
+// their wave, in CSR order.  Longer rows are split into four contiguous quarters (quarter length
+// ceil(deg/4)), each summed in CSR order, and combined left to right, ((q0 + q1) + q2) + q3, before the
+// division: by the front blocks of the grid when the rows were listed (see seg_list.h), else by the four
+// waves of the row's own block behind its other rows.
+constexpr int FWD_ROWS_PER_BLOCK = HC_WAVES_PER_BLOCK;
+constexpr int FWD_XCD_CHUNK = 256;  // consecutive blocks (1024 rows) that share an XCD
+
+// One long row summed by the four waves of the calling block (all of them must call this), whole rows per
+// load: wave w takes the w-th quarter.
+template <typename T, typename TH, int VEC, int CHUNKS, int UNROLL, bool SRC, int WMODE>
+__device__ __forceinline__ void fwd_long_row(const FwdArgs &a, int64_t lrow, int lane, int wave,
+                                             float (*part)[HC_WAVE * VEC * CHUNKS]) {
+  const int64_t lb = a.ptr[lrow];
+  const int64_t le = a.ptr[lrow + 1];
+  const int64_t deg = le - lb;
+  const int64_t q = (deg + HC_WAVES_PER_BLOCK - 1) / HC_WAVES_PER_BLOCK;
+  int64_t sb = lb + wave * q;
+  int64_t se = sb + q;
+  if (sb > le) sb = le;
+  if (se > le) se = le;
+  const int tiles = (a.slots + HC_WAVE * CHUNKS - 1) / (HC_WAVE * CHUNKS);
+  for (int tile = 0; tile < (CHUNKS == 4 ? tiles : 1); ++tile) {
+    const FwdCols<VEC, CHUNKS> col(a, tile, lane, false);
+    float acc[CHUNKS][VEC];
+#pragma unroll
+    for (int c = 0; c < CHUNKS; ++c)
+#pragma unroll
+      for (int i = 0; i < VEC; ++i) acc[c][i] = 0.0f;
+    fwd_accumulate<T, TH, VEC, CHUNKS, UNROLL, SRC, WMODE>(a, col, sb, se, lane, acc);
+    if (wave > 0) {
+#pragma unroll
+      for (int c = 0; c < CHUNKS; ++c)
+#pragma unroll
+        for (int i = 0; i < VEC; ++i) part[wave - 1][(c * HC_WAVE + lane) * VEC + i] = acc[c][i];
+    }
+    __syncthreads();
+    if (wave == 0) {
+      const float fdeg = (float)(int)deg;
+      float *__restrict__ orow = a.vout + lrow * a.F;
+#pragma unroll
+      for (int c = 0; c < CHUNKS; ++c) {
+        float o[VEC];
+#pragma unroll
+        for (int i = 0; i < VEC; ++i) {
+          float t2 = acc[c][i];
+#pragma unroll
+          for (int pw = 0; pw < HC_WAVES_PER_BLOCK - 1; ++pw) t2 += part[pw][(c * HC_WAVE + lane) * VEC + i];
+          o[i] = WMODE != W_NONE ? t2 : (deg > 0 ? t2 / fdeg : 0.0f);
+        }
+        if (col.on[c]) {
+          if constexpr (SRC) hc_store_f32_nt<VEC>(orow + col.off[c], o);
+          else hc_store_f32<VEC>(orow + col.off[c], o);
+        }
+      }
+    }
+    __syncthreads();
+  }
+}
+
+// A slice is one cache line of a row: 32 fp32 columns, or 64 of a half-precision row in 32 lanes of two (a
+// wave-wide load of single half-precision elements takes the address unit three times as long as one of whole
+// words: 350 us instead of 150 us for 20 000 edges).  Half-precision rows of odd length, whose elements cannot be
+// paired, are loaded one by one.
+constexpr int FWD_SLICE_LANES = 32;
+
+// Blocks of at most this many rows need no lists: their front blocks look the rows through themselves.
+constexpr int64_t FWD_SELF_ROWS = 4096;
+constexpr int FWD_SELF_ITEMS = 512;
+
+// The front blocks: slices of the longest rows (one block per task, wave = quarter; rows of several heads: one
+// wave per task), then the other listed rows as whole rows.
+template <typename T, typename TH, int VEC, int CHUNKS, int UNROLL, bool SRC, int WMODE>
+__device__ __forceinline__ void fwd_front(const FwdArgs &a, int64_t far_above, int lane, int wave,
+                                          float (*part)[HC_WAVE * VEC * CHUNKS], int *self_rows, int *self_n) {
+  constexpr int SV = sizeof(T) == 2 && VEC > 1 ? 2 : 1;
+  constexpr int SL = FWD_SLICE_LANES * SV;
+  const int ns = (int)((a.F + SL - 1) / SL);
+  SegIndex far_index;
+  int n_far;
+  if (a.n_tiles > 0) {
+    far_index = seg_index(a.far.count, a.n_tiles, lane);
+    n_far = far_index.total;
+  } else {
+    // Few rows: look them through here (at most FWD_SELF_ITEMS of them can be long, see `listed`).  Wave w takes
+    // a contiguous run of rows and the runs are joined in order, so that every block arrives at the same list.
+    constexpr int IT = (int)(FWD_SELF_ROWS / HC_BLOCK);
+    unsigned long long m[IT];
+    int mine = 0;
+#pragma unroll
+    for (int it = 0; it < IT; ++it) {
+      const int64_t r = ((int64_t)wave * IT + it) * HC_WAVE + lane;
+      const bool is_long = r < a.R && a.ptr[r + 1] - a.ptr[r] > far_above && (SRC || a.hmap == nullptr || a.hmap[r] == -1);
+      m[it] = __ballot(is_long);
+      mine += __popcll(m[it]);
+    }
+    if (lane == 0) self_n[wave] = mine;
+    __syncthreads();
+    int at = 0;
+    n_far = 0;
+#pragma unroll
+    for (int w = 0; w < HC_WAVES_PER_BLOCK; ++w) {
+      if (w < wave) at += self_n[w];
+      n_far += self_n[w];
+    }
+    const unsigned long long below = (1ull << lane) - 1ull;
+#pragma unroll
+    for (int it = 0; it < IT; ++it) {
+      if ((m[it] >> lane) & 1ull) self_rows[at + __popcll(m[it] & below)] = (wave * IT + it) * HC_WAVE + lane;
+      at += __popcll(m[it]);
+    }
+    __syncthreads();
+  }
+  const auto far_row = [&](int e) -> int64_t {
+    if (a.n_tiles == 0) return (int64_t)__builtin_amdgcn_readfirstlane(self_rows[e]);
+    int t, w;
+    seg_locate(far_index, e, lane, &t, &w);
+    return (int64_t)__builtin_amdgcn_readfirstlane(a.far.item[seg_part(a.ptr, (int64_t)t * a.tile, far_above) + w]);
+  };
+  // the lane's columns of slice `sl`; lanes behind the slice or the row read its last ones again
+  const auto columns = [&](int sl, bool &on) -> uint32_t {
+    const int c = (sl * FWD_SLICE_LANES + (lane < FWD_SLICE_LANES ? lane : FWD_SLICE_LANES - 1)) * SV;
+    on = lane < FWD_SLICE_LANES && c < a.F;
+    return (uint32_t)(c < a.F ? c : a.F - SV);
+  };
+  const int64_t tasks = (int64_t)n_far * ns;
+  if (WMODE == W_EDGE_HEAD || a.split_above == 0) {
+    for (int64_t t = (int64_t)wave * a.front + blockIdx.x; t < tasks; t += (int64_t)HC_WAVES_PER_BLOCK * a.front) {
+      const int64_t row = far_row((int)(t / ns));
+      bool on;
+      const uint32_t c = columns((int)(t % ns), on);
+      const int64_t b = a.ptr[row], e = a.ptr[row + 1];
+      float s[SV];
+      if constexpr (WMODE == W_EDGE_HEAD) {
+        // every column of the slice in one head: its weights are staged with the ids, 64 at a time
+        const int fh = (int)(a.F / a.n_head);
+        const int c0 = (int)(t % ns) * SL;
+        const int c1 = (c0 + SL < a.F ? c0 + SL : (int)a.F) - 1;
+        if (c0 / fh == c1 / fh)
+          fwd_slice_any<T, TH, SV, SRC, W_EDGE, 32>(a, c, b, e, lane, a.ev + c0 / fh, a.n_head, s);
+        else
+          fwd_slice_sum<T, TH, SV, SRC, W_EDGE_HEAD, 16, false>(a, c, b, e, lane, a.ev, 0, s);
+      } else {
+        fwd_slice_any<T, TH, SV, SRC, WMODE, 16>(a, c, b, e, lane, a.ev, 1, s);
+      }
+#pragma unroll
+      for (int i = 0; i < SV; ++i)
+        if (on) a.vout[row * a.F + c + i] = WMODE != W_NONE ? s[i] : s[i] / (float)(int)(e - b);
+    }
+    return;
+  }
+  constexpr int LMODE = WMODE == W_EDGE_HEAD ? W_EDGE : WMODE;
+  for (int64_t t = blockIdx.x; t < tasks; t += a.front) {
+    const int64_t row = far_row((int)(t / ns));
+    bool on;
+    const uint32_t c = columns((int)(t % ns), on);
+    const int64_t lb = a.ptr[row], le = a.ptr[row + 1];
+    const int64_t q = (le - lb + HC_WAVES_PER_BLOCK - 1) / HC_WAVES_PER_BLOCK;
+    int64_t sb = lb + wave * q, se = sb + q;
+    if (sb > le) sb = le;
+    if (se > le) se = le;
+    float s[SV];
+    fwd_slice_any<T, TH, SV, SRC, LMODE, 16>(a, c, sb, se, lane, a.ev, 1, s);
+    if (wave > 0 && lane < FWD_SLICE_LANES) {
+#pragma unroll
+      for (int i = 0; i < SV; ++i) part[wave - 1][lane * SV + i] = s[i];
+    }
+    __syncthreads();
+    if (wave == 0 && on) {
+#pragma unroll
+      for (int i = 0; i < SV; ++i) {
+#pragma unroll
+        for (int pw = 0; pw < HC_WAVES_PER_BLOCK - 1; ++pw) s[i] += part[pw][lane * SV + i];
+        a.vout[row * a.F + c + i] = WMODE != W_NONE ? s[i] : s[i] / (float)(int)(le - lb);
+      }
+    }
+    __syncthreads();
+  }
+  if (a.n_tiles == 0) return;
+  const SegIndex near_index = seg_index(a.near.count, a.n_tiles, lane);
+  for (int t = (int)blockIdx.x; t < near_index.total; t += a.front) {
+    int tile, w;
+    seg_locate(near_index, t, lane, &tile, &w);
+    const int64_t row = (int64_t)__builtin_amdgcn_readfirstlane(
+        a.near.item[seg_part(a.ptr, (int64_t)tile * a.tile, a.slice_above) + w]);
+    fwd_long_row<T, TH, VEC, CHUNKS, UNROLL, SRC, LMODE>(a, row, lane, wave, part);
+  }
+}
+
+template <typename T, typename TH, int VEC, int CHUNKS, int UNROLL, bool SRC, int WMODE>
+__global__ __launch_bounds__(HC_BLOCK) void fwd_rows(FwdArgs a) {
+  // without heads the rows may be split: the split code is compiled for those modes only
+  constexpr int LMODE = WMODE == W_EDGE_HEAD ? W_EDGE : WMODE;
+  __shared__ float part[HC_WAVES_PER_BLOCK - 1][HC_WAVE * VEC * CHUNKS];
+  __shared__ int self_rows[FWD_SELF_ITEMS];
+  __shared__ int long_rows[FWD_ROWS_PER_BLOCK];    // (front blocks: the waves' counts)
+  __shared__ int n_long_s;
+  const int lane = hc_lane();
+  const int wave = hc_wave_in_block();
+  // every thread of the grid reads the same two words, so the decision is uniform: the lists hold every long row
+  int64_t far_above = 0;
+  bool listed = false;
+  if (a.front > 0) {
+    const int64_t total = a.ptr[a.R] - a.ptr[0];
+    far_above = fwd_far_above(a, total);
+    if (a.n_tiles > 0)
+      listed = total / (far_above + 1) <= a.far.cap &&
+               (a.split_above == 0 || total / (a.slice_above + 1) <= a.near.cap);
+    else
+      listed = total / (far_above + 1) <= FWD_SELF_ITEMS && far_above == a.slice_above;
+    if ((int)blockIdx.x < a.front) {
+      if (listed)
+        fwd_front<T, TH, VEC, CHUNKS, UNROLL, SRC, WMODE>(a, far_above, lane, wave, part, self_rows, long_rows);
+      return;
+    }
+  }
+  const int64_t row0 = hc_xcd_block<FWD_XCD_CHUNK>((int64_t)blockIdx.x - a.front,
+                                                   (int64_t)gridDim.x - a.front) * FWD_ROWS_PER_BLOCK;
+  const int64_t rest = a.R - row0;
+  const int nrows = rest < FWD_ROWS_PER_BLOCK ? (int)rest : FWD_ROWS_PER_BLOCK;
+  const bool in_block = a.split_above > 0 && !listed;      // the block sums its own long rows afterwards
+
+  if (in_block) {
+    if (threadIdx.x == 0) n_long_s = 0;
+    __syncthreads();
+  }
+
+  if (wave < nrows) {
+    const int64_t row = row0 + wave;
+    float *__restrict__ orow = a.vout + row * a.F;
+    bool hist = false;
+    if (!SRC && a.hmap != nullptr) hist = a.hmap[row] != -1;
+    if (hist) {
+      if (WMODE == W_EDGE_HEAD && a.hsize != a.F) {      // one history row shared by the heads
+        const int64_t fh = a.F / a.n_head;
+        for (int h = 0; h < a.n_head; ++h) copy_row_any(a.hbuf, a.hist_dtype, row * a.hsize, orow + h * fh, fh, lane);
+      } else {
+        copy_row_any(a.hbuf, a.hist_dtype, row * a.hsize, orow, a.F, lane);
+      }
+    } else {
+      const int64_t begin = a.ptr[row];
+      const int64_t end = a.ptr[row + 1];
+      const int64_t deg = end - begin;
+      if (listed && deg > a.slice_above) {
+        // summed by the front blocks
+      } else if (in_block && deg > a.split_above) {
+        if (lane == 0) long_rows[atomicAdd(&n_long_s, 1)] = wave;
+      } else {
+        const int tiles = (a.slots + HC_WAVE * CHUNKS - 1) / (HC_WAVE * CHUNKS);
+        for (int tile = 0; tile < (CHUNKS == 4 ? tiles : 1); ++tile) {
+          const FwdCols<VEC, CHUNKS> col(a, tile, lane, WMODE == W_EDGE_HEAD);
+          float acc[CHUNKS][VEC];
+#pragma unroll
+          for (int c = 0; c < CHUNKS; ++c)
+#pragma unroll
+            for (int i = 0; i < VEC; ++i) acc[c][i] = 0.0f;
+          fwd_accumulate<T, TH, VEC, CHUNKS, UNROLL, SRC, WMODE>(a, col, begin, end, lane, acc);
+          const float fdeg = (float)(int)deg;
+#pragma unroll
+          for (int c = 0; c < CHUNKS; ++c) {
+            float o[VEC];
+#pragma unroll
+            for (int i = 0; i < VEC; ++i) o[i] = WMODE != W_NONE ? acc[c][i] : (deg > 0 ? acc[c][i] / fdeg : 0.0f);
+            if (col.on[c]) {
+              if constexpr (SRC) hc_store_f32_nt<VEC>(orow + col.off[c], o);
+              else hc_store_f32<VEC>(orow + col.off[c], o);
+            }
+          }
+        }
+      }
+    }
+  }
+  if (!in_block) return;  // the whole grid takes the same branch
+  __syncthreads();
+  const int n_long = n_long_s;
+  // The order in which long rows were noted does not matter: each is summed on its own.
+  for (int t = 0; t < n_long; ++t)
+    fwd_long_row<T, TH, VEC, CHUNKS, UNROLL, SRC, LMODE>(a, row0 + long_rows[t], lane, wave, part);
+}
+
+// One translation unit each (the kernels take a minute to compile).
+__attribute__((visibility("hidden"))) int fwd_dispatch_f32(FwdArgs &a, bool src_mode, int n_head, hipStream_t st);
+__attribute__((visibility("hidden"))) int fwd_dispatch_f16(FwdArgs &a, bool src_mode, int n_head, hipStream_t st);
+__attribute__((visibility("hidden"))) int fwd_dispatch_bf16(FwdArgs &a, bool src_mode, int n_head, hipStream_t st);
+
+#ifdef FWD_INSTANTIATE
+namespace {
+
+template <typename T, int VEC, int CHUNKS>
+int launch_rows(const FwdArgs &a, bool src_mode, hipStream_t st) {
+  constexpr int per = VEC * CHUNKS;
+  constexpr int UNROLL = per >= 16 ? 4 : (per >= 4 ? 8 : 16);
+  const int64_t blocks = (a.R + FWD_ROWS_PER_BLOCK - 1) / FWD_ROWS_PER_BLOCK + a.front;
+  if (!hc_grid_ok(blocks)) return HC_EUNSUPPORTED;
+  const dim3 grid((unsigned)blocks), block(HC_BLOCK);
+#define HC_FWD_LAUNCH(TH, SRC, WMODE) fwd_rows<T, TH, VEC, CHUNKS, UNROLL, SRC, WMODE><<<grid, block, 0, st>>>(a)
+  if (a.ev != nullptr && a.n_head > 1) HC_FWD_LAUNCH(T, false, W_EDGE_HEAD);
+  else if (a.ev != nullptr) HC_FWD_LAUNCH(T, false, W_EDGE);
+  else if (src_mode && a.hmap != nullptr) {
+    // the table of a per-source substitution may be narrower than fp32 features
+    if constexpr (std::is_same<T, float>::value) {
+      if (a.hist_dtype == HC_F16) HC_FWD_LAUNCH(__half, true, W_NONE);
+      else if (a.hist_dtype == HC_BF16) HC_FWD_LAUNCH(__hip_bfloat16, true, W_NONE);
+      else HC_FWD_LAUNCH(T, true, W_NONE);
+    } else HC_FWD_LAUNCH(T, true, W_NONE);
+  } else HC_FWD_LAUNCH(T, false, W_NONE);
+#undef HC_FWD_LAUNCH
+  return hc_launch_status();
+}
+
+template <typename T, int VEC>
+int launch_chunks(const FwdArgs &a, bool src_mode, hipStream_t st) {
+  const int chunks = (a.slots + HC_WAVE - 1) / HC_WAVE;
+  if (chunks <= 1) return launch_rows<T, VEC, 1>(a, src_mode, st);
+  if (chunks == 2) return launch_rows<T, VEC, 2>(a, src_mode, st);
+  if (chunks == 3) return launch_rows<T, VEC, 3>(a, src_mode, st);
+  return launch_rows<T, VEC, 4>(a, src_mode, st);       // wider rows: column tiles of 256 slots
+}
+
+// Elements per lane and load: the widest power of two that the row length, a head's width and the pointers
+// allow, halved while the row still fits the wave (all lanes busy rather than wide loads by a few) and a lane
+// loads at least a word (loads of single half-precision elements are slow, see FWD_SLICE_LANES).
+template <typename T>
+int dispatch(FwdArgs &a, bool src_mode, int n_head, hipStream_t st) {
+  const int64_t fh = a.F / n_head;
+  const size_t hesz = a.hist_dtype == HC_F32 ? 4 : 2;
+  const auto fits = [&](int v) {
+    if (fh % v != 0) return false;
+    if (reinterpret_cast<uintptr_t>(a.vin) % (v * sizeof(T)) != 0) return false;
+    if (reinterpret_cast<uintptr_t>(a.vout) % (v > 4 ? 16 : v * sizeof(float)) != 0) return false;
+    if (src_mode && a.hmap != nullptr &&
+        (reinterpret_cast<uintptr_t>(a.hbuf) % (v * hesz) != 0 || a.hsize % v != 0)) return false;
+    return true;
+  };
+  int v = 16 / (int)sizeof(T);
+  while (v > 1 && (!fits(v) || (a.F / (v / 2) <= HC_WAVE && v * sizeof(T) > 4))) v /= 2;
+  if (a.F / v > 0x3fffffffLL) return HC_EUNSUPPORTED;
+  a.slots = (int)(a.F / v);
+  if constexpr (sizeof(T) == 2)
+    if (v == 8) return launch_chunks<T, 8>(a, src_mode, st);
+  if (v == 4) return launch_chunks<T, 4>(a, src_mode, st);
+  if (v == 2) return launch_chunks<T, 2>(a, src_mode, st);
+  return launch_chunks<T, 1>(a, src_mode, st);
+}
+
+}  // namespace
+#endif  // FWD_INSTANTIATE

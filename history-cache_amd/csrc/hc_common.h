@@ -6,6 +6,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 #include "hiscache_hip.h"
 
 #define HC_WAVE 64
@@ -178,6 +180,63 @@ struct hc_vec {
     }
   }
 };
+
+// ---- pieces of a row whose base address is a wave-uniform integer ------------
+// Loads through an explicit global pointer (base in scalar registers, 32-bit byte offset per lane).  A pointer
+// made from an integer is otherwise taken as generic: flat loads, which also occupy the LDS counter, so that a
+// wave can only wait for all of them at once.  `raw_t` keeps the element type until the value is used.
+#define HC_GLOBAL __attribute__((address_space(1)))
+template <int BYTES>
+struct hc_piece_raw;
+template <>
+struct hc_piece_raw<2> { typedef uint16_t type; };
+template <>
+struct hc_piece_raw<4> { typedef uint32_t type; };
+template <>
+struct hc_piece_raw<8> { typedef uint32_t type __attribute__((ext_vector_type(2))); };
+template <>
+struct hc_piece_raw<16> { typedef uint32_t type __attribute__((ext_vector_type(4))); };
+
+template <typename T, int VEC>
+struct hc_piece {
+  typedef typename hc_piece_raw<sizeof(T) * VEC>::type raw_t;
+  // base + byte must be aligned to sizeof(T) * VEC
+  template <bool NT>
+  __device__ __forceinline__ static raw_t load(int64_t base, uint32_t byte) {
+    const HC_GLOBAL char *p = (const HC_GLOBAL char *)base + byte;
+    if constexpr (NT) return __builtin_nontemporal_load((const HC_GLOBAL raw_t *)p);
+    else return *(const HC_GLOBAL raw_t *)p;
+  }
+  __device__ __forceinline__ static float widen(const raw_t &r, int i) {
+    if constexpr (std::is_same<T, float>::value) {
+      if constexpr (VEC == 1) return __uint_as_float(r);
+      else return __uint_as_float(r[i]);
+    } else {
+      uint32_t w;
+      if constexpr (VEC <= 2) w = r;
+      else w = r[i >> 1];
+      if constexpr (std::is_same<T, __hip_bfloat16>::value) {
+        return __uint_as_float((i & 1) ? (w & 0xffff0000u) : (w << 16));
+      } else {
+        const uint16_t h = (uint16_t)((i & 1) ? (w >> 16) : w);
+        return __half2float(__builtin_bit_cast(__half, h));
+      }
+    }
+  }
+};
+
+// One word (or half word) of a row at a wave-uniform 32-bit offset from a matrix of less than 4 GiB: a buffer
+// load takes the row's offset from a scalar register and the lane's from a vector register, which leaves one
+// v_readlane per row as address arithmetic.
+typedef __amdgpu_buffer_rsrc_t hc_buffer;
+__device__ __forceinline__ hc_buffer hc_make_buffer(const void *base) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(base), 0, 0xffffffffu, 0x00027000);
+}
+template <typename RAW>
+__device__ __forceinline__ RAW hc_buffer_load(hc_buffer b, uint32_t lane_byte, uint32_t row_byte) {
+  if constexpr (sizeof(RAW) == 2) return __builtin_amdgcn_raw_buffer_load_b16(b, lane_byte, row_byte, 0);
+  else return __builtin_amdgcn_raw_buffer_load_b32(b, lane_byte, row_byte, 0);
+}
 
 // Store VEC consecutive fp32 values (VEC may exceed one 16-byte store).
 template <int VEC>

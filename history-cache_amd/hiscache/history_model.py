@@ -83,7 +83,8 @@ class _SageConvFunction(torch.autograd.Function):
     def forward(ctx, x, w_l, b_l, w_r, ptr, idx, hmap, hbuf, hsize, num_node, num_edge, sink, view=None):
         be = hiscache_backend
         R = int(num_node) if num_node else ptr.numel() - 1
-        agg = be._aggr_fwd(be.SUBST_ROW, ptr, idx, x, hmap, hbuf, hsize, None, R)
+        agg = be._aggr_fwd(be.SUBST_ROW, ptr, idx, x, hmap, hbuf, hsize, None, R,
+                           max_degree=None if view is None else view.max_out_degree)
         # plain GEMMs and a separate bias add: a GEMM with a bias epilogue goes to hipBLASLt whatever
         # library is preferred, and its per-shape set-up costs the host more than the extra launch
         out = agg @ w_l.t()
@@ -384,7 +385,8 @@ class _RgcnConvFunction(torch.autograd.Function):
         K, Fin, H = weight.shape
         ptr2, idx2, _cnt, _deg, w2 = be.typed_csr(ptr, idx, edge_types, K, R, x.shape[0], used_mask,
                                                   want_weights=True)
-        agg = be._aggr_fwd(be.SUBST_ROW, ptr2, idx2, x, None, None, 0, w2, R * K).view(R, K, Fin)
+        agg = be._aggr_fwd(be.SUBST_ROW, ptr2, idx2, x, None, None, 0, w2, R * K,
+                           max_degree=None if view is None else view.max_out_degree).view(R, K, Fin)
         out = _rel_matmul(agg, weight)
         hit = None
         if hmap is not None:

@@ -103,12 +103,15 @@ class RecordedIteration:
         # a view known to hold no source above the backward's chunk length is recorded without the hub launches
         if view is not None and view.max_in_degree is not None and view.max_in_degree <= self._hub_edges:
             view_kind += 10
+        # ... and one whose rows are bounded (by the sampler's fanout) without the look for long rows
+        if view is not None and view.max_out_degree is not None and view.max_out_degree <= _be.MAX_DEGREE_WITHOUT_LISTS:
+            view_kind += 20
         return nnl, n_edges, view_kind, getattr(batch, "edge_type", None)
 
     # ------------------------------------------------------------------ records
     def _new_record(self, j, view_kind, pre_like, etype):
         L, dev = self.L, self.device
-        hubless, view_kind = view_kind >= 10, view_kind % 10
+        hubless, bounded, view_kind = view_kind // 10 % 2 == 1, view_kind >= 20, view_kind % 10
         has_view = view_kind > 0
         caps, e_cap = self._shape(j)
         r = _Record()
@@ -135,7 +138,8 @@ class RecordedIteration:
             r.have = torch.zeros(caps[L], dtype=torch.uint8, device=dev)
             r.src_ids = torch.full((caps[L],), -1, **i64)
             pre = SimpleNamespace(rows=r.x_pre, have=r.have, src_ids=r.src_ids)
-        view = (_be.BatchView(r.ptrT, r.rowT, r.edgeT, caps[L - 1], caps[L], e_cap, 0 if hubless else None)
+        view = (_be.BatchView(r.ptrT, r.rowT, r.edgeT, caps[L - 1], caps[L], e_cap, 0 if hubless else None,
+                              _be.MAX_DEGREE_WITHOUT_LISTS if bounded else None)
                 if has_view else None)
         r.batch = SimpleNamespace(
             ptr=r.ptr, idx=r.idx, sub_to_full=r.s2f, y=r.y, x=None, edge_type=r.etype, typed_num_node_in_layer=None,

@@ -127,7 +127,8 @@ class NeighborSampler:
             ptrT, rowT, edgeT = out[4], out[5], out[6]
             n_e = max(nel[-1], 1)
             view = _be.BatchView(ptrT[: nnl[L] + 1], rowT[:n_e], None if edgeT is None else edgeT[:n_e],
-                                 nnl[L - 1], nnl[L], nel[-1], max_in_degree=c[2 * L + 1])
+                                 nnl[L - 1], nnl[L], nel[-1], max_in_degree=c[2 * L + 1],
+                                 max_out_degree=max(self.fanout))
         if stream != cur:
             # arrays of a replay slot belong to its graph and are never handed back to the allocator
             for t in ((seeds,) if pooled else (ptr, idx, s2f, seeds)) + (() if y is None else (y,)):

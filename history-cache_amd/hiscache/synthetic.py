@@ -106,6 +106,7 @@ def make_batch(sample, labels, device, emit_view=False, view_edges=False):
         # known here at no cost (the arrays are on the host): lets the backward leave its hub path out
         idx = sample["idx"]
         batch.view.max_in_degree = int(np.bincount(idx, minlength=1).max()) if len(idx) else 0
+        batch.view.max_out_degree = int(np.diff(sample["ptr"]).max()) if len(sample["ptr"]) > 1 else 0
     return batch
 
 

@@ -34,6 +34,7 @@ HC_F32, HC_F16, HC_BF16 = 0, 1, 2
 SUBST_ROW, SUBST_SRC = 0, 1
 NORM_L2, NORM_L1 = 0, 1
 CMP_LT, CMP_NOT_GT = 0, 1
+MAX_DEGREE_WITHOUT_LISTS = 128         # rows of up to this many edges are never listed (hc_aggr_fwd_bounded)
 GRAD_CHECK_STATIC_MAX_ROWS = 1 << 24   # HC_GRAD_CHECK_STATIC_MAX_ROWS
 
 _DTYPES = {torch.float32: HC_F32, torch.float16: HC_F16, torch.bfloat16: HC_BF16}
@@ -51,6 +52,8 @@ _SIGNATURES = {
     "hc_aggr_fwd_workspace_bytes": (_c_sz, [_c_int, _c_i64, _c_i64, _c_i64]),
     "hc_aggr_fwd": (_c_int, [_c_int, _c_p, _c_p, _c_p, _c_int, _c_p, _c_p, _c_int, _c_i64, _c_p, _c_i64,
                              _c_p, _c_i64, _c_i64, _c_i64, _c_p, _c_sz, _c_p]),
+    "hc_aggr_fwd_bounded": (_c_int, [_c_int, _c_p, _c_p, _c_p, _c_int, _c_p, _c_p, _c_int, _c_i64, _c_p, _c_i64,
+                                     _c_p, _c_i64, _c_i64, _c_i64, _c_i64, _c_p, _c_sz, _c_p]),
     "hc_aggr_fwd_long_row_edges": (_c_i64, [_c_i64, _c_int]),
     "hc_transpose_workspace_bytes": (_c_sz, [_c_i64, _c_i64, _c_i64]),
     "hc_build_transpose": (_c_int, [_c_p, _c_p, _c_p, _c_p, _c_i64, _c_i64, _c_i64, _c_p, _c_p, _c_p, _c_p,
@@ -260,7 +263,9 @@ def check_csr(ptr, idx, num_node, n_src):
 
 
 # ----------------------------------------------------------------------------- raw launchers
-def _aggr_fwd(mode, ptr, idx, x, hmap, hbuf, hsize, edge_value, num_node):
+def _aggr_fwd(mode, ptr, idx, x, hmap, hbuf, hsize, edge_value, num_node, max_degree=None):
+    """``max_degree`` (optional): a bound on the rows' edges that the caller knows, e.g. a sampled batch's largest
+    fanout; the library then does not look for long rows."""
     lib = load_library()
     _dev(ptr, "ptr", torch.int64)
     _dev(idx, "idx", torch.int64)
@@ -291,13 +296,16 @@ def _aggr_fwd(mode, ptr, idx, x, hmap, hbuf, hsize, edge_value, num_node):
         check_csr(ptr, idx, R, n_src)
     out_shape = (R, F) if n_head == 1 and x.dim() == 2 else (R, n_head, F)
     out = torch.empty(out_shape, dtype=torch.float32, device=x.device)
-    # scratch for the long-row list (large blocks only: the library reports 0 bytes otherwise)
-    ws_bytes = int(lib.hc_aggr_fwd_workspace_bytes(mode, R, idx.numel(), n_src)) if n_head == 1 else 0
+    # scratch for the lists of long rows (the library reports 0 bytes where it needs none)
+    bound = -1 if max_degree is None else int(max_degree)
+    ws_bytes = 0
+    if mode == SUBST_SRC or not 0 <= bound <= MAX_DEGREE_WITHOUT_LISTS:
+        ws_bytes = int(lib.hc_aggr_fwd_workspace_bytes(mode, R, idx.numel(), n_src))
     ws = _workspace(ws_bytes, x.device) if ws_bytes > 0 else None
-    rc = lib.hc_aggr_fwd(mode, _ptr(ptr), _ptr(idx), _ptr(x), _float_dtype(x, "input"),
-                         _ptr(hmap), _ptr(hbuf), _float_dtype(hbuf, "history_buffer") if hmap is not None else 0,
-                         int(hsize), _ptr(edge_value), n_head, _ptr(out), R, F, n_src, _ptr(ws), ws_bytes,
-                         _stream())
+    rc = lib.hc_aggr_fwd_bounded(mode, _ptr(ptr), _ptr(idx), _ptr(x), _float_dtype(x, "input"),
+                                 _ptr(hmap), _ptr(hbuf), _float_dtype(hbuf, "history_buffer") if hmap is not None else 0,
+                                 int(hsize), _ptr(edge_value), n_head, _ptr(out), R, F, n_src, bound, _ptr(ws), ws_bytes,
+                                 _stream())
     _check(rc, "hc_aggr_fwd")
     return out
 
@@ -379,15 +387,18 @@ class BatchView:
     ``rows`` rows.  A layer that owns the first R <= rows rows and the first n <= n_src sources uses a
     prefix of ``ptrT``; edges of other rows are stepped over in backward.  ``num_edge`` bounds the
     entries of ``rowT`` that hold edges."""
-    __slots__ = ("ptrT", "rowT", "edgeT", "rows", "n_src", "num_edge", "max_in_degree")
+    __slots__ = ("ptrT", "rowT", "edgeT", "rows", "n_src", "num_edge", "max_in_degree", "max_out_degree")
 
-    def __init__(self, ptrT, rowT, edgeT, rows, n_src, num_edge, max_in_degree=None):
+    def __init__(self, ptrT, rowT, edgeT, rows, n_src, num_edge, max_in_degree=None, max_out_degree=None):
         self.ptrT, self.rowT, self.edgeT = ptrT, rowT, edgeT
         self.rows, self.n_src, self.num_edge = int(rows), int(n_src), int(num_edge)
         # the largest number of edges that one node of the batch has in the view, when whoever made the batch
         # knows it (None: unknown).  A view without a source above the backward's chunk length needs neither
         # the chunk sums nor the launch that combines them.
         self.max_in_degree = None if max_in_degree is None else int(max_in_degree)
+        # likewise a bound on the edges of one row of the batch's CSR (a sampled batch: its largest fanout); the
+        # forward passes then look for no long rows
+        self.max_out_degree = None if max_out_degree is None else int(max_out_degree)
 
     def covers(self, num_node, n_src):
         return int(num_node) <= self.rows and int(n_src) <= self.n_src
@@ -492,7 +503,8 @@ class _AggrHistory(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, ptr, idx, edge_value, hmap, hbuf, hsize, num_node, mode, num_edge=None, view=None):
         R = int(num_node) if num_node else ptr.numel() - 1
-        out = _aggr_fwd(mode, ptr, idx, x, hmap, hbuf, hsize, edge_value, R)
+        out = _aggr_fwd(mode, ptr, idx, x, hmap, hbuf, hsize, edge_value, R,
+                        max_degree=None if view is None else view.max_out_degree)
         ctx.hc = (ptr, idx, hmap, hsize, R, mode, None if hbuf is None else tuple(hbuf.shape))
         # edge slots the first R rows can reach, when the caller knows it (a layer of a shared CSR owns a
         # prefix of idx): the transposed view then sorts that prefix only

@@ -77,15 +77,14 @@ int hc_device_count(void);
  * history, hbuf (hist_dtype), vout[R, n_head, F] fp32.  n_head >= 1; n_head > 1
  * requires edge_value.
  * Summation order (fp32, fixed, so results are bit-reproducible): a row is
- * summed in CSR order; when hc_aggr_fwd_long_row_edges() reports a threshold
- * T > 0 for the shape (mean and single-head weighted aggregation on widths
- * that are a multiple of 64), a row with more than T edges is summed as four
+ * summed in CSR order; in the mean and the single-head weighted aggregation a
+ * row with more than T = hc_aggr_fwd_long_row_edges() edges is summed as four
  * contiguous quarters of ceil(deg/4) edges, each in CSR order, combined left to
  * right ((q0+q1)+q2)+q3, then divided (mean only).
  * workspace (optional, NULL allowed; 256-byte aligned, of
  * hc_aggr_fwd_workspace_bytes(mode, R, E, n_src) bytes, E = an upper bound of
- * ptr[R]): on large blocks the long rows are listed first and scheduled at the
- * start of the launch, which shortens its tail; with HC_SUBST_SRC over a
+ * ptr[R]): the long rows are listed first and shared out over the compute
+ * units by the start of the launch, which shortens its tail; with HC_SUBST_SRC over a
  * million sources or more, one bit per source ("has an entry") is derived from
  * hmap first, so that sources without an entry never touch the map.  Results
  * do not depend on the workspace. */
@@ -95,9 +94,20 @@ int hc_aggr_fwd(int mode, const int64_t *ptr, const int64_t *idx, const void *vi
                 const float *edge_value, int64_t n_head, float *vout, int64_t R, int64_t F,
                 int64_t n_src, void *workspace, size_t workspace_bytes, void *stream);
 
-/* The long-row threshold T that hc_aggr_fwd applies to a mean aggregation with
- * rows of F elements of in_dtype; 0 when every row is summed strictly in CSR
- * order.  No reference counterpart (the reference sums every row with one
+/* hc_aggr_fwd for callers that know a bound on the rows' edges (max_degree: no
+ * row has more; negative: unknown, as hc_aggr_fwd).  Same results: with a bound
+ * of at most 128 (several heads) or hc_aggr_fwd_long_row_edges() the call is
+ * one launch that looks for no long rows.  A sampled batch is bounded by its
+ * largest fanout. */
+int hc_aggr_fwd_bounded(int mode, const int64_t *ptr, const int64_t *idx, const void *vin,
+                        int in_dtype, const int64_t *hmap, const void *hbuf, int hist_dtype,
+                        int64_t hsize, const float *edge_value, int64_t n_head, float *vout,
+                        int64_t R, int64_t F, int64_t n_src, int64_t max_degree, void *workspace,
+                        size_t workspace_bytes, void *stream);
+
+/* The long-row threshold T that hc_aggr_fwd applies to a mean or single-head
+ * weighted aggregation with rows of F elements of in_dtype; 0 for arguments
+ * that no call accepts.  No reference counterpart (the reference sums every row with one
  * warp per 32 columns, history_aggr.cu:27-37). */
 int64_t hc_aggr_fwd_long_row_edges(int64_t F, int in_dtype);
 
