@@ -199,17 +199,28 @@ int hc_build_transpose_dev_deg(const int64_t *ptr, const int64_t *idx, const int
  * Summation order (fp32, fixed): ascending destination row.  When a workspace
  * of hc_aggr_bwd_workspace_bytes() is given and hc_aggr_bwd_chunk_edges(F)
  * reports C > 0, a source with more than C incoming edges is summed in chunks
- * of C consecutive edges (each chunk in order, by its own wave) and the chunk
- * sums are combined left to right; without a workspace (NULL), and always for
- * weighted sums, every source is summed strictly in order by one wave.  The workspace must be 256-byte
- * aligned. */
+ * of C consecutive edges (each chunk in order) and the chunk sums are combined
+ * left to right; without a workspace (NULL), and always for weighted sums and
+ * the other widths, every source is summed strictly in order.  The workspace
+ * (256-byte aligned) also holds the lists that share long sources out over the
+ * compute units; with hc_aggr_bwd_workspace_bytes_for() bytes, which counts
+ * the sources too, the sources are moreover dealt to the waves by their edges
+ * (same results).  Both report 0 where a call needs none. */
 size_t hc_aggr_bwd_workspace_bytes(int64_t E_total, int64_t F);
+size_t hc_aggr_bwd_workspace_bytes_for(int64_t E_total, int64_t F, int64_t n_src);
 int64_t hc_aggr_bwd_chunk_edges(int64_t F);
 int hc_aggr_bwd(const int64_t *ptr, const int64_t *idx, const int64_t *ptrT, const int32_t *rowT,
                 const int32_t *edgeT, const float *g, const int64_t *hmap, const float *edge_value,
                 const void *vin, int in_dtype, int64_t n_head, float *grad_vin, float *grad_hbuf,
                 int64_t hsize, float *edge_grad, int64_t E_total, int64_t R, int64_t F,
                 int64_t n_src, void *workspace, size_t workspace_bytes, void *stream);
+/* hc_aggr_bwd with grad_vin of element type grad_dtype (HC_F32, HC_F16, HC_BF16): the fp32 sum of a source is
+ * rounded to it once, when it is stored. */
+int hc_aggr_bwd_as(const int64_t *ptr, const int64_t *idx, const int64_t *ptrT, const int32_t *rowT,
+                   const int32_t *edgeT, const float *g, const int64_t *hmap, const float *edge_value,
+                   const void *vin, int in_dtype, int64_t n_head, void *grad_vin, int grad_dtype, float *grad_hbuf,
+                   int64_t hsize, float *edge_grad, int64_t E_total, int64_t R, int64_t F,
+                   int64_t n_src, void *workspace, size_t workspace_bytes, void *stream);
 
 /* hc_aggr_bwd_batch_view: the mean aggregation's backward over ONE transposed
  * view of the whole mini-batch CSR, shared by every layer of the batch and
@@ -226,7 +237,8 @@ int hc_aggr_bwd(const int64_t *ptr, const int64_t *idx, const int64_t *ptrT, con
  * stepped over here instead of being left out of the view.  grad_vin[n_src, F]
  * and grad_hbuf (nullable) as in hc_aggr_bwd.  E_view bounds ptrT[n_src] (the
  * entries of rowT that may be read; it sizes the workspace:
- * hc_aggr_bwd_workspace_bytes(E_view, F)).
+ * hc_aggr_bwd_workspace_bytes(E_view, F) or
+ * hc_aggr_bwd_workspace_bytes_for(E_view, F, n_src)).
  * Summation order: ascending destination row over the live edges.  With a
  * workspace and C = hc_aggr_bwd_chunk_edges(F) > 0, a source with more than C
  * edges IN THE BATCH VIEW is summed in chunks of C consecutive view positions
@@ -238,6 +250,11 @@ int hc_aggr_bwd_batch_view(const int64_t *ptr, const int64_t *ptrT, const int32_
                            const float *g, const int64_t *hmap, float *grad_vin, float *grad_hbuf,
                            int64_t hsize, int64_t E_view, int64_t R, int64_t F, int64_t n_src,
                            void *workspace, size_t workspace_bytes, void *stream);
+/* The same with grad_vin of element type grad_dtype, as hc_aggr_bwd_as. */
+int hc_aggr_bwd_batch_view_as(const int64_t *ptr, const int64_t *ptrT, const int32_t *rowT,
+                              const float *g, const int64_t *hmap, void *grad_vin, int grad_dtype, float *grad_hbuf,
+                              int64_t hsize, int64_t E_view, int64_t R, int64_t F, int64_t n_src,
+                              void *workspace, size_t workspace_bytes, void *stream);
 
 /* hc_aggr_bwd_batch_view_typed: the input gradient of the relational layer
  * (hiscache/history_model.py:220-278; forward: hc_typed_csr, then hc_aggr_fwd
