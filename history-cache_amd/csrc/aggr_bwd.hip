@@ -1,9 +1,6 @@
 // hc_aggr_bwd: argument checks, the long sources' lists and the runs of sources, the choice of the kernel
 // (aggr_bwd_rows.h; one translation unit per element type of the gradient, aggr_bwd_f32.hip / _f16.hip /
-// _bf16.hip); the gradients of the edge weights and of the history buffer of several heads; the relational
-// layer's backward.
-//
-// edge_grad[j] = <g[r,:], vin[idx[j],:]> as in the reference (/root/reference/src/cpp/src/history_aggr.cu:258-267).
+// _bf16.hip); the gradient of the history buffer of several heads; the relational layer's backward.
 #include "aggr_bwd_rows.h"
 
 namespace {
@@ -109,232 +106,6 @@ __global__ __launch_bounds__(HC_BLOCK) void bwd_hist_generic(const float *__rest
     }
     d[c] = v;
   }
-}
-
-// edge_grad[j,h] = <g[r,h,:], vin[idx[j],h,:]> in CSR order; 0 for edges of history rows and
-// for edge slots in [ptr[R], E_total).  One wave per (row, head); extra blocks clear the tail.
-template <typename T>
-__global__ __launch_bounds__(HC_BLOCK) void bwd_edge_grad(
-    const int64_t *__restrict__ ptr, const int64_t *__restrict__ idx, const float *__restrict__ g,
-    const int64_t *__restrict__ hmap, const T *__restrict__ vin, float *__restrict__ edge_grad,
-    int64_t E_total, int64_t R, int64_t F, int64_t H, int64_t row_blocks) {
-  const int lane = hc_lane();
-  if ((int64_t)blockIdx.x >= row_blocks) {
-    const int64_t nb = (int64_t)gridDim.x - row_blocks;
-    const int64_t start = ptr[R] * H;
-    const int64_t stop = E_total * H;
-    for (int64_t i = start + ((int64_t)blockIdx.x - row_blocks) * HC_BLOCK + threadIdx.x; i < stop;
-         i += nb * HC_BLOCK)
-      edge_grad[i] = 0.0f;
-    return;
-  }
-  const int64_t vrow = (int64_t)blockIdx.x * HC_WAVES_PER_BLOCK + hc_wave_in_block();
-  if (vrow >= R * H) return;
-  const int64_t row = vrow / H;
-  const int64_t head = vrow - row * H;
-  const int64_t begin = ptr[row];
-  int64_t end = ptr[row + 1];
-  if (end > E_total) end = E_total;
-  if (hmap != nullptr && hmap[row] != -1) {
-    for (int64_t e = begin + lane; e < end; e += HC_WAVE) edge_grad[e * H + head] = 0.0f;
-    return;
-  }
-  const float *__restrict__ gr = g + vrow * F;
-  for (int64_t base = begin; base < end; base += HC_WAVE) {
-    const int64_t left = end - base;
-    const int n = left < HC_WAVE ? (int)left : HC_WAVE;
-    int64_t my_id = 0;
-    if (lane < n) my_id = idx[base + lane];
-    float my_out = 0.0f;
-    for (int j = 0; j < n; ++j) {
-      const int64_t id = hc_readlane64(my_id, j);
-      const T *__restrict__ x = vin + (id * H + head) * F;
-      float part = 0.0f;
-      for (int64_t c = lane; c < F; c += HC_WAVE) part = __fmaf_rn(gr[c], hc_to_f32<T>(x[c]), part);
-      part = hc_wave_sum_butterfly(part);
-      if (lane == j) my_out = part;
-    }
-    if (lane < n) edge_grad[(base + lane) * H + head] = my_out;
-  }
-}
-
-// edge_grad on the fast widths, single head: one wave per 64 consecutive edge slots, whatever rows
-// they belong to (a row of thousands of edges is shared by many waves).  Lane l finds the row of
-// slot base + l by binary search over the row offsets between the rows of the wave's first and last
-// slot; then, UNROLL edges at a time, the wave loads g[row] and vin[idx] (consecutive edges of one
-// row re-read the same g row from L1), forms the 64 per-lane partial dot products with fused
-// multiply-adds and sums them with the butterfly.  Slots of history rows and slots behind the last
-// row get 0.
-template <typename T, int VEC, int CHUNKS, int UNROLL>
-__global__ __launch_bounds__(HC_BLOCK) void bwd_edge_grad_fast(
-    const int64_t *__restrict__ ptr, const int64_t *__restrict__ idx, const float *__restrict__ g,
-    const int64_t *__restrict__ hmap, const T *__restrict__ vin, float *__restrict__ edge_grad,
-    int64_t E_total, int64_t R) {
-  constexpr int F = HC_WAVE * VEC * CHUNKS;
-  const int lane = hc_lane();
-  const int64_t base = ((int64_t)blockIdx.x * HC_WAVES_PER_BLOCK + hc_wave_in_block()) * HC_WAVE;
-  if (base >= E_total) return;
-  const int64_t left = E_total - base;
-  const int n = left < HC_WAVE ? (int)left : HC_WAVE;
-  // rows of the first and the last slot: largest r in [0, R] with ptr[r] <= slot
-  int64_t lo = 0, hi = R;
-  const int64_t probe = lane == 0 ? base : base + n - 1;
-  while (lo < hi) {
-    const int64_t mid = (lo + hi + 1) >> 1;
-    if (ptr[mid] <= probe) lo = mid;
-    else hi = mid - 1;
-  }
-  // lanes 0 and 1 searched for the first and the last slot (every other lane repeated the last)
-  int64_t a = hc_readlane64(lo, 0), b = hc_readlane64(lo, 1);
-  int64_t my_row = -1, my_id = 0;
-  if (lane < n) {
-    const int64_t e = base + lane;
-    while (a < b) {
-      const int64_t mid = (a + b + 1) >> 1;
-      if (ptr[mid] <= e) a = mid;
-      else b = mid - 1;
-    }
-    if (a < R && ptr[a] <= e && (hmap == nullptr || hmap[a] == -1)) {
-      my_row = a;
-      my_id = idx[e];
-    }
-  }
-  float my_out = 0.0f;
-  for (int j = 0; j < n; j += UNROLL) {
-    float x[UNROLL][CHUNKS][VEC], gr[UNROLL][CHUNKS][VEC];
-    bool live[UNROLL];
-#pragma unroll
-    for (int u = 0; u < UNROLL; ++u) {
-      live[u] = false;
-      if (j + u < n) {
-        const int64_t r = hc_readlane64(my_row, j + u);
-        if (r >= 0) {
-          live[u] = true;
-          const T *px = vin + hc_readlane64(my_id, j + u) * F + lane * VEC;
-          const float *pg = g + r * F + lane * VEC;
-#pragma unroll
-          for (int k = 0; k < CHUNKS; ++k) {
-            hc_vec<T, VEC>::load(px + k * HC_WAVE * VEC, x[u][k]);
-            hc_vec<float, VEC>::load(pg + k * HC_WAVE * VEC, gr[u][k]);
-          }
-        }
-      }
-    }
-#pragma unroll
-    for (int u = 0; u < UNROLL; ++u) {
-      if (live[u]) {  // wave-uniform
-        float part = 0.0f;
-#pragma unroll
-        for (int k = 0; k < CHUNKS; ++k)
-#pragma unroll
-          for (int i = 0; i < VEC; ++i) part = __fmaf_rn(gr[u][k][i], x[u][k][i], part);
-        part = hc_wave_sum_butterfly(part);
-        if (lane == j + u) my_out = part;
-      }
-    }
-  }
-  if (lane < n) edge_grad[base + lane] = my_out;
-}
-
-// The same for rows of n_head heads side by side (F = n_head * fh elements): edge_grad[e, h] is the dot
-// product over head h only.  A head is either a whole number of 64-lane chunks (one butterfly over the
-// wave per head) or a power-of-two group of lanes inside a chunk (a butterfly inside each group); the
-// first lane of a group stores its head's value.  Slots of history rows and behind the last row get 0.
-template <typename T, int VEC, int CHUNKS, int UNROLL>
-__global__ __launch_bounds__(HC_BLOCK) void bwd_edge_grad_fast_heads(
-    const int64_t *__restrict__ ptr, const int64_t *__restrict__ idx, const float *__restrict__ g,
-    const int64_t *__restrict__ hmap, const T *__restrict__ vin, float *__restrict__ edge_grad,
-    int64_t E_total, int64_t R, int n_head) {
-  constexpr int F = HC_WAVE * VEC * CHUNKS;
-  const int lane = hc_lane();
-  const int64_t base = ((int64_t)blockIdx.x * HC_WAVES_PER_BLOCK + hc_wave_in_block()) * HC_WAVE;
-  if (base >= E_total) return;
-  const int64_t left = E_total - base;
-  const int n = left < HC_WAVE ? (int)left : HC_WAVE;
-  const int lanes_per_head = (F / n_head) / VEC;
-  int64_t lo = 0, hi = R;
-  const int64_t probe = lane == 0 ? base : base + n - 1;
-  while (lo < hi) {
-    const int64_t mid = (lo + hi + 1) >> 1;
-    if (ptr[mid] <= probe) lo = mid;
-    else hi = mid - 1;
-  }
-  int64_t a = hc_readlane64(lo, 0), b = hc_readlane64(lo, 1);
-  int64_t my_row = -1, my_id = 0;
-  if (lane < n) {
-    const int64_t e = base + lane;
-    while (a < b) {
-      const int64_t mid = (a + b + 1) >> 1;
-      if (ptr[mid] <= e) a = mid;
-      else b = mid - 1;
-    }
-    if (a < R && ptr[a] <= e && (hmap == nullptr || hmap[a] == -1)) {
-      my_row = a;
-      my_id = idx[e];
-    }
-  }
-  for (int j = 0; j < n; j += UNROLL) {
-    float x[UNROLL][CHUNKS][VEC], gr[UNROLL][CHUNKS][VEC];
-    bool live[UNROLL];
-#pragma unroll
-    for (int u = 0; u < UNROLL; ++u) {
-      live[u] = false;
-      if (j + u < n) {
-        const int64_t r = hc_readlane64(my_row, j + u);
-        if (r >= 0) {
-          live[u] = true;
-          const T *px = vin + hc_readlane64(my_id, j + u) * F + lane * VEC;
-          const float *pg = g + r * F + lane * VEC;
-#pragma unroll
-          for (int k = 0; k < CHUNKS; ++k) {
-            hc_vec<T, VEC>::load(px + k * HC_WAVE * VEC, x[u][k]);
-            hc_vec<float, VEC>::load(pg + k * HC_WAVE * VEC, gr[u][k]);
-          }
-        }
-      }
-    }
-#pragma unroll
-    for (int u = 0; u < UNROLL; ++u) {
-      if (!live[u]) continue;  // wave-uniform
-      float *__restrict__ o = edge_grad + (base + j + u) * n_head;
-      if (lanes_per_head >= HC_WAVE) {
-        const int chunks_per_head = lanes_per_head / HC_WAVE;
-        for (int h = 0; h < n_head; ++h) {
-          float part = 0.0f;
-#pragma unroll
-          for (int k = 0; k < CHUNKS; ++k)
-            if (k / chunks_per_head == h) {
-#pragma unroll
-              for (int i = 0; i < VEC; ++i) part = __fmaf_rn(gr[u][k][i], x[u][k][i], part);
-            }
-          part = hc_wave_sum_butterfly(part);
-          if (lane == 0) o[h] = part;
-        }
-      } else {
-        const int heads_per_chunk = HC_WAVE / lanes_per_head;
-#pragma unroll
-        for (int k = 0; k < CHUNKS; ++k) {
-          float part = 0.0f;
-#pragma unroll
-          for (int i = 0; i < VEC; ++i) part = __fmaf_rn(gr[u][k][i], x[u][k][i], part);
-          for (int d = lanes_per_head >> 1; d >= 1; d >>= 1) part += __shfl_xor(part, d, HC_WAVE);
-          if (lane % lanes_per_head == 0) o[k * heads_per_chunk + lane / lanes_per_head] = part;
-        }
-      }
-    }
-  }
-  if (lane < n && my_row < 0) {
-    float *__restrict__ o = edge_grad + (base + lane) * n_head;
-    for (int h = 0; h < n_head; ++h) o[h] = 0.0f;
-  }
-}
-
-// Can bwd_edge_grad_fast_heads<.., VEC, ..> take rows of n_head heads of fh elements?
-inline bool edge_grad_heads_ok(int64_t fh, int vec) {
-  if (fh % vec != 0) return false;
-  const int64_t lanes = fh / vec;
-  if (lanes >= HC_WAVE) return lanes % HC_WAVE == 0;
-  return lanes >= 1 && (lanes & (lanes - 1)) == 0;
 }
 
 // The sums of the sources (and grad_hbuf of a single head).  `vin_dtype` is grad_vin's element type.
@@ -518,74 +289,7 @@ int aggr_bwd_impl(const int64_t *ptr, const int64_t *idx, const int64_t *ptrT,
     bwd_hist_generic<<<dim3((unsigned)hb), dim3(HC_BLOCK), 0, st>>>(g, hmap, grad_hbuf, hsize, R, F, n_head);
     if (hc_launch_status() != HC_OK) return HC_ELAUNCH;
   }
-  bool eg_done = false;
-  if (edge_grad && E_total > 0 && n_head == 1 && (reinterpret_cast<uintptr_t>(vin) % 16 == 0) &&
-      (reinterpret_cast<uintptr_t>(g) % 16 == 0)) {
-    const int64_t wb = ((E_total + HC_WAVE - 1) / HC_WAVE + HC_WAVES_PER_BLOCK - 1) / HC_WAVES_PER_BLOCK;
-    if (!hc_grid_ok(wb)) return HC_EUNSUPPORTED;
-    dim3 gr((unsigned)wb), bl(HC_BLOCK);
-    eg_done = true;
-#define HC_EG(T, V, C)                                                                                 \
-  if (F == 64 * (V) * (C))                                                                             \
-    bwd_edge_grad_fast<T, V, C, ((V) * (C) >= 16 ? 2 : ((V) * (C) >= 8 ? 4 : 8))><<<gr, bl, 0, st>>>(     \
-        ptr, idx, g, hmap, static_cast<const T *>(vin), edge_grad, E_total, R);                         \
-  else
-    if (in_dtype == HC_F32) {
-      HC_EG(float, 4, 1) HC_EG(float, 4, 2) HC_EG(float, 4, 3) HC_EG(float, 4, 4) HC_EG(float, 2, 1)
-      HC_EG(float, 1, 1) eg_done = false;
-    } else if (in_dtype == HC_F16) {
-      HC_EG(__half, 4, 1) HC_EG(__half, 4, 2) HC_EG(__half, 4, 3) HC_EG(__half, 4, 4) HC_EG(__half, 2, 1)
-      HC_EG(__half, 1, 1) eg_done = false;
-    } else {
-      HC_EG(__hip_bfloat16, 4, 1) HC_EG(__hip_bfloat16, 4, 2) HC_EG(__hip_bfloat16, 4, 3)
-      HC_EG(__hip_bfloat16, 4, 4) HC_EG(__hip_bfloat16, 2, 1) HC_EG(__hip_bfloat16, 1, 1) eg_done = false;
-    }
-#undef HC_EG
-    if (eg_done && hc_launch_status() != HC_OK) return HC_ELAUNCH;
-  }
-  if (edge_grad && E_total > 0 && !eg_done && n_head > 1 && n_head <= 64 &&
-      (reinterpret_cast<uintptr_t>(vin) % 16 == 0) && (reinterpret_cast<uintptr_t>(g) % 16 == 0)) {
-    const int64_t wb = ((E_total + HC_WAVE - 1) / HC_WAVE + HC_WAVES_PER_BLOCK - 1) / HC_WAVES_PER_BLOCK;
-    if (!hc_grid_ok(wb)) return HC_EUNSUPPORTED;
-    dim3 gr((unsigned)wb), bl(HC_BLOCK);
-    const int64_t Fall = F * n_head;
-    const int nh = (int)n_head;
-    eg_done = true;
-#define HC_EGH(T, V, C)                                                                                  \
-  if (Fall == 64 * (V) * (C) && edge_grad_heads_ok(F, V))                                                \
-    bwd_edge_grad_fast_heads<T, V, C, ((V) * (C) >= 16 ? 2 : ((V) * (C) >= 8 ? 4 : 8))><<<gr, bl, 0, st>>>( \
-        ptr, idx, g, hmap, static_cast<const T *>(vin), edge_grad, E_total, R, nh);                       \
-  else
-    if (in_dtype == HC_F32) {
-      HC_EGH(float, 4, 1) HC_EGH(float, 4, 2) HC_EGH(float, 4, 3) HC_EGH(float, 4, 4) HC_EGH(float, 2, 1)
-      HC_EGH(float, 1, 1) eg_done = false;
-    } else if (in_dtype == HC_F16) {
-      HC_EGH(__half, 4, 1) HC_EGH(__half, 4, 2) HC_EGH(__half, 4, 3) HC_EGH(__half, 4, 4) HC_EGH(__half, 2, 1)
-      HC_EGH(__half, 1, 1) eg_done = false;
-    } else {
-      HC_EGH(__hip_bfloat16, 4, 1) HC_EGH(__hip_bfloat16, 4, 2) HC_EGH(__hip_bfloat16, 4, 3)
-      HC_EGH(__hip_bfloat16, 4, 4) HC_EGH(__hip_bfloat16, 2, 1) HC_EGH(__hip_bfloat16, 1, 1) eg_done = false;
-    }
-#undef HC_EGH
-    if (eg_done && hc_launch_status() != HC_OK) return HC_ELAUNCH;
-  }
-  if (edge_grad && E_total > 0 && !eg_done) {
-    const int64_t rb = (R * n_head + HC_WAVES_PER_BLOCK - 1) / HC_WAVES_PER_BLOCK;
-    const int64_t tail_blocks = 64;
-    if (!hc_grid_ok(rb + tail_blocks)) return HC_EUNSUPPORTED;
-    dim3 gr((unsigned)(rb + tail_blocks)), bl(HC_BLOCK);
-    if (in_dtype == HC_F32)
-      bwd_edge_grad<float><<<gr, bl, 0, st>>>(ptr, idx, g, hmap, static_cast<const float *>(vin),
-                                              edge_grad, E_total, R, F, n_head, rb);
-    else if (in_dtype == HC_F16)
-      bwd_edge_grad<__half><<<gr, bl, 0, st>>>(ptr, idx, g, hmap, static_cast<const __half *>(vin),
-                                               edge_grad, E_total, R, F, n_head, rb);
-    else
-      bwd_edge_grad<__hip_bfloat16><<<gr, bl, 0, st>>>(ptr, idx, g, hmap,
-                                                       static_cast<const __hip_bfloat16 *>(vin),
-                                                       edge_grad, E_total, R, F, n_head, rb);
-    if (hc_launch_status() != HC_OK) return HC_ELAUNCH;
-  }
+  if (edge_grad) return hc_edge_grad(ptr, idx, g, hmap, vin, in_dtype, edge_grad, E_total, R, F, n_head, st);
   return HC_OK;
 }
 

@@ -40,6 +40,12 @@ __attribute__((visibility("hidden"))) int hc_fixup_rows_chunked(const void *src,
                                                                 const uint8_t *have, void *dst, int dst_dtype,
                                                                 int64_t n, int64_t F, hipStream_t st);
 
+// edge_grad.hip: the gradient of the edge weights (hc_aggr_bwd hands over; arguments are checked there).
+__attribute__((visibility("hidden"))) int hc_edge_grad(const int64_t *ptr, const int64_t *idx, const float *g,
+                                                       const int64_t *hmap, const void *vin, int in_dtype,
+                                                       float *edge_grad, int64_t E, int64_t R, int64_t F,
+                                                       int64_t n_head, hipStream_t st);
+
 #ifdef __HIPCC__
 
 __device__ __forceinline__ int hc_lane() { return (int)(threadIdx.x & (HC_WAVE - 1)); }
