@@ -320,7 +320,63 @@ __global__ __launch_bounds__(HC_BLOCK) void bn_bwd_apply(
   *reinterpret_cast<float4 *>(dx + 4 * i) = o;
 }
 
+// y = max(0, ((x + bias) - mean) * invstd * gamma + beta) with the running statistics (evaluation).  A thread keeps
+// one column group and takes BN_FLIGHT rows, so that its channels' square roots are taken once.  NaN stays NaN.
+// Bound by the memory: read x, write y.  (Bias, normalisation and ReLU as operators of their own: three passes;
+// 2 layers of an evaluation batch of 4 000 seeds, 256 channels, 330 us, 93 us in one.)
+__global__ __launch_bounds__(HC_BLOCK) void bn_eval(
+    const float *__restrict__ x, const float *__restrict__ bias, const float *__restrict__ mean,
+    const float *__restrict__ var, const float *__restrict__ gamma, const float *__restrict__ beta, float eps,
+    float *__restrict__ y, int64_t n, int G) {
+  const int P = HC_BLOCK / G;                                    // rows per pass of the block
+  const int g = (int)threadIdx.x % G, p = (int)threadIdx.x / G;
+  if (p >= P) return;
+  const int c = g * 4, C = G * 4;
+  const int64_t r0 = (int64_t)blockIdx.x * P * BN_FLIGHT + p;
+  float4 v[BN_FLIGHT];
+#pragma unroll
+  for (int k = 0; k < BN_FLIGHT; ++k) {
+    const int64_t r = r0 + (int64_t)k * P;
+    if (r < n) v[k] = bn_ld4(x + r * C + c);
+  }
+  const float4 one = make_float4(1.f, 1.f, 1.f, 1.f), zero = make_float4(0.f, 0.f, 0.f, 0.f);
+  const float4 b = bias ? bn_ld4(bias + c) : zero, m = bn_ld4(mean + c), va = bn_ld4(var + c);
+  const float4 ga = gamma ? bn_ld4(gamma + c) : one, be = beta ? bn_ld4(beta + c) : zero;
+  const float4 s = make_float4(1.0f / sqrtf(va.x + eps), 1.0f / sqrtf(va.y + eps), 1.0f / sqrtf(va.z + eps),
+                               1.0f / sqrtf(va.w + eps));
+#pragma unroll
+  for (int k = 0; k < BN_FLIGHT; ++k) {
+    const int64_t r = r0 + (int64_t)k * P;
+    if (r >= n) break;
+    float4 o;
+#define BN_EVAL(F)                                                 \
+  {                                                                \
+    const float t = bn_pre(v[k].F + b.F, m.F, s.F, ga.F, be.F);    \
+    o.F = t < 0.f ? 0.f : t;                                       \
+  }
+    BN_EVAL(x) BN_EVAL(y) BN_EVAL(z) BN_EVAL(w)
+#undef BN_EVAL
+    *reinterpret_cast<float4 *>(y + r * C + c) = o;
+  }
+}
+
 }  // namespace
+
+extern "C" int hc_bn_relu_eval(const float *x, const float *bias, const float *gamma, const float *beta,
+                               const float *running_mean, const float *running_var, float eps, float *y, int64_t n,
+                               int64_t C, void *stream) {
+  HC_REQUIRE(n >= 0 && C >= 1);
+  if (C % 4 != 0 || C > BN_MAX_C) return HC_EUNSUPPORTED;
+  if (n == 0) return HC_OK;
+  HC_REQUIRE(x && y && running_mean && running_var);
+  const int G = (int)(C / 4);
+  const int64_t rows = (int64_t)(HC_BLOCK / G) * BN_FLIGHT;
+  const int64_t blocks = (n + rows - 1) / rows;
+  if (!hc_grid_ok(blocks)) return HC_EUNSUPPORTED;
+  bn_eval<<<dim3((unsigned)blocks), dim3(HC_BLOCK), 0, static_cast<hipStream_t>(stream)>>>(
+      x, bias, running_mean, running_var, gamma, beta, eps, y, n, G);
+  return hc_launch_status();
+}
 
 extern "C" size_t hc_bn_relu_workspace_bytes(int64_t n, int64_t C) {
   BnShape sh;

@@ -149,13 +149,16 @@ def bn_relu(x, bn, bias=None, fused=True, n_dev=None):
     the GPU this is one autograd node over the library's epilogue kernels (two launches forward, two
     backward, against eight and four operator by operator); ``bias`` then must NOT have been added to
     ``x`` yet.  Otherwise the torch operators run.  ``bn``'s running statistics and batch counter are
-    updated as ``torch.nn.BatchNorm1d.forward`` updates them.  ``n_dev`` (one int64 on the device; recorded
+    updated as ``torch.nn.BatchNorm1d.forward`` updates them.  Evaluation with the running statistics and without
+    gradients is one kernel as well.  ``n_dev`` (one int64 on the device; recorded
     iterations over padded batches): the number of rows of ``x`` that are in use."""
     be = hiscache_backend
     if not (fused and bn.training and x.dim() == 2 and be.bn_relu_supported(x, x.shape[1])
             and x.shape[0] > 1):
         if n_dev is not None:
             raise ValueError("a row count on the device needs the fused epilogue (training mode, fp32 on the GPU)")
+        if fused and _evaluates(bn, x, bias):
+            return be.bias_bn_relu_eval(x, bias, bn.weight, bn.bias, bn.running_mean, bn.running_var, bn.eps)
         if bias is not None:
             x = x + bias
         return F.relu(bn(x))
@@ -170,6 +173,19 @@ def bn_relu(x, bn, bias=None, fused=True, n_dev=None):
             counter = bn.num_batches_tracked          # incremented by the statistics kernel
     return be.bias_bn_relu(x, bias, bn.weight, bn.bias, bn.running_mean if track else None,
                            bn.running_var if track else None, momentum, bn.eps, counter, n_dev)
+
+
+def _evaluates(bn, x, bias):
+    """Does ``hc_bn_relu_eval`` cover this call: the running statistics, no gradient, no autocast, plain fp32 vectors
+    on the GPU, and no hook or subclass of the normalisation that a fused call would pass by?"""
+    if bn.training or torch.is_grad_enabled() or torch.is_autocast_enabled("cuda") or type(bn) is not torch.nn.BatchNorm1d:
+        return False
+    if bn._forward_hooks or bn._forward_pre_hooks or bn.running_mean is None or x.dim() != 2 or not x.is_contiguous():
+        return False
+    vectors = [t for t in (bias, bn.weight, bn.bias, bn.running_mean, bn.running_var) if t is not None]
+    return (hiscache_backend.bn_relu_supported(x, x.shape[1]) and x.dtype == torch.float32 and x.data_ptr() % 16 == 0
+            and all(t.is_cuda and t.device == x.device and t.dtype == torch.float32 and t.is_contiguous()
+                    and t.numel() == x.shape[1] and t.data_ptr() % 16 == 0 for t in vectors))
 
 
 class MySageConvHistory(torch.nn.Module):
@@ -267,7 +283,8 @@ class HistorySAGE(torch.nn.Module):
             ne = None if nel is None else int(nel[k])
             ptr = batch.ptr if ptrs is None else ptrs[k]
             # the bias of lin_l goes to the normalisation's kernels instead of a launch of its own
-            defer = self.fused_epilogue and conv.fused and self.training and x.is_cuda
+            defer = (self.fused_epilogue and conv.fused and x.is_cuda
+                     and (self.training or not torch.is_grad_enabled()))
             if self.training and i == self.num_layers - 2:
                 # the layer whose output is one hop from the seeds uses (and produces) history
                 x, his = conv(x, ptr, batch.idx, self.table.sub2embed,

@@ -136,6 +136,7 @@ _SIGNATURES = {
                                     _c_p, _c_p, _c_i64, _c_i64, _c_p, _c_p, _c_sz, _c_p, _c_p]),
     "hc_bn_relu_bwd_dev": (_c_int, [_c_p, _c_p, _c_p, _c_p, _c_p, _c_p, _c_p, _c_p, _c_p, _c_p, _c_i64, _c_i64,
                                     _c_p, _c_p, _c_sz, _c_p, _c_p]),
+    "hc_bn_relu_eval": (_c_int, [_c_p, _c_p, _c_p, _c_p, _c_p, _c_p, ctypes.c_float, _c_p, _c_i64, _c_i64, _c_p]),
     "hc_typed_csr_workspace_bytes": (_c_sz, [_c_i64, _c_int]),
     "hc_edge_types_by_ranges": (_c_int, [_c_p, _c_p, _c_p, _c_i64, _c_p, _c_int, _c_p, _c_p, _c_i64, _c_i64, _c_p]),
     "hc_typed_csr": (_c_int, [_c_p, _c_p, _c_p, _c_p, _c_i64, _c_i64, _c_i64, _c_int, _c_p, _c_p, _c_p, _c_p,
@@ -1416,6 +1417,25 @@ def bias_bn_relu(x, bias, gamma, beta, running_mean, running_var, momentum, eps,
         _dev(n_dev, "n_dev", torch.int64)
     return _BiasBnRelu.apply(x, bias, gamma, beta, running_mean, running_var, momentum, eps, num_batches_tracked,
                              n_dev)
+
+
+def bias_bn_relu_eval(x, bias, gamma, beta, running_mean, running_var, eps):
+    """Evaluation-mode ``relu(batch_norm(x + bias))`` with the running statistics, without gradients; x is [n, C]
+    fp32 on the GPU (``bn_relu_supported``)."""
+    lib = load_library()
+    _dev(x, "x", torch.float32)
+    if x.dim() != 2 or not bn_relu_supported(x, x.shape[1]):
+        raise ValueError("hc_bn_relu_eval: [n, C] fp32 on the GPU with C % 4 == 0 and C <= 1024")
+    for name, t in (("bias", bias), ("gamma", gamma), ("beta", beta), ("running_mean", running_mean),
+                    ("running_var", running_var)):
+        if t is not None:
+            _dev(t, name, torch.float32)
+            if t.numel() != x.shape[1] or t.data_ptr() % 16 != 0:
+                raise ValueError(f"{name} must hold C = {x.shape[1]} values, 16-byte aligned")
+    y = torch.empty_like(x)
+    _check(lib.hc_bn_relu_eval(_ptr(x), _ptr(bias), _ptr(gamma), _ptr(beta), _ptr(running_mean), _ptr(running_var),
+                               float(eps), _ptr(y), x.shape[0], x.shape[1], _stream()), "hc_bn_relu_eval")
+    return y
 
 
 def evict(checkin, slot2full, full2slot, stale_iter, sub2slot=None, score=None, thres=None):

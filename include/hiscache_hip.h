@@ -658,6 +658,12 @@ int hc_bn_relu_bwd(const float *dy, const float *x, const float *gamma, const fl
                    const float *save_mean, const float *save_invstd, float *dx, float *dgamma,
                    float *dbeta, float *dbias, int64_t n, int64_t C, void *workspace,
                    size_t workspace_bytes, unsigned *ticket, void *stream);
+/* hc_bn_relu_eval: y = max(0, batch_norm(x + bias)) with the running statistics (evaluation mode, no gradient), in
+ * one pass; bias, gamma and beta are nullable, C % 4 == 0 and C <= 1024 (else HC_EUNSUPPORTED), all pointers
+ * 16-byte aligned. */
+int hc_bn_relu_eval(const float *x, const float *bias, const float *gamma, const float *beta,
+                    const float *running_mean, const float *running_var, float eps, float *y, int64_t n, int64_t C,
+                    void *stream);
 
 /* hc_weight_grad: the gradient of a layer's linear maps, dw[H, F] = g^T x for
  * g [n, H] and x [n, F] (fp32, row-major, contiguous) -- what autograd computes

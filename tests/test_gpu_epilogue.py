@@ -228,3 +228,42 @@ def test_history_buffer_that_requires_grad_takes_the_operator_spelling():
     pe = cache.produced_embedding
     assert torch.equal(gh[hit], pe.grad[hit])
     assert all(p.grad is not None for p in model.parameters())
+
+
+@pytest.mark.parametrize("n,C", [(1, 4), (7, 64), (8, 256), (65, 256), (1000, 100), (513, 1024), (300, 772)])
+@pytest.mark.parametrize("affine", [True, False])
+def test_evaluation_is_one_kernel(n, C, affine):
+    """Rows around a block's pass, the narrowest and widest rows, NaN and infinities; against fp64.  Bound: the
+    value's own rounding steps, five at the size of the largest intermediate."""
+    import hiscache_backend as be
+    from hiscache.history_model import bn_relu
+    torch.manual_seed(n + C)
+    bn = torch.nn.BatchNorm1d(C, affine=affine).to(DEV)
+    bn.running_mean.normal_()
+    bn.running_var.uniform_(0.5, 2.0)
+    if affine:
+        torch.nn.init.normal_(bn.weight)
+        torch.nn.init.normal_(bn.bias)
+    bn.eval()
+    x, bias = torch.randn(n, C, device=DEV), torch.randn(C, device=DEV)
+    x[0, 0], x[-1, 1], x[n // 2, 2] = float("nan"), float("inf"), float("-inf")
+    calls = []
+    real = be.bias_bn_relu_eval
+    be.bias_bn_relu_eval = lambda *a: (calls.append(1), real(*a))[1]
+    try:
+        with torch.no_grad():
+            got = bn_relu(x, bn, bias).double()
+            bn_relu(x[:, ::2], torch.nn.BatchNorm1d(C // 2).to(DEV).eval(), None)      # strided: torch's operators
+        bn_relu(x, bn, bias)                                                           # with gradients: torch's operators
+    finally:
+        be.bias_bn_relu_eval = real
+    assert len(calls) == 1
+    s = 1.0 / torch.sqrt(bn.running_var.double() + bn.eps)
+    g = bn.weight.double() if affine else torch.ones_like(s)
+    b = bn.bias.double() if affine else torch.zeros_like(s)
+    d = x.double() + bias.double() - bn.running_mean.double()
+    want = torch.relu(d * s * g + b)
+    size = (x.double().abs() + bias.double().abs() + bn.running_mean.double().abs()) * (s * g).abs() + b.abs()
+    fine = torch.isfinite(want) & torch.isfinite(x.double())
+    assert ((got - want).abs()[fine] <= 5 * 2.0 ** -24 * size[fine]).all()
+    assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.isinf(), want.isinf())
