@@ -18,8 +18,8 @@
 //               tile and keep a running count per bucket in LDS; a wave ranks 64 consecutive slots
 //               at a time (see vs_rank_among_equal).  value = destination row (mean aggregation)
 //               or the edge slot
-//   vs_bucket   block per bucket: counts the local ids per wave (the four waves own consecutive
-//               quarters of the bucket's pairs), scans them -- which IS this bucket's stretch of
+//   vs_bucket   block per bucket: counts the local ids per wave (the waves own consecutive equal
+//               shares of the bucket's pairs), scans them -- which IS this bucket's stretch of
 //               ptrT --, ranks the pairs in order the same way and writes rowT (and edgeT) at segment
 //               start + rank, through LDS so that the stores are whole lines
 // Every (source, slot) pair therefore lands where a stable sort by source puts it.  The cost is set
@@ -41,10 +41,12 @@ constexpr int VS_MAX_LOCAL_BITS = 13;                    // 16 bytes of LDS per 
 constexpr int64_t VS_MAX_EDGES = (int64_t)1 << 28;       // the per-tile counts stay a few hundred MB
 constexpr uint32_t VS_DEAD = 0xffffffffu;
 
-constexpr int VB_WAVES = 4;                              // waves per block of vs_bucket
-constexpr int VB_THREADS = VB_WAVES * HC_WAVE;
-constexpr int VB_ITERS = 32;                             // pairs per lane on the register path
-constexpr uint32_t VB_STAGED = VB_THREADS * VB_ITERS;    // 8192: largest bucket that takes the register path
+// Waves per block of vs_bucket.  A wave ranks its share of a bucket 64 pairs at a time, each step behind the one
+// before (0.6 us), and popular sources tend to be neighbours: of 3 M pairs over 1 M sources the fullest of 2 000
+// buckets held 90 000, which took four waves 214 us and takes sixteen 83.  Sixteen wherever their counters fit the LDS.
+constexpr int VB_WAVES_MANY = 16, VB_WAVES_FEW = 4;
+constexpr int VB_MANY_LOCAL_BITS = 11;                   // 64 bytes of counters per local id
+constexpr uint32_t VB_STAGED = 8192;                     // largest bucket that takes the register path
 
 // Tile of a block: workgroup i runs on XCD i % 8, and every XCD gets one contiguous eighth of the
 // tiles, so that the partial lines at the write front of every bucket (runs of a few pairs per tile)
@@ -431,11 +433,13 @@ __device__ __forceinline__ uint32_t vb_swz16w(uint32_t w) { return (w & ~7u) | (
 // Buckets of at most VB_STAGED pairs: the pairs are read once and stay in registers, the cursors are
 // 16 bits wide and the bucket's stretch of rowT is put together in LDS and stored line by line.
 // LDS: cur16[VB_WAVES][n_local] (as words), then stage[VB_STAGED].
-template <bool WANT_EDGES>
+template <bool WANT_EDGES, int VB_WAVES>
 __device__ __forceinline__ void vb_small(const uint2 *__restrict__ mine, uint32_t n, uint32_t p0, int64_t b,
                                          uint32_t *__restrict__ lds, uint32_t *__restrict__ s_wave,
                                          const uint32_t *__restrict__ rows, int64_t *__restrict__ ptrT,
                                          int32_t *__restrict__ rowT, int32_t *__restrict__ edgeT, const VsShape &S) {
+  constexpr int VB_THREADS = VB_WAVES * HC_WAVE;
+  constexpr int VB_ITERS = VB_STAGED / VB_THREADS;        // pairs per lane
   const int tid = (int)threadIdx.x;
   const int lane = hc_lane();
   const int wave = tid >> 6;
@@ -443,10 +447,10 @@ __device__ __forceinline__ void vb_small(const uint2 *__restrict__ mine, uint32_
   const uint32_t words = (n_local + 1u) / 2u;             // cursor words per wave
   uint32_t *stage = lds + VB_WAVES * words;
   uint32_t *my = lds + (uint32_t)wave * words;
-  // the four waves own consecutive quarters of the bucket's pairs
-  const uint32_t quarter = ((n + VB_WAVES - 1) / VB_WAVES + HC_WAVE - 1) / HC_WAVE * HC_WAVE;
-  const uint32_t q_begin = (uint32_t)wave * quarter < n ? (uint32_t)wave * quarter : n;
-  const uint32_t q_len = q_begin + quarter < n ? quarter : n - q_begin;
+  // the waves own consecutive equal shares of the bucket's pairs
+  const uint32_t share = ((n + VB_WAVES - 1) / VB_WAVES + HC_WAVE - 1) / HC_WAVE * HC_WAVE;
+  const uint32_t q_begin = (uint32_t)wave * share < n ? (uint32_t)wave * share : n;
+  const uint32_t q_len = q_begin + share < n ? share : n - q_begin;
   uint2 pr[VB_ITERS];
 #pragma unroll
   for (int j = 0; j < VB_ITERS; ++j) {
@@ -513,7 +517,7 @@ __device__ __forceinline__ void vb_small(const uint2 *__restrict__ mine, uint32_
     if (id <= S.n_src) ptrT[id] = (int64_t)p0 + ((v >> ((k & 1u) * 16u)) & 0xffffu);
   }
   __syncthreads();
-  // every wave ranks the pairs of its quarter in order, 64 at a time
+  // every wave ranks the pairs of its share in order, 64 at a time
   const unsigned long long below = (1ull << lane) - 1ull;
 #pragma unroll
   for (int j = 0; j < VB_ITERS; ++j) {
@@ -548,18 +552,19 @@ __device__ __forceinline__ void vb_small(const uint2 *__restrict__ mine, uint32_
 
 // Buckets above VB_STAGED pairs (hub sources): 32-bit cursors, the pairs are read twice and the
 // results stored as they come.  LDS: cur[VB_WAVES][n_local].
-template <bool WANT_EDGES>
+template <bool WANT_EDGES, int VB_WAVES>
 __device__ __forceinline__ void vb_large(const uint2 *__restrict__ mine, uint32_t n, uint32_t p0, int64_t b,
                                          uint32_t *__restrict__ cur, uint32_t *__restrict__ s_wave,
                                          const uint32_t *__restrict__ rows, int64_t *__restrict__ ptrT,
                                          int32_t *__restrict__ rowT, int32_t *__restrict__ edgeT, const VsShape &S) {
+  constexpr int VB_THREADS = VB_WAVES * HC_WAVE;
   const int tid = (int)threadIdx.x;
   const int lane = hc_lane();
   const int wave = tid >> 6;
   const uint32_t n_local = 1u << S.lb;
-  const uint32_t quarter = ((n + VB_WAVES - 1) / VB_WAVES + HC_WAVE - 1) / HC_WAVE * HC_WAVE;
-  const uint32_t q_begin = (uint32_t)wave * quarter < n ? (uint32_t)wave * quarter : n;
-  const uint32_t q_end = q_begin + quarter < n ? q_begin + quarter : n;
+  const uint32_t share = ((n + VB_WAVES - 1) / VB_WAVES + HC_WAVE - 1) / HC_WAVE * HC_WAVE;
+  const uint32_t q_begin = (uint32_t)wave * share < n ? (uint32_t)wave * share : n;
+  const uint32_t q_end = q_begin + share < n ? q_begin + share : n;
   uint32_t *my = cur + (uint32_t)wave * n_local;
   for (uint32_t i = tid; i < VB_WAVES * n_local; i += VB_THREADS) cur[i] = 0u;
   __syncthreads();
@@ -573,7 +578,8 @@ __device__ __forceinline__ void vb_large(const uint2 *__restrict__ mine, uint32_
     if (k0 < n_local)
       for (uint32_t k = k0; k < k0 + per; ++k) {
         const uint32_t at = vb_swz32(k);
-        sum += cur[at] + cur[n_local + at] + cur[2 * n_local + at] + cur[3 * n_local + at];
+#pragma unroll
+        for (int w = 0; w < VB_WAVES; ++w) sum += cur[(uint32_t)w * n_local + at];
       }
     const uint32_t incl = vs_wave_incl_scan(sum, lane);
     if (lane == HC_WAVE - 1) s_wave[wave] = incl;
@@ -583,12 +589,14 @@ __device__ __forceinline__ void vb_large(const uint2 *__restrict__ mine, uint32_
     if (k0 < n_local)
       for (uint32_t k = k0; k < k0 + per; ++k) {
         const uint32_t at = vb_swz32(k);
-        const uint32_t c0 = cur[at], c1 = cur[n_local + at], c2 = cur[2 * n_local + at], c3 = cur[3 * n_local + at];
-        cur[at] = run;
-        cur[n_local + at] = run + c0;
-        cur[2 * n_local + at] = run + c0 + c1;
-        cur[3 * n_local + at] = run + c0 + c1 + c2;
-        run += c0 + c1 + c2 + c3;
+        uint32_t c[VB_WAVES];
+#pragma unroll
+        for (int w = 0; w < VB_WAVES; ++w) c[w] = cur[(uint32_t)w * n_local + at];
+#pragma unroll
+        for (int w = 0; w < VB_WAVES; ++w) {
+          cur[(uint32_t)w * n_local + at] = run;
+          run += c[w];
+        }
       }
   }
   __syncthreads();
@@ -631,8 +639,8 @@ __device__ __forceinline__ void vb_large(const uint2 *__restrict__ mine, uint32_
   }
 }
 
-template <bool WANT_EDGES>
-__global__ __launch_bounds__(VB_THREADS) void vs_bucket(const uint2 *__restrict__ pairs,
+template <bool WANT_EDGES, int VB_WAVES>
+__global__ __launch_bounds__(VB_WAVES * HC_WAVE) void vs_bucket(const uint2 *__restrict__ pairs,
                                                          const uint32_t *__restrict__ bucket_off,
                                                          const uint32_t *__restrict__ rows,
                                                          int64_t *__restrict__ ptrT, int32_t *__restrict__ rowT,
@@ -642,8 +650,8 @@ __global__ __launch_bounds__(VB_THREADS) void vs_bucket(const uint2 *__restrict_
   const int64_t b = blockIdx.x;
   const uint32_t p0 = bucket_off[b];
   const uint32_t n = bucket_off[b + 1] - p0;               // block-uniform
-  if (n <= VB_STAGED) vb_small<WANT_EDGES>(pairs + p0, n, p0, b, vb_lds, s_wave, rows, ptrT, rowT, edgeT, S);
-  else vb_large<WANT_EDGES>(pairs + p0, n, p0, b, vb_lds, s_wave, rows, ptrT, rowT, edgeT, S);
+  if (n <= VB_STAGED) vb_small<WANT_EDGES, VB_WAVES>(pairs + p0, n, p0, b, vb_lds, s_wave, rows, ptrT, rowT, edgeT, S);
+  else vb_large<WANT_EDGES, VB_WAVES>(pairs + p0, n, p0, b, vb_lds, s_wave, rows, ptrT, rowT, edgeT, S);
 }
 
 struct VsLayout {
@@ -677,10 +685,11 @@ bool vs_shape(int64_t R, int64_t E, int64_t n_src, VsShape *S) {
 size_t vs_scatter_lds(const VsShape &S) {
   return (size_t)S.nbc * sizeof(uint32_t) + (size_t)VS_WAVES * S.nbc * sizeof(uint16_t);
 }
+int vs_bucket_waves(const VsShape &S) { return S.lb <= VB_MANY_LOCAL_BITS ? VB_WAVES_MANY : VB_WAVES_FEW; }
 size_t vs_bucket_lds(const VsShape &S) {
-  const size_t n_local = (size_t)1 << S.lb;
-  const size_t small = VB_WAVES * ((n_local + 1) / 2) * sizeof(uint32_t) + (size_t)VB_STAGED * sizeof(uint32_t);
-  const size_t large = VB_WAVES * n_local * sizeof(uint32_t);
+  const size_t n_local = (size_t)1 << S.lb, waves = (size_t)vs_bucket_waves(S);
+  const size_t small = waves * ((n_local + 1) / 2) * sizeof(uint32_t) + (size_t)VB_STAGED * sizeof(uint32_t);
+  const size_t large = waves * n_local * sizeof(uint32_t);
   return small > large ? small : large;
 }
 
@@ -707,16 +716,26 @@ VsLayout vs_layout(const VsShape &S) {
 // A launch with more dynamic LDS than the default limit (64 KB) has to be allowed once per kernel; the
 // compute unit has 160 KB.  The largest size allowed so far is remembered per kernel (a benign race: two
 // threads may both ask).
-template <typename K>
-bool vs_allow_lds(K kernel, size_t bytes) {
+template <auto KERNEL>
+bool vs_allow_lds(size_t bytes) {
   static size_t allowed = 60 * 1024;
   if (bytes <= allowed) return true;
-  if (hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
+  if (hipFuncSetAttribute(reinterpret_cast<const void *>(KERNEL), hipFuncAttributeMaxDynamicSharedMemorySize,
                           (int)bytes) != hipSuccess) {
     (void)hipGetLastError();
     return false;
   }
   allowed = bytes;
+  return true;
+}
+
+template <bool WANT_EDGES, int VB_WAVES>
+bool vs_launch_bucket(const uint2 *pairs, const uint32_t *bucket_off, const uint32_t *rows, int64_t *ptrT,
+                      int32_t *rowT, int32_t *edgeT, const VsShape &S, hipStream_t st) {
+  const size_t lds = vs_bucket_lds(S);
+  if (!vs_allow_lds<&vs_bucket<WANT_EDGES, VB_WAVES>>(lds)) return false;
+  vs_bucket<WANT_EDGES, VB_WAVES><<<dim3((unsigned)S.nb), dim3(VB_WAVES * HC_WAVE), lds, st>>>(pairs, bucket_off, rows,
+                                                                                             ptrT, rowT, edgeT, S);
   return true;
 }
 
@@ -756,11 +775,8 @@ int vs_launch(const int64_t *ptr, const int64_t *idx, const int64_t *hmap_row, c
     if (blocks > 0) vs_src_bits<<<dim3((unsigned)blocks), dim3(HC_BLOCK), 0, st>>>(hmap_src, n_src, bits);
     src_bits = reinterpret_cast<const uint32_t *>(bits);
   }
-  const size_t lds = vs_scatter_lds(S), blds = vs_bucket_lds(S);
-  const bool lds_ok = edgeT != nullptr
-                          ? vs_allow_lds(&vs_scatter<false>, lds) && vs_allow_lds(&vs_bucket<true>, blds)
-                          : vs_allow_lds(&vs_scatter<true>, lds) && vs_allow_lds(&vs_bucket<false>, blds);
-  if (!lds_ok) return HC_ELAUNCH;
+  const size_t lds = vs_scatter_lds(S);
+  if (!(edgeT != nullptr ? vs_allow_lds<&vs_scatter<false>>(lds) : vs_allow_lds<&vs_scatter<true>>(lds))) return HC_ELAUNCH;
   const dim3 tgrid((unsigned)S.ntiles);
   if (hmap_row != nullptr)
     vs_count<true><<<tgrid, dim3(VS_THREADS), 0, st>>>(ptr, idx, hmap_row, src_bits, key32, tile_count, S);
@@ -771,16 +787,19 @@ int vs_launch(const int64_t *ptr, const int64_t *idx, const int64_t *hmap_row, c
   vs_bucket_scan<<<dim3((unsigned)((S.nb + HC_WAVES_PER_BLOCK - 1) / HC_WAVES_PER_BLOCK)), dim3(HC_BLOCK), 0, st>>>(
       group_count, bucket_total, S);
   vs_bucket_offsets<<<dim3(1), dim3(VS_OFF_THREADS), 0, st>>>(bucket_total, bucket_off, S);
+  const bool many = vs_bucket_waves(S) == VB_WAVES_MANY;
+  bool ok;
   if (edgeT != nullptr) {
     vs_scatter<false><<<tgrid, dim3(VS_THREADS), lds, st>>>(ptr, key32, tile_count, group_count, bucket_off, pairs,
                                                            rows, S);
-    vs_bucket<true><<<dim3((unsigned)S.nb), dim3(VB_THREADS), blds, st>>>(pairs, bucket_off, rows, ptrT, rowT, edgeT,
-                                                                        S);
+    ok = many ? vs_launch_bucket<true, VB_WAVES_MANY>(pairs, bucket_off, rows, ptrT, rowT, edgeT, S, st)
+              : vs_launch_bucket<true, VB_WAVES_FEW>(pairs, bucket_off, rows, ptrT, rowT, edgeT, S, st);
   } else {
     vs_scatter<true><<<tgrid, dim3(VS_THREADS), lds, st>>>(ptr, key32, tile_count, group_count, bucket_off, pairs,
                                                           rows, S);
-    vs_bucket<false><<<dim3((unsigned)S.nb), dim3(VB_THREADS), blds, st>>>(pairs, bucket_off, rows, ptrT, rowT, edgeT,
-                                                                         S);
+    ok = many ? vs_launch_bucket<false, VB_WAVES_MANY>(pairs, bucket_off, rows, ptrT, rowT, edgeT, S, st)
+              : vs_launch_bucket<false, VB_WAVES_FEW>(pairs, bucket_off, rows, ptrT, rowT, edgeT, S, st);
   }
+  if (!ok) return HC_ELAUNCH;
   return hc_launch_status();
 }
