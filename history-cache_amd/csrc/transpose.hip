@@ -213,12 +213,16 @@ __global__ __launch_bounds__(HC_BLOCK) void tr_finalize_ptr(const uint32_t *__re
 
 // ---------------------------------------------------------------------------------------
 // Small blocks (sampled mini-batches: at most TR_SMALL_EDGES edge slots and TR_SMALL_SOURCES sources):
-// a counting sort in four launches of this file's own kernels instead of the library sort's dozen.
-//   tr_small_clear  zero the per-source counters and the ticket
+// a counting sort in a few launches of this file's own kernels instead of the library sort's dozen.
+//   tr_small_clear  zero the per-source counters
 //   tr_small_count  thread per edge slot: the slot's key (source id, or the sentinel for a dropped
 //                   slot) and destination row are saved and the source's counter is bumped (integer
-//                   atomics: the final counts do not depend on their order); the block that finishes
-//                   last turns the counters into ptrT (exclusive scan) and into per-source cursors
+//                   atomics: the final counts do not depend on their order)
+//   tr_small_sums   (more than TRS_DIRECT_TILES tiles of 4096 sources) every tile's sum
+//   tr_small_scan   block per tile: the counters become ptrT (exclusive scan) and per-source cursors; the
+//                   sum in front of the tile is added up from the tiles' sums, or from the counters
+//                   themselves where the tiles are few.  (One block that scanned all counters behind a
+//                   ticket took 100 us of a batch of 230 000 sources; the two launches take 9.)
 //   tr_small_place  thread per edge slot: takes the next free position of its source's segment
 //                   (atomic: WHICH slots a segment holds is fixed, their order inside it is not yet)
 //                   and writes (row, slot) there, into temporary arrays
@@ -228,7 +232,7 @@ __global__ __launch_bounds__(HC_BLOCK) void tr_finalize_ptr(const uint32_t *__re
 //                   ones by the whole block through a bitmap of the segment's slots in LDS (rank =
 //                   number of set bits below the slot), one window of TR_SMALL_EDGES slots at a time
 // The result is bit-identical to the sorted view of the large-block path.
-// The same four kernels serve hc_build_transpose_dev, where the block's sizes are read from device
+// The same kernels serve hc_build_transpose_dev, where the block's sizes are read from device
 // memory (TrDims) and the launches are sized by capacities of up to 2^24 edge slots / sources.
 // ---------------------------------------------------------------------------------------
 constexpr int TRS_BLOCK = 1024;
@@ -237,10 +241,8 @@ constexpr int TRS_BITMAP_WORDS = (int)(TR_SMALL_EDGES / 32);   // one bit per ed
 constexpr int TRS_ORDER_SOURCES = HC_BLOCK;                     // sources per block of tr_small_order
 constexpr int TRS_LANE_SORT = 8;                                // longest segment a single lane sorts
 
-struct TrSmallHeader {
-  unsigned ticket;
-  unsigned pad[63];
-};
+constexpr int TRS_TILE = TRS_BLOCK * 4;                         // counters per block of the scan
+constexpr int64_t TRS_DIRECT_TILES = 8;                         // up to so many tiles go without their sums
 
 // Sizes of the block: given by value, or -- when the host does not know them yet (a batch that the
 // sampler has just drawn) -- read from device memory and clamped to the bounds the launch was sized for.
@@ -268,41 +270,28 @@ __device__ __forceinline__ bool tr_dims_clamped(const TrDims &d) {
   return r < 0 || e < 0 || s < 0 || e > d.E || s > d.n_src;
 }
 
-// zero the ticket and the counters of sources [0, n_src] (rounded up to whole 16-byte groups)
+// zero the counters of sources [0, n_src] (rounded up to whole 16-byte groups)
 __global__ __launch_bounds__(HC_BLOCK) void tr_small_clear(uint32_t *__restrict__ p, TrDims dims) {
   int64_t R, E, n_src;
   tr_dims(dims, R, E, n_src);
-  const int64_t n = (int64_t)(sizeof(TrSmallHeader) / sizeof(uint32_t)) + (n_src + 1 + 3) / 4 * 4;
+  const int64_t n = (n_src + 1 + 3) / 4 * 4;
   const int64_t i = (int64_t)blockIdx.x * HC_BLOCK + threadIdx.x;
   if (i < n) p[i] = 0u;
   if (i == 0 && dims.overflow != nullptr) *dims.overflow = tr_dims_clamped(dims) ? 1 : 0;
+  if (i == 0 && dims.max_count != nullptr) *dims.max_count = 0;
 }
-
-// Read of a counter by the block that scans them.  The counters were only ever touched by atomics (which
-// work in the L2) and this block reads them behind its device-scope fence, so an ordinary load sees the
-// final values; ordinary loads, unlike atomic ones, are issued back to back.
-__device__ __forceinline__ int trs_load(const int *p) { return *p; }
 
 __global__ __launch_bounds__(TRS_BLOCK) void tr_small_count(
     const int64_t *__restrict__ ptr, const int64_t *__restrict__ idx, const int64_t *__restrict__ hmap_row,
     const int64_t *__restrict__ hmap_src, uint32_t *__restrict__ keys, int32_t *__restrict__ rows,
-    int *__restrict__ count, TrSmallHeader *__restrict__ header, int64_t *__restrict__ ptrT, TrDims dims) {
+    int *__restrict__ count, TrDims dims) {
   __shared__ int64_t s_ptr[TR_LDS_ROWS];
   __shared__ int64_t s_range[2];
-  __shared__ int s_wave[TRS_BLOCK / HC_WAVE];
-  __shared__ int s_last;
   int64_t R, E, n_src;
   tr_dims(dims, R, E, n_src);
-  // The launch may be sized for more edge slots than the block has (sizes read on the device): only the
-  // blocks that own edge slots take part, and block 0 always does, so that some block runs the scan.
-  // (Every ticket is an atomic on one address; hundreds of idle blocks queueing for it cost more than
-  // the work itself.)
-  const int64_t with_edges = R > 0 ? (E + TRS_BLOCK - 1) / TRS_BLOCK : 0;
-  const unsigned active = with_edges > 0 ? (unsigned)with_edges : 1u;
-  if (blockIdx.x >= active) return;
   const int64_t e0 = (int64_t)blockIdx.x * TRS_BLOCK;
   const int64_t e1 = e0 + TRS_BLOCK < E ? e0 + TRS_BLOCK : E;
-  if (e0 < E && R > 0) {                 // block-uniform (false only for block 0 of a block without edges)
+  if (e0 < E && R > 0) {                 // block-uniform (the launch may be sized for more edge slots)
     if (threadIdx.x < 2 * HC_WAVE) {       // the tile's first and last row, searched by two waves side by side
       const int lane0 = hc_lane();
       const int which = (int)(threadIdx.x >> 6);
@@ -337,101 +326,97 @@ __global__ __launch_bounds__(TRS_BLOCK) void tr_small_count(
       if (live) atomicAdd(count + src, 1);
     }
   }
-  // The block that takes the last ticket sees every block's counts.  One device-scope release per
-  // block, by the thread that takes the ticket, behind the block's barrier (which orders the other
-  // waves' atomics in front of it): on this multi-die part a device-scope release writes the die's L2
-  // back, and one per wave made this kernel several times longer.
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+}
+
+// Four counters per thread.  Entries between n_src and the end of the counter array are zero.
+__device__ __forceinline__ int4 trs_counters(const int *__restrict__ count, int64_t i, int64_t n_entries) {
+  return i < (n_entries + 3) / 4 * 4 ? *reinterpret_cast<const int4 *>(count + i) : make_int4(0, 0, 0, 0);
+}
+
+// Sum over the block (every thread calls it; `s_wave` is free again when it returns).
+__device__ __forceinline__ int trs_block_sum(int v, int *s_wave) {
+#pragma unroll
+  for (int d = HC_WAVE / 2; d > 0; d >>= 1) v += __shfl_xor(v, d, HC_WAVE);
+  if (hc_lane() == 0) s_wave[threadIdx.x >> 6] = v;
   __syncthreads();
-  if (threadIdx.x == 0) {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
-    s_last = atomicAdd(&header->ticket, 1u) == active - 1u ? 1 : 0;
-  }
+  int sum = 0;
+#pragma unroll
+  for (int w = 0; w < TRS_BLOCK / HC_WAVE; ++w) sum += s_wave[w];
   __syncthreads();
-  if (!s_last) return;
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-  // Exclusive scan of count[0, n_src] by this one block, TRS_SUPER entries per sweep.  Every wave owns a
-  // contiguous run of 2 048 entries of the sweep and loads it with eight 16-byte loads per lane issued
-  // together (entry = run + (g * 64 + lane) * 4 + j: each load instruction covers 1 KiB), scans its run
-  // with shuffles alone, and the sixteen waves exchange their totals once per sweep (two barriers per
-  // 32 768 entries; a block-wide scan per slab of 4 096 entries took a barrier pair per slab and made the
-  // scan of 230 000 counters 80 us long).  (One thread per contiguous run of entries would issue 64
-  // scattered requests per instruction from a single compute unit: measured 60 us for 26 000 sources.)
-  // Entries between n_src and the end of the counter array are zero.
-  constexpr int NW = TRS_BLOCK / HC_WAVE;
-  constexpr int G = 8;
-  constexpr int64_t WAVE_SPAN = (int64_t)HC_WAVE * 4 * G;
-  constexpr int64_t TRS_SUPER = WAVE_SPAN * NW;
+  return sum;
+}
+
+__global__ __launch_bounds__(TRS_BLOCK) void tr_small_sums(const int *__restrict__ count, int *__restrict__ sums,
+                                                            TrDims dims) {
+  __shared__ int s_wave[TRS_BLOCK / HC_WAVE];
+  int64_t R, E, n_src;
+  tr_dims(dims, R, E, n_src);
+  const int64_t base = (int64_t)blockIdx.x * TRS_TILE;
+  if (base > n_src) return;
+  const int4 c = trs_counters(count, base + (int64_t)threadIdx.x * 4, n_src + 1);
+  const int sum = trs_block_sum((c.x + c.y) + (c.z + c.w), s_wave);
+  if (threadIdx.x == 0) sums[blockIdx.x] = sum;
+}
+
+// `sums` nullable: the counters in front of the tile are added up here, while other blocks write their cursors (an
+// array of its own).
+__global__ __launch_bounds__(TRS_BLOCK) void tr_small_scan(const int *__restrict__ count, const int *__restrict__ sums,
+                                                            int *__restrict__ cursor, int64_t *__restrict__ ptrT,
+                                                            TrDims dims) {
+  __shared__ int s_wave[TRS_BLOCK / HC_WAVE];
+  int64_t R, E, n_src;
+  tr_dims(dims, R, E, n_src);
+  const int64_t base = (int64_t)blockIdx.x * TRS_TILE;
+  const int64_t n_entries = n_src + 1;                      // ptrT has n_src + 1 entries
+  if (base >= n_entries) return;
   const int lane = hc_lane();
   const int wave = (int)(threadIdx.x >> 6);
-  const int64_t n_entries = n_src + 1;                      // ptrT has n_src + 1 entries
-  const int64_t padded = (n_entries + 3) / 4 * 4;           // the counter array is zero-padded to 256 bytes
-  int carry = 0;
-  int longest = 0;                                          // the lane's largest counter
-  for (int64_t base = 0; base < n_entries; base += TRS_SUPER) {
-    const int64_t run0 = base + (int64_t)wave * WAVE_SPAN;
-    int4 c[G];
-#pragma unroll
-    for (int g = 0; g < G; ++g) {
-      const int64_t i = run0 + ((int64_t)g * HC_WAVE + lane) * 4;
-      c[g] = i < padded ? *reinterpret_cast<const int4 *>(count + i) : make_int4(0, 0, 0, 0);
-      longest = max(max(longest, max(c[g].x, c[g].y)), max(c[g].z, c[g].w));
-    }
-    int pre[G];                                             // entries of the run in front of the lane's four
-    int run = 0;
-#pragma unroll
-    for (int g = 0; g < G; ++g) {
-      const int mine = (c[g].x + c[g].y) + (c[g].z + c[g].w);
-      int x = mine;                                         // inclusive scan over the wave
-#pragma unroll
-      for (int d = 1; d < HC_WAVE; d <<= 1) {
-        const int y = __shfl_up(x, d, HC_WAVE);
-        if (lane >= d) x += y;
-      }
-      pre[g] = run + x - mine;
-      run += __builtin_amdgcn_readlane(x, HC_WAVE - 1);
-    }
-    if (lane == 0) s_wave[wave] = run;
-    __syncthreads();
-    int off = carry;
-    int sweep = 0;
-    for (int w = 0; w < NW; ++w) {
-      const int t = s_wave[w];
-      if (w < wave) off += t;
-      sweep += t;
-    }
-    __syncthreads();
-    carry += sweep;
-#pragma unroll
-    for (int g = 0; g < G; ++g) {
-      const int64_t i = run0 + ((int64_t)g * HC_WAVE + lane) * 4;
-      if (i < n_entries) {
-        const int p0 = off + pre[g], p1 = p0 + c[g].x, p2 = p1 + c[g].y, p3 = p2 + c[g].z;
-        if (i + 3 < n_entries) {
-          *reinterpret_cast<int4 *>(count + i) = make_int4(p0, p1, p2, p3);   // the segments' cursors
-          ptrT[i] = p0;
-          ptrT[i + 1] = p1;
-          ptrT[i + 2] = p2;
-          ptrT[i + 3] = p3;
-        } else {
-          const int p[4] = {p0, p1, p2, p3};
-          for (int j = 0; j < 4 && i + j < n_entries; ++j) {
-            count[i + j] = p[j];
-            ptrT[i + j] = p[j];
-          }
-        }
-      }
+  const int64_t i = base + (int64_t)threadIdx.x * 4;
+  const int4 c = trs_counters(count, i, n_entries);
+  int before = 0;
+  if (sums != nullptr) {
+    for (int64_t t = threadIdx.x; t < (int64_t)blockIdx.x; t += TRS_BLOCK) before += sums[t];
+  } else {
+    for (int64_t t = 0; t < (int64_t)blockIdx.x; ++t) {
+      const int4 p = trs_counters(count, t * TRS_TILE + (int64_t)threadIdx.x * 4, n_entries);
+      before += (p.x + p.y) + (p.z + p.w);
     }
   }
+  before = trs_block_sum(before, s_wave);
+  const int mine = (c.x + c.y) + (c.z + c.w);
+  int x = mine;                                             // inclusive scan over the wave
+#pragma unroll
+  for (int d = 1; d < HC_WAVE; d <<= 1) {
+    const int y = __shfl_up(x, d, HC_WAVE);
+    if (lane >= d) x += y;
+  }
+  if (lane == HC_WAVE - 1) s_wave[wave] = x;
+  __syncthreads();
+  int p0 = before + x - mine;
+  for (int w = 0; w < wave; ++w) p0 += s_wave[w];
+  const int p[4] = {p0, p0 + c.x, p0 + c.x + c.y, p0 + c.x + c.y + c.z};
+  if (i + 3 < n_entries && reinterpret_cast<uintptr_t>(ptrT) % 16 == 0) {
+    *reinterpret_cast<int4 *>(cursor + i) = make_int4(p[0], p[1], p[2], p[3]);      // the segments' cursors
+    *reinterpret_cast<longlong2 *>(ptrT + i) = make_longlong2(p[0], p[1]);
+    *reinterpret_cast<longlong2 *>(ptrT + i + 2) = make_longlong2(p[2], p[3]);
+  } else {
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      if (i + j < n_entries) {
+        cursor[i + j] = p[j];
+        ptrT[i + j] = p[j];
+      }
+  }
   if (dims.max_count != nullptr) {                          // (kernel argument: the whole block takes the branch)
+    int longest = max(max(c.x, c.y), max(c.z, c.w));
 #pragma unroll
     for (int d = HC_WAVE / 2; d > 0; d >>= 1) longest = max(longest, __shfl_xor(longest, d, HC_WAVE));
-    if (lane == 0) s_wave[wave] = longest;                  // free since the last sweep's second barrier
+    __syncthreads();                                        // s_wave is free again
+    if (lane == 0) s_wave[wave] = longest;
     __syncthreads();
-    if (threadIdx.x == 0) {
-      int m = 0;
-      for (int w = 0; w < NW; ++w) m = max(m, s_wave[w]);
-      *dims.max_count = m;
+    if (threadIdx.x == 0) {                                 // one atomic per block: they queue at one address
+      for (int w = 1; w < TRS_BLOCK / HC_WAVE; ++w) longest = max(longest, s_wave[w]);
+      if (longest > 0) atomicMax(reinterpret_cast<unsigned long long *>(dims.max_count), (unsigned long long)longest);
     }
   }
 }
@@ -468,7 +453,12 @@ __global__ __launch_bounds__(HC_BLOCK) void tr_small_order(const int64_t *__rest
   const int wave = hc_wave_in_block();
   if (threadIdx.x == 0) n_long_s = 0;
   __syncthreads();
-  const int64_t s = (int64_t)blockIdx.x * TRS_ORDER_SOURCES + threadIdx.x;
+  // Popular sources tend to be neighbours (a sampled batch numbers them early), and a block works through its
+  // long segments one after the other: the sources are dealt to the blocks eight at a time (a line of ptrT).
+  const int64_t blocks = (n_src + TRS_ORDER_SOURCES - 1) / TRS_ORDER_SOURCES;
+  if ((int64_t)blockIdx.x >= blocks) return;
+  const auto source_of = [&](int t) -> int64_t { return ((int64_t)(t >> 3) * blocks + blockIdx.x) * 8 + (t & 7); };
+  const int64_t s = source_of((int)threadIdx.x);
   int64_t b = 0;
   int len = 0;
   if (s < n_src) {
@@ -532,7 +522,7 @@ __global__ __launch_bounds__(HC_BLOCK) void tr_small_order(const int64_t *__rest
   // plus the set bits below it in its own.
   const int n_long = n_long_s;
   for (int t = 0; t < n_long; ++t) {
-    const int64_t src = (int64_t)blockIdx.x * TRS_ORDER_SOURCES + long_src[t];
+    const int64_t src = source_of(long_src[t]);
     const int64_t sb = ptrT[src];
     const int sl = (int)(ptrT[src + 1] - sb);
     int before = 0;                                  // the segment's slots in the windows already done
@@ -593,13 +583,16 @@ __global__ __launch_bounds__(HC_BLOCK) void tr_small_order(const int64_t *__rest
 }
 
 struct SmallLayout {
-  size_t count, keys, rows, tmp_row, tmp_edge, total;
+  size_t count, cursor, sums, keys, rows, tmp_row, tmp_edge, total;
 };
 SmallLayout small_layout(int64_t E, int64_t n_src) {
   SmallLayout L;
   const size_t arr = hc_align_up((size_t)(E > 0 ? E : 1) * sizeof(uint32_t), 256);
-  L.count = sizeof(TrSmallHeader);
-  L.keys = L.count + hc_align_up((size_t)(n_src + 1) * sizeof(int), 256);
+  const size_t per_source = hc_align_up((size_t)(n_src + 1) * sizeof(int), 256);
+  L.count = 0;
+  L.cursor = per_source;
+  L.sums = 2 * per_source;
+  L.keys = L.sums + hc_align_up((size_t)(n_src / TRS_TILE + 1) * sizeof(int), 256);
   L.rows = L.keys + arr;
   L.tmp_row = L.rows + arr;
   L.tmp_edge = L.tmp_row + arr;
@@ -612,26 +605,30 @@ inline bool small_block(int64_t E, int64_t n_src) { return E <= TR_SMALL_EDGES &
 // dozen launches: 600 k edges 150 us, 66 us with the bucket sort.)
 inline bool bucket_sorted(int64_t E, int64_t n_src) { return !small_block(E, n_src) && vs_supported(E, n_src); }
 
-// The four launches of the counting sort; dims.E / dims.n_src size the grids (upper bounds when the real
+// The launches of the counting sort; dims.E / dims.n_src size the grids (upper bounds when the real
 // sizes are read on the device).
 int small_launch(const int64_t *ptr, const int64_t *idx, const int64_t *hmap_row, const int64_t *hmap_src,
                  const TrDims &dims, int64_t *ptrT, int32_t *rowT, int32_t *edgeT, char *w, const SmallLayout &S,
                  hipStream_t st) {
-  TrSmallHeader *header = reinterpret_cast<TrSmallHeader *>(w);
   int *count = reinterpret_cast<int *>(w + S.count);
+  int *cursor = reinterpret_cast<int *>(w + S.cursor);
+  int *sums = reinterpret_cast<int *>(w + S.sums);
   uint32_t *keys = reinterpret_cast<uint32_t *>(w + S.keys);
   int32_t *rows = reinterpret_cast<int32_t *>(w + S.rows);
   int32_t *tmp_row = reinterpret_cast<int32_t *>(w + S.tmp_row);
   int32_t *tmp_edge = reinterpret_cast<int32_t *>(w + S.tmp_edge);
   const int64_t E = dims.E > 0 ? dims.E : 1, n_src = dims.n_src;
-  const int64_t clear_words = (int64_t)(S.keys / sizeof(uint32_t));   // header + counters
+  const int64_t clear_words = (int64_t)(S.cursor / sizeof(uint32_t));
+  const int64_t tiles = n_src / TRS_TILE + 1;
   const int64_t cb = (clear_words + HC_BLOCK - 1) / HC_BLOCK, eb = (E + TRS_BLOCK - 1) / TRS_BLOCK;
   const int64_t pb = (E + HC_BLOCK - 1) / HC_BLOCK, ob = (n_src + TRS_ORDER_SOURCES - 1) / TRS_ORDER_SOURCES;
   if (!hc_grid_ok(cb) || !hc_grid_ok(eb) || !hc_grid_ok(pb) || !hc_grid_ok(ob)) return HC_EUNSUPPORTED;
-  tr_small_clear<<<dim3((unsigned)cb), dim3(HC_BLOCK), 0, st>>>(reinterpret_cast<uint32_t *>(w), dims);
-  tr_small_count<<<dim3((unsigned)eb), dim3(TRS_BLOCK), 0, st>>>(ptr, idx, hmap_row, hmap_src, keys, rows, count,
-                                                                 header, ptrT, dims);
-  tr_small_place<<<dim3((unsigned)pb), dim3(HC_BLOCK), 0, st>>>(keys, rows, count, tmp_row, tmp_edge, dims);
+  tr_small_clear<<<dim3((unsigned)cb), dim3(HC_BLOCK), 0, st>>>(reinterpret_cast<uint32_t *>(count), dims);
+  tr_small_count<<<dim3((unsigned)eb), dim3(TRS_BLOCK), 0, st>>>(ptr, idx, hmap_row, hmap_src, keys, rows, count, dims);
+  if (tiles > TRS_DIRECT_TILES) tr_small_sums<<<dim3((unsigned)tiles), dim3(TRS_BLOCK), 0, st>>>(count, sums, dims);
+  tr_small_scan<<<dim3((unsigned)tiles), dim3(TRS_BLOCK), 0, st>>>(count, tiles > TRS_DIRECT_TILES ? sums : nullptr, cursor,
+                                                                   ptrT, dims);
+  tr_small_place<<<dim3((unsigned)pb), dim3(HC_BLOCK), 0, st>>>(keys, rows, cursor, tmp_row, tmp_edge, dims);
   if (n_src > 0)
     tr_small_order<<<dim3((unsigned)ob), dim3(HC_BLOCK), 0, st>>>(ptrT, tmp_row, tmp_edge, rowT, edgeT, dims);
   return hc_launch_status();
