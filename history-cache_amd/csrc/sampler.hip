@@ -4,26 +4,24 @@
 // external cxgnndl loader).  Sub-graph nodes are numbered seeds first, then every hop's new nodes in
 // first-seen order; one shared CSR holds the sampled neighbours of all but the last hop's nodes.
 //
-// Per hop, for the frontier rows [lo, hi):
-//   count    c(u) = min(deg(u), fanout)
-//   scan     row offsets
+// Per hop, for the frontier rows [lo, hi), four launches:
+//   count    node map <- local ids of the frontier (the previous hop's new nodes); c(u) = min(deg(u), fanout),
+//            summed up to every row inside its tile of 1024 rows, and per tile
 //   pick     neighbour j of row u is position perm_u(j) of u's adjacency list (all of them, in
 //            list order, when deg <= fanout); its full id goes to idx, and an integer atomicMin
 //            leaves the first edge slot that mentions an unseen node in the node map
-//   flag     an edge owns its node when the map holds its own slot
-//   scan     owners before every slot -> new local ids in first-seen order
-//            (count and flag stay launches of their own: read through a functor inside the scans, their
-//            random reads of the graph and of the node map made a batch a third slower)
-//   relabel  idx <- local ids; owners append to sub_to_full
-//   commit   node map <- local ids of the new nodes; its first thread writes the next hop's state
-//            (lo, hi, edges): every hop has a state of its own, so nothing it reads changes under it
+//   flag     an edge owns its node when the map holds its own slot: one bit per slot, the owners in front of every
+//            64 slots inside their tile of 1024, and per tile
+//   relabel  idx <- local ids (a new node's: the owners in front of its own, from the bits); owners append to
+//            sub_to_full; the first thread writes the next hop's state (lo, hi, edges): every hop has a state of
+//            its own, so nothing it reads changes under it
+// The tiles' sums are added up by whoever needs the offset of a tile (hundreds of tiles: one or two loads per
+// lane); beyond SP_DIRECT_TILES of them a launch of one block scans them first.  A batch is bound by its chain of
+// small launches: with the library's scans (two launches each) and the commit of the new ids a hop took nine;
+// a batch of 1000 seeds, fanouts 15, 10, 5, with its view 283 -> 246 us.
 // perm_u is a keyed bijection of [0, deg): four Feistel rounds on the next even power of two with
 // cycle walking, so the picks of a row are distinct (sampling without replacement) at O(fanout)
 // work whatever the degree.  Everything is integer work with one well-defined result.
-#include <cstring>
-
-#include <rocprim/rocprim.hpp>
-
 #include "hc_common.h"
 
 namespace {
@@ -31,6 +29,12 @@ namespace {
 constexpr int32_t SP_UNSEEN = 0x7fffffff;
 constexpr int32_t SP_PROV = 0x40000000;  // map values at or above this are edge slots, below are ids
 constexpr int SP_GROUP = 16;             // lanes that share one row in the pick kernel
+constexpr int SP_BLOCK = HC_BLOCK;       // threads of the kernels that own a tile
+constexpr int SP_ITEMS = 4;
+// Rows or edge slots per tile.  A hop has a hundred thousand of them: with tiles of 4096 (and blocks of 1024) a few
+// tens of blocks stood in the chip, each behind its own chain of loads, and the three kernels took 86 us instead of 45.
+constexpr int SP_TILE = SP_BLOCK * SP_ITEMS;
+constexpr int64_t SP_DIRECT_TILES = 4096;
 
 struct SpState {
   int64_t lo, hi;   // frontier rows of the current hop
@@ -90,22 +94,97 @@ __global__ __launch_bounds__(HC_BLOCK) void sp_init(const int64_t *__restrict__ 
   if (s >= 0 && s < num_nodes) loc[s] = (int32_t)i;
 }
 
-__global__ __launch_bounds__(HC_BLOCK) void sp_count(const int64_t *__restrict__ indptr,
+// Sums of a hop's tiles.  `before` (nullable: few tiles) holds the exclusive scan and, behind the last tile, the
+// total.
+struct SpTiles {
+  int32_t *sum;
+  int32_t *before;
+};
+
+// Sum of the first n tiles, by a whole wave; every lane ends with it.
+__device__ __forceinline__ int32_t sp_before(const SpTiles &t, int64_t n, int lane) {
+  if (t.before != nullptr) return t.before[n];
+  int32_t v = 0;
+  for (int64_t i = lane; i < n; i += HC_WAVE) v += t.sum[i];
+#pragma unroll
+  for (int d = HC_WAVE / 2; d > 0; d >>= 1) v += __shfl_xor(v, d, HC_WAVE);
+  return v;
+}
+
+__device__ __forceinline__ int64_t sp_tiles_of(int64_t n) { return (n + SP_TILE - 1) / SP_TILE; }
+
+// Exclusive sum over the block's threads (every thread calls it once per launch); *total: the block's.
+__device__ __forceinline__ int32_t sp_block_exclusive(int32_t v, int32_t *s_wave, int32_t *total) {
+  const int lane = hc_lane(), wave = (int)(threadIdx.x >> 6);
+  int32_t x = v;
+#pragma unroll
+  for (int d = 1; d < HC_WAVE; d <<= 1) {
+    const int32_t y = __shfl_up(x, d, HC_WAVE);
+    if (lane >= d) x += y;
+  }
+  if (lane == HC_WAVE - 1) s_wave[wave] = x;
+  __syncthreads();
+  int32_t base = 0, sum = 0;
+#pragma unroll
+  for (int w = 0; w < SP_BLOCK / HC_WAVE; ++w) {
+    const int32_t t = s_wave[w];
+    if (w < wave) base += t;
+    sum += t;
+  }
+  *total = sum;
+  return base + x - v;
+}
+
+// One block: before[0 .. n] of a hop's row tiles (edges: false) or edge tiles.
+__global__ __launch_bounds__(SP_BLOCK) void sp_tile_scan(SpTiles rows, SpTiles edges, const SpState *__restrict__ st,
+                                                          int of_edges) {
+  __shared__ int32_t s_wave[SP_BLOCK / HC_WAVE];
+  const int64_t n_rows = sp_tiles_of(st->hi - st->lo);
+  const int64_t n = of_edges ? sp_tiles_of(sp_before(rows, n_rows, hc_lane())) : n_rows;
+  const SpTiles t = of_edges ? edges : rows;
+  int32_t carry = 0;
+  for (int64_t base = 0; base < n; base += SP_BLOCK) {
+    const int64_t i = base + threadIdx.x;
+    const int32_t v = i < n ? t.sum[i] : 0;
+    int32_t total;
+    const int32_t x = sp_block_exclusive(v, s_wave, &total);
+    if (i < n) t.before[i] = carry + x;
+    carry += total;
+    __syncthreads();
+  }
+  if (threadIdx.x == 0) t.before[n] = carry;
+}
+
+__global__ __launch_bounds__(SP_BLOCK) void sp_count(const int64_t *__restrict__ indptr,
                                                       const int64_t *__restrict__ sub_to_full,
                                                       const SpState *__restrict__ st, int64_t fanout,
-                                                      int64_t num_nodes, int32_t *__restrict__ cnt, int64_t cap) {
-  const int64_t i = (int64_t)blockIdx.x * HC_BLOCK + threadIdx.x;
-  if (i >= cap) return;
-  const int64_t u = st->lo + i;
-  int32_t c = 0;
-  if (u < st->hi) {
-    const int64_t full = sub_to_full[u];
-    if (full >= 0 && full < num_nodes) {
-      const int64_t d = indptr[full + 1] - indptr[full];
-      c = (int32_t)(d < fanout ? (d < 0 ? 0 : d) : fanout);
+                                                      int64_t num_nodes, int hop, int32_t *__restrict__ loc,
+                                                      int32_t *__restrict__ incl, SpTiles rows) {
+  __shared__ int32_t s_wave[SP_BLOCK / HC_WAVE];
+  const int64_t lo = st->lo, n = st->hi - lo;
+  const int64_t i0 = (int64_t)blockIdx.x * SP_TILE + (int64_t)threadIdx.x * SP_ITEMS;
+  if ((int64_t)blockIdx.x * SP_TILE >= n) return;
+  int64_t full[SP_ITEMS];
+  int32_t c[SP_ITEMS];
+#pragma unroll
+  for (int k = 0; k < SP_ITEMS; ++k) full[k] = i0 + k < n ? sub_to_full[lo + i0 + k] : -1;
+#pragma unroll
+  for (int k = 0; k < SP_ITEMS; ++k) {
+    c[k] = 0;
+    if (full[k] >= 0 && full[k] < num_nodes) {
+      const int64_t d = indptr[full[k] + 1] - indptr[full[k]];
+      c[k] = (int32_t)(d < fanout ? (d < 0 ? 0 : d) : fanout);
+      if (hop > 0) loc[full[k]] = (int32_t)(lo + i0 + k);
     }
   }
-  cnt[i] = c;
+#pragma unroll
+  for (int k = 1; k < SP_ITEMS; ++k) c[k] += c[k - 1];
+  int32_t total;
+  const int32_t before = sp_block_exclusive(c[SP_ITEMS - 1], s_wave, &total);
+#pragma unroll
+  for (int k = 0; k < SP_ITEMS; ++k)
+    if (i0 + k < n) incl[i0 + k] = before + c[k];
+  if (threadIdx.x == 0) rows.sum[blockIdx.x] = total;
 }
 
 __global__ __launch_bounds__(HC_BLOCK) void sp_pick(const int64_t *__restrict__ indptr,
@@ -113,19 +192,24 @@ __global__ __launch_bounds__(HC_BLOCK) void sp_pick(const int64_t *__restrict__ 
                                                      const int64_t *__restrict__ sub_to_full,
                                                      const SpState *__restrict__ st, int64_t fanout,
                                                      int64_t num_nodes, int hop,
-                                                     const int32_t *__restrict__ incl, int32_t *__restrict__ loc,
-                                                     int64_t *__restrict__ ptr, int64_t *__restrict__ idx,
-                                                     int64_t cap) {
+                                                     const int32_t *__restrict__ incl, SpTiles rows,
+                                                     int32_t *__restrict__ loc, int64_t *__restrict__ ptr,
+                                                     int64_t *__restrict__ idx) {
   const int64_t t = (int64_t)blockIdx.x * HC_BLOCK + threadIdx.x;
   const int64_t i = t / SP_GROUP;
   const int sub = (int)(t % SP_GROUP);
-  if (i >= cap) return;
-  const int64_t u = st->lo + i;
-  if (u >= st->hi) return;
-  const int64_t begin = i > 0 ? (int64_t)incl[i - 1] : 0;  // slot of the row's first pick inside this hop
-  const int32_t c = (int32_t)((int64_t)incl[i] - begin);
+  const int64_t lo = st->lo, n = st->hi - lo;
+  constexpr int64_t ROWS = HC_BLOCK / SP_GROUP;
+  static_assert(SP_TILE % ROWS == 0, "a block's rows lie in one tile");
+  if ((int64_t)blockIdx.x * ROWS >= n) return;
+  const int32_t tile_begin = sp_before(rows, (int64_t)blockIdx.x * ROWS / SP_TILE, hc_lane());
+  if (i >= n) return;
+  const int64_t u = lo + i;
+  const int32_t in_tile = i % SP_TILE > 0 ? incl[i - 1] : 0;
+  const int64_t begin = (int64_t)tile_begin + in_tile;     // slot of the row's first pick inside this hop
+  const int32_t c = incl[i] - in_tile;
   const int64_t base = st->edges;
-  if (sub == 0) ptr[u + 1] = base + incl[i];
+  if (sub == 0) ptr[u + 1] = base + begin + c;
   if (c == 0) return;
   const int64_t full = sub_to_full[u];
   const int64_t first = indptr[full];
@@ -139,70 +223,116 @@ __global__ __launch_bounds__(HC_BLOCK) void sp_pick(const int64_t *__restrict__ 
   }
 }
 
-__global__ __launch_bounds__(HC_BLOCK) void sp_flag(const int64_t *__restrict__ idx,
-                                                     const int32_t *__restrict__ loc,
-                                                     const SpState *__restrict__ st,
-                                                     const int32_t *__restrict__ incl, int64_t cap,
-                                                     int64_t num_nodes, int32_t *__restrict__ flag,
-                                                     int64_t edge_cap) {
-  const int64_t p = (int64_t)blockIdx.x * HC_BLOCK + threadIdx.x;
-  if (p >= edge_cap) return;
-  const int64_t hop_edges = incl[cap - 1];
-  int32_t f = 0;
-  if (p < hop_edges) {
-    const int64_t v = idx[st->edges + p];
-    f = (v >= 0 && v < num_nodes && loc[v] == SP_PROV + (int32_t)p) ? 1 : 0;
-  }
-  flag[p] = f;
-}
+// The owners among a hop's edge slots: bit p % 64 of bits[p / 64], and word_before[p / 64], the owners in front of
+// those 64 slots inside their tile.
+struct SpOwners {
+  unsigned long long *bits;
+  int32_t *word_before;
+  SpTiles tiles;
+};
 
-__global__ __launch_bounds__(HC_BLOCK) void sp_relabel(int64_t *__restrict__ idx,
-                                                        const int32_t *__restrict__ loc,
-                                                        const SpState *__restrict__ st,
-                                                        const int32_t *__restrict__ incl, int64_t cap,
-                                                        int64_t num_nodes, const int32_t *__restrict__ rank_incl,
-                                                        int64_t *__restrict__ sub_to_full, int64_t edge_cap) {
-  const int64_t p = (int64_t)blockIdx.x * HC_BLOCK + threadIdx.x;
-  if (p >= edge_cap) return;
-  const int64_t hop_edges = incl[cap - 1];
-  if (p >= hop_edges) return;
-  const int64_t e = st->edges + p;
-  const int64_t v = idx[e];
-  int64_t id = -1;
-  if (v >= 0 && v < num_nodes) {
-    const int32_t t = loc[v];
-    if (t >= SP_PROV) {
-      const int32_t q = t - SP_PROV;  // the owning edge slot of this hop
-      id = st->hi + rank_incl[q] - 1;
-      if (q == (int32_t)p) sub_to_full[id] = v;
-    } else {
-      id = t;
+__global__ __launch_bounds__(SP_BLOCK) void sp_flag(const int64_t *__restrict__ idx, const int32_t *__restrict__ loc,
+                                                     const SpState *__restrict__ st, SpTiles rows, int64_t num_nodes,
+                                                     SpOwners own) {
+  __shared__ int32_t s_wave[SP_BLOCK / HC_WAVE];
+  const int lane = hc_lane(), wave = (int)(threadIdx.x >> 6);
+  const int64_t hop_edges = sp_before(rows, sp_tiles_of(st->hi - st->lo), lane);
+  const int64_t tile0 = (int64_t)blockIdx.x * SP_TILE;
+  if (tile0 >= hop_edges) return;
+  const int64_t base = st->edges;
+  const int64_t w0 = tile0 + (int64_t)wave * SP_ITEMS * HC_WAVE;       // the wave's SP_ITEMS words
+  int64_t v[SP_ITEMS];
+#pragma unroll
+  for (int k = 0; k < SP_ITEMS; ++k) {
+    const int64_t p = w0 + k * HC_WAVE + lane;
+    v[k] = p < hop_edges ? idx[base + p] : -1;
+  }
+  unsigned long long b[SP_ITEMS];
+  int32_t mine = 0;
+#pragma unroll
+  for (int k = 0; k < SP_ITEMS; ++k) {
+    const int64_t p = w0 + k * HC_WAVE + lane;
+    b[k] = __ballot(v[k] >= 0 && v[k] < num_nodes && loc[v[k]] == SP_PROV + (int32_t)p);
+    mine += (int32_t)__popcll(b[k]);
+  }
+  if (lane == 0) s_wave[wave] = mine;
+  __syncthreads();
+  int32_t before = 0, total = 0;
+#pragma unroll
+  for (int w = 0; w < SP_BLOCK / HC_WAVE; ++w) {
+    const int32_t t = s_wave[w];
+    if (w < wave) before += t;
+    total += t;
+  }
+  if (lane == 0) {
+#pragma unroll
+    for (int k = 0; k < SP_ITEMS; ++k) {
+      own.bits[w0 / HC_WAVE + k] = b[k];
+      own.word_before[w0 / HC_WAVE + k] = before;
+      before += (int32_t)__popcll(b[k]);
     }
   }
-  idx[e] = id;
+  if (threadIdx.x == 0) own.tiles.sum[blockIdx.x] = total;
 }
 
-__global__ __launch_bounds__(HC_BLOCK) void sp_commit(const int64_t *__restrict__ sub_to_full,
-                                                       const SpState *__restrict__ st, SpState *__restrict__ next,
-                                                       const int32_t *__restrict__ incl, int64_t cap,
-                                                       const int32_t *__restrict__ rank_incl,
-                                                       int32_t *__restrict__ loc, int64_t *__restrict__ counts,
-                                                       int hop, int num_hops, int64_t edge_cap) {
-  const int64_t i = (int64_t)blockIdx.x * HC_BLOCK + threadIdx.x;
-  if (i >= edge_cap) return;
-  const int64_t hop_edges = incl[cap - 1];
-  const int64_t fresh = hop_edges > 0 ? rank_incl[hop_edges - 1] : 0;
-  if (i == 0) {  // the next hop's state (this hop's is read by the other threads and stays as it is)
-    next->lo = st->hi;
-    next->hi = st->hi + fresh;
-    next->edges = st->edges + hop_edges;
-    next->key = st->key;
-    counts[hop + 1] = st->hi + fresh;
-    counts[num_hops + 1 + hop] = st->edges + hop_edges;
+__global__ __launch_bounds__(SP_BLOCK) void sp_relabel(int64_t *__restrict__ idx, const int32_t *__restrict__ loc,
+                                                        const SpState *__restrict__ st, SpState *__restrict__ next,
+                                                        SpTiles rows, int64_t num_nodes, SpOwners own,
+                                                        int64_t *__restrict__ sub_to_full,
+                                                        int64_t *__restrict__ counts, int hop, int num_hops) {
+  __shared__ int32_t s_tile[SP_DIRECT_TILES + 1];
+  __shared__ int32_t s_wave[SP_BLOCK / HC_WAVE];
+  const int lane = hc_lane();
+  const int64_t hop_edges = sp_before(rows, sp_tiles_of(st->hi - st->lo), lane);
+  const int64_t tile0 = (int64_t)blockIdx.x * SP_TILE;
+  if (tile0 >= hop_edges && blockIdx.x > 0) return;
+  const int64_t n_tiles = sp_tiles_of(hop_edges);
+  const int32_t *tile_before = own.tiles.before;
+  if (tile_before == nullptr) {                            // every block scans the tiles' sums: at most 4096 of them
+    const int per = (int)((n_tiles + SP_BLOCK - 1) / SP_BLOCK), t0 = (int)threadIdx.x * per;
+    int32_t sum = 0, total;
+    for (int t = t0; t < t0 + per && t < n_tiles; ++t) sum += own.tiles.sum[t];
+    int32_t run = sp_block_exclusive(sum, s_wave, &total);
+    for (int t = t0; t < t0 + per && t < n_tiles; ++t) {
+      s_tile[t] = run;
+      run += own.tiles.sum[t];
+    }
+    if (threadIdx.x == 0) s_tile[SP_DIRECT_TILES] = total;
+    __syncthreads();
+    tile_before = s_tile;
   }
-  if (i >= fresh) return;
-  const int64_t id = st->hi + i;
-  loc[sub_to_full[id]] = (int32_t)id;
+  const int64_t hi = st->hi, base = st->edges;
+  if (blockIdx.x == 0 && threadIdx.x == 0) {  // the next hop's state (this hop's is read by the other threads and stays as it is)
+    const int64_t fresh = own.tiles.before != nullptr ? tile_before[n_tiles] : s_tile[SP_DIRECT_TILES];
+    next->lo = hi;
+    next->hi = hi + fresh;
+    next->edges = base + hop_edges;
+    next->key = st->key;
+    counts[hop + 1] = hi + fresh;
+    counts[num_hops + 1 + hop] = base + hop_edges;
+  }
+  int64_t v[SP_ITEMS];
+  int32_t t[SP_ITEMS];
+#pragma unroll
+  for (int k = 0; k < SP_ITEMS; ++k) {
+    const int64_t p = tile0 + k * SP_BLOCK + threadIdx.x;
+    v[k] = p < hop_edges ? idx[base + p] : -1;
+  }
+#pragma unroll
+  for (int k = 0; k < SP_ITEMS; ++k) t[k] = v[k] >= 0 && v[k] < num_nodes ? loc[v[k]] : -1;
+#pragma unroll
+  for (int k = 0; k < SP_ITEMS; ++k) {
+    const int64_t p = tile0 + k * SP_BLOCK + threadIdx.x;
+    if (p >= hop_edges) continue;
+    int64_t id = t[k];                            // -1: not a node of the graph
+    if (t[k] >= SP_PROV) {
+      const int32_t q = t[k] - SP_PROV;           // the owning edge slot of this hop
+      const unsigned long long below = own.bits[q / HC_WAVE] & ((1ull << (q % HC_WAVE)) - 1ull);
+      id = hi + tile_before[q / SP_TILE] + own.word_before[q / HC_WAVE] + (int32_t)__popcll(below);
+      if (q == (int32_t)p) sub_to_full[id] = v[k];
+    }
+    idx[base + p] = id;
+  }
 }
 
 __global__ __launch_bounds__(HC_BLOCK) void sp_reset(const int64_t *__restrict__ sub_to_full,
@@ -252,35 +382,28 @@ SpCaps sp_caps(int64_t n_seed, const int64_t *fanout, int num_hops, int64_t num_
   return c;
 }
 
-size_t sp_scan_bytes(int64_t n) {
-  size_t bytes = 0;
-  int32_t *none = nullptr;
-  if (rocprim::inclusive_scan(nullptr, bytes, none, none, (size_t)(n > 0 ? n : 1), rocprim::plus<int32_t>()) !=
-      hipSuccess)
-    return 0;
-  return bytes;
-}
-
 struct SpLayout {
-  size_t state, cnt, incl, flag, rank, scan, total;
+  size_t state, incl, row_sum, row_before, bits, word_before, edge_sum, edge_before, total;
 };
+
+inline int64_t sp_tiles(int64_t n) { return (n + SP_TILE - 1) / SP_TILE; }
 
 SpLayout sp_layout(const SpCaps &c) {
   SpLayout l{};
   size_t off = 0;
-  l.state = off;                                   // one state per hop and the final one
-  off += hc_align_up(sizeof(SpState) * (HC_SAMPLE_MAX_HOPS + 1), 256);
-  l.cnt = off;
-  off += hc_align_up((size_t)(c.max_rows + 1) * 4, 256);
-  l.incl = off;
-  off += hc_align_up((size_t)(c.max_rows + 1) * 4, 256);
-  l.flag = off;
-  off += hc_align_up((size_t)(c.max_edges + 1) * 4, 256);
-  l.rank = off;
-  off += hc_align_up((size_t)(c.max_edges + 1) * 4, 256);
-  l.scan = off;
-  size_t a = sp_scan_bytes(c.max_rows), b = sp_scan_bytes(c.max_edges);
-  off += hc_align_up(a > b ? a : b, 256) + 256;
+  const auto take = [&off](size_t bytes) {
+    const size_t here = off;
+    off += hc_align_up(bytes, 256);
+    return here;
+  };
+  l.state = take(sizeof(SpState) * (HC_SAMPLE_MAX_HOPS + 1));      // one state per hop and the final one
+  l.incl = take((size_t)(c.max_rows + 1) * 4);
+  l.row_sum = take((size_t)(sp_tiles(c.max_rows) + 1) * 4);
+  l.row_before = take((size_t)(sp_tiles(c.max_rows) + 1) * 4);
+  l.bits = take((size_t)sp_tiles(c.max_edges) * (SP_TILE / HC_WAVE) * 8);
+  l.word_before = take((size_t)sp_tiles(c.max_edges) * (SP_TILE / HC_WAVE) * 4);
+  l.edge_sum = take((size_t)(sp_tiles(c.max_edges) + 1) * 4);
+  l.edge_before = take((size_t)(sp_tiles(c.max_edges) + 1) * 4);
   l.total = off;
   return l;
 }
@@ -335,33 +458,29 @@ int sample_layers_impl(const int64_t *indptr, const int64_t *indices, int64_t nu
   hipStream_t s = static_cast<hipStream_t>(stream);
   char *w = static_cast<char *>(workspace);
   SpState *states = reinterpret_cast<SpState *>(w + l.state);
-  int32_t *cnt = reinterpret_cast<int32_t *>(w + l.cnt);
   int32_t *incl = reinterpret_cast<int32_t *>(w + l.incl);
-  int32_t *flag = reinterpret_cast<int32_t *>(w + l.flag);
-  int32_t *rank = reinterpret_cast<int32_t *>(w + l.rank);
-  void *scan_ws = w + l.scan;
-  const dim3 bl(HC_BLOCK);
+  const dim3 bl(HC_BLOCK), tl(SP_BLOCK);
 
   sp_init<<<dim3(sp_blocks(n_seed)), bl, 0, s>>>(seeds, n_seed, num_nodes, node_map, sub_to_full, ptr, counts, states,
                                                  rng_seed, rng_seed_at);
   for (int k = 0; k < num_hops; ++k) {
     const int64_t cap = c.rows[k], ecap = c.edges[k];
+    const int64_t row_tiles = sp_tiles(cap), edge_tiles = sp_tiles(ecap);
     const SpState *st = states + k;
-    sp_count<<<dim3(sp_blocks(cap)), bl, 0, s>>>(indptr, sub_to_full, st, fanout[k], num_nodes, cnt, cap);
-    size_t bytes = sp_scan_bytes(cap);
-    if (rocprim::inclusive_scan(scan_ws, bytes, cnt, incl, (size_t)cap, rocprim::plus<int32_t>(), s) != hipSuccess)
-      return HC_ELAUNCH;
+    SpTiles rows{reinterpret_cast<int32_t *>(w + l.row_sum), reinterpret_cast<int32_t *>(w + l.row_before)};
+    SpOwners own{reinterpret_cast<unsigned long long *>(w + l.bits), reinterpret_cast<int32_t *>(w + l.word_before),
+                 {reinterpret_cast<int32_t *>(w + l.edge_sum), reinterpret_cast<int32_t *>(w + l.edge_before)}};
+    if (row_tiles <= SP_DIRECT_TILES) rows.before = nullptr;
+    if (edge_tiles <= SP_DIRECT_TILES) own.tiles.before = nullptr;
+    sp_count<<<dim3((unsigned)row_tiles), tl, 0, s>>>(indptr, sub_to_full, st, fanout[k], num_nodes, k, node_map, incl,
+                                                      rows);
+    if (rows.before != nullptr) sp_tile_scan<<<dim3(1), tl, 0, s>>>(rows, own.tiles, st, 0);
     sp_pick<<<dim3(sp_blocks(cap * SP_GROUP)), bl, 0, s>>>(indptr, indices, sub_to_full, st, fanout[k], num_nodes,
-                                                          k, incl, node_map, ptr, idx, cap);
-    sp_flag<<<dim3(sp_blocks(ecap)), bl, 0, s>>>(idx, node_map, st, incl, cap, num_nodes, flag, ecap);
-    bytes = sp_scan_bytes(ecap);
-    if (rocprim::inclusive_scan(scan_ws, bytes, flag, rank, (size_t)ecap, rocprim::plus<int32_t>(), s) !=
-        hipSuccess)
-      return HC_ELAUNCH;
-    sp_relabel<<<dim3(sp_blocks(ecap)), bl, 0, s>>>(idx, node_map, st, incl, cap, num_nodes, rank, sub_to_full,
-                                                   ecap);
-    sp_commit<<<dim3(sp_blocks(ecap)), bl, 0, s>>>(sub_to_full, st, states + k + 1, incl, cap, rank, node_map,
-                                                  counts, k, num_hops, ecap);
+                                                          k, incl, rows, node_map, ptr, idx);
+    sp_flag<<<dim3((unsigned)edge_tiles), tl, 0, s>>>(idx, node_map, st, rows, num_nodes, own);
+    if (own.tiles.before != nullptr) sp_tile_scan<<<dim3(1), tl, 0, s>>>(rows, own.tiles, st, 1);
+    sp_relabel<<<dim3((unsigned)edge_tiles), tl, 0, s>>>(idx, node_map, st, states + k + 1, rows, num_nodes, own,
+                                                        sub_to_full, counts, k, num_hops);
     if (hc_launch_status() != HC_OK) return HC_ELAUNCH;
   }
   const SpState *st = states + num_hops;
