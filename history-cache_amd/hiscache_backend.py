@@ -186,14 +186,14 @@ def _raw_stream(device_index=None):
     return int(torch.cuda.current_stream(device_index).cuda_stream)
 
 
+# (pointer arguments are handed over as integers: the signatures' c_void_p takes them, and building an object for
+# each costs a call with twenty of them three microseconds)
 def _stream():
-    return _c_p(_raw_stream())
+    return _raw_stream()
 
 
 def _ptr(t):
-    if t is None:
-        return _c_p(None)
-    return _c_p(t.data_ptr())
+    return None if t is None else t.data_ptr()
 
 
 def _dev(t, name, dtype=None):
