@@ -119,6 +119,22 @@ __device__ __forceinline__ int64_t fwd_row_address(const FwdArgs &a, int64_t id)
   return addr;
 }
 
+// A neighbour row that lies in the features or, in another element type, in the history table: both are loaded, the
+// one that the row does not lie in through a descriptor of no bytes, which answers with zeros and asks the memory
+// nothing.  (With a branch between the two loads the compiler waits for every row before the next one's load: 14 000
+// edges of a half-precision table took 0.18 us each.)
+template <typename T, typename TH>
+struct FwdEither {
+  hc_buffer features, table;
+  bool from_table;
+  __device__ __forceinline__ FwdEither(int64_t address, int64_t F) {
+    from_table = (address & 1) != 0;
+    const void *row = reinterpret_cast<const void *>(address & ~(int64_t)1);
+    features = hc_make_buffer(row, from_table ? 0u : (uint32_t)F * (uint32_t)sizeof(T));
+    table = hc_make_buffer(row, from_table ? (uint32_t)F * (uint32_t)sizeof(TH) : 0u);
+  }
+};
+
 // Columns of a lane: chunk k holds elements off[k] .. off[k] + VEC - 1; lanes behind the row's end read
 // the last slot again (no extra line) and store nothing.
 template <int VEC, int CHUNKS>
@@ -235,7 +251,11 @@ __device__ __forceinline__ void fwd_slice_sum(const FwdArgs &a, uint32_t c, int6
     if constexpr (BUF) return (int64_t)((uint32_t)id * row_bytes);
     else return fwd_row_address<T, TH, SRC>(a, id);
   };
-  const auto load = [&](raw_t (&x)[D], float (&w)[D], int64_t addr, int64_t base, int g, int last) {
+  // MIXED: the table's share of a row (see FwdEither), and the stage's edges that read the table
+  uint16_t yb[2][MIXED ? D : 1];
+  unsigned long long tables = 0ull, next_tables = 0ull;
+  const auto load = [&](raw_t (&x)[D], float (&w)[D], uint16_t (&y)[MIXED ? D : 1], int64_t addr, int64_t base, int g,
+                        int last) {
     uint32_t off[D];
     if constexpr (BUF) {
 #pragma unroll
@@ -254,8 +274,9 @@ __device__ __forceinline__ void fwd_slice_sum(const FwdArgs &a, uint32_t c, int6
         const int64_t p = hc_readlane64(addr, j);
         if constexpr (MIXED) {
           static_assert(!MIXED || SV == 1, "a table of another element type beside fp32 rows");
-          if ((p & 1) != 0) w[u] = hc_piece<TH, 1>::widen(hc_piece<TH, 1>::template load<true>(p - 1, c * (uint32_t)sizeof(TH)), 0);
-          else w[u] = hc_piece<T, 1>::widen(hc_piece<T, 1>::template load<true>(p, c * (uint32_t)sizeof(T)), 0);
+          const FwdEither<T, TH> row(p, a.F);
+          x[u] = hc_buffer_load_nt<raw_t>(row.features, c * (uint32_t)sizeof(T));
+          y[u] = hc_buffer_load_nt<uint16_t>(row.table, c * (uint32_t)sizeof(TH));
         } else {
           x[u] = hc_piece<T, SV>::template load<SRC>(p, c * (uint32_t)sizeof(T));
         }
@@ -263,11 +284,12 @@ __device__ __forceinline__ void fwd_slice_sum(const FwdArgs &a, uint32_t c, int6
       if constexpr (WMODE == W_EDGE_HEAD) w[u] = ev[(base + j) * a.n_head + hd];
     }
   };
-  const auto add1 = [&](const raw_t &x, float w, float my_w, int j) {
+  const auto add1 = [&](const raw_t &x, float w, uint16_t y, float my_w, int j) {
     const float w1 = WMODE == W_EDGE ? hc_readlane_f(my_w, j) : w;
 #pragma unroll
     for (int i = 0; i < SV; ++i) {
-      if constexpr (MIXED) acc[i] += w;
+      if constexpr (MIXED)
+        acc[i] += ((tables >> j) & 1ull) != 0ull ? hc_piece<TH, 1>::widen(y, 0) : hc_piece<T, SV>::widen(x, i);
       else if constexpr (WMODE == W_NONE) acc[i] += hc_piece<T, SV>::widen(x, i);
       else acc[i] = __fmaf_rn(hc_piece<T, SV>::widen(x, i), w1, acc[i]);
     }
@@ -276,9 +298,10 @@ __device__ __forceinline__ void fwd_slice_sum(const FwdArgs &a, uint32_t c, int6
   float w[2][D];
   int64_t e = begin + lane < end ? begin + lane : end - 1;
   int64_t addr = address(a.idx[e]);
+  if constexpr (MIXED) tables = __ballot((addr & 1) != 0);
   float my_w = WMODE == W_EDGE ? ev[e * ev_stride] : 0.0f;
   int last = end - begin < HC_WAVE ? (int)(end - begin) - 1 : HC_WAVE - 1;
-  load(x[0], w[0], addr, begin, 0, last);
+  load(x[0], w[0], yb[0], addr, begin, 0, last);
   int64_t base = begin;
   for (; base + HC_WAVE <= end; base += HC_WAVE) {
     const int64_t next = base + HC_WAVE;
@@ -289,27 +312,29 @@ __device__ __forceinline__ void fwd_slice_sum(const FwdArgs &a, uint32_t c, int6
 #pragma unroll
     for (int g = 0; g < G; ++g) {
       if (g + 1 < G) {
-        load(x[(g + 1) & 1], w[(g + 1) & 1], addr, base, g + 1, HC_WAVE - 1);
+        load(x[(g + 1) & 1], w[(g + 1) & 1], yb[(g + 1) & 1], addr, base, g + 1, HC_WAVE - 1);
       } else {
         addr = address(next_id);
+        if constexpr (MIXED) next_tables = __ballot((addr & 1) != 0);
         last = end - next < HC_WAVE ? (int)(end - next) - 1 : HC_WAVE - 1;
         last = last < 0 ? 0 : last;
-        load(x[0], w[0], addr, next < end ? next : end - 1, 0, last);
+        load(x[0], w[0], yb[0], addr, next < end ? next : end - 1, 0, last);
       }
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int u = 0; u < D; ++u) add1(x[g & 1][u], w[g & 1][u], my_w, g * D + u);
+      for (int u = 0; u < D; ++u) add1(x[g & 1][u], w[g & 1][u], yb[g & 1][MIXED ? u : 0], my_w, g * D + u);
       __builtin_amdgcn_sched_barrier(0);
     }
     my_w = next_w;
+    if constexpr (MIXED) tables = next_tables;
   }
   // the last, partial stage: its first group is on its way
   const int n = (int)(end - base);
   for (int g = 0; g * D < n; ++g) {
-    if (g > 0) load(x[0], w[0], addr, base, g, n - 1);
+    if (g > 0) load(x[0], w[0], yb[0], addr, base, g, n - 1);
 #pragma unroll
     for (int u = 0; u < D; ++u)
-      if (g * D + u < n) add1(x[0][u], w[0][u], my_w, g * D + u);
+      if (g * D + u < n) add1(x[0][u], w[0][u], yb[0][MIXED ? u : 0], my_w, g * D + u);
   }
 }
 
@@ -514,7 +539,11 @@ __device__ __forceinline__ void fwd_front(const FwdArgs &a, int64_t far_above, i
   }
 }
 
-template <typename T, typename TH, int VEC, int CHUNKS, int UNROLL, bool SRC, int WMODE>
+// PART: the front blocks and the rows' in one launch, or one of the two.  A table of another element type beside the
+// features takes two launches: the slices' code needs 170 registers there, which would leave the rows three waves per
+// SIMD (11 M edges x 128 in one launch 2.55 ms, in two 1.96 ms).
+constexpr int FWD_ALL = 0, FWD_FRONT = 1, FWD_BODY = 2;
+template <typename T, typename TH, int VEC, int CHUNKS, int UNROLL, bool SRC, int WMODE, int PART>
 __global__ __launch_bounds__(HC_BLOCK) void fwd_rows(FwdArgs a) {
   // without heads the rows may be split: the split code is compiled for those modes only
   constexpr int LMODE = WMODE == W_EDGE_HEAD ? W_EDGE : WMODE;
@@ -535,14 +564,18 @@ __global__ __launch_bounds__(HC_BLOCK) void fwd_rows(FwdArgs a) {
                (a.split_above == 0 || total / (a.slice_above + 1) <= a.near.cap);
     else
       listed = total / (far_above + 1) <= FWD_SELF_ITEMS && far_above == a.slice_above;
-    if ((int)blockIdx.x < a.front) {
-      if (listed)
-        fwd_front<T, TH, VEC, CHUNKS, UNROLL, SRC, WMODE>(a, far_above, lane, wave, part, self_rows, long_rows);
-      return;
+    if constexpr (PART != FWD_BODY) {
+      if ((int)blockIdx.x < a.front) {
+        if (listed)
+          fwd_front<T, TH, VEC, CHUNKS, UNROLL, SRC, WMODE>(a, far_above, lane, wave, part, self_rows, long_rows);
+        return;
+      }
     }
   }
-  const int64_t row0 = hc_xcd_block<FWD_XCD_CHUNK>((int64_t)blockIdx.x - a.front,
-                                                   (int64_t)gridDim.x - a.front) * FWD_ROWS_PER_BLOCK;
+  if constexpr (PART == FWD_FRONT) return;
+  const int ahead = PART == FWD_BODY ? 0 : a.front;
+  const int64_t row0 = hc_xcd_block<FWD_XCD_CHUNK>((int64_t)blockIdx.x - ahead, (int64_t)gridDim.x - ahead) *
+                       FWD_ROWS_PER_BLOCK;
   const int64_t rest = a.R - row0;
   const int nrows = rest < FWD_ROWS_PER_BLOCK ? (int)rest : FWD_ROWS_PER_BLOCK;
   const bool in_block = a.split_above > 0 && !listed;      // the block sums its own long rows afterwards
@@ -617,21 +650,29 @@ template <typename T, int VEC, int CHUNKS>
 int launch_rows(const FwdArgs &a, bool src_mode, hipStream_t st) {
   constexpr int per = VEC * CHUNKS;
   constexpr int UNROLL = per >= 16 ? 4 : (per >= 4 ? 8 : 16);
-  const int64_t blocks = (a.R + FWD_ROWS_PER_BLOCK - 1) / FWD_ROWS_PER_BLOCK + a.front;
+  const int64_t row_blocks = (a.R + FWD_ROWS_PER_BLOCK - 1) / FWD_ROWS_PER_BLOCK;
+  const int64_t blocks = row_blocks + a.front;
   if (!hc_grid_ok(blocks)) return HC_EUNSUPPORTED;
   const dim3 grid((unsigned)blocks), block(HC_BLOCK);
-#define HC_FWD_LAUNCH(TH, SRC, WMODE) fwd_rows<T, TH, VEC, CHUNKS, UNROLL, SRC, WMODE><<<grid, block, 0, st>>>(a)
+#define HC_FWD_LAUNCH(TH, SRC, WMODE) fwd_rows<T, TH, VEC, CHUNKS, UNROLL, SRC, WMODE, FWD_ALL><<<grid, block, 0, st>>>(a)
+#define HC_FWD_LAUNCH_TWO(TH)                                                                                           \
+  {                                                                                                                     \
+    if (a.front > 0)                                                                                                    \
+      fwd_rows<T, TH, VEC, CHUNKS, UNROLL, true, W_NONE, FWD_FRONT><<<dim3((unsigned)a.front), block, 0, st>>>(a);      \
+    fwd_rows<T, TH, VEC, CHUNKS, UNROLL, true, W_NONE, FWD_BODY><<<dim3((unsigned)row_blocks), block, 0, st>>>(a);      \
+  }
   if (a.ev != nullptr && a.n_head > 1) HC_FWD_LAUNCH(T, false, W_EDGE_HEAD);
   else if (a.ev != nullptr) HC_FWD_LAUNCH(T, false, W_EDGE);
   else if (src_mode && a.hmap != nullptr) {
     // the table of a per-source substitution may be narrower than fp32 features
     if constexpr (std::is_same<T, float>::value) {
-      if (a.hist_dtype == HC_F16) HC_FWD_LAUNCH(__half, true, W_NONE);
-      else if (a.hist_dtype == HC_BF16) HC_FWD_LAUNCH(__hip_bfloat16, true, W_NONE);
+      if (a.hist_dtype == HC_F16) HC_FWD_LAUNCH_TWO(__half)
+      else if (a.hist_dtype == HC_BF16) HC_FWD_LAUNCH_TWO(__hip_bfloat16)
       else HC_FWD_LAUNCH(T, true, W_NONE);
     } else HC_FWD_LAUNCH(T, true, W_NONE);
   } else HC_FWD_LAUNCH(T, false, W_NONE);
 #undef HC_FWD_LAUNCH
+#undef HC_FWD_LAUNCH_TWO
   return hc_launch_status();
 }
 

@@ -235,13 +235,23 @@ struct hc_piece {
 // load takes the row's offset from a scalar register and the lane's from a vector register, which leaves one
 // v_readlane per row as address arithmetic.
 typedef __amdgpu_buffer_rsrc_t hc_buffer;
-__device__ __forceinline__ hc_buffer hc_make_buffer(const void *base) {
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(base), 0, 0xffffffffu, 0x00027000);
+__device__ __forceinline__ hc_buffer hc_make_buffer(const void *base, uint32_t bytes = 0xffffffffu) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(base), 0, bytes, 0x00027000);
 }
 template <typename RAW>
 __device__ __forceinline__ RAW hc_buffer_load(hc_buffer b, uint32_t lane_byte, uint32_t row_byte) {
   if constexpr (sizeof(RAW) == 2) return __builtin_amdgcn_raw_buffer_load_b16(b, lane_byte, row_byte, 0);
   else return __builtin_amdgcn_raw_buffer_load_b32(b, lane_byte, row_byte, 0);
+}
+
+// A piece of a row that has a descriptor of its own, with the non-temporal hint; behind its end: zeros.
+template <typename RAW>
+__device__ __forceinline__ RAW hc_buffer_load_nt(hc_buffer b, uint32_t lane_byte) {
+  constexpr int NT = 2;
+  if constexpr (sizeof(RAW) == 2) return __builtin_bit_cast(RAW, __builtin_amdgcn_raw_buffer_load_b16(b, lane_byte, 0, NT));
+  else if constexpr (sizeof(RAW) == 4) return __builtin_bit_cast(RAW, __builtin_amdgcn_raw_buffer_load_b32(b, lane_byte, 0, NT));
+  else if constexpr (sizeof(RAW) == 8) return __builtin_bit_cast(RAW, __builtin_amdgcn_raw_buffer_load_b64(b, lane_byte, 0, NT));
+  else return __builtin_bit_cast(RAW, __builtin_amdgcn_raw_buffer_load_b128(b, lane_byte, 0, NT));
 }
 
 // Store VEC consecutive fp32 values (VEC may exceed one 16-byte store).
