@@ -17,19 +17,13 @@
 // A bias added in front of the normalisation cancels in y; it only shifts the mean that the running
 // statistics see, and its gradient is zero.  Nothing here depends on scheduling: slabs are fixed by
 // (n, C) and added in a fixed order.  The reducing kernels run 1024-thread blocks over at most 128
-// slabs (256 and a second launch for large matrices): the block that adds the slabs reads all partial sums
-// through one compute unit, so their number is kept small and the sixteen waves split them.
+// slabs: the block that adds the slabs reads all partial sums through one compute unit, so their
+// number is kept small and the sixteen waves split them.
 #include "hc_common.h"
 
 namespace {
 
 constexpr int BN_MAX_SLABS = 128;
-// From this many rows on the matrix is cut into twice as many slabs, one per compute unit, and their sums are added
-// by a launch of their own, a block per 64 columns: the block that arrives last reads them through one compute unit
-// (two layers of a 100 000-row batch, 256 channels: statistics 43 -> 30 us, sums of the backward 60 -> 44 us).  Below, the extra launch costs more than it saves.
-constexpr int64_t BN_LARGE_ROWS = 16384;
-constexpr int BN_LARGE_SLABS = 256;
-constexpr int BN_FINAL_GROUPS = 16;   // float4 groups per block of the adding launch
 constexpr int BN_MAX_C = 1024;
 constexpr int BN_BLOCK = 1024;   // threads per block of the two reducing kernels
 constexpr int BN_FLIGHT = 8;     // rows a thread has in flight
@@ -46,8 +40,7 @@ static bool bn_shape(int64_t n, int64_t C, BnShape *s) {
   s->groups = (int)(C / 4);
   s->rows_per_pass = BN_BLOCK / s->groups;
   const int64_t p = s->rows_per_pass;
-  const int64_t most = n >= BN_LARGE_ROWS ? BN_LARGE_SLABS : BN_MAX_SLABS;
-  int64_t rows = (n + most - 1) / most;
+  int64_t rows = (n + BN_MAX_SLABS - 1) / BN_MAX_SLABS;
   if (rows < 2 * p) rows = 2 * p;
   rows = (rows + p - 1) / p * p;
   s->slab_rows = rows;
@@ -92,10 +85,10 @@ __device__ __forceinline__ bool bn_last_block(unsigned *ticket, int *s_flag) {
   return true;
 }
 
-// Sum over the slabs of the two partial sums of column group g0 + g, by one block with G groups:
+// Sum over the slabs of the two partial sums of column group g, by the block that arrived last:
 // part[slab][2][C].  Thread (g, p) adds slabs p, p + P, ... in that order, thread (g, 0) then adds the
 // P results in order of p.  Ends with the totals in the threads with p == 0.
-__device__ __forceinline__ void bn_sum_slabs(const float *__restrict__ part, int64_t slabs, int C, int g0, int G, int P,
+__device__ __forceinline__ void bn_sum_slabs(const float *__restrict__ part, int64_t slabs, int C, int G, int P,
                                              int g, int p, float4 (*s_red)[BN_BLOCK], float4 &t1, float4 &t2) {
   t1 = make_float4(0.f, 0.f, 0.f, 0.f);
   t2 = t1;
@@ -106,8 +99,8 @@ __device__ __forceinline__ void bn_sum_slabs(const float *__restrict__ part, int
       float4 a[4], b[4];
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
-        a[j] = bn_ld4(part + (k + (int64_t)j * P) * 2 * C + 4 * (g0 + g));
-        b[j] = bn_ld4(part + (k + (int64_t)j * P) * 2 * C + C + 4 * (g0 + g));
+        a[j] = bn_ld4(part + (k + (int64_t)j * P) * 2 * C + 4 * g);
+        b[j] = bn_ld4(part + (k + (int64_t)j * P) * 2 * C + C + 4 * g);
       }
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
@@ -116,8 +109,8 @@ __device__ __forceinline__ void bn_sum_slabs(const float *__restrict__ part, int
       }
     }
     for (; k < slabs; k += P) {
-      bn_add4(t1, bn_ld4(part + k * 2 * C + 4 * (g0 + g)));
-      bn_add4(t2, bn_ld4(part + k * 2 * C + C + 4 * (g0 + g)));
+      bn_add4(t1, bn_ld4(part + k * 2 * C + 4 * g));
+      bn_add4(t2, bn_ld4(part + k * 2 * C + C + 4 * g));
     }
   }
   s_red[0][threadIdx.x] = t1;
@@ -130,43 +123,12 @@ __device__ __forceinline__ void bn_sum_slabs(const float *__restrict__ part, int
     }
 }
 
-struct BnStatsOut {
-  const float *bias;
-  float *save_mean, *save_invstd, *running_mean, *running_var;
-  int64_t *batches_tracked;
-  float momentum, eps;
-};
-
-// Mean, 1/sqrt(var + eps) and running statistics of column group g from the totals of (x - sft) and (x - sft)^2.
-__device__ __forceinline__ void bn_finish_stats(const BnStatsOut &f, int64_t n, int g, const float4 &sft,
-                                                const float4 &t1, const float4 &t2) {
-  const float cnt = (float)n;
-  const float a1[4] = {t1.x, t1.y, t1.z, t1.w}, a2[4] = {t2.x, t2.y, t2.z, t2.w};
-  const float sf[4] = {sft.x, sft.y, sft.z, sft.w};
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const int c = 4 * g + j;
-    const float d = a1[j] / cnt;            // mean - shift
-    float m2 = a2[j] - a1[j] * d;           // sum of squared deviations from the mean
-    if (m2 < 0.f) m2 = 0.f;
-    const float mean = sf[j] + d;
-    const float var = m2 / cnt;
-    f.save_mean[c] = mean;
-    f.save_invstd[c] = 1.0f / sqrtf(var + f.eps);
-    if (f.running_mean != nullptr) {
-      const float shift = f.bias != nullptr ? f.bias[c] : 0.f;
-      f.running_mean[c] = (1.0f - f.momentum) * f.running_mean[c] + f.momentum * (mean + shift);
-    }
-    if (f.running_var != nullptr) {
-      const float unb = n > 1 ? m2 / (cnt - 1.f) : var;
-      f.running_var[c] = (1.0f - f.momentum) * f.running_var[c] + f.momentum * unb;
-    }
-  }
-}
-
 // part[slab][2][C]: S1 = sum (x - s), S2 = sum (x - s)^2 with s = x[0, :]
 __global__ __launch_bounds__(BN_BLOCK) void bn_stats(
-    const float *__restrict__ x, float *__restrict__ part, BnStatsOut f, int64_t n_cap, const int64_t *__restrict__ n_dev, int C, BnShape sh, unsigned *__restrict__ ticket) {
+    const float *__restrict__ x, const float *__restrict__ bias, float *__restrict__ part,
+    float *__restrict__ save_mean, float *__restrict__ save_invstd, float *__restrict__ running_mean,
+    float *__restrict__ running_var, int64_t *__restrict__ batches_tracked, float momentum, float eps,
+    int64_t n_cap, const int64_t *__restrict__ n_dev, int C, BnShape sh, unsigned *__restrict__ ticket) {
   __shared__ float4 s_red[2][BN_BLOCK];
   __shared__ int s_flag;
   const int64_t n = bn_rows(n_cap, n_dev);
@@ -208,27 +170,33 @@ __global__ __launch_bounds__(BN_BLOCK) void bn_stats(
     *reinterpret_cast<float4 *>(o) = s1;
     *reinterpret_cast<float4 *>(o + C) = s2;
   }
-  if (ticket == nullptr) return;                            // bn_stats_final adds the slabs
   if (!bn_last_block(ticket, &s_flag)) return;
-  if (threadIdx.x == 0 && f.batches_tracked != nullptr) *f.batches_tracked += 1;   // BatchNorm1d's batch counter
+  if (threadIdx.x == 0 && batches_tracked != nullptr) *batches_tracked += 1;   // BatchNorm1d's batch counter
   float4 t1, t2;
-  bn_sum_slabs(part, sh.slabs, C, 0, G, P, g, p, s_red, t1, t2);
-  if (p == 0) bn_finish_stats(f, n, g, sft, t1, t2);
-}
-
-// The slabs' sums added by a block per BN_FINAL_GROUPS column groups.
-__global__ __launch_bounds__(BN_BLOCK) void bn_stats_final(const float *__restrict__ x, const float *__restrict__ part,
-                                                            BnStatsOut f, int64_t n_cap,
-                                                            const int64_t *__restrict__ n_dev, int C, int64_t slabs) {
-  __shared__ float4 s_red[2][BN_BLOCK];
-  const int g0 = (int)blockIdx.x * BN_FINAL_GROUPS;
-  const int G = C / 4 - g0 < BN_FINAL_GROUPS ? C / 4 - g0 : BN_FINAL_GROUPS;
-  const int P = BN_BLOCK / G < 64 ? BN_BLOCK / G : 64;
-  const int g = (int)threadIdx.x % G, p = (int)threadIdx.x / G;
-  if (blockIdx.x == 0 && threadIdx.x == 0 && f.batches_tracked != nullptr) *f.batches_tracked += 1;
-  float4 t1, t2;
-  bn_sum_slabs(part, slabs, C, g0, G, P, g, p, s_red, t1, t2);
-  if (p == 0) bn_finish_stats(f, bn_rows(n_cap, n_dev), g0 + g, bn_ld4(x + 4 * (g0 + g)), t1, t2);
+  bn_sum_slabs(part, sh.slabs, C, G, P, g, p, s_red, t1, t2);
+  if (p != 0) return;
+  const float cnt = (float)n;
+  const float a1[4] = {t1.x, t1.y, t1.z, t1.w}, a2[4] = {t2.x, t2.y, t2.z, t2.w};
+  const float sf[4] = {sft.x, sft.y, sft.z, sft.w};
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const int c = 4 * g + j;
+    const float d = a1[j] / cnt;            // mean - shift
+    float m2 = a2[j] - a1[j] * d;           // sum of squared deviations from the mean
+    if (m2 < 0.f) m2 = 0.f;
+    const float mean = sf[j] + d;
+    const float var = m2 / cnt;
+    save_mean[c] = mean;
+    save_invstd[c] = 1.0f / sqrtf(var + eps);
+    if (running_mean != nullptr) {
+      const float shift = bias != nullptr ? bias[c] : 0.f;
+      running_mean[c] = (1.0f - momentum) * running_mean[c] + momentum * (mean + shift);
+    }
+    if (running_var != nullptr) {
+      const float unb = n > 1 ? m2 / (cnt - 1.f) : var;
+      running_var[c] = (1.0f - momentum) * running_var[c] + momentum * unb;
+    }
+  }
 }
 
 __global__ __launch_bounds__(HC_BLOCK) void bn_apply(
@@ -251,13 +219,6 @@ __global__ __launch_bounds__(HC_BLOCK) void bn_apply(
   o.z = fmaxf(bn_pre(v.z, m.z, s.z, ga.z, be.z), 0.f);
   o.w = fmaxf(bn_pre(v.w, m.w, s.w, ga.w, be.w), 0.f);
   *reinterpret_cast<float4 *>(y + 4 * i) = o;
-}
-
-__device__ __forceinline__ void bn_finish_bwd(float *__restrict__ dgamma, float *__restrict__ dbeta,
-                                              float *__restrict__ dbias, int g, const float4 &t1, const float4 &t2) {
-  *reinterpret_cast<float4 *>(dbeta + 4 * g) = t1;
-  *reinterpret_cast<float4 *>(dgamma + 4 * g) = t2;
-  if (dbias != nullptr) *reinterpret_cast<float4 *>(dbias + 4 * g) = make_float4(0.f, 0.f, 0.f, 0.f);
 }
 
 // part[slab][2][C]: sum dy', sum dy' * xhat
@@ -319,24 +280,13 @@ __global__ __launch_bounds__(BN_BLOCK) void bn_bwd_reduce(
     *reinterpret_cast<float4 *>(o) = s1;
     *reinterpret_cast<float4 *>(o + C) = s2;
   }
-  if (ticket == nullptr) return;                            // bn_bwd_final adds the slabs
   if (!bn_last_block(ticket, &s_flag)) return;
   float4 t1, t2;
-  bn_sum_slabs(part, sh.slabs, C, 0, G, P, g, p, s_red, t1, t2);
-  if (p == 0) bn_finish_bwd(dgamma, dbeta, dbias, g, t1, t2);
-}
-
-__global__ __launch_bounds__(BN_BLOCK) void bn_bwd_final(const float *__restrict__ part, float *__restrict__ dgamma,
-                                                          float *__restrict__ dbeta, float *__restrict__ dbias, int C,
-                                                          int64_t slabs) {
-  __shared__ float4 s_red[2][BN_BLOCK];
-  const int g0 = (int)blockIdx.x * BN_FINAL_GROUPS;
-  const int G = C / 4 - g0 < BN_FINAL_GROUPS ? C / 4 - g0 : BN_FINAL_GROUPS;
-  const int P = BN_BLOCK / G < 64 ? BN_BLOCK / G : 64;
-  const int g = (int)threadIdx.x % G, p = (int)threadIdx.x / G;
-  float4 t1, t2;
-  bn_sum_slabs(part, slabs, C, g0, G, P, g, p, s_red, t1, t2);
-  if (p == 0) bn_finish_bwd(dgamma, dbeta, dbias, g0 + g, t1, t2);
+  bn_sum_slabs(part, sh.slabs, C, G, P, g, p, s_red, t1, t2);
+  if (p != 0) return;
+  *reinterpret_cast<float4 *>(dbeta + 4 * g) = t1;
+  *reinterpret_cast<float4 *>(dgamma + 4 * g) = t2;
+  if (dbias != nullptr) *reinterpret_cast<float4 *>(dbias + 4 * g) = make_float4(0.f, 0.f, 0.f, 0.f);
 }
 
 __global__ __launch_bounds__(HC_BLOCK) void bn_bwd_apply(
@@ -448,13 +398,9 @@ extern "C" int hc_bn_relu_fwd_dev(const float *x, const float *bias, const float
   const int64_t blocks = (n4 + HC_BLOCK - 1) / HC_BLOCK;
   if (!hc_grid_ok(blocks)) return HC_ELAUNCH;
   hipStream_t st = static_cast<hipStream_t>(stream);
-  float *part = static_cast<float *>(workspace);
-  const BnStatsOut f{bias, save_mean, save_invstd, running_mean, running_var, num_batches_tracked, momentum, eps};
-  const bool large = n >= BN_LARGE_ROWS;
-  bn_stats<<<dim3((unsigned)sh.slabs), dim3(BN_BLOCK), 0, st>>>(x, part, f, n, n_dev, (int)C, sh, large ? nullptr : ticket);
-  if (large)
-    bn_stats_final<<<dim3((unsigned)((sh.groups + BN_FINAL_GROUPS - 1) / BN_FINAL_GROUPS)), dim3(BN_BLOCK), 0, st>>>(
-        x, part, f, n, n_dev, (int)C, sh.slabs);
+  bn_stats<<<dim3((unsigned)sh.slabs), dim3(BN_BLOCK), 0, st>>>(
+      x, bias, static_cast<float *>(workspace), save_mean, save_invstd, running_mean, running_var,
+      num_batches_tracked, momentum, eps, n, n_dev, (int)C, sh, ticket);
   bn_apply<<<dim3((unsigned)blocks), dim3(HC_BLOCK), 0, st>>>(x, save_mean, save_invstd, gamma, beta, y, n4,
                                                               sh.groups, n, n_dev);
   return hc_launch_status();
@@ -482,14 +428,9 @@ extern "C" int hc_bn_relu_bwd_dev(const float *dy, const float *x, const float *
   const int64_t blocks = (n4 + HC_BLOCK - 1) / HC_BLOCK;
   if (!hc_grid_ok(blocks)) return HC_ELAUNCH;
   hipStream_t st = static_cast<hipStream_t>(stream);
-  float *part = static_cast<float *>(workspace);
-  const bool large = n >= BN_LARGE_ROWS;
   bn_bwd_reduce<<<dim3((unsigned)sh.slabs), dim3(BN_BLOCK), 0, st>>>(
-      dy, x, save_mean, save_invstd, gamma, beta, part, dgamma, dbeta, dbias, n, n_dev, (int)C, sh,
-      large ? nullptr : ticket);
-  if (large)
-    bn_bwd_final<<<dim3((unsigned)((sh.groups + BN_FINAL_GROUPS - 1) / BN_FINAL_GROUPS)), dim3(BN_BLOCK), 0, st>>>(
-        part, dgamma, dbeta, dbias, (int)C, sh.slabs);
+      dy, x, save_mean, save_invstd, gamma, beta, static_cast<float *>(workspace), dgamma, dbeta, dbias, n, n_dev,
+      (int)C, sh, ticket);
   bn_bwd_apply<<<dim3((unsigned)blocks), dim3(HC_BLOCK), 0, st>>>(
       dy, x, save_mean, save_invstd, gamma, beta, dgamma, dbeta, dx, n4, sh.groups, n, n_dev);
   return hc_launch_status();
