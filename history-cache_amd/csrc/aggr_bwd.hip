@@ -9,8 +9,10 @@ namespace {
 // source; source n_src stands for the end.
 constexpr int BWD_PREP_BLOCK = 1024;     // at most SEG_MAX_REGIONS blocks: large ones, to fill the chip
 __global__ __launch_bounds__(BWD_PREP_BLOCK) void bwd_prepare(BwdArgs a, int64_t runs) {
-  __shared__ int n_mid, n_hub;
-  if (threadIdx.x == 0) n_mid = n_hub = 0;
+  __shared__ int n_mid, n_hub, n_giant;
+  if (threadIdx.x == 0) n_mid = n_hub = n_giant = 0;
+  for (int64_t i = (int64_t)blockIdx.x * BWD_PREP_BLOCK + threadIdx.x; i < a.n_tickets; i += (int64_t)gridDim.x * BWD_PREP_BLOCK)
+    a.ticket[i] = 0u;
   __syncthreads();
   const int64_t first = (int64_t)blockIdx.x * a.tile;
   int64_t last = first + a.tile;
@@ -18,6 +20,7 @@ __global__ __launch_bounds__(BWD_PREP_BLOCK) void bwd_prepare(BwdArgs a, int64_t
   const bool at_end = last == a.n_src;
   const int64_t mid0 = seg_part(a.ptrT, first, a.long_above);
   const int64_t hub0 = a.chunk > 0 ? seg_part(a.ptrT, first, a.chunk) : 0;
+  const int64_t giant0 = a.giant.cap > 0 ? seg_part(a.ptrT, first, BWD_SPAN) : 0;
   constexpr int ITEMS = 4;
   for (int64_t s0 = first; s0 < last + (at_end ? 1 : 0); s0 += BWD_PREP_BLOCK * ITEMS) {
     int64_t p[ITEMS], p1[ITEMS], pm[ITEMS];
@@ -41,7 +44,10 @@ __global__ __launch_bounds__(BWD_PREP_BLOCK) void bwd_prepare(BwdArgs a, int64_t
       }
       const int64_t deg = p1[it] - p[it];
       if (deg <= a.long_above) continue;
-      if (a.chunk > 0 && deg > a.chunk) {
+      if (a.giant.cap > 0 && deg > BWD_SPAN) {
+        const int64_t at = giant0 + atomicAdd(&n_giant, 1);
+        if (at < a.giant.cap) a.giant.item[at] = (int32_t)s;
+      } else if (a.chunk > 0 && deg > a.chunk) {
         const int64_t at = hub0 + atomicAdd(&n_hub, 1);
         if (at < a.hub.cap) a.hub.item[at] = (int32_t)s;
       } else {
@@ -54,6 +60,7 @@ __global__ __launch_bounds__(BWD_PREP_BLOCK) void bwd_prepare(BwdArgs a, int64_t
   if (threadIdx.x == 0) {
     a.mid.count[blockIdx.x] = n_mid;
     a.hub.count[blockIdx.x] = n_hub;
+    a.giant.count[blockIdx.x] = n_giant;
   }
 }
 
@@ -61,20 +68,26 @@ bool bwd_fast_shape(int64_t F) {
   return F == 64 || F == 128 || F == 192 || F == 256 || F == 384 || F == 512 || F == 768 || F == 1024;
 }
 
-// Workspace: the lists' counts and entries, then the runs' starts.  A block of up to BWD_LONG edges has no long
-// source and needs neither.
+// Workspace: the lists' counts and entries, the giants' tickets and chunk sums (F: the width of a chunked sum, else 0),
+// then the runs' starts.  A block of up to BWD_LONG edges has no long source and needs none of them.
 struct BwdWsLayout {
-  size_t mid, hub, lists, run_start, total;
-  int64_t mid_cap, hub_cap, runs;
+  size_t mid, hub, giant, ticket, partial, lists, run_start, total;
+  int64_t mid_cap, hub_cap, giant_cap, tickets, runs;
 };
-BwdWsLayout bwd_ws_layout(int64_t E, int64_t n_src) {
+BwdWsLayout bwd_ws_layout(int64_t E, int64_t F, int64_t n_src) {
   BwdWsLayout L{};
   if (E <= BWD_LONG) return L;
   L.mid_cap = E / (BWD_LONG + 1) + 1;
   L.hub_cap = E / (BWD_CHUNK + 1) + 1;
-  L.mid = 2 * SEG_MAX_REGIONS * sizeof(int32_t);
+  L.giant_cap = F > 0 && E > BWD_SPAN ? E / (BWD_SPAN + 1) + 1 : 0;
+  L.tickets = L.giant_cap * ((F + BWD_SLICE - 1) / BWD_SLICE);
+  L.mid = 3 * SEG_MAX_REGIONS * sizeof(int32_t);
   L.hub = L.mid + (size_t)L.mid_cap * sizeof(int32_t);
-  L.lists = hc_align_up(L.hub + (size_t)L.hub_cap * sizeof(int32_t), 256);
+  L.giant = L.hub + (size_t)L.hub_cap * sizeof(int32_t);
+  L.ticket = L.giant + (size_t)L.giant_cap * sizeof(int32_t);
+  L.partial = hc_align_up(L.ticket + (size_t)L.tickets * sizeof(int32_t), 256);
+  L.lists = L.partial;
+  if (L.giant_cap > 0) L.lists += hc_align_up((size_t)(2 * (E / BWD_CHUNK + 1)) * (size_t)F * sizeof(float), 256);
   L.run_start = L.lists;
   L.runs = (E + BWD_SRC_COST * n_src) / BWD_UNIT + 1;
   L.total = L.lists + hc_align_up((size_t)L.runs * sizeof(int32_t), 256);
@@ -112,7 +125,8 @@ __global__ __launch_bounds__(HC_BLOCK) void bwd_hist_generic(const float *__rest
 int bwd_sum_sources(BwdArgs &a, int64_t E, void *workspace, size_t workspace_bytes, int vin_dtype, bool masked,
                     hipStream_t st) {
   a.hist_blocks = (a.grad_hbuf && a.n_head == 1) ? (a.R + HC_WAVES_PER_BLOCK - 1) / HC_WAVES_PER_BLOCK : 0;
-  const BwdWsLayout L = bwd_ws_layout(E, a.n_src);
+  const bool chunked = a.ev == nullptr && bwd_fast_shape(a.F);
+  const BwdWsLayout L = bwd_ws_layout(E, chunked ? a.F : 0, a.n_src);
   char *ws = static_cast<char *>(workspace);
   // fixed runs: enough of them for the chip, at most BWD_MAX_RUN sources (two layers of a sampled batch: 31 us, in
   // runs of 32 whatever their number 40 us)
@@ -121,11 +135,17 @@ int bwd_sum_sources(BwdArgs &a, int64_t E, void *workspace, size_t workspace_byt
   int64_t waves = (a.n_src + a.run - 1) / a.run;
   if (L.lists > 0 && a.n_src > 0 && ws != nullptr && workspace_bytes >= L.lists && reinterpret_cast<uintptr_t>(ws) % 256 == 0) {
     a.long_above = BWD_LONG;
-    a.chunk = a.ev == nullptr && bwd_fast_shape(a.F) ? BWD_CHUNK : 0;
+    a.chunk = chunked ? BWD_CHUNK : 0;
     a.tile = seg_tile(a.n_src);
     a.n_tiles = (int)((a.n_src + a.tile - 1) / a.tile);
     a.mid.count = reinterpret_cast<int32_t *>(ws);
     a.hub.count = a.mid.count + SEG_MAX_REGIONS;
+    a.giant.count = a.hub.count + SEG_MAX_REGIONS;
+    a.giant.item = reinterpret_cast<int32_t *>(ws + L.giant);
+    a.giant.cap = L.giant_cap;
+    a.ticket = reinterpret_cast<uint32_t *>(ws + L.ticket);
+    a.n_tickets = L.tickets;
+    a.partial = reinterpret_cast<float *>(ws + L.partial);
     a.mid.item = reinterpret_cast<int32_t *>(ws + L.mid);
     a.hub.item = reinterpret_cast<int32_t *>(ws + L.hub);
     a.mid.cap = L.mid_cap;
@@ -228,12 +248,12 @@ __global__ __launch_bounds__(HC_BLOCK) void bwd_typed_batch_view(
 
 extern "C" size_t hc_aggr_bwd_workspace_bytes(int64_t E_total, int64_t F) {
   if (E_total < 0 || F <= 0) return 0;
-  return bwd_ws_layout(E_total, 0).lists;
+  return bwd_ws_layout(E_total, bwd_fast_shape(F) ? F : 0, 0).lists;
 }
 
 extern "C" size_t hc_aggr_bwd_workspace_bytes_for(int64_t E_total, int64_t F, int64_t n_src) {
   if (E_total < 0 || F <= 0 || n_src < 0) return 0;
-  return bwd_ws_layout(E_total, n_src).total;
+  return bwd_ws_layout(E_total, bwd_fast_shape(F) ? F : 0, n_src).total;
 }
 
 extern "C" int64_t hc_aggr_bwd_chunk_edges(int64_t F) { return bwd_fast_shape(F) ? BWD_CHUNK : 0; }

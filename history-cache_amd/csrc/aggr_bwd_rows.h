@@ -39,6 +39,10 @@ constexpr int BWD_XCD_CHUNK = 64;   // consecutive blocks that share an XCD
 // in chunks of BWD_CHUNK edges, the chunk sums added left to right.
 constexpr int BWD_CHUNK = 512;
 constexpr int BWD_LONG = 128;       // sources with more edges are the front blocks' tasks
+// A chunked source above this many edges is several blocks' work: each leaves its chunks' sums in the workspace and
+// the one that arrives last adds them left to right.  (A compute unit brings in about 65 lines a microsecond, whatever
+// its waves do.  4 M edges x 256 with a source of 1.0 M and 70 above 4 096: 3.5 ms by a wave per chunk, 1.2 ms so.)
+constexpr int BWD_SPAN = 8 * BWD_CHUNK;
 constexpr int BWD_UNIT = 128;       // a wave's run of sources: edges + BWD_SRC_COST per source
 constexpr int BWD_SRC_COST = 4;
 constexpr int BWD_MAX_RUN = 32;     // BWD_UNIT / BWD_SRC_COST; fixed runs have at most this many sources too
@@ -61,7 +65,10 @@ struct BwdArgs {
   bool small_matrix;            // g holds less than 4 GiB
   int64_t long_above;           // sources with more edges are left to the front blocks (0: none)
   int64_t chunk;                // sources with more edges are summed in chunks (0: never); >= long_above
-  SegList mid, hub;             // long sources up to `chunk` (or all of them), the others
+  SegList mid, hub, giant;      // long sources up to `chunk` (or all of them), up to BWD_SPAN, the others
+  uint32_t *ticket;             // per giant and slice, zeroed by bwd_prepare
+  int64_t n_tickets;
+  float *partial;               // chunk sums of the giants, two rows per BWD_CHUNK positions of the view
   int n_tiles;
   int64_t tile;
   int front;
@@ -236,6 +243,58 @@ __device__ __forceinline__ void bwd_front(const BwdArgs &a, int lane, int wave) 
     return (uint32_t)(c < a.F ? c : a.F - 1);
   };
   TO *__restrict__ out = static_cast<TO *>(a.grad_vin);
+  if (WMODE == W_NONE && a.giant.cap > 0) {
+    __shared__ int s_last;
+    const SegIndex index = seg_index(a.giant.count, a.n_tiles, lane);
+    int64_t t = blockIdx.x;                                  // this block's next task, counted from the giant's first
+    for (int i = 0; i < index.total; ++i) {                  // block-uniform
+      const int64_t s = source(a.giant, index, BWD_SPAN, i);
+      const int64_t b = a.ptrT[s], e = a.ptrT[s + 1];
+      const int64_t spans = (e - b + BWD_SPAN - 1) / BWD_SPAN;
+      // chunk k starts at position b + k * BWD_CHUNK; its window holds one other start at most, a first chunk's
+      const auto row = [&](int64_t k) -> float * {
+        return a.partial + (2 * ((b + k * BWD_CHUNK) / BWD_CHUNK) + (k == 0 ? 1 : 0)) * a.F;
+      };
+      for (; t < spans * ns; t += a.front) {
+        const int sl = (int)(t % ns);
+        bool on;
+        const uint32_t c = column(sl, on);
+        for (int64_t k = t / ns * (BWD_SPAN / BWD_CHUNK) + wave; k < (t / ns + 1) * (BWD_SPAN / BWD_CHUNK);
+             k += HC_WAVES_PER_BLOCK) {
+          const int64_t mb = b + k * BWD_CHUNK;
+          if (mb >= e) break;
+          const float v = bwd_slice_any<W_NONE, MASKED>(a, c, mb, mb + BWD_CHUNK < e ? mb + BWD_CHUNK : e, lane);
+          if (on) row(k)[c] = v;
+        }
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+        __syncthreads();
+        if (threadIdx.x == 0) {
+          __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+          s_last = atomicAdd(a.ticket + (int64_t)i * ns + sl, 1u) == (uint32_t)(spans - 1) ? 1 : 0;
+        }
+        __syncthreads();
+        if (s_last != 0) {
+          __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+          if (wave == 0) {
+            const int64_t n = (e - b + BWD_CHUNK - 1) / BWD_CHUNK;
+            float sum = row(0)[c];
+            int64_t k = 1;
+            for (; k + 8 <= n; k += 8) {
+              float v[8];
+#pragma unroll
+              for (int u = 0; u < 8; ++u) v[u] = row(k + u)[c];
+#pragma unroll
+              for (int u = 0; u < 8; ++u) sum += v[u];
+            }
+            for (; k < n; ++k) sum += row(k)[c];
+            if (on) out[s * a.F + c] = hc_from_f32<TO>(sum);
+          }
+        }
+        __syncthreads();
+      }
+      t -= spans * ns;
+    }
+  }
   if (WMODE == W_NONE && a.chunk > 0) {
     const SegIndex index = seg_index(a.hub.count, a.n_tiles, lane);
     const int64_t tasks = (int64_t)index.total * ns;

@@ -377,7 +377,7 @@ def _aggr_bwd(ptr, idx, tr, g, hmap, edge_value, x, want_edge_grad, hbuf_shape, 
     E_total = rowT.numel()
     if edge_value is not None:
         E_total = max(E_total, edge_value.shape[0]) if edge_grad is None else edge_value.shape[0]
-    nbytes = lib.hc_aggr_bwd_workspace_bytes_for(E_total, F, n_src)
+    nbytes = lib.hc_aggr_bwd_workspace_bytes_for(E_total, F if edge_value is None else 1, n_src)   # (weighted: no chunks)
     ws = _workspace(nbytes, dev) if nbytes else None
     rc = lib.hc_aggr_bwd_as(_ptr(ptr), _ptr(idx), _ptr(ptrT), _ptr(rowT), _ptr(edgeT), _ptr(g), _ptr(hmap),
                          _ptr(edge_value), _ptr(x) if want_edge_grad else _c_p(None),

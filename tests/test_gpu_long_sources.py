@@ -23,8 +23,10 @@ def T(a, dtype=None):
     return t if dtype is None else t.to(dtype)
 
 
-# in-degrees around every threshold: 64 edges of a stage, 128 (long), 512 (chunk), four chunks of a block's waves
-DEGREES = {0: 1700, 1: 513, 2: 512, 3: 129, 4: 128, 5: 127, 6: 65, 7: 0, 8: 64, 9: 2048, 10: 2049, 300: 640, -1: 2600, -2: 1}
+# in-degrees around every threshold: 64 edges of a stage, 128 (long), 512 (chunk), four chunks of a block's waves,
+# 4096 (several blocks) and its multiples
+DEGREES = {0: 1700, 1: 513, 2: 512, 3: 129, 4: 128, 5: 127, 6: 65, 7: 0, 8: 64, 9: 2048, 10: 2049, 300: 640,
+           301: 4096, 302: 4097, 303: 8192, 304: 23456, -3: 9000, -1: 2600, -2: 1}
 
 
 def block(rng, R, N, extra=4):
