@@ -400,8 +400,8 @@ class BatchView:
         self.ptrT, self.rowT, self.edgeT = ptrT, rowT, edgeT
         self.rows, self.n_src, self.num_edge = int(rows), int(n_src), int(num_edge)
         # the largest number of edges that one node of the batch has in the view, when whoever made the batch
-        # knows it (None: unknown).  A view without a source above the backward's chunk length needs neither
-        # the chunk sums nor the launch that combines them.
+        # knows it (None: unknown).  A view without a source above the backward's chunk length goes without the
+        # launch that lists the long ones.
         self.max_in_degree = None if max_in_degree is None else int(max_in_degree)
         # likewise a bound on the edges of one row of the batch's CSR (a sampled batch: its largest fanout); the
         # forward passes then look for no long rows
