@@ -29,7 +29,7 @@
 #include <type_traits>
 
 // Rows with more edges than this are summed as four quarters (mean, single-head weights).
-// The CPU checker applies the same rule; the header documents it.
+// The oracle applies the same rule; the header documents it.
 constexpr int64_t HC_LONG_ROW_EDGES = 256;
 // Rows of several heads are never split into quarters; those above this many edges are summed slice by
 // slice on several compute units (each slice strictly in CSR order).

@@ -91,7 +91,7 @@ __device__ __forceinline__ int64_t hc_xcd_block(int64_t bid, int64_t n) {
 
 // Butterfly sum over the 64 lanes, partner distance 32,16,8,4,2,1.  Every lane
 // ends with the same bits (fp add is commutative), and the order is the one
-// the CPU checker reproduces.
+// the oracle reproduces.
 __device__ __forceinline__ float hc_wave_sum_butterfly(float v) {
 #pragma unroll
   for (int d = 32; d >= 1; d >>= 1) v = v + __shfl_xor(v, d, HC_WAVE);
