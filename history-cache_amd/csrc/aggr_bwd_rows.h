@@ -266,15 +266,7 @@ __device__ __forceinline__ void bwd_front(const BwdArgs &a, int lane, int wave) 
           const float v = bwd_slice_any<W_NONE, MASKED>(a, c, mb, mb + BWD_CHUNK < e ? mb + BWD_CHUNK : e, lane);
           if (on) row(k)[c] = v;
         }
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-        __syncthreads();
-        if (threadIdx.x == 0) {
-          __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
-          s_last = atomicAdd(a.ticket + (int64_t)i * ns + sl, 1u) == (uint32_t)(spans - 1) ? 1 : 0;
-        }
-        __syncthreads();
-        if (s_last != 0) {
-          __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+        if (hc_arrives_last(a.ticket + (int64_t)i * ns + sl, (unsigned)spans, &s_last)) {
           if (wave == 0) {
             const int64_t n = (e - b + BWD_CHUNK - 1) / BWD_CHUNK;
             float sum = row(0)[c];

@@ -67,24 +67,6 @@ __device__ __forceinline__ void bn_add4(float4 &a, const float4 &b) {
   a.x += b.x; a.y += b.y; a.z += b.z; a.w += b.w;
 }
 
-// One ticket per launch: true in the block that arrives last.  The counter is zero again when the
-// kernel ends.  One device-scope release per block, by the thread that takes the ticket, behind the
-// block's barrier.
-__device__ __forceinline__ bool bn_last_block(unsigned *ticket, int *s_flag) {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
-    const unsigned t = atomicAdd(ticket, 1u);
-    *s_flag = t == gridDim.x - 1 ? 1 : 0;
-    if (t == gridDim.x - 1) atomicExch(ticket, 0u);
-  }
-  __syncthreads();
-  if (!*s_flag) return false;
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-  return true;
-}
-
 // Sum over the slabs of the two partial sums of column group g, by the block that arrived last:
 // part[slab][2][C].  Thread (g, p) adds slabs p, p + P, ... in that order, thread (g, 0) then adds the
 // P results in order of p.  Ends with the totals in the threads with p == 0.
@@ -170,7 +152,7 @@ __global__ __launch_bounds__(BN_BLOCK) void bn_stats(
     *reinterpret_cast<float4 *>(o) = s1;
     *reinterpret_cast<float4 *>(o + C) = s2;
   }
-  if (!bn_last_block(ticket, &s_flag)) return;
+  if (!hc_arrives_last(ticket, gridDim.x, &s_flag)) return;
   if (threadIdx.x == 0 && batches_tracked != nullptr) *batches_tracked += 1;   // BatchNorm1d's batch counter
   float4 t1, t2;
   bn_sum_slabs(part, sh.slabs, C, G, P, g, p, s_red, t1, t2);
@@ -280,7 +262,7 @@ __global__ __launch_bounds__(BN_BLOCK) void bn_bwd_reduce(
     *reinterpret_cast<float4 *>(o) = s1;
     *reinterpret_cast<float4 *>(o + C) = s2;
   }
-  if (!bn_last_block(ticket, &s_flag)) return;
+  if (!hc_arrives_last(ticket, gridDim.x, &s_flag)) return;
   float4 t1, t2;
   bn_sum_slabs(part, sh.slabs, C, G, P, g, p, s_red, t1, t2);
   if (p != 0) return;

@@ -98,6 +98,28 @@ __device__ __forceinline__ float hc_wave_sum_butterfly(float v) {
   return v;
 }
 
+// The calling block arrives at a counter that `of` blocks take (every thread of them calls this).  True in every
+// thread of the block that arrives last, which then sees what all of them had stored; the counter is zero again.
+// Every wave waits for its own stores in front of the barrier: a release of workgroup scope waits for the LDS alone,
+// and the device-scope release that thread 0 makes behind the barrier waits for its own wave's stores only, before
+// it writes the die's L2 back.  (One release of device scope per wave would do as well, at one write-back each.)
+__device__ __forceinline__ bool hc_arrives_last(unsigned *ticket, unsigned of, int *s_flag) {
+  constexpr int VMCNT_0 = 0x0f70;      // s_waitcnt: vmcnt 0, the other counters at their largest
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+  __builtin_amdgcn_s_waitcnt(VMCNT_0);
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+    const unsigned t = atomicAdd(ticket, 1u);
+    *s_flag = t == of - 1u ? 1 : 0;
+    if (t == of - 1u) atomicExch(ticket, 0u);
+  }
+  __syncthreads();
+  if (*s_flag == 0) return false;
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+  return true;
+}
+
 // ---- element conversion ----------------------------------------------------
 template <typename T>
 __device__ __forceinline__ float hc_to_f32(T v);

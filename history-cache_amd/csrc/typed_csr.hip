@@ -127,8 +127,7 @@ __device__ __forceinline__ void tc_scan_row_totals(int64_t *__restrict__ p, int6
 }
 
 // tc_count for small blocks (row totals into ptr2, see above), and the scan of the totals by the block that
-// arrives last (one device-scope release per block, by the thread that takes the ticket, behind the block's
-// barrier; the ticket is zero again when the kernel ends)
+// arrives last (the ticket is zero again when the kernel ends)
 __global__ __launch_bounds__(TCS_BLOCK) void tc_count_scan(const int64_t *__restrict__ ptr,
                                                             const int64_t *__restrict__ idx,
                                                             const int64_t *__restrict__ et,
@@ -159,17 +158,7 @@ __global__ __launch_bounds__(TCS_BLOCK) void tc_count_scan(const int64_t *__rest
       ptr2[(row + 1) * K] = total;
     }
   }
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
-    const unsigned t = atomicAdd(ticket, 1u);
-    s_last = t == gridDim.x - 1 ? 1 : 0;
-    if (t == gridDim.x - 1) atomicExch(ticket, 0u);
-  }
-  __syncthreads();
-  if (!s_last) return;
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+  if (!hc_arrives_last(ticket, gridDim.x, &s_last)) return;
   if (threadIdx.x == 0) ptr2[0] = 0;
   tc_scan_row_totals(ptr2, R, K, s_wave);
 }
