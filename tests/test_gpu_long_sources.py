@@ -148,3 +148,26 @@ def test_half_precision_features_through_autograd(be, orc, dtype):
     assert x.grad.dtype == dtype
     ref, _ = orc.bwd_mean_row(ptr, idx, g, None, N, chunk=be.bwd_chunk_edges(F))
     assert torch.equal(x.grad.cpu(), torch.from_numpy(ref).to(dtype))
+
+
+@pytest.mark.parametrize("F", [64, 100])
+def test_layer_without_rows_over_a_view_of_long_sources(be, F):
+    """Every edge of the view is stepped over and there is no gradient row: zeros, whatever the sources' lengths."""
+    rng = np.random.default_rng(13)
+    R, N = 3000, 900
+    ptr, idx = block(rng, R, N)
+    tp, ti = T(ptr), T(idx)
+    view = be.build_batch_view(tp, ti, R, N)
+    lib = be.load_library()
+    ws = torch.empty(lib.hc_aggr_bwd_workspace_bytes_for(len(idx), F, N), dtype=torch.uint8, device=DEV)
+    out = torch.full((N, F), float("nan"), device=DEV)
+    rc = lib.hc_aggr_bwd_batch_view(tp.data_ptr(), view.ptrT.data_ptr(), view.rowT.data_ptr(), None, None, out.data_ptr(),
+                                    None, 0, len(idx), 0, F, N, ws.data_ptr(), ws.numel(),
+                                    torch.cuda.current_stream().cuda_stream)
+    assert rc == 0 and not out.any()
+    none = torch.empty(0, device=DEV)
+    x = T(rng.standard_normal((N, F)).astype(np.float32)).requires_grad_(True)
+    y = be.aggr_forward_history(x, tp[:1], ti, none, none, 0, 0, view=view)
+    assert y.shape == (0, F)
+    y.sum().backward()
+    assert x.grad.shape == (N, F) and not x.grad.any()
