@@ -135,6 +135,7 @@ int bwd_sum_sources(BwdArgs &a, int64_t E, void *workspace, size_t workspace_byt
   int64_t waves = (a.n_src + a.run - 1) / a.run;
   // (without rows every edge of a shared view is stepped over: nothing to share out, and no row of g to read instead)
   if (L.lists > 0 && a.n_src > 0 && a.R > 0 && ws != nullptr && workspace_bytes >= L.lists && reinterpret_cast<uintptr_t>(ws) % 256 == 0) {
+    a.E = E;
     a.long_above = BWD_LONG;
     a.chunk = chunked ? BWD_CHUNK : 0;
     a.tile = seg_tile(a.n_src);

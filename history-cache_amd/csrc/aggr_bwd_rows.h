@@ -60,6 +60,7 @@ struct BwdArgs {
   float *grad_hbuf;             // nullable
   int64_t hsize;
   int64_t R, n_src;
+  int64_t E;                    // entries of the view that the lists and the runs are sized for
   int64_t F;                    // a row is all heads side by side
   int slots;                    // F / VEC
   bool small_matrix;            // g holds less than 4 GiB
@@ -336,8 +337,11 @@ template <typename TO, int VEC, int CHUNKS, int UNROLL, int WMODE, bool MASKED>
 __global__ __launch_bounds__(HC_BLOCK) void bwd_sources(BwdArgs a) {
   const int lane = hc_lane();
   const int wave = hc_wave_in_block();
+  // every thread of the grid reads the same two words, so the decision is uniform: a view of more entries than its
+  // caller announced is summed as if there were neither lists nor runs (they would not hold it)
+  const bool listed = a.front > 0 && a.ptrT[a.n_src] - a.ptrT[0] <= a.E;
   if ((int)blockIdx.x < a.front) {
-    bwd_front<TO, WMODE, MASKED>(a, lane, wave);
+    if (listed) bwd_front<TO, WMODE, MASKED>(a, lane, wave);
     return;
   }
   const int64_t block = (int64_t)blockIdx.x - a.front;
@@ -366,14 +370,15 @@ __global__ __launch_bounds__(HC_BLOCK) void bwd_sources(BwdArgs a) {
   }
   const int64_t unit = hc_xcd_block<BWD_XCD_CHUNK>(block, a.src_blocks) * HC_WAVES_PER_BLOCK + wave;
   int64_t s0, s1;
-  if (a.run_start != nullptr) {
+  if (a.run_start != nullptr && listed) {
     const int64_t last = bwd_run_of(a, a.n_src);
     if (unit > last) return;
     s0 = a.run_start[unit];
     s1 = unit < last ? a.run_start[unit + 1] : a.n_src;
   } else {
-    s0 = unit * a.run;
-    s1 = s0 + a.run < a.n_src ? s0 + a.run : a.n_src;
+    const int64_t run = a.run_start != nullptr ? BWD_MAX_RUN : a.run;      // the runs' waves are no fewer than those
+    s0 = unit * run;
+    s1 = s0 + run < a.n_src ? s0 + run : a.n_src;
   }
   s0 = hc_uniform64(s0);
   s1 = hc_uniform64(s1);
@@ -384,7 +389,7 @@ __global__ __launch_bounds__(HC_BLOCK) void bwd_sources(BwdArgs a) {
   const int64_t my_p1 = a.ptrT[s0 + (lane + 1 < ns ? lane + 1 : ns)];
   // sources summed by the front blocks: their segments are stepped over and not stored here
   const unsigned long long long_mask =
-      a.long_above > 0 ? __ballot(lane < ns && (my_p1 - my_p) > a.long_above) : 0ull;
+      listed ? __ballot(lane < ns && (my_p1 - my_p) > a.long_above) : 0ull;
   const int tiles = CHUNKS == 4 ? (a.slots + HC_WAVE * CHUNKS - 1) / (HC_WAVE * CHUNKS) : 1;
   for (int tile = 0; tile < tiles; ++tile) {
     const BwdCols<VEC, CHUNKS> col(a, tile, lane, WMODE == W_EDGE_HEAD);

@@ -171,3 +171,33 @@ def test_layer_without_rows_over_a_view_of_long_sources(be, F):
     assert y.shape == (0, F)
     y.sum().backward()
     assert x.grad.shape == (N, F) and not x.grad.any()
+
+
+@pytest.mark.parametrize("F", [47, 128])
+@pytest.mark.parametrize("runs", [False, True])
+@pytest.mark.parametrize("announced", [200, 5000])
+def test_view_of_more_entries_than_announced(be, orc, F, runs, announced):
+    """The lists and runs are sized by the caller's number of entries; a view that holds more is summed without them,
+    strictly in order, with nothing left out and nothing written behind the scratch."""
+    rng = np.random.default_rng(F)
+    R, N = 4000, 9000
+    ptr, idx = block(rng, R, N)
+    g = rng.standard_normal((R, F)).astype(np.float32)
+    tp, tg = T(ptr), T(g)
+    view = be.build_batch_view(tp, T(idx), R, N)
+    lib = be.load_library()
+    need = (lib.hc_aggr_bwd_workspace_bytes_for(announced, F, N) if runs else lib.hc_aggr_bwd_workspace_bytes(announced, F))
+    ws = torch.full((need + 4096,), 0x5a, dtype=torch.uint8, device=DEV)
+    want, _ = orc.bwd_mean_row(ptr, idx, g, None, N, chunk=0)
+    st = torch.cuda.current_stream().cuda_stream
+    for masked in (False, True):
+        out = torch.full((N, F), float("nan"), device=DEV)
+        if masked:
+            rc = lib.hc_aggr_bwd_batch_view(tp.data_ptr(), view.ptrT.data_ptr(), view.rowT.data_ptr(), tg.data_ptr(), None,
+                                            out.data_ptr(), None, 0, announced, R, F, N, ws.data_ptr(), need, st)
+        else:
+            rc = lib.hc_aggr_bwd(tp.data_ptr(), None, view.ptrT.data_ptr(), view.rowT.data_ptr(), None, tg.data_ptr(), None,
+                                 None, None, 0, 1, out.data_ptr(), None, 0, None, announced, R, F, N, ws.data_ptr(), need, st)
+        assert rc == 0
+        np.testing.assert_array_equal(out.cpu().numpy(), want)
+        assert (ws[need:] == 0x5a).all()
