@@ -13,6 +13,7 @@ import weakref
 
 import torch
 import torch.nn.functional as F
+from torch.nn.modules.module import _has_any_global_hook
 
 import hiscache_backend
 
@@ -175,15 +176,27 @@ def bn_relu(x, bn, bias=None, fused=True, n_dev=None):
                            bn.running_var if track else None, momentum, bn.eps, counter, n_dev)
 
 
+def _unobserved(module, kind):
+    """Is ``module`` a plain ``kind`` whose call nothing watches or replaces: no hook of its own or of all modules, no
+    ``forward`` of its own, no autocast, no tracing, function transform, forward-mode level or dispatch mode?  Only then
+    may evaluation fold it into a library call, or hand a part of it to the next layer."""
+    return (type(module) is kind and "forward" not in module.__dict__
+            and not (module._forward_hooks or module._forward_pre_hooks or _has_any_global_hook())
+            and not torch.is_autocast_enabled("cuda") and not torch.jit.is_tracing()
+            and torch.autograd.forward_ad._current_level < 0 and torch._C._len_torch_dispatch_stack() == 0
+            and torch._C._functorch.peek_interpreter_stack() is None)
+
+
 def _evaluates(bn, x, bias):
-    """Does ``hc_bn_relu_eval`` cover this call: the running statistics, no gradient, no autocast, plain fp32 vectors
-    on the GPU, and no hook or subclass of the normalisation that a fused call would pass by?"""
-    if bn.training or torch.is_grad_enabled() or torch.is_autocast_enabled("cuda") or type(bn) is not torch.nn.BatchNorm1d:
+    """Does ``hc_bn_relu_eval`` cover this call: the running statistics, no gradient, plain fp32 vectors on the current
+    GPU, and nothing that a fused call would pass by?"""
+    if bn.training or torch.is_grad_enabled() or not _unobserved(bn, torch.nn.BatchNorm1d):
         return False
-    if bn._forward_hooks or bn._forward_pre_hooks or bn.running_mean is None or x.dim() != 2 or not x.is_contiguous():
+    if bn.running_mean is None or x.dim() != 2 or not x.is_contiguous():
         return False
     vectors = [t for t in (bias, bn.weight, bn.bias, bn.running_mean, bn.running_var) if t is not None]
-    return (hiscache_backend.bn_relu_supported(x, x.shape[1]) and x.dtype == torch.float32 and x.data_ptr() % 16 == 0
+    return (hiscache_backend.bn_relu_supported(x, x.shape[1]) and x.data_ptr() % 16 == 0
+            and x.device.index == torch.cuda.current_device()
             and all(t.is_cuda and t.device == x.device and t.dtype == torch.float32 and t.is_contiguous()
                     and t.numel() == x.shape[1] and t.data_ptr() % 16 == 0 for t in vectors))
 
@@ -282,9 +295,10 @@ class HistorySAGE(torch.nn.Module):
             n = batch.num_node_in_layer[k]
             ne = None if nel is None else int(nel[k])
             ptr = batch.ptr if ptrs is None else ptrs[k]
-            # the bias of lin_l goes to the normalisation's kernels instead of a launch of its own
+            # the bias of lin_l goes to the normalisation's kernels instead of a launch of its own (in evaluation where
+            # nobody sees the layer's output without it)
             defer = (self.fused_epilogue and conv.fused and x.is_cuda
-                     and (self.training or not torch.is_grad_enabled()))
+                     and (self.training or (not torch.is_grad_enabled() and _unobserved(conv, MySageConvHistory))))
             if self.training and i == self.num_layers - 2:
                 # the layer whose output is one hop from the seeds uses (and produces) history
                 x, his = conv(x, ptr, batch.idx, self.table.sub2embed,

@@ -267,3 +267,51 @@ def test_evaluation_is_one_kernel(n, C, affine):
     fine = torch.isfinite(want) & torch.isfinite(x.double())
     assert ((got - want).abs()[fine] <= 5 * 2.0 ** -24 * size[fine]).all()
     assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.isinf(), want.isinf())
+
+
+def test_evaluation_shows_its_layers_to_whoever_watches():
+    """Hooks of a hidden layer (its own, or those of all modules) see its output with the bias, and the
+    normalisation's are called, as in an evaluation with gradients; the transforms reach the normalisation."""
+    from types import SimpleNamespace
+    from torch.autograd import forward_ad
+    from torch.nn.modules.module import register_module_forward_hook
+    from hiscache import HistorySAGE, make_config
+    from hiscache.history_model import bn_relu
+    from hiscache.synthetic import direct_power_law_batch, make_batch
+    N, Fin, H, C, L = 20_000, 64, 64, 8, 3
+    rng = np.random.default_rng(5)
+    smp = direct_power_law_batch(N, 100, [5, 4, 3], 2.0, 9, degree_scale=2.0)
+    torch.manual_seed(6)
+    model = HistorySAGE(Fin, H, C, L, 0.0, "CSR_Layer", make_config(Fin, C, H, L, device=DEV),
+                        SimpleNamespace(method="")).to(DEV).eval()
+    b = make_batch(smp, rng.integers(0, C, size=N), DEV)
+    b.x = torch.from_numpy(rng.standard_normal((len(smp["sub_to_full"]), Fin)).astype(np.float32)).to(DEV)
+
+    def seen(register, grad):
+        out = []
+
+        def hook(module, args, result):
+            out.append((type(module).__name__, (result[0] if isinstance(result, tuple) else result).detach().clone()))
+        handles = register(hook)
+        try:
+            with torch.set_grad_enabled(grad):
+                model(b)
+        finally:
+            for h in handles:
+                h.remove()
+        return out
+
+    for register in (lambda hook: [conv.register_forward_hook(hook) for conv in model.convs],
+                     lambda hook: [register_module_forward_hook(hook)]):
+        watched, want = seen(register, False), seen(register, True)
+        assert [name for name, _ in watched] == [name for name, _ in want] and len(want) >= L
+        for (name, got), (_, ref) in zip(watched, want):
+            assert torch.allclose(got, ref, rtol=1e-5, atol=1e-5), name
+    bn = model.bns[0]
+    with torch.no_grad():
+        x = torch.randn(6, 10, H, device=DEV)
+        want = torch.stack([F.relu(bn(v)) for v in x])
+        assert torch.allclose(torch.vmap(lambda v: bn_relu(v, bn))(x), want, rtol=1e-5, atol=1e-5)
+        with forward_ad.dual_level():
+            y = bn_relu(forward_ad.make_dual(x[0], torch.ones_like(x[0])), bn)
+            assert forward_ad.unpack_dual(y).tangent is not None
