@@ -83,11 +83,14 @@ __device__ __forceinline__ int64_t bwd_run_of(const BwdArgs &a, int64_t s) {
   return (a.ptrT[s] + (int64_t)BWD_SRC_COST * s) / BWD_UNIT;
 }
 
-// v / d rounded once, from r = 1 / d rounded once: the quotient's residual is exact in a fused multiply-add, and
-// adding residual * r rounds to the quotient (Markstein, IBM J. Res. Dev. 34, 1990; a whole divisor below 2^22
-// keeps quotients further from the rounding boundaries than the residual's error).  The fix-up passes infinities,
-// NaN and signed zeros on as a division does.  Five instructions shorter than the division, which took more
-// issue slots of a row than its loads.
+// v / d from r = 1 / d rounded once: the quotient's residual is exact in a fused multiply-add, and adding
+// residual * r rounds to the quotient (Markstein, IBM J. Res. Dev. 34, 1990).  These are the division's bits where the
+// quotient is normal and the whole divisor is below 2^22: such a quotient lies further from the rounding boundaries
+// than the residual's error reaches.  A subnormal quotient that is an exact tie may become either of its two nearest
+// neighbours (9 * 2^-149 / 6 the odd one), and above 2^22 one that close to a tie may; the error is no larger than a
+// division's.  The fix-up passes infinities, NaN and signed zeros on as a division does.  Five instructions shorter
+// than the division, which took more issue slots of a row than its loads.  (Looking every quotient over, to divide
+// where it is subnormal: 14 M edges x 64 1.33 -> 1.39 ms, slices of a long source 104 -> 120 us.)
 __device__ __forceinline__ float bwd_div(float v, float d, float r) {
   const float q = __fmul_rn(v, r);
   return __builtin_amdgcn_div_fixupf(__fmaf_rn(__fmaf_rn(-q, d, v), r, q), d, v);

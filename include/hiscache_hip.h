@@ -206,7 +206,10 @@ int hc_build_transpose_dev_deg(const int64_t *ptr, const int64_t *idx, const int
  * compute units; with hc_aggr_bwd_workspace_bytes_for() bytes, which counts
  * the sources too, the sources are moreover dealt to the waves by their edges
  * (same results).  Both report 0 where a call needs none.  A view of more than
- * E_total entries is summed as without a workspace. */
+ * E_total entries is summed as without a workspace.
+ * g[r,h,:]/deg(r) is the correctly rounded quotient, except that a subnormal
+ * quotient half way between two numbers may become either of them (and one
+ * within 2^-23 of half way, for a degree of 2^22 or more). */
 size_t hc_aggr_bwd_workspace_bytes(int64_t E_total, int64_t F);
 size_t hc_aggr_bwd_workspace_bytes_for(int64_t E_total, int64_t F, int64_t n_src);
 int64_t hc_aggr_bwd_chunk_edges(int64_t F);

@@ -201,3 +201,25 @@ def test_view_of_more_entries_than_announced(be, orc, F, runs, announced):
         assert rc == 0
         np.testing.assert_array_equal(out.cpu().numpy(), want)
         assert (ws[need:] == 0x5a).all()
+
+
+@pytest.mark.parametrize("F", [64, 100])
+def test_underflowing_gradient(be, orc, F):
+    """Gradients around and below the smallest normal number.  A subnormal quotient is one of the two numbers next to
+    the exact one, and sums of subnormals are exact: a source of n edges lies within n * 2^-149 of the divisions' sum.
+    Above, the quotients are the divisions' and the sums have the same bits."""
+    rng = np.random.default_rng(14)
+    R, N = 3000, 900
+    ptr, idx = block(rng, R, N)
+    count = np.bincount(idx, minlength=N)[:, None]
+    tr = be.build_transpose(T(ptr), T(idx), None, R, N, want_edges=False)
+    longest = int(np.diff(ptr).max())
+    for low, high in ((0, 40), (0, 1 << 13), (longest << 23, longest << 25)):      # in units of 2^-149
+        g = np.ldexp(rng.integers(low, high, size=(R, F)).astype(np.float32), -149)
+        gx, _, _ = be._aggr_bwd(T(ptr), T(idx), tr, T(g), None, None, None, False, None, 0, R, N)
+        ref, _ = orc.bwd_mean_row(ptr, idx, g, None, N, chunk=be.bwd_chunk_edges(F))
+        if low == 0:
+            assert np.abs(ref).max() < 2.0 ** -125              # (up to there the sums are exact)
+            assert (np.abs(gx.cpu().numpy().astype(np.float64) - ref) <= count * 2.0 ** -149).all()
+        else:
+            np.testing.assert_array_equal(gx.cpu().numpy(), ref)
