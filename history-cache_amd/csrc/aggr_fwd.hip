@@ -37,6 +37,11 @@ __global__ __launch_bounds__(HC_BLOCK) void fwd_find_long(FwdArgs a) {
   }
   __syncthreads();
   if (threadIdx.x == 0) {
+    if (blockIdx.x == 0) {
+      a.plan->far_above = far_above;
+      a.plan->listed = total / (far_above + 1) <= a.far.cap &&
+                       (a.split_above == 0 || total / (a.slice_above + 1) <= a.near.cap) ? 1 : 0;
+    }
     a.near.count[blockIdx.x] = n_near;
     a.far.count[blockIdx.x] = n_far;
   }
@@ -54,10 +59,11 @@ struct FwdScratch {
   size_t bytes;
 };
 
-// Workspace of a forward launch: the two lists (their counts, then their entries: a third of the room for
+// Workspace of a forward launch: the two lists (their counts and the plan, then their entries: a third of the room for
 // whole rows, two thirds for sliced ones), then one bit per source (per-source substitution over many
 // sources).  Either part may be absent (0 bytes).
 constexpr size_t FWD_COUNT_BYTES = 2 * SEG_MAX_REGIONS * sizeof(int32_t);
+constexpr size_t FWD_HEAD_BYTES = FWD_COUNT_BYTES + 256;
 struct FwdWsLayout {
   size_t list_bytes, bits_bytes, total;
 };
@@ -65,7 +71,7 @@ FwdWsLayout fwd_ws_layout(int mode, int64_t R, int64_t E, int64_t n_src) {
   FwdWsLayout L{0, 0, 0};
   if (E > FWD_HEAD_SLICE_EDGES && !(R <= FWD_SELF_ROWS && E <= FWD_SELF_EDGES)) {
     const int64_t near = E / (HC_LONG_ROW_EDGES + 1) + 1;
-    L.list_bytes = hc_align_up(FWD_COUNT_BYTES + (size_t)(3 * near + 3) * sizeof(int32_t), 256);
+    L.list_bytes = hc_align_up(FWD_HEAD_BYTES + (size_t)(3 * near + 3) * sizeof(int32_t), 256);
   }
   if (mode == HC_SUBST_SRC && n_src >= FWD_BITS_MIN_SRC) L.bits_bytes = hc_align_up((size_t)((n_src + 63) / 64) * 8, 256);
   L.total = L.list_bytes + L.bits_bytes;
@@ -106,13 +112,14 @@ int fwd_prepare_lists(FwdArgs &a, bool src_mode, FwdScratch ws, int64_t n_src, i
     return HC_OK;
   }
   if (a.R > 0x7fffffffLL) return HC_OK;
-  if (room > FWD_COUNT_BYTES + 3 * sizeof(int32_t)) {
+  if (room > FWD_HEAD_BYTES + 3 * sizeof(int32_t)) {
     a.tile = seg_tile(a.R);
     a.n_tiles = (int)((a.R + a.tile - 1) / a.tile);
-    const int64_t items = (int64_t)((room - FWD_COUNT_BYTES) / sizeof(int32_t));
+    const int64_t items = (int64_t)((room - FWD_HEAD_BYTES) / sizeof(int32_t));
     a.near.count = static_cast<int32_t *>(ws.ptr);
     a.far.count = a.near.count + SEG_MAX_REGIONS;
-    a.near.item = a.far.count + SEG_MAX_REGIONS;
+    a.plan = reinterpret_cast<FwdPlan *>(static_cast<char *>(ws.ptr) + FWD_COUNT_BYTES);
+    a.near.item = reinterpret_cast<int32_t *>(static_cast<char *>(ws.ptr) + FWD_HEAD_BYTES);
     a.near.cap = items / 3;
     a.far.item = a.near.item + a.near.cap;
     a.far.cap = items - a.near.cap;

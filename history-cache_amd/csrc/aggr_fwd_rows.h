@@ -69,6 +69,12 @@ __device__ __forceinline__ void copy_row_any(const void *hbuf, int hist_dtype, i
 // elements of a chunk lie inside one head, whose weight the lane loads itself.
 constexpr int W_NONE = 0, W_EDGE = 1, W_EDGE_HEAD = 2;
 
+// What the main launch does with the lists.  (Worked out by each of its waves, with two 64-bit divisions, it took 1 M
+// rows of 3 edges of 64 columns from 443 to 526 us.)
+struct FwdPlan {
+  int64_t far_above, listed;
+};
+
 struct FwdArgs {
   const int64_t *ptr, *idx;
   const void *vin;
@@ -88,6 +94,7 @@ struct FwdArgs {
   SegList near, far;          // whole-row and slice-wise tasks of the front blocks
   int n_tiles;                // tiles of the lists; 0: every front block looks the rows through itself
   int64_t tile;
+  FwdPlan *plan;              // with lists: written by the launch that makes them
   int front;                  // blocks at the start of the grid that work through the lists
 };
 
@@ -153,6 +160,9 @@ struct FwdCols {
   }
 };
 
+template <int N>
+using FwdInt = std::integral_constant<int, N>;
+
 // Sum of the neighbour rows of edges [begin, end), added to acc in edge order by the calling wave.
 // SRC (per-source substitution): neighbour rows and ids are loaded with the non-temporal hint.  Every edge
 // also looks its source up in the map, and the map (not the rows, which are too many to be reused) is what
@@ -172,15 +182,22 @@ __device__ __forceinline__ void fwd_accumulate(const FwdArgs &a, const FwdCols<V
       my_addr = fwd_row_address<T, TH, SRC>(a, id);
       if constexpr (WMODE == W_EDGE) my_w = a.ev[base + lane];
     }
-    for (int j = 0; j < n; j += UNROLL) {
-      typename hc_piece<T, VEC>::raw_t v[UNROLL][CHUNKS];
-      float vm[MIXED ? UNROLL : 1][CHUNKS][VEC];
-      float wh[WMODE == W_EDGE_HEAD ? UNROLL : 1][CHUNKS];
+    const auto add = [&](const auto &x, float w1, const float (&wh)[CHUNKS]) {
 #pragma unroll
-      for (int u = 0; u < UNROLL; ++u) {
-        if (j + u < n) {
-          const int64_t p = hc_readlane64(my_addr, j + u);
-          if constexpr (MIXED) {
+      for (int k = 0; k < CHUNKS; ++k)
+#pragma unroll
+        for (int i = 0; i < VEC; ++i) {
+          if constexpr (WMODE == W_NONE) acc[k][i] += x(k, i);
+          else acc[k][i] = __fmaf_rn(x(k, i), WMODE == W_EDGE_HEAD ? wh[k] : w1, acc[k][i]);
+        }
+    };
+    if constexpr (MIXED) {
+      for (int j = 0; j < n; j += UNROLL) {
+        float vm[UNROLL][CHUNKS][VEC];
+#pragma unroll
+        for (int u = 0; u < UNROLL; ++u) {
+          if (j + u < n) {
+            const int64_t p = hc_readlane64(my_addr, j + u);
             if ((p & 1) != 0) {      // a row of the history table, in its own element type
               typename hc_piece<TH, VEC>::raw_t h[CHUNKS];
 #pragma unroll
@@ -190,37 +207,74 @@ __device__ __forceinline__ void fwd_accumulate(const FwdArgs &a, const FwdCols<V
 #pragma unroll
                 for (int i = 0; i < VEC; ++i) vm[u][k][i] = hc_piece<TH, VEC>::widen(h[k], i);
             } else {
+              typename hc_piece<T, VEC>::raw_t v[CHUNKS];
 #pragma unroll
-              for (int k = 0; k < CHUNKS; ++k) v[0][k] = hc_piece<T, VEC>::template load<true>(p, col.off[k] * (uint32_t)sizeof(T));
+              for (int k = 0; k < CHUNKS; ++k) v[k] = hc_piece<T, VEC>::template load<true>(p, col.off[k] * (uint32_t)sizeof(T));
 #pragma unroll
               for (int k = 0; k < CHUNKS; ++k)
 #pragma unroll
-                for (int i = 0; i < VEC; ++i) vm[u][k][i] = hc_piece<T, VEC>::widen(v[0][k], i);
-            }
-          } else {
-#pragma unroll
-            for (int k = 0; k < CHUNKS; ++k) {
-              v[u][k] = hc_piece<T, VEC>::template load<SRC>(p, col.off[k] * (uint32_t)sizeof(T));
-              if constexpr (WMODE == W_EDGE_HEAD) wh[u][k] = a.ev[(base + j + u) * a.n_head + col.hd[k]];
+                for (int i = 0; i < VEC; ++i) vm[u][k][i] = hc_piece<T, VEC>::widen(v[k], i);
             }
           }
         }
+#pragma unroll
+        for (int u = 0; u < UNROLL; ++u)
+          if (j + u < n) add([&](int k, int i) { return vm[u][k][i]; }, 0.0f, {});
       }
+    } else {
+      typename hc_piece<T, VEC>::raw_t v[UNROLL][CHUNKS];
+      float wh[WMODE == W_EDGE_HEAD ? UNROLL : 1][CHUNKS];
+      // COUNT rows from place `at` of the stage into slots SLOT ... ; loads first, then the adds in order
+      const auto load = [&](auto slot, auto count, int at) {
 #pragma unroll
-      for (int u = 0; u < UNROLL; ++u) {
-        if (j + u < n) {
-          const float w1 = WMODE == W_EDGE ? hc_readlane_f(my_w, j + u) : 0.0f;
+        for (int k = 0; k < CHUNKS; ++k) {
+          uint32_t byte = col.off[k] * (uint32_t)sizeof(T);
+          asm("" : "+v"(byte));      // seen as 32 bits beside the loads, which then take the row's address from scalar registers
 #pragma unroll
-          for (int k = 0; k < CHUNKS; ++k)
-#pragma unroll
-            for (int i = 0; i < VEC; ++i) {
-              float x;
-              if constexpr (MIXED) x = vm[u][k][i];
-              else x = hc_piece<T, VEC>::widen(v[u][k], i);
-              if constexpr (WMODE == W_NONE) acc[k][i] += x;
-              else acc[k][i] = __fmaf_rn(x, WMODE == W_EDGE_HEAD ? wh[u][k] : w1, acc[k][i]);
-            }
+          for (int u = 0; u < count.value; ++u)
+            v[slot.value + u][k] = hc_piece<T, VEC>::template load<SRC>(hc_readlane64(my_addr, at + u), byte);
         }
+        if constexpr (WMODE == W_EDGE_HEAD) {
+#pragma unroll
+          for (int u = 0; u < count.value; ++u)
+#pragma unroll
+            for (int k = 0; k < CHUNKS; ++k) wh[slot.value + u][k] = a.ev[(base + at + u) * a.n_head + col.hd[k]];
+        }
+      };
+      const auto sum = [&](auto slot, auto count, int at) {
+#pragma unroll
+        for (int u = 0; u < count.value; ++u) {
+          const float w1 = WMODE == W_EDGE ? hc_readlane_f(my_w, at + u) : 0.0f;
+          add([&](int k, int i) { return hc_piece<T, VEC>::widen(v[slot.value + u][k], i); }, w1,
+              wh[WMODE == W_EDGE_HEAD ? slot.value + u : 0]);
+        }
+      };
+      int j = 0;
+      for (; j + UNROLL <= n; j += UNROLL) {
+        load(FwdInt<0>(), FwdInt<UNROLL>(), j);
+        sum(FwdInt<0>(), FwdInt<UNROLL>(), j);
+      }
+      // the rest in parts of 8, 4, 2 and 1, all of their loads first.  (Asking of every row of a batch whether it is
+      // there took five scalar instructions a row: 1 M rows of 3 edges of 64 columns 443 us instead of 336.)
+      const int rest = n - j;
+      if (rest > 0) {
+        const int j4 = j + (rest & 8), j2 = j4 + (rest & 4), j1 = j2 + (rest & 2);
+        constexpr FwdInt<0> s8;
+        constexpr FwdInt<UNROLL - 8> s4;      // slots behind the larger parts'
+        constexpr FwdInt<UNROLL - 4> s2;
+        constexpr FwdInt<UNROLL - 2> s1;
+        if constexpr (UNROLL > 8)
+          if ((rest & 8) != 0) load(s8, FwdInt<8>(), j);
+        if constexpr (UNROLL > 4)
+          if ((rest & 4) != 0) load(s4, FwdInt<4>(), j4);
+        if ((rest & 2) != 0) load(s2, FwdInt<2>(), j2);
+        if ((rest & 1) != 0) load(s1, FwdInt<1>(), j1);
+        if constexpr (UNROLL > 8)
+          if ((rest & 8) != 0) sum(s8, FwdInt<8>(), j);
+        if constexpr (UNROLL > 4)
+          if ((rest & 4) != 0) sum(s4, FwdInt<4>(), j4);
+        if ((rest & 2) != 0) sum(s2, FwdInt<2>(), j2);
+        if ((rest & 1) != 0) sum(s1, FwdInt<1>(), j1);
       }
     }
   }
@@ -544,7 +598,9 @@ __device__ __forceinline__ void fwd_front(const FwdArgs &a, int64_t far_above, i
 // SIMD (11 M edges x 128 in one launch 2.55 ms, in two 1.96 ms).
 constexpr int FWD_ALL = 0, FWD_FRONT = 1, FWD_BODY = 2;
 template <typename T, typename TH, int VEC, int CHUNKS, int UNROLL, bool SRC, int WMODE, int PART>
-__global__ __launch_bounds__(HC_BLOCK) void fwd_rows(FwdArgs a) {
+// At most 80 scalar registers: above, fewer waves of short rows fit the chip.  (The slices would take 106, and with them
+// 1 M rows of 3 edges of 64 columns 433 us instead of 388, 700 k rows of 20 edges 664 instead of 638.)
+__global__ __launch_bounds__(HC_BLOCK) __attribute__((amdgpu_num_sgpr(80))) void fwd_rows(FwdArgs a) {
   // without heads the rows may be split: the split code is compiled for those modes only
   constexpr int LMODE = WMODE == W_EDGE_HEAD ? W_EDGE : WMODE;
   __shared__ float part[HC_WAVES_PER_BLOCK - 1][HC_WAVE * VEC * CHUNKS];
@@ -553,17 +609,18 @@ __global__ __launch_bounds__(HC_BLOCK) void fwd_rows(FwdArgs a) {
   __shared__ int n_long_s;
   const int lane = hc_lane();
   const int wave = hc_wave_in_block();
-  // every thread of the grid reads the same two words, so the decision is uniform: the lists hold every long row
+  // every thread of the grid reads the same words, so the decision is uniform: the lists hold every long row
   int64_t far_above = 0;
   bool listed = false;
   if (a.front > 0) {
-    const int64_t total = a.ptr[a.R] - a.ptr[0];
-    far_above = fwd_far_above(a, total);
-    if (a.n_tiles > 0)
-      listed = total / (far_above + 1) <= a.far.cap &&
-               (a.split_above == 0 || total / (a.slice_above + 1) <= a.near.cap);
-    else
-      listed = total / (far_above + 1) <= FWD_SELF_ITEMS && far_above == a.slice_above;
+    if (a.n_tiles > 0) {
+      far_above = a.plan->far_above;
+      listed = a.plan->listed != 0;
+    } else {
+      const int64_t total = a.ptr[a.R] - a.ptr[0];
+      far_above = fwd_far_above(a, total);
+      listed = total < (FWD_SELF_ITEMS + 1) * (far_above + 1) && far_above == a.slice_above;
+    }
     if constexpr (PART != FWD_BODY) {
       if ((int)blockIdx.x < a.front) {
         if (listed)

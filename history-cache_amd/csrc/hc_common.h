@@ -82,11 +82,10 @@ __device__ __forceinline__ float hc_readlane_f(float v, int lane) {
 #define HC_NUM_XCD 8
 template <int CHUNK>
 __device__ __forceinline__ int64_t hc_xcd_block(int64_t bid, int64_t n) {
-  constexpr int64_t GROUP = (int64_t)HC_NUM_XCD * CHUNK;
-  const int64_t g = bid / GROUP;
-  if ((g + 1) * GROUP > n) return bid;
-  const int64_t in = bid - g * GROUP;
-  return g * GROUP + (in % HC_NUM_XCD) * CHUNK + in / HC_NUM_XCD;
+  constexpr uint32_t GROUP = (uint32_t)HC_NUM_XCD * CHUNK;       // a power of two; a grid has less than 2^24 blocks
+  const uint32_t b = (uint32_t)bid, in = b % GROUP, first = b - in;
+  if (first + GROUP > (uint32_t)n) return bid;
+  return first + (in % HC_NUM_XCD) * CHUNK + in / HC_NUM_XCD;
 }
 
 // Butterfly sum over the 64 lanes, partner distance 32,16,8,4,2,1.  Every lane

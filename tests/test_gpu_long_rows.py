@@ -137,3 +137,28 @@ def test_unaligned_rows(be, orc):
         out = be._aggr_fwd(be.SUBST_ROW, T(ptr), T(idx), x, None, None, 0, None, R)
         ref = orc.fwd_mean_row(ptr, idx, x.float().cpu().numpy(), None, None, split_above=256)
         np.testing.assert_array_equal(out.cpu().numpy(), ref)
+
+
+@pytest.mark.parametrize("F,dtype", [(64, torch.float32), (128, torch.float32), (256, torch.float32), (1024, torch.float32),
+                                     (512, torch.bfloat16), (47, torch.float16)])
+def test_rows_of_every_short_length(be, orc, F, dtype):
+    """0 to 70 edges: every remainder of a batch of 16, 8 and 4 rows in flight, plain and weighted, a head and two."""
+    rng = np.random.default_rng(F)
+    N = 300
+    deg = rng.permutation(np.repeat(np.arange(71), 3))
+    ptr = np.concatenate([[0], np.cumsum(deg)]).astype(np.int64)
+    R, E = len(deg), int(ptr[-1])
+    idx = rng.integers(0, N, size=E, dtype=np.int64)
+    x = T(rng.standard_normal((N, F)).astype(np.float32), dtype)
+    x32 = x.float().cpu().numpy()
+    out = be._aggr_fwd(be.SUBST_ROW, T(ptr), T(idx), x, None, None, 0, None, R)
+    np.testing.assert_array_equal(out.cpu().numpy(), orc.fwd_mean_row(ptr, idx, x32, None, None))
+    hist = T(rng.standard_normal((40, F)).astype(np.float32), dtype)
+    hmap = np.where(rng.random(N) < 0.4, rng.integers(0, 40, size=N), -1).astype(np.int64)
+    out = be.aggr_forward_source_history(x, T(ptr), T(idx), T(hmap), hist)
+    np.testing.assert_array_equal(out.cpu().numpy(), orc.fwd_mean_src(ptr, idx, x32, hmap, hist.float().cpu().numpy()))
+    for H in ((1,) if F % 2 else (1, 2)):
+        ev = rng.standard_normal((E, H) if H > 1 else (E,)).astype(np.float32)
+        shape = (N, H, F // H) if H > 1 else (N, F)
+        out = be._aggr_fwd(be.SUBST_ROW, T(ptr), T(idx), x.view(shape), None, None, 0, T(ev), R)
+        np.testing.assert_array_equal(out.cpu().numpy(), orc.fwd_edge_value(ptr, idx, ev, x32.reshape(shape), None, None))
