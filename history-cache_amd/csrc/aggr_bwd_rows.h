@@ -25,6 +25,8 @@
 //   * sources of more than BWD_LONG edges are listed by the same launch and summed by the front blocks of the
 //     main one, a cache line's columns at a time (seg_list.h): 32 loads of one line in flight instead of eight
 //     of whole rows, and one source on several compute units.
+// Of a shared view's long sources the front blocks visit the live edges only (BwdLive): a layer of 50 rows over a view
+// with sources of 10 000 edges takes 24 us (101 when every dead edge cost a load, 50 before there were lists).
 // Measured on MI355X, before (fixed runs of 32 sources; widths off a multiple of 64 element by element; the
 // conversion of a half-precision gradient as a pass of its own) and after, lists included: 3 M edges x 256 to
 // 1 M bf16 sources 2.37 -> 0.38 ms, 1 M edges x 4 heads of 32 to 200 k sources 0.95 -> 0.08 ms, 600 k edges x 100
@@ -106,7 +108,7 @@ struct BwdEdge {
   int edge;     // W_EDGE_HEAD: the edge's slot
 };
 template <int WMODE, bool MASKED>
-__device__ __forceinline__ BwdEdge bwd_edge(const BwdArgs &a, int64_t pos, int row, int64_t ev_stride, int head) {
+__device__ __forceinline__ BwdEdge bwd_edge(const BwdArgs &a, int64_t pos, int row) {
   BwdEdge e{row, 1.0f, 1.0f, 0};
   if constexpr (MASKED) {
     if (row >= a.R || row < 0) e.row = -1;
@@ -115,7 +117,7 @@ __device__ __forceinline__ BwdEdge bwd_edge(const BwdArgs &a, int64_t pos, int r
   if constexpr (WMODE == W_EDGE_HEAD) {
     e.edge = a.edgeT[pos];
   } else if constexpr (WMODE == W_EDGE) {
-    e.d = a.ev[a.edgeT[pos] * ev_stride + head];
+    e.d = a.ev[a.edgeT[pos]];
   } else if (!MASKED || e.row >= 0) {
     e.d = (float)(int)(a.ptr[e.row + 1] - a.ptr[e.row]);
     if (MASKED && e.d == 0.0f) {
@@ -145,11 +147,18 @@ struct BwdCols {
   }
 };
 
+// Element c of a row of g (wave-uniform).
+template <bool BUF>
+__device__ __forceinline__ float bwd_element(const BwdArgs &a, hc_buffer buf, uint32_t row_bytes, int row, uint32_t c) {
+  if constexpr (BUF) return __uint_as_float(hc_buffer_load<uint32_t>(buf, c * 4u, (uint32_t)row * row_bytes));
+  else return __uint_as_float(hc_piece<float, 1>::template load<false>(reinterpret_cast<int64_t>(a.g + (int64_t)row * a.F), c * 4u));
+}
+
 // One column per lane of transposed edges [begin, end), added in edge order, D to 2 D gradient rows in flight:
 // the loads of a group of D rows are issued before the adds of the group in front of it, the rows of the next 64
 // edges at the start of this stage and their degrees or weights behind its first group.
 // BUF: g is smaller than 4 GiB and its rows are addressed by 32-bit offsets from scalar registers.
-template <int WMODE, bool MASKED, bool BUF>
+template <int WMODE, bool BUF>
 __device__ __forceinline__ float bwd_slice_sum(const BwdArgs &a, uint32_t c, int64_t begin, int64_t end, int lane) {
   constexpr int D = 16;
   constexpr int G = HC_WAVE / D;
@@ -165,26 +174,18 @@ __device__ __forceinline__ float bwd_slice_sum(const BwdArgs &a, uint32_t c, int
     for (int u = 0; u < D; ++u) {
       int j = g * D + u;
       j = j < last ? j : last;                               // behind the end: the last row again, not added
-      int row = __builtin_amdgcn_readlane(e.row, j);
-      if constexpr (MASKED) row = row < 0 ? 0 : row;         // stepped over: some row, not added
-      if constexpr (BUF) x[h][u] = __uint_as_float(hc_buffer_load<uint32_t>(buf, c * 4u, (uint32_t)row * row_bytes));
-      else x[h][u] = __uint_as_float(hc_piece<float, 1>::template load<false>(reinterpret_cast<int64_t>(a.g + (int64_t)row * a.F), c * 4u));
+      const int row = __builtin_amdgcn_readlane(e.row, j);
+      x[h][u] = bwd_element<BUF>(a, buf, row_bytes, row, c);
       if constexpr (WMODE == W_EDGE_HEAD) w[h][u] = a.ev[(int64_t)__builtin_amdgcn_readlane(e.edge, j) * a.n_head + hd];
     }
   };
   const auto add1 = [&](int h, int u, const BwdEdge &e, int j) {
-    if constexpr (WMODE == W_EDGE_HEAD) {
-      acc += __fmul_rn(x[h][u], w[h][u]);
-    } else if constexpr (WMODE == W_EDGE) {
-      acc += __fmul_rn(x[h][u], hc_readlane_f(e.d, j));
-    } else {
-      const float q = bwd_div(x[h][u], hc_readlane_f(e.d, j), hc_readlane_f(e.r, j));
-      if constexpr (MASKED) acc += __builtin_amdgcn_readlane(e.row, j) < 0 ? 0.0f : q;   // acc is never -0
-      else acc += q;
-    }
+    if constexpr (WMODE == W_EDGE_HEAD) acc += __fmul_rn(x[h][u], w[h][u]);
+    else if constexpr (WMODE == W_EDGE) acc += __fmul_rn(x[h][u], hc_readlane_f(e.d, j));
+    else acc += bwd_div(x[h][u], hc_readlane_f(e.d, j), hc_readlane_f(e.r, j));
   };
   int64_t p = begin + lane < end ? begin + lane : end - 1;
-  BwdEdge cur = bwd_edge<WMODE, MASKED>(a, p, a.rowT[p], 1, 0);
+  BwdEdge cur = bwd_edge<WMODE, false>(a, p, a.rowT[p]);
   int last = end - begin < HC_WAVE ? (int)(end - begin) - 1 : HC_WAVE - 1;
   load(0, cur, 0, last);
   int64_t base = begin;
@@ -206,7 +207,7 @@ __device__ __forceinline__ float bwd_slice_sum(const BwdArgs &a, uint32_t c, int
 #pragma unroll
       for (int u = 0; u < D; ++u) add1(g & 1, u, cur, g * D + u);
       __builtin_amdgcn_sched_barrier(0);
-      if (g == 0) ahead = bwd_edge<WMODE, MASKED>(a, p, next_row, 1, 0);
+      if (g == 0) ahead = bwd_edge<WMODE, false>(a, p, next_row);
     }
     cur = ahead;
   }
@@ -221,10 +222,124 @@ __device__ __forceinline__ float bwd_slice_sum(const BwdArgs &a, uint32_t c, int
   return acc;
 }
 
+// The live edges of a stretch of a shared view, put together 64 at a time: BWD_WINDOWS windows of 64 positions are
+// looked at together and the rows that are live go to a ring in the LDS.
+constexpr int BWD_WINDOWS = 4, BWD_RING = 512;       // a ring holds what is left of a stage and all of the windows
+struct BwdLive {
+  int *ring;
+  int64_t pos, end;                                  // next position to be looked at
+  int head, count;
+  int next[BWD_WINDOWS];                             // the rows from `pos` on, on their way
+  __device__ __forceinline__ BwdLive(const BwdArgs &a, int *ring_, int64_t begin, int64_t end_, int lane)
+      : ring(ring_), pos(begin), end(end_), head(0), count(0) {
+    fetch(a, lane);
+  }
+  __device__ __forceinline__ void fetch(const BwdArgs &a, int lane) {
+#pragma unroll
+    for (int w = 0; w < BWD_WINDOWS; ++w) {
+      const int64_t p = pos + w * HC_WAVE + lane;
+      next[w] = a.rowT[p < end ? p : end - 1];
+    }
+  }
+  // The next up to 64 live edges, in order; their number.  Lanes behind them hold the last one again.
+  __device__ __forceinline__ int take(const BwdArgs &a, int lane, BwdEdge &e) {
+    const unsigned long long below = (1ull << lane) - 1ull;
+    while (count < HC_WAVE && pos < end) {           // wave-uniform
+      int row[BWD_WINDOWS];
+      bool live[BWD_WINDOWS];
+      int64_t slot[BWD_WINDOWS];
+#pragma unroll
+      for (int w = 0; w < BWD_WINDOWS; ++w) {
+        row[w] = next[w];
+        live[w] = pos + w * HC_WAVE + lane < end && row[w] >= 0 && row[w] < a.R;
+      }
+      pos += BWD_WINDOWS * HC_WAVE;
+      fetch(a, lane);
+#pragma unroll
+      for (int w = 0; w < BWD_WINDOWS; ++w) slot[w] = live[w] && a.hmap != nullptr ? a.hmap[row[w]] : -1;
+#pragma unroll
+      for (int w = 0; w < BWD_WINDOWS; ++w) {
+        live[w] = live[w] && slot[w] == -1;
+        const unsigned long long b = __ballot(live[w]);
+        if (live[w]) ring[(head + count + __popcll(b & below)) % BWD_RING] = row[w];
+        count += __popcll(b);
+      }
+    }
+    const int n = count < HC_WAVE ? count : HC_WAVE;
+    if (n == 0) return 0;
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");     // (the LDS serves a wave in order)
+    e = BwdEdge{ring[(head + (lane < n ? lane : n - 1)) % BWD_RING], 1.0f, 1.0f, 0};
+    head = (head + n) % BWD_RING;
+    count -= n;
+    e.d = (float)(int)(a.ptr[e.row + 1] - a.ptr[e.row]);
+    if (e.d == 0.0f) {
+      e.row = -1;
+      e.d = 1.0f;
+    }
+    e.r = 1.0f / e.d;
+    return n;
+  }
+};
+
+// bwd_slice_sum of the mean over the live edges of a shared view.
+template <bool BUF>
+__device__ __forceinline__ float bwd_live_sum(const BwdArgs &a, uint32_t c, int64_t begin, int64_t end, int lane, int *ring) {
+  constexpr int D = 16;
+  constexpr int G = HC_WAVE / D;
+  float acc = 0.0f;
+  if (begin >= end) return acc;
+  const hc_buffer buf = hc_make_buffer(a.g);
+  const uint32_t row_bytes = (uint32_t)a.F * 4u;
+  float x[2][D];
+  const auto load = [&](int h, const BwdEdge &e, int g, int last) {
+#pragma unroll
+    for (int u = 0; u < D; ++u) {
+      int j = g * D + u;
+      j = j < last ? j : last;                               // behind the end: the last row again, not added
+      const int row = __builtin_amdgcn_readlane(e.row, j);
+      x[h][u] = bwd_element<BUF>(a, buf, row_bytes, row < 0 ? 0 : row, c);       // without edges of its own: not added
+    }
+  };
+  const auto add1 = [&](int h, int u, const BwdEdge &e, int j) {
+    const float q = bwd_div(x[h][u], hc_readlane_f(e.d, j), hc_readlane_f(e.r, j));
+    acc += __builtin_amdgcn_readlane(e.row, j) < 0 ? 0.0f : q;                   // acc is never -0
+  };
+  BwdLive live(a, ring, begin, end, lane);
+  BwdEdge cur{0, 1.0f, 1.0f, 0};
+  int n = live.take(a, lane, cur);
+  if (n > 0) load(0, cur, 0, n - 1);
+  while (n == HC_WAVE) {
+    BwdEdge ahead = cur;
+    int m = 0;
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+      if (g + 1 < G) load((g + 1) & 1, cur, g + 1, HC_WAVE - 1);
+      else load(0, ahead, 0, m > 0 ? m - 1 : 0);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int u = 0; u < D; ++u) add1(g & 1, u, cur, g * D + u);
+      __builtin_amdgcn_sched_barrier(0);
+      if (g == 0) m = live.take(a, lane, ahead);
+    }
+    cur = ahead;
+    n = m;
+  }
+  for (int g = 0; g * D < n; ++g) {
+    if (g > 0) load(0, cur, g, n - 1);
+#pragma unroll
+    for (int u = 0; u < D; ++u)
+      if (g * D + u < n) add1(0, u, cur, g * D + u);
+  }
+  return acc;
+}
+
 template <int WMODE, bool MASKED>
-__device__ __forceinline__ float bwd_slice_any(const BwdArgs &a, uint32_t c, int64_t begin, int64_t end, int lane) {
-  return a.small_matrix ? bwd_slice_sum<WMODE, MASKED, true>(a, c, begin, end, lane)
-                        : bwd_slice_sum<WMODE, MASKED, false>(a, c, begin, end, lane);
+__device__ __forceinline__ float bwd_slice_any(const BwdArgs &a, uint32_t c, int64_t begin, int64_t end, int lane, int *ring) {
+  if constexpr (MASKED)
+    return a.small_matrix ? bwd_live_sum<true>(a, c, begin, end, lane, ring) : bwd_live_sum<false>(a, c, begin, end, lane, ring);
+  else
+    return a.small_matrix ? bwd_slice_sum<WMODE, true>(a, c, begin, end, lane) : bwd_slice_sum<WMODE, false>(a, c, begin, end, lane);
 }
 
 constexpr int BWD_SLICE = 32;       // columns of a task: one cache line of g
@@ -234,6 +349,8 @@ constexpr int BWD_SLICE = 32;       // columns of a task: one cache line of g
 template <typename TO, int WMODE, bool MASKED>
 __device__ __forceinline__ void bwd_front(const BwdArgs &a, int lane, int wave) {
   __shared__ float part[HC_WAVES_PER_BLOCK][BWD_SLICE];
+  __shared__ int rings[MASKED ? HC_WAVES_PER_BLOCK : 1][MASKED ? BWD_RING : 1];
+  int *ring = rings[MASKED ? wave : 0];
   const int ns = (int)((a.F + BWD_SLICE - 1) / BWD_SLICE);
   const auto source = [&](const SegList &list, const SegIndex &index, int64_t above, int e) -> int64_t {
     int t, w;
@@ -267,7 +384,7 @@ __device__ __forceinline__ void bwd_front(const BwdArgs &a, int lane, int wave) 
              k += HC_WAVES_PER_BLOCK) {
           const int64_t mb = b + k * BWD_CHUNK;
           if (mb >= e) break;
-          const float v = bwd_slice_any<W_NONE, MASKED>(a, c, mb, mb + BWD_CHUNK < e ? mb + BWD_CHUNK : e, lane);
+          const float v = bwd_slice_any<W_NONE, MASKED>(a, c, mb, mb + BWD_CHUNK < e ? mb + BWD_CHUNK : e, lane, ring);
           if (on) row(k)[c] = v;
         }
         if (hc_arrives_last(a.ticket + (int64_t)i * ns + sl, (unsigned)spans, &s_last)) {
@@ -303,7 +420,7 @@ __device__ __forceinline__ void bwd_front(const BwdArgs &a, int lane, int wave) 
       for (int64_t c0 = b; c0 < e; c0 += HC_WAVES_PER_BLOCK * BWD_CHUNK) {     // block-uniform
         const int64_t mb = c0 + wave * BWD_CHUNK < e ? c0 + wave * BWD_CHUNK : e;
         const int64_t me = mb + BWD_CHUNK < e ? mb + BWD_CHUNK : e;
-        const float v = bwd_slice_any<W_NONE, MASKED>(a, c, mb, me, lane);
+        const float v = bwd_slice_any<W_NONE, MASKED>(a, c, mb, me, lane, ring);
         if (lane < BWD_SLICE) part[wave][lane] = v;
         __syncthreads();
         if (wave == 0 && lane < BWD_SLICE) {
@@ -324,7 +441,7 @@ __device__ __forceinline__ void bwd_front(const BwdArgs &a, int lane, int wave) 
     const int64_t s = source(a.mid, index, a.long_above, (int)(t / ns));
     bool on;
     const uint32_t c = column((int)(t % ns), on);
-    const float v = bwd_slice_any<WMODE, MASKED>(a, c, a.ptrT[s], a.ptrT[s + 1], lane);
+    const float v = bwd_slice_any<WMODE, MASKED>(a, c, a.ptrT[s], a.ptrT[s + 1], lane, ring);
     if (on) out[s * a.F + c] = hc_from_f32<TO>(v);
   }
 }
@@ -337,7 +454,7 @@ __device__ __forceinline__ void bwd_front(const BwdArgs &a, int lane, int wave) 
 // TO: element type of grad_vin; the fp32 sums are rounded once when a source is stored.
 // Blocks: front blocks, blocks of source runs, rows of grad_hbuf.
 template <typename TO, int VEC, int CHUNKS, int UNROLL, int WMODE, bool MASKED>
-__global__ __launch_bounds__(HC_BLOCK) void bwd_sources(BwdArgs a) {
+__device__ __forceinline__ void bwd_block(const BwdArgs &a) {
   const int lane = hc_lane();
   const int wave = hc_wave_in_block();
   // every thread of the grid reads the same two words, so the decision is uniform: a view of more entries than its
@@ -433,7 +550,7 @@ __global__ __launch_bounds__(HC_BLOCK) void bwd_sources(BwdArgs a) {
       const int64_t left = stop - base;
       const int n = left < HC_WAVE ? (int)left : HC_WAVE;
       BwdEdge my{-1, 1.0f, 1.0f, 0};
-      if (lane < n) my = bwd_edge<WMODE, MASKED>(a, base + lane, a.rowT[base + lane], 1, 0);
+      if (lane < n) my = bwd_edge<WMODE, MASKED>(a, base + lane, a.rowT[base + lane]);
       // MASKED: only the live edges of the stage are visited (lowest position first), so that UNROLL rows are
       // in flight however many edges of other layers lie between them
       unsigned long long todo = 0ull;
@@ -499,6 +616,16 @@ __global__ __launch_bounds__(HC_BLOCK) void bwd_sources(BwdArgs a) {
   }
 }
 
+template <typename TO, int VEC, int CHUNKS, int UNROLL, int WMODE>
+__global__ __launch_bounds__(HC_BLOCK) void bwd_sources(BwdArgs a) {
+  bwd_block<TO, VEC, CHUNKS, UNROLL, WMODE, false>(a);
+}
+
+template <typename TO, int VEC, int CHUNKS, int UNROLL>
+__global__ __launch_bounds__(HC_BLOCK) void bwd_sources_of_view(BwdArgs a) {
+  bwd_block<TO, VEC, CHUNKS, UNROLL, W_NONE, true>(a);
+}
+
 // One translation unit per element type of grad_vin.
 __attribute__((visibility("hidden"))) int bwd_dispatch_f32(BwdArgs &a, bool masked, hipStream_t st);
 __attribute__((visibility("hidden"))) int bwd_dispatch_f16(BwdArgs &a, bool masked, hipStream_t st);
@@ -514,10 +641,10 @@ int bwd_launch(const BwdArgs &a, bool masked, hipStream_t st) {
   const int64_t blocks = a.front + a.src_blocks + a.hist_blocks;
   if (!hc_grid_ok(blocks)) return HC_EUNSUPPORTED;
   const dim3 grid((unsigned)blocks), block(HC_BLOCK);
-  if (masked) bwd_sources<TO, VEC, CHUNKS, UNROLL, W_NONE, true><<<grid, block, 0, st>>>(a);
-  else if (a.ev != nullptr && a.n_head > 1) bwd_sources<TO, VEC, CHUNKS, UNROLL, W_EDGE_HEAD, false><<<grid, block, 0, st>>>(a);
-  else if (a.ev != nullptr) bwd_sources<TO, VEC, CHUNKS, UNROLL, W_EDGE, false><<<grid, block, 0, st>>>(a);
-  else bwd_sources<TO, VEC, CHUNKS, UNROLL, W_NONE, false><<<grid, block, 0, st>>>(a);
+  if (masked) bwd_sources_of_view<TO, VEC, CHUNKS, UNROLL><<<grid, block, 0, st>>>(a);
+  else if (a.ev != nullptr && a.n_head > 1) bwd_sources<TO, VEC, CHUNKS, UNROLL, W_EDGE_HEAD><<<grid, block, 0, st>>>(a);
+  else if (a.ev != nullptr) bwd_sources<TO, VEC, CHUNKS, UNROLL, W_EDGE><<<grid, block, 0, st>>>(a);
+  else bwd_sources<TO, VEC, CHUNKS, UNROLL, W_NONE><<<grid, block, 0, st>>>(a);
   return hc_launch_status();
 }
 

@@ -462,7 +462,8 @@ def _aggr_bwd_batch_view(ptr, view, g, hmap, hbuf_shape, hsize, num_node, n_src,
         if grad_h.numel() != R * hsize:
             grad_h.zero_()
     # a sampled batch whose popular sources are short enough for one wave does without the extra launch (two
-    # layers of a batch of 1000 seeds: 31 us without, 64 us with the lists)
+    # layers of a batch of 1000 seeds, 256 columns, no source above 412 edges: 35 us without, 52 us with the lists;
+    # of 4000 seeds, one source of 1376: 117 and 99 us)
     short = view.max_in_degree is not None and view.max_in_degree <= MAX_IN_DEGREE_WITHOUT_LISTS
     nbytes = 0 if short else lib.hc_aggr_bwd_workspace_bytes_for(view.num_edge, F, int(n_src))
     ws = _workspace(nbytes, dev) if nbytes else None

@@ -223,3 +223,23 @@ def test_underflowing_gradient(be, orc, F):
             assert (np.abs(gx.cpu().numpy().astype(np.float64) - ref) <= count * 2.0 ** -149).all()
         else:
             np.testing.assert_array_equal(gx.cpu().numpy(), ref)
+
+
+@pytest.mark.parametrize("F", [64, 100, 256])
+@pytest.mark.parametrize("rows", [1, 40, 700, 2999, 3000])
+def test_inner_layer_over_a_view_of_long_sources(be, orc, F, rows):
+    """A layer that owns a few of the view's rows: stretches of hundreds of positions without a live edge, stages put
+    together from several of them, and (all rows) stages taken as they come."""
+    rng = np.random.default_rng(rows + F)
+    R, N = 3000, 900
+    ptr, idx = block(rng, R, N)
+    hmap = np.where(rng.random(rows) < 0.2, 3, -1).astype(np.int64)
+    g = special(rng, rows, F)
+    view = be.build_batch_view(T(ptr), T(idx), R, N)
+    want, _ = orc.bwd_mean_row_batch_view(ptr, idx, g, hmap, N, R, hbuf_shape=(rows, F), chunk=be.bwd_chunk_edges(F))
+    for m in (hmap, None):
+        if m is None:
+            want, _ = orc.bwd_mean_row_batch_view(ptr, idx, g, m, N, R, chunk=be.bwd_chunk_edges(F))
+        gx, _ = be._aggr_bwd_batch_view(T(ptr), view, T(g), None if m is None else T(m), None, 0, rows, N,
+                                        want_hist_grad=False)
+        np.testing.assert_array_equal(gx.cpu().numpy(), want)
