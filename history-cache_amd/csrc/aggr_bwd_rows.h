@@ -616,11 +616,13 @@ __device__ __forceinline__ void bwd_block(const BwdArgs &a) {
   }
 }
 
+// At most 80 scalar registers: above, fewer waves fit the chip (14 M edges x 64 1326 us, 1295 so).
 template <typename TO, int VEC, int CHUNKS, int UNROLL, int WMODE>
-__global__ __launch_bounds__(HC_BLOCK) void bwd_sources(BwdArgs a) {
+__global__ __launch_bounds__(HC_BLOCK) __attribute__((amdgpu_num_sgpr(80))) void bwd_sources(BwdArgs a) {
   bwd_block<TO, VEC, CHUNKS, UNROLL, WMODE, false>(a);
 }
 
+// The vector registers of the live edges' slices leave four waves per SIMD, whatever the scalar ones.
 template <typename TO, int VEC, int CHUNKS, int UNROLL>
 __global__ __launch_bounds__(HC_BLOCK) void bwd_sources_of_view(BwdArgs a) {
   bwd_block<TO, VEC, CHUNKS, UNROLL, W_NONE, true>(a);
