@@ -600,10 +600,22 @@ SmallLayout small_layout(int64_t E, int64_t n_src) {
   return L;
 }
 inline bool small_block(int64_t E, int64_t n_src) { return E <= TR_SMALL_EDGES && n_src <= TR_SMALL_SOURCES; }
+// Few edges over more sources than the small path takes: the library sorts them in one or two blocks, while the bucket
+// sort's passes over a thousand buckets cost the same for any number of edges (us, library / buckets: 1000 edges over
+// 2 M sources 24 / 50, over 5 M 38 / 46, over 20 M 104 / 98; 10 000 edges over 1.1 M 41 / 43, over 5 M 66 / 51).  Above
+// 22 M sources the buckets' counters fill a compute unit's LDS (1000 edges over 40 M: 192 / 243).
+constexpr int64_t TR_FEW_EDGES = 1 << 13;
+constexpr int64_t TR_FEW_PRODUCT = (int64_t)1 << 34;
+constexpr int64_t TR_WIDE_SOURCES = 22'000'000;
+inline bool few_edges(int64_t E, int64_t n_src) {
+  return E <= TR_FEW_EDGES && (E * n_src <= TR_FEW_PRODUCT || n_src > TR_WIDE_SOURCES);
+}
 // Larger blocks go to the bucket sort of view_sort.hip; what it does not cover (more than 2^28 edge slots or
 // about 44 M sources) stays with the library sort below.  (Between 2^18 and 2^20 edges the library merges in a
 // dozen launches: 600 k edges 150 us, 66 us with the bucket sort.)
-inline bool bucket_sorted(int64_t E, int64_t n_src) { return !small_block(E, n_src) && vs_supported(E, n_src); }
+inline bool bucket_sorted(int64_t E, int64_t n_src) {
+  return !small_block(E, n_src) && !few_edges(E, n_src) && vs_supported(E, n_src);
+}
 
 // The launches of the counting sort; dims.E / dims.n_src size the grids (upper bounds when the real
 // sizes are read on the device).

@@ -137,3 +137,24 @@ def test_bucket_sorted_view_on_adversarial_blocks(be):
             np.testing.assert_array_equal(rowT.cpu().numpy()[:n], rows, err_msg=name)
             if want_edges:
                 np.testing.assert_array_equal(edgeT.cpu().numpy()[:n], order, err_msg=name)
+
+
+@pytest.mark.parametrize("E,N", [(300, 2_000_000), (8191, 2_000_000), (8193, 2_000_000), (3436, 5_000_000), (3437, 5_000_000),
+                                 (100, 1_048_577), (262_145, 50), (8192, 22_000_001), (8193, 22_000_001), (1, 1 << 24)])
+def test_few_edges_over_many_sources(be, E, N):
+    """Around the lines between the counting sort, the library's sort and the bucket sort."""
+    rng = np.random.default_rng(E)
+    R = E // 7 + 1
+    ptr = np.concatenate([[0], np.sort(rng.integers(0, E + 1, size=R - 1)), [E]]).astype(np.int64)
+    idx = rng.integers(0, N, size=E, dtype=np.int64)
+    idx[::5] = idx[0]
+    hrow = np.where(rng.random(R) < 0.2, 1, -1).astype(np.int64)
+    for m in (None, hrow):
+        ptrT, rowT, edgeT = be.build_transpose(T(ptr), T(idx), None if m is None else T(m), R, N, want_edges=True)
+        _, rows_only, _ = be.build_transpose(T(ptr), T(idx), None if m is None else T(m), R, N, want_edges=False)
+        want_ptr, want_edge, want_row = stable_view(ptr, idx, R, N, E, m)
+        kept = len(want_edge)
+        np.testing.assert_array_equal(ptrT.cpu().numpy(), want_ptr)
+        np.testing.assert_array_equal(edgeT[:kept].cpu().numpy(), want_edge)
+        np.testing.assert_array_equal(rowT[:kept].cpu().numpy(), want_row)
+        np.testing.assert_array_equal(rows_only[:kept].cpu().numpy(), want_row)
