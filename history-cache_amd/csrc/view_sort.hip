@@ -47,6 +47,12 @@ constexpr uint32_t VS_DEAD = 0xffffffffu;
 constexpr int VB_WAVES_MANY = 16, VB_WAVES_FEW = 4;
 constexpr int VB_MANY_LOCAL_BITS = 11;                   // 64 bytes of counters per local id
 constexpr uint32_t VB_STAGED = 8192;                     // largest bucket that takes the register path
+// Of the sixteen, four sort a bucket of up to VB_FEW_PAIRS pairs and the others leave at once, which makes room for the
+// next blocks: 3 M pairs evenly over 1 M sources 80 -> 67 us (65 with four waves for every bucket), with popular ones
+// among them 130 -> 126.  (Up to 8192 pairs: 74, above 2^10 local ids, whose counters leave a compute unit two blocks
+// at most: 81 -> 86.)
+constexpr uint32_t VB_FEW_PAIRS = 4096;
+constexpr int VB_FEW_LOCAL_BITS = 10;
 
 // Tile of a block: workgroup i runs on XCD i % 8, and every XCD gets one contiguous eighth of the
 // tiles, so that the partial lines at the write front of every bucket (runs of a few pairs per tile)
@@ -430,16 +436,16 @@ __device__ __forceinline__ uint32_t vb_swz32(uint32_t k) { return (k & ~15u) | (
 // 16-bit cursors (buckets of at most VB_STAGED pairs), two to a word: word k / 2 -> vb_swz16w(k / 2).
 __device__ __forceinline__ uint32_t vb_swz16w(uint32_t w) { return (w & ~7u) | ((w & 7u) ^ ((w >> 5) & 7u)); }
 
-// Buckets of at most VB_STAGED pairs: the pairs are read once and stay in registers, the cursors are
+// Buckets of at most STAGED pairs: the pairs are read once and stay in registers, the cursors are
 // 16 bits wide and the bucket's stretch of rowT is put together in LDS and stored line by line.
-// LDS: cur16[VB_WAVES][n_local] (as words), then stage[VB_STAGED].
-template <bool WANT_EDGES, int VB_WAVES>
+// LDS: cur16[VB_WAVES][n_local] (as words), then stage[STAGED].
+template <bool WANT_EDGES, int VB_WAVES, uint32_t STAGED>
 __device__ __forceinline__ void vb_small(const uint2 *__restrict__ mine, uint32_t n, uint32_t p0, int64_t b,
                                          uint32_t *__restrict__ lds, uint32_t *__restrict__ s_wave,
                                          const uint32_t *__restrict__ rows, int64_t *__restrict__ ptrT,
                                          int32_t *__restrict__ rowT, int32_t *__restrict__ edgeT, const VsShape &S) {
   constexpr int VB_THREADS = VB_WAVES * HC_WAVE;
-  constexpr int VB_ITERS = VB_STAGED / VB_THREADS;        // pairs per lane
+  constexpr int VB_ITERS = STAGED / VB_THREADS;           // pairs per lane
   const int tid = (int)threadIdx.x;
   const int lane = hc_lane();
   const int wave = tid >> 6;
@@ -650,7 +656,14 @@ __global__ __launch_bounds__(VB_WAVES * HC_WAVE) void vs_bucket(const uint2 *__r
   const int64_t b = blockIdx.x;
   const uint32_t p0 = bucket_off[b];
   const uint32_t n = bucket_off[b + 1] - p0;               // block-uniform
-  if (n <= VB_STAGED) vb_small<WANT_EDGES, VB_WAVES>(pairs + p0, n, p0, b, vb_lds, s_wave, rows, ptrT, rowT, edgeT, S);
+  if constexpr (VB_WAVES > VB_WAVES_FEW) {
+    if (n <= VB_FEW_PAIRS && S.lb <= VB_FEW_LOCAL_BITS) {
+      if (threadIdx.x >= VB_WAVES_FEW * HC_WAVE) return;     // whole waves; the barriers go on without them
+      vb_small<WANT_EDGES, VB_WAVES_FEW, VB_FEW_PAIRS>(pairs + p0, n, p0, b, vb_lds, s_wave, rows, ptrT, rowT, edgeT, S);
+      return;
+    }
+  }
+  if (n <= VB_STAGED) vb_small<WANT_EDGES, VB_WAVES, VB_STAGED>(pairs + p0, n, p0, b, vb_lds, s_wave, rows, ptrT, rowT, edgeT, S);
   else vb_large<WANT_EDGES, VB_WAVES>(pairs + p0, n, p0, b, vb_lds, s_wave, rows, ptrT, rowT, edgeT, S);
 }
 

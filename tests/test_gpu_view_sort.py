@@ -158,3 +158,26 @@ def test_few_edges_over_many_sources(be, E, N):
         np.testing.assert_array_equal(edgeT[:kept].cpu().numpy(), want_edge)
         np.testing.assert_array_equal(rowT[:kept].cpu().numpy(), want_row)
         np.testing.assert_array_equal(rows_only[:kept].cpu().numpy(), want_row)
+
+
+@pytest.mark.parametrize("N", [2_000, 500_000, 1_000_000, 2_000_000, 4_000_000])
+def test_buckets_around_the_sizes_that_take_other_paths(be, N):
+    """Buckets of 4096 pairs (four waves), one more (sixteen), 8192 (pairs in registers) and one more, with one id and
+    with all ids of the bucket in use, from one to 2^11 ids to a bucket."""
+    rng = np.random.default_rng(N)
+    bits = max(int(N).bit_length() - 11, 0)
+    ids = []
+    for k, n in enumerate((4095, 4096, 4097, 8191, 8192, 8193, 1, 63, 64, 65)):
+        first = (3 * k + 1) << bits
+        ids += [np.full(n, first), first + (1 << bits) * 31 + rng.integers(0, 1 << bits, size=n)]
+    idx = np.concatenate(ids + [rng.integers(100 << bits, N, size=260_000)])
+    rng.shuffle(idx)
+    E, R = len(idx), 9_000
+    ptr = np.concatenate([[0], np.sort(rng.integers(0, E + 1, size=R - 1)), [E]]).astype(np.int64)
+    want_ptr, order, rows = stable_view(ptr, idx, R, N, E)
+    for want_edges in (False, True):
+        ptrT, rowT, edgeT = be.build_transpose(T(ptr), T(idx), None, R, N, want_edges=want_edges)
+        np.testing.assert_array_equal(ptrT.cpu().numpy(), want_ptr)
+        np.testing.assert_array_equal(rowT.cpu().numpy(), rows)
+        if want_edges:
+            np.testing.assert_array_equal(edgeT.cpu().numpy(), order)
