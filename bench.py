@@ -353,7 +353,7 @@ def run_c2(args, row_mode=False):
                    "40%% history hits (%s substitution), mean fwd + transpose build + bwd"
                    % (R, E, N, F, "per-row" if row_mode else "per-source")},
         "roofline": {"bound": "hbm",
-                     "kernel": "fwd_rows<float,float,4,1,8,%s,0>" % ("false" if row_mode else "true"),
+                     "kernel": "fwd_rows<float,float,4,1,8,false,0>" if row_mode else "fwd_rows_wide<float,float,4,1,8,true,0>",
                      "achieved": bytes_f / (t_f * 1e-3) / 1e9,
                      "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": bytes_f / (t_f * 1e-3) / 1e9 / HBM_PEAK_GBS,
                      "traffic": MEASURED_TRAFFIC["c2row" if row_mode else "c2"] if s == 1.0 else None,
@@ -428,7 +428,7 @@ def run_c2w(args):
         "config": {"workload": "c2w: weighted aggregation (edge_value) on the c2 block, R=%d, E=%d, %d sources x %d "
                                "fp32 in %d head(s): fwd + transposed view with edge slots + bwd (input gradient and "
                                "edge gradient)" % (R, E, N, F, H)},
-        "roofline": {"bound": "hbm", "kernel": "fwd_rows<float,float,4,1,8,false,%d>" % (2 if H > 1 else 1),
+        "roofline": {"bound": "hbm", "kernel": "fwd_rows_wide<float,float,4,1,8,false,%d>" % (2 if H > 1 else 1),
                      "achieved": bytes_f / (t_f * 1e-3) / 1e9, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": bytes_f / (t_f * 1e-3) / 1e9 / HBM_PEAK_GBS, "traffic": None,
                      "algorithmic_bytes": bytes_f, "launch_ms": t_f},

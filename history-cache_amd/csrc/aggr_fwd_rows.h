@@ -598,9 +598,7 @@ __device__ __forceinline__ void fwd_front(const FwdArgs &a, int64_t far_above, i
 // SIMD (11 M edges x 128 in one launch 2.55 ms, in two 1.96 ms).
 constexpr int FWD_ALL = 0, FWD_FRONT = 1, FWD_BODY = 2;
 template <typename T, typename TH, int VEC, int CHUNKS, int UNROLL, bool SRC, int WMODE, int PART>
-// At most 80 scalar registers: above, fewer waves of short rows fit the chip.  (The slices would take 106, and with them
-// 1 M rows of 3 edges of 64 columns 433 us instead of 388, 700 k rows of 20 edges 664 instead of 638.)
-__global__ __launch_bounds__(HC_BLOCK) __attribute__((amdgpu_num_sgpr(80))) void fwd_rows(FwdArgs a) {
+__device__ __forceinline__ void fwd_block(const FwdArgs &a) {
   // without heads the rows may be split: the split code is compiled for those modes only
   constexpr int LMODE = WMODE == W_EDGE_HEAD ? W_EDGE : WMODE;
   __shared__ float part[HC_WAVES_PER_BLOCK - 1][HC_WAVE * VEC * CHUNKS];
@@ -695,6 +693,23 @@ __global__ __launch_bounds__(HC_BLOCK) __attribute__((amdgpu_num_sgpr(80))) void
     fwd_long_row<T, TH, VEC, CHUNKS, UNROLL, SRC, LMODE>(a, row0 + long_rows[t], lane, wave, part);
 }
 
+// Plain rows, and rows beside a table of another element type: at most 80 scalar registers;
+// above, fewer waves fit the chip.  (The slices would take 106, and with them 1 M rows of 3 edges of 64 columns 433 us
+// instead of 388, 700 k rows of 20 edges 664 instead of 638; 6 M edges x 100 beside a half-precision table 1214 us
+// instead of 1063.)
+template <typename T, typename TH, int VEC, int CHUNKS, int UNROLL, bool SRC, int WMODE, int PART>
+__global__ __launch_bounds__(HC_BLOCK) __attribute__((amdgpu_num_sgpr(80))) void fwd_rows(FwdArgs a) {
+  fwd_block<T, TH, VEC, CHUNKS, UNROLL, SRC, WMODE, PART>(a);
+}
+
+// Weights, substituted sources: with the heads' and the substitution's vector registers there is room for four or five
+// waves whatever the scalar ones, and the slices are the faster with more of these (20 M edges x 256 over 20 GB 4.19 ms,
+// 4.24 with 80; a row of 27 000 weighted edges x 256 198 us, 202 with 80).
+template <typename T, typename TH, int VEC, int CHUNKS, int UNROLL, bool SRC, int WMODE, int PART>
+__global__ __launch_bounds__(HC_BLOCK) void fwd_rows_wide(FwdArgs a) {
+  fwd_block<T, TH, VEC, CHUNKS, UNROLL, SRC, WMODE, PART>(a);
+}
+
 // One translation unit each (the kernels take a minute to compile).
 __attribute__((visibility("hidden"))) int fwd_dispatch_f32(FwdArgs &a, bool src_mode, int n_head, hipStream_t st);
 __attribute__((visibility("hidden"))) int fwd_dispatch_f16(FwdArgs &a, bool src_mode, int n_head, hipStream_t st);
@@ -711,24 +726,26 @@ int launch_rows(const FwdArgs &a, bool src_mode, hipStream_t st) {
   const int64_t blocks = row_blocks + a.front;
   if (!hc_grid_ok(blocks)) return HC_EUNSUPPORTED;
   const dim3 grid((unsigned)blocks), block(HC_BLOCK);
-#define HC_FWD_LAUNCH(TH, SRC, WMODE) fwd_rows<T, TH, VEC, CHUNKS, UNROLL, SRC, WMODE, FWD_ALL><<<grid, block, 0, st>>>(a)
+#define HC_FWD_LAUNCH(WMODE) fwd_rows<T, T, VEC, CHUNKS, UNROLL, false, WMODE, FWD_ALL><<<grid, block, 0, st>>>(a)
+#define HC_FWD_LAUNCH_WIDE(SRC, WMODE) fwd_rows_wide<T, T, VEC, CHUNKS, UNROLL, SRC, WMODE, FWD_ALL><<<grid, block, 0, st>>>(a)
 #define HC_FWD_LAUNCH_TWO(TH)                                                                                           \
   {                                                                                                                     \
     if (a.front > 0)                                                                                                    \
       fwd_rows<T, TH, VEC, CHUNKS, UNROLL, true, W_NONE, FWD_FRONT><<<dim3((unsigned)a.front), block, 0, st>>>(a);      \
     fwd_rows<T, TH, VEC, CHUNKS, UNROLL, true, W_NONE, FWD_BODY><<<dim3((unsigned)row_blocks), block, 0, st>>>(a);      \
   }
-  if (a.ev != nullptr && a.n_head > 1) HC_FWD_LAUNCH(T, false, W_EDGE_HEAD);
-  else if (a.ev != nullptr) HC_FWD_LAUNCH(T, false, W_EDGE);
+  if (a.ev != nullptr && a.n_head > 1) HC_FWD_LAUNCH_WIDE(false, W_EDGE_HEAD);
+  else if (a.ev != nullptr) HC_FWD_LAUNCH_WIDE(false, W_EDGE);
   else if (src_mode && a.hmap != nullptr) {
     // the table of a per-source substitution may be narrower than fp32 features
     if constexpr (std::is_same<T, float>::value) {
       if (a.hist_dtype == HC_F16) HC_FWD_LAUNCH_TWO(__half)
       else if (a.hist_dtype == HC_BF16) HC_FWD_LAUNCH_TWO(__hip_bfloat16)
-      else HC_FWD_LAUNCH(T, true, W_NONE);
-    } else HC_FWD_LAUNCH(T, true, W_NONE);
-  } else HC_FWD_LAUNCH(T, false, W_NONE);
+      else HC_FWD_LAUNCH_WIDE(true, W_NONE);
+    } else HC_FWD_LAUNCH_WIDE(true, W_NONE);
+  } else HC_FWD_LAUNCH(W_NONE);
 #undef HC_FWD_LAUNCH
+#undef HC_FWD_LAUNCH_WIDE
 #undef HC_FWD_LAUNCH_TWO
   return hc_launch_status();
 }
