@@ -354,7 +354,7 @@ __device__ __forceinline__ void bwd_front(const BwdArgs &a, int lane, int wave) 
   const int ns = (int)((a.F + BWD_SLICE - 1) / BWD_SLICE);
   const auto source = [&](const SegList &list, const SegIndex &index, int64_t above, int e) -> int64_t {
     int t, w;
-    seg_locate(index, e, lane, &t, &w);
+    seg_locate(index, e, &t, &w);
     return (int64_t)__builtin_amdgcn_readfirstlane(list.item[seg_part(a.ptrT, (int64_t)t * a.tile, above) + w]);
   };
   // the lane's column of slice `sl`; lanes behind the slice or the row read its last one again

@@ -520,7 +520,7 @@ __device__ __forceinline__ void fwd_front(const FwdArgs &a, int64_t far_above, i
   const auto far_row = [&](int e) -> int64_t {
     if (a.n_tiles == 0) return (int64_t)__builtin_amdgcn_readfirstlane(self_rows[e]);
     int t, w;
-    seg_locate(far_index, e, lane, &t, &w);
+    seg_locate(far_index, e, &t, &w);
     return (int64_t)__builtin_amdgcn_readfirstlane(a.far.item[seg_part(a.ptr, (int64_t)t * a.tile, far_above) + w]);
   };
   // the lane's columns of slice `sl`; lanes behind the slice or the row read its last ones again
@@ -530,66 +530,62 @@ __device__ __forceinline__ void fwd_front(const FwdArgs &a, int64_t far_above, i
     return (uint32_t)(c < a.F ? c : a.F - SV);
   };
   const int64_t tasks = (int64_t)n_far * ns;
-  if (WMODE == W_EDGE_HEAD || a.split_above == 0) {
+  if constexpr (WMODE == W_EDGE_HEAD) {                  // rows of several heads are never split: one wave per task
     for (int64_t t = (int64_t)wave * a.front + blockIdx.x; t < tasks; t += (int64_t)HC_WAVES_PER_BLOCK * a.front) {
       const int64_t row = far_row((int)(t / ns));
       bool on;
       const uint32_t c = columns((int)(t % ns), on);
       const int64_t b = a.ptr[row], e = a.ptr[row + 1];
       float s[SV];
-      if constexpr (WMODE == W_EDGE_HEAD) {
-        // every column of the slice in one head: its weights are staged with the ids, 64 at a time
-        const int fh = (int)(a.F / a.n_head);
-        const int c0 = (int)(t % ns) * SL;
-        const int c1 = (c0 + SL < a.F ? c0 + SL : (int)a.F) - 1;
-        if (c0 / fh == c1 / fh)
-          fwd_slice_any<T, TH, SV, SRC, W_EDGE, 32>(a, c, b, e, lane, a.ev + c0 / fh, a.n_head, s);
-        else
-          fwd_slice_sum<T, TH, SV, SRC, W_EDGE_HEAD, 16, false>(a, c, b, e, lane, a.ev, 0, s);
-      } else {
-        fwd_slice_any<T, TH, SV, SRC, WMODE, 16>(a, c, b, e, lane, a.ev, 1, s);
-      }
+      // every column of the slice in one head: its weights are staged with the ids, 64 at a time
+      const int fh = (int)(a.F / a.n_head);
+      const int c0 = (int)(t % ns) * SL;
+      const int c1 = (c0 + SL < a.F ? c0 + SL : (int)a.F) - 1;
+      if (c0 / fh == c1 / fh)
+        fwd_slice_any<T, TH, SV, SRC, W_EDGE, 32>(a, c, b, e, lane, a.ev + c0 / fh, a.n_head, s);
+      else
+        fwd_slice_sum<T, TH, SV, SRC, W_EDGE_HEAD, 16, false>(a, c, b, e, lane, a.ev, 0, s);
 #pragma unroll
       for (int i = 0; i < SV; ++i)
-        if (on) a.vout[row * a.F + c + i] = WMODE != W_NONE ? s[i] : s[i] / (float)(int)(e - b);
+        if (on) a.vout[row * a.F + c + i] = s[i];
     }
     return;
-  }
-  constexpr int LMODE = WMODE == W_EDGE_HEAD ? W_EDGE : WMODE;
-  for (int64_t t = blockIdx.x; t < tasks; t += a.front) {
-    const int64_t row = far_row((int)(t / ns));
-    bool on;
-    const uint32_t c = columns((int)(t % ns), on);
-    const int64_t lb = a.ptr[row], le = a.ptr[row + 1];
-    const int64_t q = (le - lb + HC_WAVES_PER_BLOCK - 1) / HC_WAVES_PER_BLOCK;
-    int64_t sb = lb + wave * q, se = sb + q;
-    if (sb > le) sb = le;
-    if (se > le) se = le;
-    float s[SV];
-    fwd_slice_any<T, TH, SV, SRC, LMODE, 16>(a, c, sb, se, lane, a.ev, 1, s);
-    if (wave > 0 && lane < FWD_SLICE_LANES) {
+  } else {
+    for (int64_t t = blockIdx.x; t < tasks; t += a.front) {
+      const int64_t row = far_row((int)(t / ns));
+      bool on;
+      const uint32_t c = columns((int)(t % ns), on);
+      const int64_t lb = a.ptr[row], le = a.ptr[row + 1];
+      const int64_t q = (le - lb + HC_WAVES_PER_BLOCK - 1) / HC_WAVES_PER_BLOCK;
+      int64_t sb = lb + wave * q, se = sb + q;
+      if (sb > le) sb = le;
+      if (se > le) se = le;
+      float s[SV];
+      fwd_slice_any<T, TH, SV, SRC, WMODE, 16>(a, c, sb, se, lane, a.ev, 1, s);
+      if (wave > 0 && lane < FWD_SLICE_LANES) {
 #pragma unroll
-      for (int i = 0; i < SV; ++i) part[wave - 1][lane * SV + i] = s[i];
-    }
-    __syncthreads();
-    if (wave == 0 && on) {
-#pragma unroll
-      for (int i = 0; i < SV; ++i) {
-#pragma unroll
-        for (int pw = 0; pw < HC_WAVES_PER_BLOCK - 1; ++pw) s[i] += part[pw][lane * SV + i];
-        a.vout[row * a.F + c + i] = WMODE != W_NONE ? s[i] : s[i] / (float)(int)(le - lb);
+        for (int i = 0; i < SV; ++i) part[wave - 1][lane * SV + i] = s[i];
       }
+      __syncthreads();
+      if (wave == 0 && on) {
+#pragma unroll
+        for (int i = 0; i < SV; ++i) {
+#pragma unroll
+          for (int pw = 0; pw < HC_WAVES_PER_BLOCK - 1; ++pw) s[i] += part[pw][lane * SV + i];
+          a.vout[row * a.F + c + i] = WMODE != W_NONE ? s[i] : s[i] / (float)(int)(le - lb);
+        }
+      }
+      __syncthreads();
     }
-    __syncthreads();
-  }
-  if (a.n_tiles == 0) return;
-  const SegIndex near_index = seg_index(a.near.count, a.n_tiles, lane);
-  for (int t = (int)blockIdx.x; t < near_index.total; t += a.front) {
-    int tile, w;
-    seg_locate(near_index, t, lane, &tile, &w);
-    const int64_t row = (int64_t)__builtin_amdgcn_readfirstlane(
-        a.near.item[seg_part(a.ptr, (int64_t)tile * a.tile, a.slice_above) + w]);
-    fwd_long_row<T, TH, VEC, CHUNKS, UNROLL, SRC, LMODE>(a, row, lane, wave, part);
+    if (a.n_tiles == 0) return;
+    const SegIndex near_index = seg_index(a.near.count, a.n_tiles, lane);
+    for (int t = (int)blockIdx.x; t < near_index.total; t += a.front) {
+      int tile, w;
+      seg_locate(near_index, t, &tile, &w);
+      const int64_t row = (int64_t)__builtin_amdgcn_readfirstlane(
+          a.near.item[seg_part(a.ptr, (int64_t)tile * a.tile, a.slice_above) + w]);
+      fwd_long_row<T, TH, VEC, CHUNKS, UNROLL, SRC, WMODE>(a, row, lane, wave, part);
+    }
   }
 }
 

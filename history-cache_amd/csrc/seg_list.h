@@ -49,7 +49,7 @@ __device__ __forceinline__ SegIndex seg_index(const int32_t *__restrict__ count,
 }
 
 // Tile and place inside its part of list entry e (wave-uniform, e < total).
-__device__ __forceinline__ void seg_locate(const SegIndex &x, int e, int lane, int *tile, int *within) {
+__device__ __forceinline__ void seg_locate(const SegIndex &x, int e, int *tile, int *within) {
   const int l = __builtin_ctzll(__ballot(x.incl > e));
   int rem = e - (l > 0 ? __builtin_amdgcn_readlane(x.incl, l - 1) : 0);
   int k = 0;
@@ -63,7 +63,6 @@ __device__ __forceinline__ void seg_locate(const SegIndex &x, int e, int lane, i
   }
   *tile = l * 8 + k;
   *within = rem;
-  (void)lane;
 }
 
 // Segments per tile: at least 1 024, few enough tiles for the readers.
