@@ -85,7 +85,7 @@ class _SageConvFunction(torch.autograd.Function):
         be = hiscache_backend
         R = int(num_node) if num_node else ptr.numel() - 1
         agg = be._aggr_fwd(be.SUBST_ROW, ptr, idx, x, hmap, hbuf, hsize, None, R,
-                           max_degree=None if view is None else view.max_out_degree)
+                           max_degree=None if view is None else view.row_bound(R, x.shape[0]))
         # plain GEMMs and a separate bias add: a GEMM with a bias epilogue goes to hipBLASLt whatever
         # library is preferred, and its per-shape set-up costs the host more than the extra launch
         out = agg @ w_l.t()
@@ -417,7 +417,7 @@ class _RgcnConvFunction(torch.autograd.Function):
         ptr2, idx2, _cnt, _deg, w2 = be.typed_csr(ptr, idx, edge_types, K, R, x.shape[0], used_mask,
                                                   want_weights=True)
         agg = be._aggr_fwd(be.SUBST_ROW, ptr2, idx2, x, None, None, 0, w2, R * K,
-                           max_degree=None if view is None else view.max_out_degree).view(R, K, Fin)
+                           max_degree=None if view is None else view.row_bound(R, x.shape[0])).view(R, K, Fin)
         out = _rel_matmul(agg, weight)
         hit = None
         if hmap is not None:

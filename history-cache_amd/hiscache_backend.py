@@ -410,6 +410,16 @@ class BatchView:
     def covers(self, num_node, n_src):
         return int(num_node) <= self.rows and int(n_src) <= self.n_src
 
+    def row_bound(self, num_node, n_src):
+        """The bound on the edges of a row, for a layer that is this batch's (None: unknown)."""
+        return self.max_out_degree if self.covers(num_node, n_src) else None
+
+    def __setstate__(self, state):
+        # a view that was saved before it carried all of its present fields: what it does not say is unknown
+        fields = state[1] if isinstance(state, tuple) else state
+        for name in self.__slots__:
+            setattr(self, name, fields.get(name))
+
     def record_stream(self, stream):
         for t in (self.ptrT, self.rowT, self.edgeT):
             if t is not None:
@@ -515,7 +525,7 @@ class _AggrHistory(torch.autograd.Function):
     def forward(ctx, x, ptr, idx, edge_value, hmap, hbuf, hsize, num_node, mode, num_edge=None, view=None):
         R = int(num_node) if num_node else ptr.numel() - 1
         out = _aggr_fwd(mode, ptr, idx, x, hmap, hbuf, hsize, edge_value, R,
-                        max_degree=None if view is None else view.max_out_degree)
+                        max_degree=None if view is None else view.row_bound(R, x.shape[0]))
         ctx.hc = (ptr, idx, hmap, hsize, R, mode, None if hbuf is None else tuple(hbuf.shape))
         # edge slots the first R rows can reach, when the caller knows it (a layer of a shared CSR owns a
         # prefix of idx): the transposed view then sorts that prefix only

@@ -379,3 +379,21 @@ def test_trainer_hands_out_every_batch_once_and_reads_one_batch_ahead():
     cfg = make_config(8, 2, 8, 2)
     assert _option(cfg, "train.model.num_layers", 7) == 2
     assert _option(cfg, "train.train.num_epochs", 7) == 7 and _option(cfg, "dl.sampler.train.batch_size", None) is None
+
+
+def test_batch_view_fields_of_saved_and_foreign_views():
+    """A view that was saved when it had fewer fields comes back with them unknown, and a view of another, smaller batch
+    bounds no layer's rows (it is not used for its backward either)."""
+    import copy
+    import pickle
+    import torch
+    import hiscache_backend as be
+    ptrT, rowT = torch.tensor([0, 1, 2]), torch.zeros(2, dtype=torch.int32)
+    view = be.BatchView(ptrT, rowT, None, 3, 2, 2, max_in_degree=1, max_out_degree=1)
+    again = pickle.loads(pickle.dumps(view))
+    assert (again.rows, again.n_src, again.max_in_degree, again.max_out_degree) == (3, 2, 1, 1)
+    assert copy.copy(view).max_out_degree == 1
+    old = be.BatchView.__new__(be.BatchView)
+    old.__setstate__((None, {k: getattr(view, k) for k in ("ptrT", "rowT", "edgeT", "rows", "n_src", "num_edge")}))
+    assert old.max_in_degree is None and old.max_out_degree is None and old.covers(3, 2)
+    assert view.row_bound(3, 2) == 1 and view.row_bound(4, 2) is None and view.row_bound(3, 3) is None
