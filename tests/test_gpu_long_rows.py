@@ -162,3 +162,19 @@ def test_rows_of_every_short_length(be, orc, F, dtype):
         shape = (N, H, F // H) if H > 1 else (N, F)
         out = be._aggr_fwd(be.SUBST_ROW, T(ptr), T(idx), x.view(shape), None, None, 0, T(ev), R)
         np.testing.assert_array_equal(out.cpu().numpy(), orc.fwd_edge_value(ptr, idx, ev, x32.reshape(shape), None, None))
+
+
+def test_rows_behind_four_gigabytes(be):
+    """Features of more than 4 GiB, whose rows the slices address in 64 bits: the bits of the same call over the matrix's
+    last rows alone, which are addressed in 32."""
+    rng = np.random.default_rng(11)
+    N, few, R, F = (1 << 24) + 777, 500, 300, 64
+    ptr, idx = block(rng, R, few, LENGTHS)
+    x = torch.empty(N, F, device=DEV)
+    x[N - few:] = torch.randn(few, F, device=DEV)
+    tp, far, near = T(ptr), T(idx + (N - few)), T(idx)
+    for H in (0, 1, 4):
+        ev = T(rng.random((len(idx), H) if H > 1 else len(idx)).astype(np.float32)) if H else None
+        out = [be._aggr_fwd(be.SUBST_ROW, tp, ids, m.view(-1, H, F // H) if H > 1 else m, None, None, 0, ev, R)
+               for ids, m in ((far, x), (near, x[N - few:]))]
+        assert torch.equal(*out), H

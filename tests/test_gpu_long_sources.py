@@ -122,6 +122,12 @@ def test_weighted(be, orc, F, H):
     ref, ref_h, ref_e = orc.bwd_edge_value(ptr, idx, ev, g, hmap, x, N, hsize=F * H, want_edge_grad=True)
     np.testing.assert_array_equal(gx.cpu().numpy(), ref)
     np.testing.assert_array_equal(gh.cpu().numpy().reshape(ref_h.shape), ref_h)
+    # (F products in any order against the oracle's: each within (F + 2) ulp/2 of the sum of their magnitudes)
+    row = np.repeat(np.arange(R), np.diff(ptr))
+    size = np.abs(g.reshape(R, H, F)[row].astype(np.float64) * x.reshape(N, H, F)[idx]).sum(2)
+    size[hmap[row] != -1] = 0.0
+    far = np.abs(eg.cpu().numpy().reshape(-1, H).astype(np.float64) - ref_e.reshape(-1, H))
+    assert (far <= 2 * (F + 2) * 2.0 ** -24 * size).all()
 
 
 def test_unaligned_gradient(be, orc):
@@ -243,3 +249,29 @@ def test_inner_layer_over_a_view_of_long_sources(be, orc, F, rows):
         gx, _ = be._aggr_bwd_batch_view(T(ptr), view, T(g), None if m is None else T(m), None, 0, rows, N,
                                         want_hist_grad=False)
         np.testing.assert_array_equal(gx.cpu().numpy(), want)
+
+
+def test_gradient_rows_behind_four_gigabytes(be):
+    """A gradient of more than 4 GiB, whose rows the slices address in 64 bits: the bits of the same call over its last
+    rows alone, which are addressed in 32."""
+    rng = np.random.default_rng(15)
+    few, N, F = 2000, 900, 64
+    ptr, idx = block(rng, few, N)
+    R = (1 << 24) + 4321
+    skip = R - few
+    wide = torch.cat([torch.zeros(skip, dtype=torch.int64, device=DEV), T(ptr)])
+    g = torch.empty(R, F, device=DEV)
+    g[skip:] = torch.randn(few, F, device=DEV)
+    ti, E = T(idx), len(idx)
+    for H in (0, 1, 4):
+        ev = T(rng.random((E, H) if H > 1 else E).astype(np.float32)) if H else None
+        out = []
+        for p, gr, n in ((wide, g, R), (T(ptr), g[skip:], few)):
+            gr = gr.view(n, H, F // H) if H > 1 else gr
+            tr = be.build_transpose(p, ti, None, n, N, want_edges=H > 0)
+            out.append(be._aggr_bwd(p, ti, tr, gr, None, ev, None, False, None, 0, n, N)[0])
+        assert torch.equal(*out), H
+    views = [be.build_batch_view(p, ti, n, N) for p, n in ((wide, R), (T(ptr), few))]
+    out = [be._aggr_bwd_batch_view(p, v, gr, None, None, 0, n, N)[0]
+           for p, v, gr, n in ((wide, views[0], g, R), (T(ptr), views[1], g[skip:], few))]
+    assert torch.equal(*out)
