@@ -42,10 +42,9 @@ AGE_LIMIT_ITERS = 100_000
 # the c3 / c5 training iterations that the default line reports beside the kernels' figures
 ITERATION_STEPS, ITERATION_WARMUP = 200, 20
 # HBM bytes per launch by the counters (rocprofv3 --pmc FETCH_SIZE / WRITE_SIZE, scaled by a 4 GiB copy), measured
-# with the library built from commit 6072fbd: profiles/aggr_c2_hbm_traffic.md, rows "C2 fwd_mean_fast" (c2),
-# "C4 gc_pass1 + gc_pass3_ring" (c4) and the three "batched layer" rows (c3_batched); c2row from the same
-# procedure over `--workload c2row` at commit 173ecbf (that kernel has not changed since).
-MEASURED_TRAFFIC = {"c2": 23.08e9, "c2row": 13.93e9, "c4": 3.49e9, "c3_batched": 51.97e9}
+# with the library built from commit 83d9576: profiles/aggr_c2_hbm_traffic.md, rows "C2 fwd_rows_wide" (c2), "C2, per-row
+# substitution" (c2row), "C4 gc_pass1 + gc_pass3_ring" (c4), "batched layer" fwd_rows, bwd_sources and gc_* (c3_batched).
+MEASURED_TRAFFIC = {"c2": 23.87e9, "c2row": 14.01e9, "c4": 3.49e9, "c3_batched": 51.34e9}
 
 
 def parse():
