@@ -58,9 +58,10 @@ __global__ __launch_bounds__(BWD_PREP_BLOCK) void bwd_prepare(BwdArgs a, int64_t
   }
   __syncthreads();
   if (threadIdx.x == 0) {
-    a.mid.count[blockIdx.x] = n_mid;
-    a.hub.count[blockIdx.x] = n_hub;
-    a.giant.count[blockIdx.x] = n_giant;
+    const bool fits = a.ptrT[a.n_src] - a.ptrT[0] <= a.E;      // else the lists may lack entries: none is used
+    a.mid.count[blockIdx.x] = fits ? n_mid : 0;
+    a.hub.count[blockIdx.x] = fits ? n_hub : 0;
+    a.giant.count[blockIdx.x] = fits ? n_giant : 0;
   }
 }
 

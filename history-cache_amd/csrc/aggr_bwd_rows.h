@@ -457,11 +457,8 @@ template <typename TO, int VEC, int CHUNKS, int UNROLL, int WMODE, bool MASKED>
 __device__ __forceinline__ void bwd_block(const BwdArgs &a) {
   const int lane = hc_lane();
   const int wave = hc_wave_in_block();
-  // every thread of the grid reads the same two words, so the decision is uniform: a view of more entries than its
-  // caller announced is summed as if there were neither lists nor runs (they would not hold it)
-  const bool listed = a.front > 0 && a.ptrT[a.n_src] - a.ptrT[0] <= a.E;
   if ((int)blockIdx.x < a.front) {
-    if (listed) bwd_front<TO, WMODE, MASKED>(a, lane, wave);
+    bwd_front<TO, WMODE, MASKED>(a, lane, wave);
     return;
   }
   const int64_t block = (int64_t)blockIdx.x - a.front;
@@ -490,6 +487,10 @@ __device__ __forceinline__ void bwd_block(const BwdArgs &a) {
   }
   const int64_t unit = hc_xcd_block<BWD_XCD_CHUNK>(block, a.src_blocks) * HC_WAVES_PER_BLOCK + wave;
   int64_t s0, s1;
+  // every thread of the grid reads the same two words, so the decision is uniform: a view of more entries than its
+  // caller announced is summed as if there were neither lists (bwd_prepare leaves them empty) nor runs, which would not
+  // hold it
+  const bool listed = a.front > 0 && a.ptrT[a.n_src] - a.ptrT[0] <= a.E;
   if (a.run_start != nullptr && listed) {
     const int64_t last = bwd_run_of(a, a.n_src);
     if (unit > last) return;
@@ -616,9 +617,15 @@ __device__ __forceinline__ void bwd_block(const BwdArgs &a) {
   }
 }
 
-// At most 80 scalar registers: above, fewer waves fit the chip (14 M edges x 64 1326 us, 1295 so).
-template <typename TO, int VEC, int CHUNKS, int UNROLL, int WMODE>
+// The mean: at most 80 scalar registers; above, fewer waves fit the chip (14 M edges x 64 1326 us, 1295 so).
+template <typename TO, int VEC, int CHUNKS, int UNROLL>
 __global__ __launch_bounds__(HC_BLOCK) __attribute__((amdgpu_num_sgpr(80))) void bwd_sources(BwdArgs a) {
+  bwd_block<TO, VEC, CHUNKS, UNROLL, W_NONE, false>(a);
+}
+
+// Weights: what their slices take.
+template <typename TO, int VEC, int CHUNKS, int UNROLL, int WMODE>
+__global__ __launch_bounds__(HC_BLOCK) void bwd_sources_weighted(BwdArgs a) {
   bwd_block<TO, VEC, CHUNKS, UNROLL, WMODE, false>(a);
 }
 
@@ -644,9 +651,9 @@ int bwd_launch(const BwdArgs &a, bool masked, hipStream_t st) {
   if (!hc_grid_ok(blocks)) return HC_EUNSUPPORTED;
   const dim3 grid((unsigned)blocks), block(HC_BLOCK);
   if (masked) bwd_sources_of_view<TO, VEC, CHUNKS, UNROLL><<<grid, block, 0, st>>>(a);
-  else if (a.ev != nullptr && a.n_head > 1) bwd_sources<TO, VEC, CHUNKS, UNROLL, W_EDGE_HEAD><<<grid, block, 0, st>>>(a);
-  else if (a.ev != nullptr) bwd_sources<TO, VEC, CHUNKS, UNROLL, W_EDGE><<<grid, block, 0, st>>>(a);
-  else bwd_sources<TO, VEC, CHUNKS, UNROLL, W_NONE><<<grid, block, 0, st>>>(a);
+  else if (a.ev != nullptr && a.n_head > 1) bwd_sources_weighted<TO, VEC, CHUNKS, UNROLL, W_EDGE_HEAD><<<grid, block, 0, st>>>(a);
+  else if (a.ev != nullptr) bwd_sources_weighted<TO, VEC, CHUNKS, UNROLL, W_EDGE><<<grid, block, 0, st>>>(a);
+  else bwd_sources<TO, VEC, CHUNKS, UNROLL><<<grid, block, 0, st>>>(a);
   return hc_launch_status();
 }
 
