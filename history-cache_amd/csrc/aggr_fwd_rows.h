@@ -14,8 +14,8 @@
 // What bounds it: the bulk of a block is bound by the memory system (5 - 6 TB/s of random rows once the chip is
 // full), the rest by its longest rows, which are therefore shared out slice by slice (seg_list.h).  Measured on
 // MI355X, before (rows of four waves, widths off a multiple of 64 element by element) and after: 3 M edges x 256
-// bf16 with a row of 14 000 edges 1.42 -> 0.30 ms; 600 k edges x 100 fp32 0.64 -> 0.055 ms; 20 M edges x 256 fp32
-// over 20 GB 4.21 -> 4.22 ms (its long rows are short beside the launch).
+// bf16 with a row of 14 000 edges 1.42 -> 0.26 ms; 600 k edges x 100 fp32 0.64 -> 0.047 ms; 20 M edges x 256 fp32
+// over 20 GB 4.20 -> 4.20 ms (its long rows are short beside the launch).
 //
 // Semantics follow the reference kernels gen_fwd_history_v2,
 // gen_fwd_history_v2_edge_value and gen_fwd_history_v2_edge_value_multi_head
