@@ -86,14 +86,19 @@ class _SageConvFunction(torch.autograd.Function):
         R = int(num_node) if num_node else ptr.numel() - 1
         agg = be._aggr_fwd(be.SUBST_ROW, ptr, idx, x, hmap, hbuf, hsize, None, R,
                            max_degree=None if view is None else view.row_bound(R, x.shape[0]))
-        # plain GEMMs and a separate bias add: a GEMM with a bias epilogue goes to hipBLASLt whatever
-        # library is preferred, and its per-shape set-up costs the host more than the extra launch
-        out = agg @ w_l.t()
+        root = None
         if w_r is not None:
             root = x[:R] if x.dtype == agg.dtype else x[:R].to(agg.dtype)
-            out.addmm_(root, w_r.t())
-        if b_l is not None:
-            out += b_l
+        if be.linear_supported(agg, w_l, root, w_r, b_l):
+            out = be.linear(agg, w_l, root, w_r, b_l)
+        else:
+            # plain GEMMs and a separate bias add: a GEMM with a bias epilogue goes to hipBLASLt whatever
+            # library is preferred, and its per-shape set-up costs the host more than the extra launch
+            out = agg @ w_l.t()
+            if w_r is not None:
+                out.addmm_(root, w_r.t())
+            if b_l is not None:
+                out += b_l
         ctx.save_for_backward(x, agg, w_l, w_r if w_r is not None else w_l.new_empty(0))
         ctx.hc = (ptr, idx, hmap, hsize, R, num_edge, b_l is not None, w_r is not None, sink)
         ctx.view = view if view is not None and view.covers(R, x.shape[0]) else None
@@ -111,11 +116,14 @@ class _SageConvFunction(torch.autograd.Function):
             return (None,) * 13
         g_out = g_out.contiguous()
         need = ctx.needs_input_grad
-        g_agg = g_out @ w_l                                   # gradient reaching the aggregation output
-        if sink is not None and sink.target is not None:
-            his = sink.target()
-            if his is not None:
-                his.grad = g_agg
+        own = be.linear_supported(g_out, w_l, w_r if has_root else None)
+        # gradient reaching the aggregation output; a feature layer that keeps none has no use for it
+        his = sink.target() if sink is not None and sink.target is not None else None
+        g_agg = None
+        if need[0] or his is not None:
+            g_agg = be.linear(g_out, w_l, transposed=True) if own else g_out @ w_l
+        if his is not None:
+            his.grad = g_agg
         g_bl = _column_sums(g_out) if has_bias and need[2] else None
         g_wl = g_wr = None
         root = None
@@ -138,7 +146,9 @@ class _SageConvFunction(torch.autograd.Function):
                 tr = be.build_transpose(ptr, idx, hmap, R, n_src, num_edge=num_edge, want_edges=False)
                 g_x, _, _ = be._aggr_bwd(ptr, idx, tr, g_agg, hmap, None, x, False, None, hsize, R, n_src,
                                          want_hist_grad=False)
-            if has_root:
+            if has_root and own:
+                be.linear(g_out, w_r, transposed=True, out=g_x[:R])
+            elif has_root:
                 g_x[:R].addmm_(g_out, w_r)
             if g_x.dtype != x.dtype:
                 g_x = g_x.to(x.dtype)

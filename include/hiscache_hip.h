@@ -669,6 +669,19 @@ int hc_bn_relu_eval(const float *x, const float *bias, const float *gamma, const
                     const float *running_mean, const float *running_var, float eps, float *y, int64_t n, int64_t C,
                     void *stream);
 
+/* hc_linear: out[M, N] = a0 op(w0) + a1 op(w1) + add + bias for row-major fp32
+ * matrices a0, a1 [M, K]: a layer's `lin_l(out) + lin_r(x[:n])` and its input
+ * gradients (hiscache/history_model.py:94-98).  w_is_kn == 0: w [N, K], as
+ * torch.nn.Linear keeps a weight, op = transpose; != 0: w [K, N] as it is.
+ * a1 and w1, add [M, N] and bias [N] may be NULL; add may be out (the product is
+ * added to what is there).  Every product is summed in fp32 from zero in
+ * ascending k, then first + second + add + bias: a row's result does not depend
+ * on M.  HC_EUNSUPPORTED: N or K above 2^20, N * K of 2^30 or more, more than
+ * 2^24 tiles. */
+int hc_linear(const float *a0, const float *w0, const float *a1, const float *w1, int w_is_kn,
+              const float *bias, const float *add, float *out, int64_t M, int64_t N, int64_t K,
+              void *stream);
+
 /* hc_weight_grad: the gradient of a layer's linear maps, dw[H, F] = g^T x for
  * g [n, H] and x [n, F] (fp32, row-major, contiguous) -- what autograd computes
  * for `self.lin_l(out)` and `self.lin_r(x[:num_node])`
