@@ -4,15 +4,17 @@
 
 namespace {
 
-// Notes the long rows of a tile in the two lists.
+// Notes the long rows of a tile in the lists.
 __global__ __launch_bounds__(HC_BLOCK) void fwd_find_long(FwdArgs a) {
-  __shared__ int n_near, n_far;
-  if (threadIdx.x == 0) n_near = n_far = 0;
+  __shared__ int n_near, n_far, n_staged;
+  if (threadIdx.x == 0) n_near = n_far = n_staged = 0;
   __syncthreads();
   const int64_t total = a.ptr[a.R] - a.ptr[0];
   const int64_t far_above = fwd_far_above(a, total);
   const int64_t first = (int64_t)blockIdx.x * a.tile;
   const int64_t last = first + a.tile < a.R ? first + a.tile : a.R;
+  const int64_t staged_above = a.stage != nullptr ? fwd_staged_above(a, total) : INT64_MAX;
+  const int64_t staged0 = a.stage != nullptr ? seg_part(a.ptr, first, staged_above) : 0;
   const int64_t near0 = seg_part(a.ptr, first, a.slice_above), far0 = seg_part(a.ptr, first, far_above);
   constexpr int ITEMS = 4;
   for (int64_t r0 = first; r0 < last; r0 += HC_BLOCK * ITEMS) {
@@ -26,7 +28,10 @@ __global__ __launch_bounds__(HC_BLOCK) void fwd_find_long(FwdArgs a) {
     for (int it = 0; it < ITEMS; ++it) {
       const int64_t r = r0 + it * HC_BLOCK + threadIdx.x;
       if (deg[it] <= a.slice_above || (a.hmap != nullptr && a.hmap[r] != -1)) continue;
-      if (deg[it] > far_above) {
+      if (deg[it] > staged_above) {
+        const int64_t p = staged0 + atomicAdd(&n_staged, 1);
+        if (p < a.staged.cap) a.staged.item[p] = (int32_t)r;
+      } else if (deg[it] > far_above) {
         const int64_t p = far0 + atomicAdd(&n_far, 1);
         if (p < a.far.cap) a.far.item[p] = (int32_t)r;
       } else {
@@ -39,11 +44,13 @@ __global__ __launch_bounds__(HC_BLOCK) void fwd_find_long(FwdArgs a) {
   if (threadIdx.x == 0) {
     if (blockIdx.x == 0) {
       a.plan->far_above = far_above;
+      a.plan->staged_above = staged_above;
       a.plan->listed = total / (far_above + 1) <= a.far.cap &&
                        (a.split_above == 0 || total / (a.slice_above + 1) <= a.near.cap) ? 1 : 0;
     }
     a.near.count[blockIdx.x] = n_near;
     a.far.count[blockIdx.x] = n_far;
+    if (a.stage != nullptr) a.staged.count[blockIdx.x] = n_staged;
   }
 }
 
@@ -64,6 +71,20 @@ struct FwdScratch {
 // sources).  Either part may be absent (0 bytes).
 constexpr size_t FWD_COUNT_BYTES = 2 * SEG_MAX_REGIONS * sizeof(int32_t);
 constexpr size_t FWD_HEAD_BYTES = FWD_COUNT_BYTES + 256;
+// For rows of several heads, 4 adjacent columns of a row in one head: the list of the rows to be staged and the room for their
+// copies, in front of the other lists.  Blocks of fewer edges are not worth the launch that copies (3 us where there is
+// nothing to copy); a copy of all edges is not needed, and copies of more than 96 MB would be bound by the memory
+// like the launch itself.
+constexpr int64_t FWD_STAGE_MIN_EDGES = (int64_t)1 << 18;
+constexpr int64_t FWD_STAGE_BYTES = (int64_t)96 << 20;
+constexpr size_t FWD_STAGE_LIST_BYTES = (SEG_MAX_REGIONS + FWD_STAGED_ROWS) * sizeof(int32_t);
+size_t fwd_stage_bytes(int mode, int64_t E, int64_t F, int64_t n_head) {
+  if (mode != HC_SUBST_ROW || n_head <= 1 || F % FWD_STAGED_COLS != 0 || E < FWD_STAGE_MIN_EDGES || F > 0x3fffffffLL / n_head) return 0;
+  const int64_t edge = (F + 1) * n_head * (int64_t)sizeof(float);
+  const int64_t most = E + FWD_STAGED_ROWS * FWD_STAGED_UNIT;      // every row's copy is a whole number of units
+  return FWD_STAGE_LIST_BYTES + (size_t)(most < FWD_STAGE_BYTES / edge ? hc_align_up((size_t)(most * edge), 256) : FWD_STAGE_BYTES);
+}
+
 struct FwdWsLayout {
   size_t list_bytes, bits_bytes, total;
 };
@@ -93,8 +114,18 @@ __global__ __launch_bounds__(HC_BLOCK) void fwd_src_bits(const int64_t *__restri
 }
 
 // The lists' launch and the front blocks of the main one.  `max_degree` >= 0: no row has more edges.
-int fwd_prepare_lists(FwdArgs &a, bool src_mode, FwdScratch ws, int64_t n_src, int64_t max_degree, hipStream_t st) {
+int fwd_prepare_lists(FwdArgs &a, bool src_mode, FwdScratch ws, int64_t n_src, int64_t max_degree, size_t stage_bytes,
+                      hipStream_t st) {
   const bool ws_ok = ws.ptr != nullptr && reinterpret_cast<uintptr_t>(ws.ptr) % 256 == 0;
+  if (ws_ok && stage_bytes > 0 && ws.bytes > stage_bytes + FWD_HEAD_BYTES && max_degree < 0 && a.R <= 0x7fffffffLL) {
+    a.staged.count = static_cast<int32_t *>(ws.ptr);
+    a.staged.item = a.staged.count + SEG_MAX_REGIONS;
+    a.staged.cap = FWD_STAGED_ROWS;
+    a.stage = reinterpret_cast<float *>(a.staged.item + FWD_STAGED_ROWS);
+    a.stage_floats = (int64_t)((stage_bytes - FWD_STAGE_LIST_BYTES) / sizeof(float));
+    ws.ptr = static_cast<char *>(ws.ptr) + stage_bytes;
+    ws.bytes -= stage_bytes;
+  }
   // the caller sized the workspace with hc_aggr_fwd_workspace_bytes(mode, R, E, n_src): the bitmap, when
   // there is one, takes the last bits_bytes bytes and the lists what lies in front of it
   size_t room = ws_ok ? ws.bytes : 0;
@@ -131,6 +162,7 @@ int fwd_prepare_lists(FwdArgs &a, bool src_mode, FwdScratch ws, int64_t n_src, i
   } else if (a.R <= FWD_SELF_ROWS) {
     a.front = FWD_SELF_FRONT_BLOCKS;
   }
+  if (a.n_tiles == 0) a.stage = nullptr;       // no room for the lists behind the copies
   return HC_OK;
 }
 
@@ -160,6 +192,20 @@ extern "C" int hc_aggr_fwd_bounded(int mode, const int64_t *ptr, const int64_t *
                                    int64_t hsize, const float *edge_value, int64_t n_head, float *vout,
                                    int64_t R, int64_t F, int64_t n_src, int64_t max_degree, void *workspace,
                                    size_t workspace_bytes, void *stream) {
+  return hc_aggr_fwd_for(mode, ptr, idx, vin, in_dtype, hmap, hbuf, hist_dtype, hsize, edge_value, n_head, vout, R, F,
+                         n_src, -1, max_degree, workspace, workspace_bytes, stream);
+}
+
+extern "C" size_t hc_aggr_fwd_workspace_bytes_for(int mode, int64_t R, int64_t E, int64_t n_src, int64_t F, int64_t n_head) {
+  if (R < 0 || E < 0 || n_src < 0 || F < 1 || n_head < 1) return 0;
+  const size_t lists = fwd_ws_layout(mode, R, E, n_src).total;
+  return lists > 0 ? lists + fwd_stage_bytes(mode, E, F, n_head) : 0;
+}
+
+extern "C" int hc_aggr_fwd_for(int mode, const int64_t *ptr, const int64_t *idx, const void *vin, int in_dtype,
+                               const int64_t *hmap, const void *hbuf, int hist_dtype, int64_t hsize,
+                               const float *edge_value, int64_t n_head, float *vout, int64_t R, int64_t F, int64_t n_src,
+                               int64_t E, int64_t max_degree, void *workspace, size_t workspace_bytes, void *stream) {
   const FwdScratch ws{workspace, workspace ? workspace_bytes : 0};
   HC_REQUIRE(R >= 0 && F > 0 && n_src >= 0 && n_head >= 1);
   if (R == 0) return HC_OK;
@@ -198,7 +244,8 @@ extern "C" int hc_aggr_fwd_bounded(int mode, const int64_t *ptr, const int64_t *
   a.split_above = n_head > 1 ? 0 : HC_LONG_ROW_EDGES;
   a.slice_above = n_head > 1 ? FWD_HEAD_SLICE_EDGES : HC_LONG_ROW_EDGES;
   hipStream_t st = static_cast<hipStream_t>(stream);
-  const int rc = fwd_prepare_lists(a, src_mode != 0 && hmap != nullptr, ws, n_src, max_degree, st);
+  const int rc = fwd_prepare_lists(a, src_mode != 0 && hmap != nullptr, ws, n_src, max_degree,
+                                   fwd_stage_bytes(mode, E, F, n_head), st);
   if (rc != HC_OK) return rc;
   if (in_dtype == HC_F32) return fwd_dispatch_f32(a, src_mode != 0, (int)n_head, st);
   if (in_dtype == HC_F16) return fwd_dispatch_f16(a, src_mode != 0, (int)n_head, st);

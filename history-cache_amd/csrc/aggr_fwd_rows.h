@@ -27,6 +27,7 @@
 #include "seg_list.h"
 
 #include <type_traits>
+#include <utility>
 
 // Rows with more edges than this are summed as four quarters (mean, single-head weights).
 // The oracle applies the same rule; the header documents it.
@@ -72,8 +73,21 @@ constexpr int W_NONE = 0, W_EDGE = 1, W_EDGE_HEAD = 2;
 // What the main launch does with the lists.  (Worked out by each of its waves, with two 64-bit divisions, it took 1 M
 // rows of 3 edges of 64 columns from 443 to 526 us.)
 struct FwdPlan {
-  int64_t far_above, listed;
+  int64_t far_above, listed, staged_above;
 };
+
+// Rows of several heads are never split: the longest of them is one chain of additions, and a wave that follows it
+// through the matrix gets 64 lines a microsecond.  Where such a row takes longer than everything else in the launch, a
+// launch of its own copies its source rows side by side first (fwd_stage), in slices of 4 columns, four edges of a
+// column adjacent: a cache line then holds eight edges of a slice instead of one, 32 compute units share a row of
+// 128 columns, and a wave reads ahead in whole lines.  Same order, same bits.  1 M edges x 128 fp32
+// columns with a row of 27 000: 428 us, now 127 and 13 for the copy.  In slices of 8 columns 142 us, and 185 without
+// reading the next values from the LDS while some are summed.  Four units ahead keep the kernel at 119 registers; six
+// take 129, and with them a wave per SIMD, at the same time.
+constexpr int FWD_STAGED_COLS = 4;
+constexpr int FWD_STAGED_UNIT = 64;         // edges per read of a slice: a kilobyte
+constexpr int FWD_STAGED_ROWS = 512;        // at most
+constexpr int64_t FWD_STAGED_MIN = 2048;    // edges: below, the copy takes longer than it saves
 
 struct FwdArgs {
   const int64_t *ptr, *idx;
@@ -92,6 +106,9 @@ struct FwdArgs {
   int64_t split_above;        // rows with more edges are summed as four quarters (0: never)
   int64_t slice_above;        // rows with more edges belong to the front blocks, when there are any (0: none)
   SegList near, far;          // whole-row and slice-wise tasks of the front blocks
+  SegList staged;             // rows that are copied side by side first, ...
+  float *stage;               // ... and the room for that (several heads; nullable)
+  int64_t stage_floats;
   int n_tiles;                // tiles of the lists; 0: every front block looks the rows through itself
   int64_t tile;
   FwdPlan *plan;              // with lists: written by the launch that makes them
@@ -104,6 +121,227 @@ struct FwdArgs {
 __device__ __forceinline__ int64_t fwd_far_above(const FwdArgs &a, int64_t total) {
   const int64_t t = total / 8192;
   return a.split_above > 0 && t > a.slice_above ? t : a.slice_above;
+}
+
+// Rows above this many edges are staged: alone they would take longer (64 edges a microsecond) than the launch moves its
+// rows' bytes (5 TB/s).  At most FWD_STAGED_ROWS - 1 rows are that long.
+__device__ __forceinline__ int64_t fwd_staged_above(const FwdArgs &a, int64_t total) {
+  int64_t t = total / 20000 * a.F;
+  if (t < total / FWD_STAGED_ROWS) t = total / FWD_STAGED_ROWS;
+  return t < FWD_STAGED_MIN ? FWD_STAGED_MIN : t;
+}
+
+// The staged rows: row i's copy starts at unit unit[i] (of FWD_STAGED_UNIT edges), F + n_head floats per edge: the row's
+// slices one after the other, then its weights, head by head.
+struct FwdStaged {
+  int32_t row[FWD_STAGED_ROWS];
+  int32_t unit[FWD_STAGED_ROWS + 1];
+  int32_t sum[HC_WAVES_PER_BLOCK];
+};
+
+// Exclusive sums of two values per thread over the block; `total` in every thread.
+__device__ __forceinline__ void fwd_block_scan(int32_t *sum, int lane, int wave, int a0, int a1, int &x0, int &x1, int &total) {
+  int incl = a0 + a1;
+#pragma unroll
+  for (int d = 1; d < HC_WAVE; d <<= 1) {
+    const int y = __shfl_up(incl, d, HC_WAVE);
+    if (lane >= d) incl += y;
+  }
+  __syncthreads();
+  if (lane == HC_WAVE - 1) sum[wave] = incl;
+  __syncthreads();
+  x0 = incl - a0 - a1;
+  total = 0;
+#pragma unroll
+  for (int w = 0; w < HC_WAVES_PER_BLOCK; ++w) {
+    if (w < wave) x0 += sum[w];
+    total += sum[w];
+  }
+  x1 = x0 + a0;
+}
+
+// Reads the list of the rows to be staged (all threads of the block).  Returns how many of them have room; they are the
+// first of the list, `*n` rows.  Every block arrives at the same result.
+__device__ __forceinline__ int fwd_read_staged(const FwdArgs &a, FwdStaged &s, int lane, int wave, int *n) {
+  static_assert(SEG_MAX_REGIONS == 2 * HC_BLOCK && FWD_STAGED_ROWS == 2 * HC_BLOCK, "two tiles and two rows per thread");
+  *n = 0;
+  if (a.plan->listed == 0) return 0;
+  const int64_t above = a.plan->staged_above;
+  const int t = (int)threadIdx.x;
+  const int c0 = 2 * t < a.n_tiles ? a.staged.count[2 * t] : 0, c1 = 2 * t + 1 < a.n_tiles ? a.staged.count[2 * t + 1] : 0;
+  int x0, x1, rows;
+  fwd_block_scan(s.sum, lane, wave, c0, c1, x0, x1, rows);
+  if (rows == 0) return 0;
+  for (int k = 0; k < c0 + c1; ++k) {
+    const int64_t part = seg_part(a.ptr, (int64_t)(k < c0 ? 2 * t : 2 * t + 1) * a.tile, above);
+    s.row[x0 + k] = a.staged.item[part + (k < c0 ? k : k - c0)];
+  }
+  __syncthreads();
+  const auto units = [&](int i) -> int {
+    if (i >= rows) return 0;
+    const int64_t r = s.row[i];
+    return (int)((a.ptr[r + 1] - a.ptr[r] + FWD_STAGED_UNIT - 1) / FWD_STAGED_UNIT);
+  };
+  const int u0 = units(2 * t), u1 = units(2 * t + 1);
+  int all;
+  fwd_block_scan(s.sum, lane, wave, u0, u1, x0, x1, all);
+  s.unit[2 * t] = x0;
+  s.unit[2 * t + 1] = x1;
+  if (t == HC_BLOCK - 1) s.unit[FWD_STAGED_ROWS] = all;
+  const int64_t room = a.stage_floats / (FWD_STAGED_UNIT * (a.F + a.n_head));
+  const int fit = __syncthreads_count(2 * t < rows && x0 + u0 <= room) + __syncthreads_count(2 * t + 1 < rows && x1 + u1 <= room);
+  *n = rows;
+  return fit;
+}
+
+// Copies the staged rows side by side, widened to fp32: a wave takes 64 edges, 64 columns at a time, a lane one column.
+template <typename T>
+__global__ __launch_bounds__(HC_BLOCK) void fwd_stage(FwdArgs a) {
+  __shared__ FwdStaged s;
+  const int lane = hc_lane(), wave = hc_wave_in_block();
+  int n;
+  const int fit = fwd_read_staged(a, s, lane, wave, &n);
+  if (fit == 0) return;
+  const int units = s.unit[fit];
+  for (int u = (int)blockIdx.x * HC_WAVES_PER_BLOCK + wave; u < units; u += (int)gridDim.x * HC_WAVES_PER_BLOCK) {
+    int lo = 0, hi = fit - 1;
+    while (lo < hi) {
+      const int mid = (lo + hi + 1) >> 1;
+      if (s.unit[mid] <= u) lo = mid;
+      else hi = mid - 1;
+    }
+    lo = __builtin_amdgcn_readfirstlane(lo);
+    const int64_t row = s.row[lo], first = a.ptr[row];
+    const int64_t e0 = (int64_t)(u - s.unit[lo]) * FWD_STAGED_UNIT, deg = a.ptr[row + 1] - first;
+    const int64_t len = (int64_t)(s.unit[lo + 1] - s.unit[lo]) * FWD_STAGED_UNIT;
+    float *to = a.stage + (int64_t)s.unit[lo] * FWD_STAGED_UNIT * (a.F + a.n_head);
+    // behind the row's end: its last edge again, not added
+    static_assert(FWD_STAGED_UNIT == HC_WAVE, "a lane per edge");
+    const int64_t e = e0 + lane < deg ? e0 + lane : deg - 1;
+    const int64_t at = a.idx[first + e] * a.F;
+    // (lanes behind the row's last column read it again: the lanes' ids are broadcast, so all must be here)
+    for (int64_t c0 = 0; c0 < a.F; c0 += HC_WAVE) {
+      const int64_t c = c0 + lane < a.F ? c0 + lane : a.F - 1;
+      float *col = to + c / FWD_STAGED_COLS * len * FWD_STAGED_COLS + e0 * FWD_STAGED_COLS + c % FWD_STAGED_COLS * 4;
+      constexpr int AT_ONCE = 32;
+      for (int i0 = 0; i0 < FWD_STAGED_UNIT; i0 += AT_ONCE) {
+        T v[AT_ONCE];
+#pragma unroll
+        for (int i = 0; i < AT_ONCE; ++i) v[i] = static_cast<const T *>(a.vin)[hc_readlane64(at, i0 + i) + c];
+#pragma unroll
+        for (int i = 0; i < AT_ONCE; i += 4) {
+          const float o[4] = {hc_to_f32<T>(v[i]), hc_to_f32<T>(v[i + 1]), hc_to_f32<T>(v[i + 2]), hc_to_f32<T>(v[i + 3])};
+          if (c0 + lane < a.F) hc_store_f32<4>(col + (i0 + i) * FWD_STAGED_COLS, o);
+        }
+      }
+    }
+    float *w = to + len * a.F;
+    for (int h = 0; h < a.n_head; ++h) w[h * len + e0 + lane] = a.ev[(first + e) * a.n_head + h];
+  }
+}
+
+template <int N>
+using FwdInt = std::integral_constant<int, N>;
+
+template <int... I, typename F>
+__device__ __forceinline__ void fwd_each(std::integer_sequence<int, I...>, F f) {
+  (f(FwdInt<I>()), ...);
+}
+
+// A wave's LDS for one slice of a staged row: two units of 64 edges x 4 columns, and their weights.
+struct FwdSlice {
+  float x[2][FWD_STAGED_UNIT * FWD_STAGED_COLS];
+  float w[2][FWD_STAGED_UNIT];
+};
+
+// Columns 4 slice .. 4 slice + 3 of staged row i, summed in edge order by one wave: every lane reads 16 bytes of a unit
+// (four units ahead, into registers) and passes them through the LDS; lane l then adds up column l % 4.
+__device__ __forceinline__ void fwd_sum_staged(const FwdArgs &a, const FwdStaged &s, FwdSlice &b, int i, int slice, int lane) {
+  constexpr int AHEAD = 4;
+  typedef float quad __attribute__((ext_vector_type(4)));
+  const int64_t row = s.row[i], deg = a.ptr[row + 1] - a.ptr[row];
+  const int units = s.unit[i + 1] - s.unit[i];
+  const int64_t len = (int64_t)units * FWD_STAGED_UNIT;
+  const float *from = a.stage + (int64_t)s.unit[i] * FWD_STAGED_UNIT * (a.F + a.n_head);
+  const int h = (int)((int64_t)slice * FWD_STAGED_COLS / (a.F / a.n_head));
+  const quad *x = reinterpret_cast<const quad *>(from + (int64_t)slice * len * FWD_STAGED_COLS) + lane;
+  const float *w = from + len * a.F + h * len + lane;
+  quad rx[AHEAD];
+  float rw[AHEAD];
+  constexpr std::make_integer_sequence<int, AHEAD> slots{};      // (a loop's counter as an index sends the arrays to scratch memory)
+  const auto load = [&](auto r, int u) {
+    u = u < units ? u : units - 1;
+    rx[r.value] = x[(int64_t)u * HC_WAVE];
+    rw[r.value] = w[(int64_t)u * FWD_STAGED_UNIT];
+  };
+  const auto pass = [&](auto r) {
+    *reinterpret_cast<quad *>(&b.x[r.value & 1][lane * 4]) = rx[r.value];
+    b.w[r.value & 1][lane] = rw[r.value];
+  };
+  float acc = 0.0f;
+  const int c = lane & (FWD_STAGED_COLS - 1);
+  // A quarter of a unit: the values of the next quarter are read from the LDS while one is summed.
+  constexpr int PART = FWD_STAGED_UNIT / 4 / 4;
+  quad v[2][PART], m[2][PART];
+  const auto read = [&](auto r, auto part) {
+#pragma unroll
+    for (int q = 0; q < PART; ++q) {
+      v[part.value & 1][q] = *reinterpret_cast<const quad *>(&b.x[r.value & 1][((part.value * PART + q) * FWD_STAGED_COLS + c) * 4]);
+      m[part.value & 1][q] = *reinterpret_cast<const quad *>(&b.w[r.value & 1][(part.value * PART + q) * 4]);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  const auto add = [&](auto part) {
+#pragma unroll
+    for (int q = 0; q < PART; ++q)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) acc = __fmaf_rn(v[part.value & 1][q][e], m[part.value & 1][q][e], acc);
+    asm("" : "+v"(acc));      // here, not behind the next reads
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  constexpr FwdInt<0> q0;
+  constexpr FwdInt<1> q1;
+  constexpr FwdInt<2> q2;
+  constexpr FwdInt<3> q3;
+  fwd_each(slots, [&](auto r) { load(r, r.value); });
+  pass(q0);
+  const int whole = (int)(deg / FWD_STAGED_UNIT);
+  int u = 0;
+  read(q0, q0);
+  for (; u + AHEAD <= whole; u += AHEAD)
+    fwd_each(slots, [&](auto r) {
+      constexpr FwdInt<(r.value + 1) % AHEAD> next;
+      load(r, u + r.value + AHEAD);
+      read(r, q1);
+      add(q0);
+      read(r, q2);
+      add(q1);
+      read(r, q3);
+      add(q2);
+      pass(next);
+      read(next, q0);
+      add(q3);
+    });
+  // the last units, which are on their way, and the last edges
+  fwd_each(slots, [&](auto r) {
+    const int64_t left = deg - (int64_t)(u + r.value) * FWD_STAGED_UNIT;
+    if (left <= 0) return;
+    if (r.value > 0) pass(r);
+    if (left >= FWD_STAGED_UNIT) {
+      read(r, q0);
+      read(r, q1);
+      add(q0);
+      read(r, q2);
+      add(q1);
+      read(r, q3);
+      add(q2);
+      add(q3);
+      return;
+    }
+    for (int e = 0; e < (int)left; ++e)
+      acc = __fmaf_rn(b.x[r.value & 1][(e / 4 * FWD_STAGED_COLS + c) * 4 + e % 4], b.w[r.value & 1][e], acc);
+  });
+  if (lane < FWD_STAGED_COLS) a.vout[row * a.F + slice * FWD_STAGED_COLS + lane] = acc;
 }
 
 // Address of the neighbour row that edge `e` reads (and its weight).
@@ -159,9 +397,6 @@ struct FwdCols {
     }
   }
 };
-
-template <int N>
-using FwdInt = std::integral_constant<int, N>;
 
 // Sum of the neighbour rows of edges [begin, end), added to acc in edge order by the calling wave.
 // SRC (per-source substitution): neighbour rows and ids are loaded with the non-temporal hint.  Every edge
@@ -478,7 +713,8 @@ constexpr int FWD_SELF_ITEMS = 512;
 // wave per task), then the other listed rows as whole rows.
 template <typename T, typename TH, int VEC, int CHUNKS, int UNROLL, bool SRC, int WMODE>
 __device__ __forceinline__ void fwd_front(const FwdArgs &a, int64_t far_above, int lane, int wave,
-                                          float (*part)[HC_WAVE * VEC * CHUNKS], int *self_rows, int *self_n) {
+                                          float (*part)[HC_WAVE * VEC * CHUNKS], int *self_rows, int *self_n,
+                                          FwdStaged *staged, FwdSlice *slice) {
   constexpr int SV = sizeof(T) == 2 && VEC > 1 ? 2 : 1;
   constexpr int SL = FWD_SLICE_LANES * SV;
   const int ns = (int)((a.F + SL - 1) / SL);
@@ -531,15 +767,14 @@ __device__ __forceinline__ void fwd_front(const FwdArgs &a, int64_t far_above, i
   };
   const int64_t tasks = (int64_t)n_far * ns;
   if constexpr (WMODE == W_EDGE_HEAD) {                  // rows of several heads are never split: one wave per task
-    for (int64_t t = (int64_t)wave * a.front + blockIdx.x; t < tasks; t += (int64_t)HC_WAVES_PER_BLOCK * a.front) {
-      const int64_t row = far_row((int)(t / ns));
+    const auto slice_of = [&](int64_t row, int sl) {
       bool on;
-      const uint32_t c = columns((int)(t % ns), on);
+      const uint32_t c = columns(sl, on);
       const int64_t b = a.ptr[row], e = a.ptr[row + 1];
       float s[SV];
       // every column of the slice in one head: its weights are staged with the ids, 64 at a time
       const int fh = (int)(a.F / a.n_head);
-      const int c0 = (int)(t % ns) * SL;
+      const int c0 = sl * SL;
       const int c1 = (c0 + SL < a.F ? c0 + SL : (int)a.F) - 1;
       if (c0 / fh == c1 / fh)
         fwd_slice_any<T, TH, SV, SRC, W_EDGE, 32>(a, c, b, e, lane, a.ev + c0 / fh, a.n_head, s);
@@ -548,7 +783,20 @@ __device__ __forceinline__ void fwd_front(const FwdArgs &a, int64_t far_above, i
 #pragma unroll
       for (int i = 0; i < SV; ++i)
         if (on) a.vout[row * a.F + c + i] = s[i];
+    };
+    if (a.stage != nullptr && seg_index(a.staged.count, a.n_tiles, lane).total > 0) {
+      int rows;
+      const int fit = fwd_read_staged(a, *staged, lane, wave, &rows);
+      const int pieces = (int)(a.F / FWD_STAGED_COLS);
+      if (wave == 0)
+        for (int64_t t = blockIdx.x; t < (int64_t)fit * pieces; t += a.front)
+          fwd_sum_staged(a, *staged, *slice, (int)(t / pieces), (int)(t % pieces), lane);
+      // rows that found no room are summed like the other long ones
+      for (int64_t t = (int64_t)wave * a.front + blockIdx.x; t < (int64_t)(rows - fit) * ns; t += (int64_t)HC_WAVES_PER_BLOCK * a.front)
+        slice_of((int64_t)staged->row[fit + (int)(t / ns)], (int)(t % ns));
     }
+    for (int64_t t = (int64_t)wave * a.front + blockIdx.x; t < tasks; t += (int64_t)HC_WAVES_PER_BLOCK * a.front)
+      slice_of(far_row((int)(t / ns)), (int)(t % ns));
     return;
   } else {
     for (int64_t t = blockIdx.x; t < tasks; t += a.front) {
@@ -600,6 +848,14 @@ __device__ __forceinline__ void fwd_block(const FwdArgs &a) {
   __shared__ float part[HC_WAVES_PER_BLOCK - 1][HC_WAVE * VEC * CHUNKS];
   __shared__ int self_rows[FWD_SELF_ITEMS];
   __shared__ int long_rows[FWD_ROWS_PER_BLOCK];    // (front blocks: the waves' counts)
+  FwdStaged *staged = nullptr;
+  FwdSlice *slice = nullptr;
+  if constexpr (WMODE == W_EDGE_HEAD) {
+    __shared__ FwdStaged staged_s;
+    __shared__ __attribute__((aligned(16))) FwdSlice slice_s;
+    staged = &staged_s;
+    slice = &slice_s;
+  }
   __shared__ int n_long_s;
   const int lane = hc_lane();
   const int wave = hc_wave_in_block();
@@ -618,7 +874,8 @@ __device__ __forceinline__ void fwd_block(const FwdArgs &a) {
     if constexpr (PART != FWD_BODY) {
       if ((int)blockIdx.x < a.front) {
         if (listed)
-          fwd_front<T, TH, VEC, CHUNKS, UNROLL, SRC, WMODE>(a, far_above, lane, wave, part, self_rows, long_rows);
+          fwd_front<T, TH, VEC, CHUNKS, UNROLL, SRC, WMODE>(a, far_above, lane, wave, part, self_rows, long_rows, staged,
+                                                               slice);
         return;
       }
     }
@@ -714,6 +971,8 @@ __attribute__((visibility("hidden"))) int fwd_dispatch_bf16(FwdArgs &a, bool src
 #ifdef FWD_INSTANTIATE
 namespace {
 
+constexpr int FWD_STAGE_BLOCKS = 512;
+
 template <typename T, int VEC, int CHUNKS>
 int launch_rows(const FwdArgs &a, bool src_mode, hipStream_t st) {
   constexpr int per = VEC * CHUNKS;
@@ -730,7 +989,10 @@ int launch_rows(const FwdArgs &a, bool src_mode, hipStream_t st) {
       fwd_rows<T, TH, VEC, CHUNKS, UNROLL, true, W_NONE, FWD_FRONT><<<dim3((unsigned)a.front), block, 0, st>>>(a);      \
     fwd_rows<T, TH, VEC, CHUNKS, UNROLL, true, W_NONE, FWD_BODY><<<dim3((unsigned)row_blocks), block, 0, st>>>(a);      \
   }
-  if (a.ev != nullptr && a.n_head > 1) HC_FWD_LAUNCH_WIDE(false, W_EDGE_HEAD);
+  if (a.ev != nullptr && a.n_head > 1) {
+    if (a.stage != nullptr) fwd_stage<T><<<dim3(FWD_STAGE_BLOCKS), block, 0, st>>>(a);
+    HC_FWD_LAUNCH_WIDE(false, W_EDGE_HEAD);
+  }
   else if (a.ev != nullptr) HC_FWD_LAUNCH_WIDE(false, W_EDGE);
   else if (src_mode && a.hmap != nullptr) {
     // the table of a per-source substitution may be narrower than fp32 features

@@ -55,6 +55,9 @@ _SIGNATURES = {
                              _c_p, _c_i64, _c_i64, _c_i64, _c_p, _c_sz, _c_p]),
     "hc_aggr_fwd_bounded": (_c_int, [_c_int, _c_p, _c_p, _c_p, _c_int, _c_p, _c_p, _c_int, _c_i64, _c_p, _c_i64,
                                      _c_p, _c_i64, _c_i64, _c_i64, _c_i64, _c_p, _c_sz, _c_p]),
+    "hc_aggr_fwd_workspace_bytes_for": (_c_sz, [_c_int, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64]),
+    "hc_aggr_fwd_for": (_c_int, [_c_int, _c_p, _c_p, _c_p, _c_int, _c_p, _c_p, _c_int, _c_i64, _c_p, _c_i64,
+                                 _c_p, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_p, _c_sz, _c_p]),
     "hc_aggr_fwd_long_row_edges": (_c_i64, [_c_i64, _c_int]),
     "hc_transpose_workspace_bytes": (_c_sz, [_c_i64, _c_i64, _c_i64]),
     "hc_build_transpose": (_c_int, [_c_p, _c_p, _c_p, _c_p, _c_i64, _c_i64, _c_i64, _c_p, _c_p, _c_p, _c_p,
@@ -308,12 +311,12 @@ def _aggr_fwd(mode, ptr, idx, x, hmap, hbuf, hsize, edge_value, num_node, max_de
     bound = -1 if max_degree is None else int(max_degree)
     ws_bytes = 0
     if mode == SUBST_SRC or not 0 <= bound <= MAX_DEGREE_WITHOUT_LISTS:
-        ws_bytes = int(lib.hc_aggr_fwd_workspace_bytes(mode, R, idx.numel(), n_src))
+        ws_bytes = int(lib.hc_aggr_fwd_workspace_bytes_for(mode, R, idx.numel(), n_src, F, n_head))
     ws = _workspace(ws_bytes, x.device) if ws_bytes > 0 else None
-    rc = lib.hc_aggr_fwd_bounded(mode, _ptr(ptr), _ptr(idx), _ptr(x), _float_dtype(x, "input"),
-                                 _ptr(hmap), _ptr(hbuf), _float_dtype(hbuf, "history_buffer") if hmap is not None else 0,
-                                 int(hsize), _ptr(edge_value), n_head, _ptr(out), R, F, n_src, bound, _ptr(ws), ws_bytes,
-                                 _stream())
+    rc = lib.hc_aggr_fwd_for(mode, _ptr(ptr), _ptr(idx), _ptr(x), _float_dtype(x, "input"), _ptr(hmap), _ptr(hbuf),
+                             _float_dtype(hbuf, "history_buffer") if hmap is not None else 0, int(hsize),
+                             _ptr(edge_value), n_head, _ptr(out), R, F, n_src, idx.numel(), bound, _ptr(ws), ws_bytes,
+                             _stream())
     _check(rc, "hc_aggr_fwd")
     return out
 

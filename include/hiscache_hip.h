@@ -105,6 +105,18 @@ int hc_aggr_fwd_bounded(int mode, const int64_t *ptr, const int64_t *idx, const 
                         int64_t R, int64_t F, int64_t n_src, int64_t max_degree, void *workspace,
                         size_t workspace_bytes, void *stream);
 
+/* hc_aggr_fwd_bounded for callers that know an upper bound E of ptr[R]
+ * (negative: unknown, as hc_aggr_fwd_bounded) and give a workspace of
+ * hc_aggr_fwd_workspace_bytes_for(mode, R, E, n_src, F, n_head) bytes, with the
+ * same E.  Same results.  With several heads of a multiple of 4 columns each and
+ * 2^18 edges or more the workspace also holds copies of the source rows of the
+ * longest rows (up to 96 MB), which shortens their sums. */
+size_t hc_aggr_fwd_workspace_bytes_for(int mode, int64_t R, int64_t E, int64_t n_src, int64_t F, int64_t n_head);
+int hc_aggr_fwd_for(int mode, const int64_t *ptr, const int64_t *idx, const void *vin, int in_dtype,
+                    const int64_t *hmap, const void *hbuf, int hist_dtype, int64_t hsize,
+                    const float *edge_value, int64_t n_head, float *vout, int64_t R, int64_t F, int64_t n_src,
+                    int64_t E, int64_t max_degree, void *workspace, size_t workspace_bytes, void *stream);
+
 /* The long-row threshold T that hc_aggr_fwd applies to a mean or single-head
  * weighted aggregation with rows of F elements of in_dtype; 0 for arguments
  * that no call accepts.  No reference counterpart (the reference sums every row with one
