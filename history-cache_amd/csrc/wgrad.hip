@@ -2,28 +2,37 @@
 // sampled layer (thousands to a hundred thousand), H and F a few hundred.  What torch's autograd computes
 // for `self.lin_l(out)` and `self.lin_r(x[:num_node])` (/root/reference/hiscache/history_model.py:94-98)
 // as one GEMM each.  A short, wide product with a very long inner dimension: the work is split over the
-// rows, every block multiplies its slab of rows on the matrix cores into a partial [256, 64] tile
-// (v_mfma_f32_32x32x2_f32, fp32 in and out), and a second launch adds the slabs' tiles in slab order.
-// Two operands that share g (the aggregated rows and the root rows) go through the same launches.
-// No atomics: the result does not depend on scheduling.
+// rows, every block multiplies its slab of rows on the matrix cores into a partial tile, and a second launch
+// adds the slabs' tiles in slab order.  Two operands that share g (the aggregated rows and the root rows) go
+// through the same launches.  No atomics: the result does not depend on scheduling.
 //
-//   A operand of the instruction (32 x 2): A[i][k] = g[row0 + k][h0 + i]   lane l holds i = l % 32, k = l / 32
-//   B operand (2 x 32):                    B[k][j] = x[row0 + k][f0 + j]   lane l holds j = l % 32, k = l / 32
-//   D (32 x 32, 16 values per lane):       D[8 * (v / 4) + 4 * (l / 32) + v % 4][l % 32], v = 0..15
-// so a lane's loads are one element of row (row0 + l / 32) of g and of x: two 128-byte runs per wave.
+// Bound by the matrix pipes (see dense.hip) where the rows are many, by the partial tiles' way through memory and two
+// launches where they are few.  Both launches, two operands, each wave loading its rows straight into registers (the
+// form before: tiles of 256 x 64, one block per compute unit) / this: 1 000 rows, 256 x 128 12.6 / 9.1 us; 3 000, 256 x 256
+// 24.7 / 20.9; 25 800, 256 x 128 44.6 / 40.8; 200 000, 256 x 128 272 / 248 (106 TFLOP/s); 89 000, 64 x 64 65 / 30 (three of
+// its four waves had no work); one operand, 4 200 rows, 3 840 x 256 138 / 88.  Tiles of 128 x 64 and 128 x 128, pieces of
+// 16 rows, 512 or 2 048 blocks instead of 1 024: between 5% faster and 40% slower, and 512 blocks sum twice the rows in one
+// chain.  Slabs of 64 rows at least: with 128, 1 500 rows of 256 x 256 take 14 instead of 16 us but a tenth more error.
+//
+// A block of four waves stages pieces of WG_PIECE rows of g and of x through two LDS buffers, the loads of a piece
+// issued in front of the matrix instructions of the one before it and kept there by a scheduling barrier.  Both
+// operands lie in LDS as in memory, the row index outside; a staged row is 16 words longer than the tile, so that the
+// 4 rows x 16 columns that a wave reads at once lie in 64 banks.  Rows behind the slab are read through a buffer
+// descriptor that ends there and are zeros.
+//
+//   A operand (16 x 4): x[row k + l / 16][f0 + l % 16]        B operand (4 x 16): g[row k + l / 16][h0 + l % 16]
+//   D (16 x 16, 4 values per lane): dW row h0 + l % 16, columns f0 + 4 (l / 16) .. + 3: one 16-byte store
 #include "hc_common.h"
 
 namespace {
 
-typedef float wg_acc __attribute__((ext_vector_type(16)));
+typedef float wg_acc __attribute__((ext_vector_type(4)));
+typedef uint32_t wg_quad __attribute__((ext_vector_type(4)));
 
-constexpr int WG_TILE_H = 256;      // output rows per block: 64 per wave
-constexpr int WG_TILE_F = 64;       // output columns per block
-constexpr int WG_STAGE = 16;        // k-steps (pairs of rows) whose loads are in flight ahead of the matrix instructions
-// One block per compute unit: with 512 or 1024 blocks the partial tiles' traffic grows faster than the
-// matrix pipes gain (n = 25 800, F = 128, two operands: 48 us with 256 blocks, 57 with 512, 70 with 1024);
-// 16 k-steps in flight against 8: 98 against 90 TFLOP/s at n = 89 000.
-constexpr int WG_TARGET_BLOCKS = 256;
+constexpr int WG_TILE_H = 64;       // rows of dW per block
+constexpr int WG_TILE_F = 64;       // columns of dW per block
+constexpr int WG_PIECE = 32;        // rows of g and x per piece
+constexpr int WG_TARGET_BLOCKS = 1024;
 constexpr int WG_MIN_SLAB_ROWS = 64;
 
 struct WgShape {
@@ -32,145 +41,156 @@ struct WgShape {
 };
 
 static bool wg_shape(int64_t n, int64_t H, int64_t F, int n_op, WgShape *s) {
-  if (n < 1 || H < 64 || H % 64 != 0 || F < WG_TILE_F || F % WG_TILE_F != 0 || H > 4096 || F > 4096) return false;
+  if (n < 1 || H < WG_TILE_H || H % WG_TILE_H != 0 || F < WG_TILE_F || F % WG_TILE_F != 0 || H > 4096 || F > 4096) return false;
   if (n_op < 1 || n_op > 2) return false;
-  s->tiles_h = (int)((H + WG_TILE_H - 1) / WG_TILE_H);
+  s->tiles_h = (int)(H / WG_TILE_H);
   s->tiles_f = (int)(F / WG_TILE_F);
   const int64_t per_slab = (int64_t)s->tiles_h * s->tiles_f * n_op;
   int64_t slabs = (WG_TARGET_BLOCKS + per_slab - 1) / per_slab;
   const int64_t most = (n + WG_MIN_SLAB_ROWS - 1) / WG_MIN_SLAB_ROWS;
   if (slabs > most) slabs = most;
-  if (slabs < 1) slabs = 1;
-  int64_t rows = (n + slabs - 1) / slabs;
-  rows = (rows + 1) / 2 * 2;                         // a k-step is two rows
-  s->slab_rows = rows;
-  s->slabs = (n + rows - 1) / rows;
+  const int64_t rows = (n + slabs - 1) / slabs;
+  s->slab_rows = (rows + 3) / 4 * 4;                 // a matrix instruction takes four rows
+  s->slabs = (n + s->slab_rows - 1) / s->slab_rows;
   return true;
 }
 
-__global__ __launch_bounds__(HC_BLOCK) void wg_partial(const float *__restrict__ g, const float *__restrict__ x0,
-                                                        const float *__restrict__ x1, float *__restrict__ part,
-                                                        int64_t n, int H, int F, WgShape sh) {
-  const float *__restrict__ x = blockIdx.z == 0 ? x0 : x1;
-  const int tile = (int)blockIdx.y;
-  const int tf = tile % sh.tiles_f, th = tile / sh.tiles_f;
-  const int wave = hc_wave_in_block(), lane = hc_lane();
-  const int h0 = th * WG_TILE_H + wave * 64;
-  if (h0 >= H) return;                                // narrow outputs leave the upper waves idle
-  const int f0 = tf * WG_TILE_F;
-  const int64_t lo = (int64_t)blockIdx.x * sh.slab_rows;
-  const int64_t hi = lo + sh.slab_rows < n ? lo + sh.slab_rows : n;
-  const int kk = lane >> 5, c = lane & 31;
-  wg_acc acc00 = {0.f}, acc01 = {0.f}, acc10 = {0.f}, acc11 = {0.f};
-  const float *gp = g + (lo + kk) * (int64_t)H + h0 + c;
-  const float *xp = x + (lo + kk) * (int64_t)F + f0 + c;
-  int64_t r = lo;
-  // Full stages of WG_STAGE k-steps (2 * WG_STAGE rows).  The loads of the next stage are issued before the
-  // matrix instructions of the current one, so that a wave keeps its matrix pipe busy while they are in flight.
-  float a0[WG_STAGE], a1[WG_STAGE], b0[WG_STAGE], b1[WG_STAGE];
-  bool have = r + 2 * WG_STAGE <= hi;
-  if (have) {
+template <bool VEC>
+__device__ __forceinline__ wg_quad wg_load(hc_buffer b, uint32_t at) {
+  if constexpr (VEC) {
+    return __builtin_bit_cast(wg_quad, __builtin_amdgcn_raw_buffer_load_b128(b, at, 0, 0));
+  } else {
+    wg_quad v;
 #pragma unroll
-    for (int s = 0; s < WG_STAGE; ++s) {
-      a0[s] = gp[(int64_t)2 * s * H];
-      a1[s] = gp[(int64_t)2 * s * H + 32];
-      b0[s] = xp[(int64_t)2 * s * F];
-      b1[s] = xp[(int64_t)2 * s * F + 32];
-    }
-  }
-  while (have) {
-    gp += (int64_t)2 * WG_STAGE * H;
-    xp += (int64_t)2 * WG_STAGE * F;
-    r += 2 * WG_STAGE;
-    const bool more = r + 2 * WG_STAGE <= hi;
-    float na0[WG_STAGE], na1[WG_STAGE], nb0[WG_STAGE], nb1[WG_STAGE];
-    if (more) {
-#pragma unroll
-      for (int s = 0; s < WG_STAGE; ++s) {
-        na0[s] = gp[(int64_t)2 * s * H];
-        na1[s] = gp[(int64_t)2 * s * H + 32];
-        nb0[s] = xp[(int64_t)2 * s * F];
-        nb1[s] = xp[(int64_t)2 * s * F + 32];
-      }
-    }
-#pragma unroll
-    for (int s = 0; s < WG_STAGE; ++s) {
-      acc00 = __builtin_amdgcn_mfma_f32_32x32x2f32(a0[s], b0[s], acc00, 0, 0, 0);
-      acc01 = __builtin_amdgcn_mfma_f32_32x32x2f32(a0[s], b1[s], acc01, 0, 0, 0);
-      acc10 = __builtin_amdgcn_mfma_f32_32x32x2f32(a1[s], b0[s], acc10, 0, 0, 0);
-      acc11 = __builtin_amdgcn_mfma_f32_32x32x2f32(a1[s], b1[s], acc11, 0, 0, 0);
-    }
-    if (more) {
-#pragma unroll
-      for (int s = 0; s < WG_STAGE; ++s) {
-        a0[s] = na0[s];
-        a1[s] = na1[s];
-        b0[s] = nb0[s];
-        b1[s] = nb1[s];
-      }
-    }
-    have = more;
-  }
-  // tail: k-steps whose second row may lie behind the slab
-  for (; r < hi; r += 2) {
-    const bool ok = r + kk < hi;
-    const float a0 = ok ? gp[0] : 0.f, a1 = ok ? gp[32] : 0.f;
-    const float b0 = ok ? xp[0] : 0.f, b1 = ok ? xp[32] : 0.f;
-    acc00 = __builtin_amdgcn_mfma_f32_32x32x2f32(a0, b0, acc00, 0, 0, 0);
-    acc01 = __builtin_amdgcn_mfma_f32_32x32x2f32(a0, b1, acc01, 0, 0, 0);
-    acc10 = __builtin_amdgcn_mfma_f32_32x32x2f32(a1, b0, acc10, 0, 0, 0);
-    acc11 = __builtin_amdgcn_mfma_f32_32x32x2f32(a1, b1, acc11, 0, 0, 0);
-    gp += (int64_t)2 * H;
-    xp += (int64_t)2 * F;
-  }
-  // partial tile of this block: [WG_TILE_H][WG_TILE_F], tiles ordered (operand, tile, slab)
-  const int64_t tiles = (int64_t)sh.tiles_h * sh.tiles_f;
-  float *o = part + (((int64_t)blockIdx.z * tiles + tile) * sh.slabs + blockIdx.x) * (WG_TILE_H * WG_TILE_F) +
-             (int64_t)(wave * 64) * WG_TILE_F;
-#pragma unroll
-  for (int v = 0; v < 16; ++v) {
-    const int i = 8 * (v / 4) + 4 * kk + (v % 4);
-    o[(int64_t)i * WG_TILE_F + c] = acc00[v];
-    o[(int64_t)i * WG_TILE_F + 32 + c] = acc01[v];
-    o[(int64_t)(32 + i) * WG_TILE_F + c] = acc10[v];
-    o[(int64_t)(32 + i) * WG_TILE_F + 32 + c] = acc11[v];
+    for (int q = 0; q < 4; ++q) v[q] = __builtin_amdgcn_raw_buffer_load_b32(b, at, 4 * q, 0);
+    return v;
   }
 }
 
-// dW[op][h][f] = sum over the slabs, in slab order, of the partial tiles; one thread per four columns
-__global__ __launch_bounds__(HC_BLOCK) void wg_reduce(const float *__restrict__ part, float *__restrict__ dw0,
-                                                       float *__restrict__ dw1, int H, int F, WgShape sh,
-                                                       int64_t per_op) {
-  const int64_t t = (int64_t)blockIdx.x * HC_BLOCK + threadIdx.x;
-  if (t >= per_op) return;
-  const int op = (int)blockIdx.y;
-  constexpr int Q = WG_TILE_F / 4;                     // float4 groups per tile row
-  const int q = (int)(t % Q);
-  const int hl = (int)((t / Q) % WG_TILE_H);
-  const int tile = (int)(t / ((int64_t)Q * WG_TILE_H));
-  const int tf = tile % sh.tiles_f, th = tile / sh.tiles_f;
-  const int h = th * WG_TILE_H + hl;
-  if (h >= H) return;
-  const int64_t tiles = (int64_t)sh.tiles_h * sh.tiles_f;
-  const float *p = part + (((int64_t)op * tiles + tile) * sh.slabs) * (WG_TILE_H * WG_TILE_F) +
-                   (int64_t)hl * WG_TILE_F + 4 * q;
-  float4 s = make_float4(0.f, 0.f, 0.f, 0.f);
-  int64_t k = 0;
-  for (; k + 8 <= sh.slabs; k += 8) {
-    float4 v[8];
+template <bool VEC>
+__global__ __launch_bounds__(HC_BLOCK) void wg_partial(const float *__restrict__ g, const float *__restrict__ x0,
+                                                        const float *__restrict__ x1, float *__restrict__ part,
+                                                        int64_t n, int H, int F, int per_slab, WgShape sh) {
+  constexpr int BM = WG_TILE_H, BN = WG_TILE_F, BK = WG_PIECE;
+  constexpr int WM = BM / 2, WN = BN / 2, TM = WM / 16, TN = WN / 16, LDG = BM + 16, LDX = BN + 16;
+  constexpr int QG = BM / 4, QX = BN / 4, NG = BK * QG / HC_BLOCK, NX = BK * QX / HC_BLOCK;
+  __shared__ __attribute__((aligned(16))) float sg[2][BK * LDG], sx[2][BK * LDX];
+  // blocks of one slab lie side by side: they read the same rows
+  const int64_t b = hc_xcd_block<16>(blockIdx.x, gridDim.x);
+  const int64_t slab = b / per_slab;
+  const int in_slab = (int)(b % per_slab), tiles = sh.tiles_h * sh.tiles_f;
+  const int op = in_slab / tiles, tile = in_slab % tiles;
+  const int f0 = tile % sh.tiles_f * BN, h0 = tile / sh.tiles_f * BM;
+  const float *__restrict__ x = op == 0 ? x0 : x1;
+  const int64_t lo = slab * sh.slab_rows, hi = lo + sh.slab_rows < n ? lo + sh.slab_rows : n;
+  const int t = (int)threadIdx.x, lane = hc_lane(), wave = hc_wave_in_block();
+  const int wm = (wave & 1) * WM, wn = (wave >> 1) * WN;
+  const int l16 = lane & 15, k4 = lane >> 4;
+  uint32_t at_g[NG], at_x[NX];
 #pragma unroll
-    for (int j = 0; j < 8; ++j) v[j] = *reinterpret_cast<const float4 *>(p + (k + j) * (WG_TILE_H * WG_TILE_F));
+  for (int i = 0; i < NG; ++i) {
+    const int f = t + i * HC_BLOCK;
+    at_g[i] = (uint32_t)(f / QG * H + h0 + f % QG * 4) * 4u;
+  }
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      s.x += v[j].x; s.y += v[j].y; s.z += v[j].z; s.w += v[j].w;
+  for (int i = 0; i < NX; ++i) {
+    const int f = t + i * HC_BLOCK;
+    at_x[i] = (uint32_t)(f / QX * F + f0 + f % QX * 4) * 4u;
+  }
+  wg_quad rg[NG], rx[NX];
+  const auto load = [&](int64_t r) {
+    const uint32_t rows = (uint32_t)(hi - r < BK ? hi - r : BK);
+    const hc_buffer bg = hc_make_buffer(g + r * H, rows * (uint32_t)H * 4u), bx = hc_make_buffer(x + r * F, rows * (uint32_t)F * 4u);
+#pragma unroll
+    for (int i = 0; i < NG; ++i) rg[i] = wg_load<VEC>(bg, at_g[i]);
+#pragma unroll
+    for (int i = 0; i < NX; ++i) rx[i] = wg_load<VEC>(bx, at_x[i]);
+  };
+  const auto stage = [&](int s) {
+#pragma unroll
+    for (int i = 0; i < NG; ++i) {
+      const int f = t + i * HC_BLOCK;
+      *reinterpret_cast<wg_quad *>(&sg[s][f / QG * LDG + f % QG * 4]) = rg[i];
     }
+#pragma unroll
+    for (int i = 0; i < NX; ++i) {
+      const int f = t + i * HC_BLOCK;
+      *reinterpret_cast<wg_quad *>(&sx[s][f / QX * LDX + f % QX * 4]) = rx[i];
+    }
+  };
+  wg_acc acc[TM][TN];
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j) acc[i][j] = wg_acc{0.f, 0.f, 0.f, 0.f};
+  const auto step = [&](int s, int k) {
+    float u[TM], v[TN];
+#pragma unroll
+    for (int i = 0; i < TM; ++i) u[i] = sg[s][(k + k4) * LDG + wm + i * 16 + l16];
+#pragma unroll
+    for (int j = 0; j < TN; ++j) v[j] = sx[s][(k + k4) * LDX + wn + j * 16 + l16];
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[j], u[i], acc[i][j], 0, 0, 0);
+  };
+  load(lo);
+  stage(0);
+  int s = 0;
+  int64_t r = lo;
+  for (; r + BK < hi; r += BK) {
+    __syncthreads();
+    load(r + BK);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int k = 0; k < BK; k += 4) step(s, k);
+    __builtin_amdgcn_sched_barrier(0);
+    s ^= 1;
+    stage(s);
   }
-  for (; k < sh.slabs; ++k) {
-    const float4 v = *reinterpret_cast<const float4 *>(p + k * (WG_TILE_H * WG_TILE_F));
-    s.x += v.x; s.y += v.y; s.z += v.z; s.w += v.w;
+  __syncthreads();
+  for (int k = 0; k < (int)(hi - r); k += 4) step(s, k);           // the last piece: 1 to WG_PIECE rows
+  // partial tile of this block, tiles ordered (operand, tile, slab)
+  float *o = part + ((int64_t)in_slab * sh.slabs + slab) * (BM * BN);
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+      *reinterpret_cast<wg_acc *>(o + (wm + i * 16 + l16) * BN + wn + j * 16 + 4 * k4) = acc[i][j];
+}
+
+// dW[op][h][f]: a quarter of the slabs per wave, in slab order, then the quarters in order.  Four columns per lane;
+// four waves share them because a lane's loads, one per slab, are what the launch waits for (89 000 rows, 64 x 64, two
+// operands, 512 slabs: both launches 44 us with one wave's chain, 30 with four).
+__global__ __launch_bounds__(HC_BLOCK) void wg_reduce(const float *__restrict__ part, float *__restrict__ dw0,
+                                                       float *__restrict__ dw1, int F, WgShape sh) {
+  constexpr int Q = WG_TILE_F / 4, FLIGHT = 8;         // float4 groups per tile row
+  __shared__ float4 s_part[3][HC_WAVE];
+  const int lane = hc_lane(), wave = hc_wave_in_block();
+  const int64_t t = (int64_t)blockIdx.x * HC_WAVE + lane;          // the grid covers whole tiles
+  const int q = (int)(t % Q), hl = (int)(t / Q % WG_TILE_H), tile = (int)(t / (Q * WG_TILE_H));
+  const int op = (int)blockIdx.y;
+  constexpr int64_t TILE = WG_TILE_H * WG_TILE_F;
+  const float *p = part + ((int64_t)op * sh.tiles_h * sh.tiles_f + tile) * sh.slabs * TILE + (int64_t)hl * WG_TILE_F + 4 * q;
+  int64_t k = sh.slabs * wave / 4;
+  const int64_t end = sh.slabs * (wave + 1) / 4;
+  float4 s = make_float4(0.f, 0.f, 0.f, 0.f);
+  const auto plus = [&](const float4 &v) { s.x += v.x; s.y += v.y; s.z += v.z; s.w += v.w; };
+  for (; k + FLIGHT <= end; k += FLIGHT) {
+    float4 v[FLIGHT];
+#pragma unroll
+    for (int j = 0; j < FLIGHT; ++j) v[j] = *reinterpret_cast<const float4 *>(p + (k + j) * TILE);
+#pragma unroll
+    for (int j = 0; j < FLIGHT; ++j) plus(v[j]);
   }
-  float *dw = op == 0 ? dw0 : dw1;
-  *reinterpret_cast<float4 *>(dw + (int64_t)h * F + tf * WG_TILE_F + 4 * q) = s;
+  for (; k < end; ++k) plus(*reinterpret_cast<const float4 *>(p + k * TILE));
+  if (wave > 0) s_part[wave - 1][lane] = s;
+  __syncthreads();
+  if (wave > 0) return;
+#pragma unroll
+  for (int w = 0; w < 3; ++w) plus(s_part[w][lane]);
+  const int h = tile / sh.tiles_f * WG_TILE_H + hl, f = tile % sh.tiles_f * WG_TILE_F + 4 * q;
+  *reinterpret_cast<float4 *>((op == 0 ? dw0 : dw1) + (int64_t)h * F + f) = s;
 }
 
 }  // namespace
@@ -194,10 +214,13 @@ extern "C" int hc_weight_grad(const float *g, const float *x0, const float *x1, 
     return HC_EINVAL;
   hipStream_t st = static_cast<hipStream_t>(stream);
   float *part = static_cast<float *>(workspace);
-  wg_partial<<<dim3((unsigned)sh.slabs, (unsigned)(sh.tiles_h * sh.tiles_f), (unsigned)n_op), dim3(HC_BLOCK), 0,
-               st>>>(g, x0, x1, part, n, (int)H, (int)F, sh);
-  const int64_t per_op = (int64_t)sh.tiles_h * sh.tiles_f * WG_TILE_H * (WG_TILE_F / 4);
-  wg_reduce<<<dim3((unsigned)((per_op + HC_BLOCK - 1) / HC_BLOCK), (unsigned)n_op), dim3(HC_BLOCK), 0, st>>>(
-      part, dw0, dw1, (int)H, (int)F, sh, per_op);
+  const int per_slab = sh.tiles_h * sh.tiles_f * n_op;
+  const int64_t blocks = sh.slabs * per_slab;
+  if (!hc_grid_ok(blocks)) return HC_EUNSUPPORTED;
+  const bool vec = (reinterpret_cast<uintptr_t>(g) | reinterpret_cast<uintptr_t>(x0) | reinterpret_cast<uintptr_t>(x1)) % 16 == 0;
+  const auto kernel = vec ? wg_partial<true> : wg_partial<false>;
+  kernel<<<dim3((unsigned)blocks), dim3(HC_BLOCK), 0, st>>>(g, x0, x1, part, n, (int)H, (int)F, per_slab, sh);
+  const int64_t quads = (int64_t)sh.tiles_h * sh.tiles_f * WG_TILE_H * (WG_TILE_F / 4);
+  wg_reduce<<<dim3((unsigned)(quads / HC_WAVE), (unsigned)n_op), dim3(HC_BLOCK), 0, st>>>(part, dw0, dw1, (int)F, sh);
   return hc_launch_status();
 }

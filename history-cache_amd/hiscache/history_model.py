@@ -34,8 +34,9 @@ class _GradSink:
 # 72 - 131 and 107 - 193 us: linear in n.  Below this many rows the single GEMM is used (21 us at 5 800).
 _WGRAD_SLAB_ROWS = 1024
 _WGRAD_SPLIT_MIN_ROWS = 8192
-# The library's own kernel (hc_weight_grad: both operands of a SAGE layer in one pair of launches, 59 us at
-# n = 25 800 and F = 128, 102 us at n = 55 000) takes over from this many rows when the widths fit it.
+# The library's own kernel (hc_weight_grad: both operands of a SAGE layer in one pair of launches, 41 us at
+# n = 25 800 and F = 128, 77 us at n = 55 000) takes over when the widths fit it; with fewer rows too (1 000 rows,
+# F = 128: 9 us for both operands; two GEMMs 40 to 227, by the kernel chosen) unless something watches the operators.
 _WGRAD_KERNEL_MIN_ROWS = 2048
 
 
@@ -129,7 +130,8 @@ class _SageConvFunction(torch.autograd.Function):
         root = None
         if has_root and need[3]:
             root = x[:R] if x.dtype == g_out.dtype else x[:R].to(g_out.dtype)
-        if need[1] and root is not None and R >= _WGRAD_KERNEL_MIN_ROWS and be.weight_grad_supported(g_out, agg):
+        if (need[1] and root is not None and be.weight_grad_supported(g_out, agg)
+                and (R >= _WGRAD_KERNEL_MIN_ROWS or be.plain_operands(g_out, agg, root))):
             g_wl, g_wr = be.weight_grad(g_out, agg, root)          # both products in one pair of launches
         else:
             if need[1]:
@@ -401,6 +403,9 @@ def _rel_weight_grad(agg, g):
     """agg^T @ g in the weight's layout: agg [n, K, F], g [n, H] -> [K, F, H]."""
     n, K, Fin = agg.shape
     a2 = agg.reshape(n, K * Fin)
+    # (4 200 rows, 3 840 x 256: 88 us against 150 for the slabs' batched GEMM and their sum)
+    if hiscache_backend.weight_grad_supported(a2, g) and hiscache_backend.plain_operands(a2, g):
+        return hiscache_backend.weight_grad(a2, g).view(K, Fin, -1)
     S = max(_REL_WGRAD_SLABS, n // _WGRAD_SLAB_ROWS)
     m = n // S * S
     if K * Fin < _REL_SPLIT_MIN_INNER or m == 0:

@@ -1407,16 +1407,22 @@ def weight_grad(g, x0, x1=None):
 _PLAIN = (torch.Tensor, torch.nn.Parameter)
 
 
-def linear_supported(a, *others):
-    """Does :func:`linear` cover a product of these tensors as the torch operators would compute it: plain, packed fp32
-    tensors on the current GPU, no autocast, nothing that records or replaces operators?  An inner size off a multiple of
-    four is read element by element, and the library is the faster one above 256 (2 000 rows of 602 to 64: 23 against 25 us)."""
-    k = a.shape[1]
-    return (a.shape[0] > 0 and (k % 4 == 0 or k <= 256) and a.is_cuda and a.device.index == torch.cuda.current_device()
+def plain_operands(a, *others):
+    """May a library call stand for torch operators on these tensors: plain, packed fp32 tensors on the current GPU, no
+    autocast, nothing that records or replaces operators?"""
+    return (a.is_cuda and a.device.index == torch.cuda.current_device()
             and all(t is None or (type(t) in _PLAIN and t.dtype == torch.float32 and t.device == a.device
                                   and t.is_contiguous() and t.numel() > 0) for t in (a, *others))
             and not torch.is_grad_enabled() and not torch.is_autocast_enabled("cuda")
             and torch._C._len_torch_dispatch_stack() == 0)
+
+
+def linear_supported(a, *others):
+    """Does :func:`linear` cover a product of these tensors as the torch operators would compute it?  An inner size off a
+    multiple of four is read element by element, and the library is the faster one above 256 (2 000 rows of 602 to 64: 23
+    against 25 us)."""
+    k = a.shape[1]
+    return (k % 4 == 0 or k <= 256) and plain_operands(a, *others)
 
 
 def linear(a0, w0, a1=None, w1=None, bias=None, transposed=False, out=None):

@@ -1,0 +1,38 @@
+"""hc_weight_grad at the edges of its pieces (32 rows), matrix instructions (4 rows) and slabs (64 rows), with operands off
+16-byte boundaries, and the relational layer's weight gradient through it."""
+import pytest
+import torch
+
+import hiscache_backend as be
+from hiscache import history_model as hm
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def _close(got, g, x, n):
+    # n products and their additions in fp32, each off by at most half a unit of the sum of magnitudes
+    bound = 1.01 * (n + 1) * 2.0 ** -24 * (g.double().abs().t() @ x.double().abs())
+    assert bool(((got.double() - g.double().t() @ x.double()).abs() <= bound).all())
+
+
+@pytest.mark.parametrize("n", (1, 3, 4, 5, 31, 32, 33, 63, 65, 96, 127, 129, 1025, 16_390))
+@pytest.mark.parametrize("H,F", ((64, 64), (128, 192)))
+def test_weight_grad_at_the_edges_of_pieces_and_slabs(n, H, F):
+    gen = torch.Generator(device=DEV).manual_seed(n + H)
+    g, x0, x1 = (torch.randn(n, c, device=DEV, generator=gen) for c in (H, F, F))
+    both = be.weight_grad(g, x0, x1)
+    for got, x in zip(both, (x0, x1)):
+        _close(got, g, x, n)
+    shifted = torch.empty(n * H + 1, device=DEV)[1:].view(n, H).copy_(g)
+    assert all(torch.equal(a, b) for a, b in zip(be.weight_grad(shifted, x0, x1), both))
+
+
+@pytest.mark.parametrize("n,K,F,H", ((1, 5, 64, 64), (301, 5, 128, 64), (4_200, 5, 768, 256), (90, 3, 20, 64), (2_100, 5, 64, 10)))
+def test_relational_weight_gradient(n, K, F, H):
+    gen = torch.Generator(device=DEV).manual_seed(n + F)
+    agg, g = torch.randn(n, K, F, device=DEV, generator=gen), torch.randn(n, H, device=DEV, generator=gen)
+    with torch.no_grad():
+        got = hm._rel_weight_grad(agg, g)
+    assert tuple(got.shape) == (K, F, H)
+    _close(got.view(K * F, H), agg.view(n, K * F), g, n)
