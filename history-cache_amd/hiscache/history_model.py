@@ -70,6 +70,15 @@ def _column_sums(g):
     return torch.mv(g.t(), ones[:n])
 
 
+def _linear_fits(a, w, root=None, w_root=None, bias=None):
+    """Does ``hiscache_backend.linear`` take these operands?  Shapes that do not fit are left to the operators, which say
+    so."""
+    return (a.dim() == 2 and w.dim() == 2 and w.shape[1] == a.shape[1]
+            and (w_root is None or (w_root.shape == w.shape and root.shape == a.shape))
+            and (bias is None or bias.shape == w.shape[:1])
+            and hiscache_backend.linear_supported(a, w, root, w_root, bias))
+
+
 class _SageConvFunction(torch.autograd.Function):
     """``lin_l(aggregate(x)) + lin_r(x[:n])`` as ONE autograd node.
 
@@ -90,7 +99,7 @@ class _SageConvFunction(torch.autograd.Function):
         root = None
         if w_r is not None:
             root = x[:R] if x.dtype == agg.dtype else x[:R].to(agg.dtype)
-        if be.linear_supported(agg, w_l, root, w_r, b_l):
+        if _linear_fits(agg, w_l, root, w_r, b_l):
             out = be.linear(agg, w_l, root, w_r, b_l)
         else:
             # plain GEMMs and a separate bias add: a GEMM with a bias epilogue goes to hipBLASLt whatever
@@ -199,18 +208,19 @@ def _unobserved(module, kind):
             and torch._C._functorch.peek_interpreter_stack() is None)
 
 
-def _evaluates(bn, x, bias):
+def _evaluates(bn, x, bias, width=None):
     """Does ``hc_bn_relu_eval`` cover this call: the running statistics, no gradient, plain fp32 vectors on the current
-    GPU, and nothing that a fused call would pass by?"""
+    GPU, and nothing that a fused call would pass by?  ``width``: of the matrix to be normalised, if it is not ``x``."""
     if bn.training or torch.is_grad_enabled() or not _unobserved(bn, torch.nn.BatchNorm1d):
         return False
     if bn.running_mean is None or x.dim() != 2 or not x.is_contiguous():
         return False
+    width = x.shape[1] if width is None else width
     vectors = [t for t in (bias, bn.weight, bn.bias, bn.running_mean, bn.running_var) if t is not None]
-    return (hiscache_backend.bn_relu_supported(x, x.shape[1]) and x.data_ptr() % 16 == 0
+    return (hiscache_backend.bn_relu_supported(x, width) and x.data_ptr() % 16 == 0
             and x.device.index == torch.cuda.current_device()
             and all(t.is_cuda and t.device == x.device and t.dtype == torch.float32 and t.is_contiguous()
-                    and t.numel() == x.shape[1] and t.data_ptr() % 16 == 0 for t in vectors))
+                    and t.numel() == width and t.data_ptr() % 16 == 0 for t in vectors))
 
 
 class MySageConvHistory(torch.nn.Module):
@@ -311,6 +321,11 @@ class HistorySAGE(torch.nn.Module):
             # nobody sees the layer's output without it)
             defer = (self.fused_epilogue and conv.fused and x.is_cuda
                      and (self.training or (not torch.is_grad_enabled() and _unobserved(conv, MySageConvHistory))))
+            if defer and not self.training:
+                y = self._evaluated(conv, self.bns[i], x, ptr, batch.idx, n, view) if dev is None else None
+                if y is not None:
+                    x = F.dropout(y, p=self.dropout, training=False)
+                    continue
             if self.training and i == self.num_layers - 2:
                 # the layer whose output is one hop from the seeds uses (and produces) history
                 x, his = conv(x, ptr, batch.idx, self.table.sub2embed,
@@ -325,6 +340,22 @@ class HistorySAGE(torch.nn.Module):
         x, his = self.convs[-1](x, batch.ptr if ptrs is None else ptrs[0], batch.idx, none, none, 0,
                                 batch.num_node_in_layer[0], None if nel is None else int(nel[0]), view=view)
         return x.log_softmax(dim=-1)
+
+    def _evaluated(self, conv, bn, x, ptr, idx, num_node, view):
+        """A hidden layer's ``relu(bn(conv(x)))`` in evaluation, bias, normalisation and ReLU on the way out of the dense
+        half; None where something does not fit it.  (The caller has looked at ``conv``.)"""
+        be = hiscache_backend
+        R = int(num_node) or ptr.numel() - 1
+        w_r = conv.lin_r.weight if conv.root_weight else None
+        root = x[:R]
+        if not (0 < R <= x.shape[0] and x.dim() == 2
+                and _linear_fits(root, conv.lin_l.weight, root, w_r, conv.lin_l.bias)
+                and _evaluates(bn, x, conv.lin_l.bias, conv.lin_l.weight.shape[0])):
+            return None
+        agg = be._aggr_fwd(be.SUBST_ROW, ptr, idx, x, None, None, 0, None, R,
+                           max_degree=None if view is None else view.row_bound(R, x.shape[0]))
+        return be.linear(agg, conv.lin_l.weight, None if w_r is None else root, w_r, conv.lin_l.bias,
+                         norm=(bn.weight, bn.bias, bn.running_mean, bn.running_var, bn.eps))
 
     def init_convs(self, **kwargs):
         need_grad = self.table.method == "grad"

@@ -127,6 +127,8 @@ _SIGNATURES = {
     "hc_bn_relu_bwd": (_c_int, [_c_p, _c_p, _c_p, _c_p, _c_p, _c_p, _c_p, _c_p, _c_p, _c_p, _c_i64, _c_i64,
                                 _c_p, _c_sz, _c_p, _c_p]),
     "hc_linear": (_c_int, [_c_p, _c_p, _c_p, _c_p, _c_int, _c_p, _c_p, _c_p, _c_i64, _c_i64, _c_i64, _c_p]),
+    "hc_linear_bn_relu": (_c_int, [_c_p, _c_p, _c_p, _c_p, _c_p, _c_p, _c_p, _c_p, _c_p, ctypes.c_float, _c_p, _c_i64,
+                                   _c_i64, _c_i64, _c_p]),
     "hc_weight_grad_workspace_bytes": (_c_sz, [_c_i64, _c_i64, _c_i64, _c_int]),
     "hc_weight_grad": (_c_int, [_c_p, _c_p, _c_p, _c_i64, _c_i64, _c_i64, _c_p, _c_p, _c_p, _c_sz, _c_p]),
     "hc_stage_arrays": (_c_int, [_c_p, _c_p, _c_p, _c_p, _c_p, _c_p, _c_int, _c_p, _c_p, _c_int, _c_p]),
@@ -1425,9 +1427,11 @@ def linear_supported(a, *others):
     return (k % 4 == 0 or k <= 256) and plain_operands(a, *others)
 
 
-def linear(a0, w0, a1=None, w1=None, bias=None, transposed=False, out=None):
+def linear(a0, w0, a1=None, w1=None, bias=None, transposed=False, out=None, norm=None):
     """``a0 @ w0.t() + a1 @ w1.t() + bias`` for fp32 a [n, K], w [N, K] on the matrix cores, in one launch;
-    ``transposed``: ``a0 @ w0`` for w [K, N].  ``out`` (contiguous [n, N]): the result is added to what it holds."""
+    ``transposed``: ``a0 @ w0`` for w [K, N].  ``out`` (contiguous [n, N]): the result is added to what it holds.
+    ``norm`` (gamma, beta, running_mean, running_var, eps; the first two may be None): :func:`bias_bn_relu_eval` of the
+    result, in the same launch."""
     lib = load_library()
     for name, t in (("a0", a0), ("w0", w0), ("a1", a1), ("w1", w1), ("bias", bias), ("out", out)):
         if t is not None:
@@ -1442,8 +1446,19 @@ def linear(a0, w0, a1=None, w1=None, bias=None, transposed=False, out=None):
         raise ValueError(f"bias must hold {N} values")
     if out is not None and out.shape != (n, N):
         raise ValueError(f"out must be [{n}, {N}]")
+    if norm is not None:
+        if transposed or out is not None:
+            raise ValueError("the normalisation follows a plain product")
+        for name, t in zip(("gamma", "beta", "running_mean", "running_var"), norm):
+            if (t is not None or name.startswith("running")) and _dev(t, name, torch.float32).shape != (N,):
+                raise ValueError(f"{name} must hold {N} values")
     res = out if out is not None else torch.empty((n, N), dtype=torch.float32, device=a0.device)
-    if res.numel() > 0:
+    if res.numel() > 0 and norm is not None:
+        gamma, beta, mean, var, eps = norm
+        _check(lib.hc_linear_bn_relu(_ptr(a0), _ptr(w0), _ptr(a1), _ptr(w1), _ptr(bias), _ptr(gamma), _ptr(beta),
+                                     _ptr(mean), _ptr(var), float(eps), _ptr(res), n, N, K, _stream()),
+               "hc_linear_bn_relu")
+    elif res.numel() > 0:
         _check(lib.hc_linear(_ptr(a0), _ptr(w0), _ptr(a1), _ptr(w1), int(transposed), _ptr(bias), _ptr(out), _ptr(res),
                              n, N, K, _stream()), "hc_linear")
     return res

@@ -694,6 +694,14 @@ int hc_linear(const float *a0, const float *w0, const float *a1, const float *w1
               const float *bias, const float *add, float *out, int64_t M, int64_t N, int64_t K,
               void *stream);
 
+/* hc_linear_bn_relu: hc_linear (w [N, K], bias [N] or NULL) with hc_bn_relu_eval
+ * behind it in the same launch: relu(batch_norm(a0 w0^T + a1 w1^T + bias)) with
+ * the running statistics, bit for bit what the two calls give.  gamma and beta
+ * [N] may be NULL.  Limits as hc_linear. */
+int hc_linear_bn_relu(const float *a0, const float *w0, const float *a1, const float *w1, const float *bias,
+                      const float *gamma, const float *beta, const float *running_mean, const float *running_var,
+                      float eps, float *out, int64_t M, int64_t N, int64_t K, void *stream);
+
 /* hc_weight_grad: the gradient of a layer's linear maps, dw[H, F] = g^T x for
  * g [n, H] and x [n, F] (fp32, row-major, contiguous) -- what autograd computes
  * for `self.lin_l(out)` and `self.lin_r(x[:num_node])`
