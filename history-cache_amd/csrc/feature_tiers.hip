@@ -16,7 +16,7 @@ namespace {
 constexpr int TV = 4;   // elements per lane per step when rows allow
 
 template <typename TS, typename TD>
-__device__ __forceinline__ bool tier_vec_ok(const TS *src, const TD *dst, int64_t F) {
+__host__ __device__ __forceinline__ bool tier_vec_ok(const TS *src, const TD *dst, int64_t F) {
   return (F % TV == 0) && (reinterpret_cast<uintptr_t>(src) % (sizeof(TS) * TV) == 0) &&
          (reinterpret_cast<uintptr_t>(dst) % (sizeof(TD) * TV) == 0);
 }
@@ -44,14 +44,17 @@ __device__ __forceinline__ void tier_copy_row(const TS *__restrict__ s, TD *__re
 // A wave serves HOT_ROWS consecutive requested rows: one lane per row reads the row's mask byte, id and slot (three
 // dependent reads for all rows at once instead of once per row), then the wave copies the rows HOT_INFLIGHT at a
 // time, every row's load issued before the first store.  With a wave per row the launch is a chain of four round
-// trips per 512-byte row and runs at a fraction of the memory rate.
+// trips per 512-byte row and runs at a fraction of the memory rate.  Rows of at most 32 (16) steps of TV elements are
+// copied two (four) at a time by one load, so that no lane is idle and all 16 rows are on their way at once.
+// 300 000 rows out of 2 M, all / half of them asked for, one row per load and then: 512 bytes 66 / 54 us, 63 / 42 (4.9 / 5.5
+// TB/s); 400 bytes 60 / 45, 55 / 35; 256 bytes 36 / 30, 30 / 20; 128 bytes (fp16) 33 / 29, 19 / 14.
 constexpr int HOT_ROWS = 16;
-constexpr int HOT_INFLIGHT = 4;
+constexpr int hot_loads(int rpl) { return rpl == 1 ? 4 : HOT_ROWS / rpl; }      // loads in flight per wave
 constexpr int ROW_ZERO = 0, ROW_COPY = 1, ROW_SKIP = 2;
 
 // TIERED = false: the plain gather of a matrix in device memory (hot is the matrix, a node's row is its id, no row
-// is left to another launch).
-template <typename TS, typename TD, bool TIERED>
+// is left to another launch).  RPL: rows per load; above 1 only where a row's steps fit that share of the lanes.
+template <typename TS, typename TD, bool TIERED, int RPL>
 __global__ __launch_bounds__(HC_BLOCK) void tier_hot_kernel(const TS *__restrict__ hot, int64_t n_hot,
                                                              const int32_t *__restrict__ slot_map, int64_t n_map,
                                                              const int64_t *__restrict__ ids,
@@ -78,40 +81,48 @@ __global__ __launch_bounds__(HC_BLOCK) void tier_hot_kernel(const TS *__restrict
     if constexpr (TIERED) cold[i] = is_cold ? 1 : 0;
     state = is_cold ? ROW_SKIP : (take ? ROW_COPY : ROW_ZERO);     // a cold row is written by the other launch
   }
-  const bool vec_ok = tier_vec_ok(hot, dst, F);
+  constexpr int LOADS = hot_loads(RPL), LANES = HC_WAVE / RPL;
+  const bool vec_ok = RPL > 1 || tier_vec_ok(hot, dst, F);
 #pragma unroll
-  for (int r0 = 0; r0 < HOT_ROWS; r0 += HOT_INFLIGHT) {
-    int st[HOT_INFLIGHT];
-    const TS *s[HOT_INFLIGHT];
+  for (int r0 = 0; r0 < HOT_ROWS; r0 += LOADS * RPL) {
+    int st[LOADS];
+    const TS *s[LOADS];
     bool any = false;
 #pragma unroll
-    for (int k = 0; k < HOT_INFLIGHT; ++k) {
-      st[k] = __builtin_amdgcn_readlane(state, r0 + k);
-      s[k] = hot + hc_readlane64(slot, r0 + k) * F;
+    for (int k = 0; k < LOADS; ++k) {
+      if constexpr (RPL == 1) {
+        st[k] = __builtin_amdgcn_readlane(state, r0 + k);
+        s[k] = hot + hc_readlane64(slot, r0 + k) * F;
+      } else {
+        const int row = r0 + k * RPL + lane / LANES;
+        st[k] = __shfl(state, row, HC_WAVE);
+        s[k] = hot + __shfl(slot, row, HC_WAVE) * F;
+      }
       any = any || st[k] != ROW_SKIP;
     }
-    if (!any) continue;                                            // wave-uniform
+    if (!any) continue;
     TD *o = dst + (base + r0) * F;
     if (vec_ok) {
-      for (int64_t c = (int64_t)lane * TV; c < F; c += HC_WAVE * TV) {
-        float v[HOT_INFLIGHT][TV];
+      o += (int64_t)(lane / LANES) * F;
+      for (int64_t c = (int64_t)(lane % LANES) * TV; c < F; c += LANES * TV) {
+        float v[LOADS][TV];
 #pragma unroll
-        for (int k = 0; k < HOT_INFLIGHT; ++k) {
+        for (int k = 0; k < LOADS; ++k) {
 #pragma unroll
           for (int e = 0; e < TV; ++e) v[k][e] = 0.0f;
           if (st[k] == ROW_COPY) hc_vec<TS, TV>::load(s[k] + c, v[k]);
         }
 #pragma unroll
-        for (int k = 0; k < HOT_INFLIGHT; ++k)
-          if (st[k] != ROW_SKIP) hc_vec<TD, TV>::store(o + k * F + c, v[k]);
+        for (int k = 0; k < LOADS; ++k)
+          if (st[k] != ROW_SKIP) hc_vec<TD, TV>::store(o + (int64_t)k * RPL * F + c, v[k]);
       }
     } else {
       for (int64_t c = lane; c < F; c += HC_WAVE) {
-        float v[HOT_INFLIGHT];
+        float v[LOADS];
 #pragma unroll
-        for (int k = 0; k < HOT_INFLIGHT; ++k) v[k] = st[k] == ROW_COPY ? hc_to_f32<TS>(s[k][c]) : 0.0f;
+        for (int k = 0; k < LOADS; ++k) v[k] = st[k] == ROW_COPY ? hc_to_f32<TS>(s[k][c]) : 0.0f;
 #pragma unroll
-        for (int k = 0; k < HOT_INFLIGHT; ++k)
+        for (int k = 0; k < LOADS; ++k)
           if (st[k] != ROW_SKIP) o[k * F + c] = hc_from_f32<TD>(v[k]);
       }
     }
@@ -180,21 +191,31 @@ __global__ __launch_bounds__(HC_BLOCK) void gather_flagged_kernel(const TS *__re
   }
 }
 
+template <typename TS, typename TD, bool TIERED>
+void launch_hot_to(const TS *hot, int64_t n_hot, const int32_t *slot_map, int64_t n_map, const int64_t *ids,
+                   const uint8_t *mask, TD *dst, uint8_t *cold, int64_t n, int64_t F, dim3 g, hipStream_t st) {
+  const dim3 bl(HC_BLOCK);
+  const bool vec = tier_vec_ok(hot, dst, F);
+  if (vec && F <= HC_WAVE / 4 * TV)
+    tier_hot_kernel<TS, TD, TIERED, 4><<<g, bl, 0, st>>>(hot, n_hot, slot_map, n_map, ids, mask, dst, cold, n, F);
+  else if (vec && F <= HC_WAVE / 2 * TV)
+    tier_hot_kernel<TS, TD, TIERED, 2><<<g, bl, 0, st>>>(hot, n_hot, slot_map, n_map, ids, mask, dst, cold, n, F);
+  else
+    tier_hot_kernel<TS, TD, TIERED, 1><<<g, bl, 0, st>>>(hot, n_hot, slot_map, n_map, ids, mask, dst, cold, n, F);
+}
+
 template <typename TS, bool TIERED>
 int launch_hot(const void *hot, int64_t n_hot, const int32_t *slot_map, int64_t n_map, const int64_t *ids,
                const uint8_t *mask, void *dst, int dst_dtype, uint8_t *cold, int64_t n, int64_t F, dim3 g,
                hipStream_t st) {
   const TS *h = static_cast<const TS *>(hot);
-  const dim3 bl(HC_BLOCK);
   if (dst_dtype == HC_F32)
-    tier_hot_kernel<TS, float, TIERED><<<g, bl, 0, st>>>(h, n_hot, slot_map, n_map, ids, mask,
-                                                         static_cast<float *>(dst), cold, n, F);
+    launch_hot_to<TS, float, TIERED>(h, n_hot, slot_map, n_map, ids, mask, static_cast<float *>(dst), cold, n, F, g, st);
   else if (dst_dtype == HC_F16)
-    tier_hot_kernel<TS, __half, TIERED><<<g, bl, 0, st>>>(h, n_hot, slot_map, n_map, ids, mask,
-                                                          static_cast<__half *>(dst), cold, n, F);
+    launch_hot_to<TS, __half, TIERED>(h, n_hot, slot_map, n_map, ids, mask, static_cast<__half *>(dst), cold, n, F, g, st);
   else
-    tier_hot_kernel<TS, __hip_bfloat16, TIERED><<<g, bl, 0, st>>>(h, n_hot, slot_map, n_map, ids, mask,
-                                                                  static_cast<__hip_bfloat16 *>(dst), cold, n, F);
+    launch_hot_to<TS, __hip_bfloat16, TIERED>(h, n_hot, slot_map, n_map, ids, mask, static_cast<__hip_bfloat16 *>(dst),
+                                              cold, n, F, g, st);
   return hc_launch_status();
 }
 
