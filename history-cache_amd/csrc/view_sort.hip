@@ -21,7 +21,8 @@
 //   vs_bucket   block per bucket: counts the local ids per wave (the waves own consecutive equal
 //               shares of the bucket's pairs), scans them -- which IS this bucket's stretch of
 //               ptrT --, ranks the pairs in order the same way and writes rowT (and edgeT) at segment
-//               start + rank, through LDS so that the stores are whole lines
+//               start + rank, through LDS so that the stores are whole lines; a bucket that is too much
+//               for one compute unit is shared by several blocks (parts of its local ids)
 // Every (source, slot) pair therefore lands where a stable sort by source puts it.  The cost is set
 // by the number of memory requests rather than by bytes: the scattered 8-byte stores of vs_scatter
 // are one request per live slot, which is why there are two levels and not three, and why everything
@@ -43,16 +44,30 @@ constexpr uint32_t VS_DEAD = 0xffffffffu;
 
 // Waves per block of vs_bucket.  A wave ranks its share of a bucket 64 pairs at a time, each step behind the one
 // before (0.6 us), and popular sources tend to be neighbours: of 3 M pairs over 1 M sources the fullest of 2 000
-// buckets held 90 000, which took four waves 214 us and takes sixteen 83.  Sixteen wherever their counters fit the LDS.
+// buckets held 90 000, which took four waves 214 us and sixteen 83 (before it was split, see below).  Sixteen wherever their counters fit the LDS.
 constexpr int VB_WAVES_MANY = 16, VB_WAVES_FEW = 4;
 constexpr int VB_MANY_LOCAL_BITS = 11;                   // 64 bytes of counters per local id
 constexpr uint32_t VB_STAGED = 8192;                     // largest bucket that takes the register path
 // Of the sixteen, four sort a bucket of up to VB_FEW_PAIRS pairs and the others leave at once, which makes room for the
-// next blocks: 3 M pairs evenly over 1 M sources 80 -> 67 us (65 with four waves for every bucket), with popular ones
-// among them 130 -> 126.  (Up to 8192 pairs: 74, above 2^10 local ids, whose counters leave a compute unit two blocks
+// next blocks: 3 M pairs evenly over 1 M sources 80 -> 67 us (65 with four waves for every bucket).  (Up to 8192 pairs: 74, above 2^10 local ids, whose counters leave a compute unit two blocks
 // at most: 81 -> 86.)
 constexpr uint32_t VB_FEW_PAIRS = 4096;
 constexpr int VB_FEW_LOCAL_BITS = 10;
+// A bucket of more pairs than a compute unit gets on average, and more than VB_HEAVY_PAIRS, would outlast the launch: it is
+// sorted by up to 32 blocks of their own, each of which reads all of its pairs and places those of one stretch of local
+// ids.  The whole view, rows / rows and slots: 3 M pairs over 1 M sources, popular ones among them, 127 / 284 -> 109 / 141 us;
+// 14 M over 3 M 633 / 1526 -> 399 / 722; 1 M over 200 000 75 / 110 -> 61 / 70; evenly spread ones as before (up to 1 us for the
+// blocks without work).  Parts of 4096 or 8192 pairs: 2 to 15% slower with up to 1 M pairs, 2 to 4% faster or slower above; 128
+// blocks instead of 512: up to 17% slower.  (Ranking several shares of a bucket side by side in a wave changed nothing:
+// it is the work, not the chain, that one compute unit is too small for.)
+constexpr uint32_t VB_HEAVY_PAIRS = VB_STAGED, VB_PART_PAIRS = 2048;
+constexpr int VB_PARTS_BITS = 5;                         // at most 32 parts
+constexpr int VB_PART_BLOCKS = 512;                      // blocks that work through the parts
+constexpr int VB_MAX_PARTS = 256 << VB_PARTS_BITS;       // fewer than 256 buckets hold more than a 256th of the pairs
+
+__host__ __device__ __forceinline__ uint32_t vb_heavy_above(uint32_t live) {
+  return live / 256 > VB_HEAVY_PAIRS ? live / 256 : VB_HEAVY_PAIRS;
+}
 
 // Tile of a block: workgroup i runs on XCD i % 8, and every XCD gets one contiguous eighth of the
 // tiles, so that the partial lines at the write front of every bucket (runs of a few pairs per tile)
@@ -298,8 +313,10 @@ __global__ __launch_bounds__(HC_BLOCK) void vs_bucket_scan(uint32_t *__restrict_
 // One block: bucket_off[0 .. nb] = exclusive scan of the bucket totals (bucket_off[nb] = live slots).
 constexpr int VS_OFF_THREADS = 1024;
 __global__ __launch_bounds__(VS_OFF_THREADS) void vs_bucket_offsets(const uint32_t *__restrict__ bucket_total,
-                                                                     uint32_t *__restrict__ bucket_off, VsShape S) {
+                                                                     uint32_t *__restrict__ bucket_off,
+                                                                     uint32_t *__restrict__ parts, VsShape S) {
   __shared__ uint32_t s_wave[VS_OFF_THREADS / HC_WAVE];
+  __shared__ uint32_t n_parts;
   constexpr int PER = (VS_MAX_BUCKETS + VS_OFF_THREADS - 1) / VS_OFF_THREADS;
   const int tid = (int)threadIdx.x;
   const int lane = hc_lane();
@@ -313,16 +330,31 @@ __global__ __launch_bounds__(VS_OFF_THREADS) void vs_bucket_offsets(const uint32
   }
   const uint32_t incl = vs_wave_incl_scan(sum, lane);
   if (lane == HC_WAVE - 1) s_wave[wave] = incl;
+  if (tid == 0) n_parts = 0u;
   __syncthreads();
-  uint32_t run = incl - sum;
-  for (int w = 0; w < wave; ++w) run += s_wave[w];
+  uint32_t run = incl - sum, live = 0u;
+  for (int w = 0; w < VS_OFF_THREADS / HC_WAVE; ++w) {
+    const uint32_t v = s_wave[w];
+    if (w < wave) run += v;
+    live += v;
+  }
+  const uint32_t heavy_above = vb_heavy_above(live);
 #pragma unroll
   for (int q = 0; q < PER; ++q) {
     const int b = tid * PER + q;
     if (b < S.nb) bucket_off[b] = run;
     run += c[q];
     if (b == S.nb - 1) bucket_off[S.nb] = run;
+    if (c[q] > heavy_above) {                            // parts[1 + i]: bucket, part, log2 of the number of parts
+      int bits = 1;
+      while (bits < VB_PARTS_BITS && ((uint32_t)VB_PART_PAIRS << bits) < c[q]) ++bits;
+      if (bits > S.lb) bits = S.lb;
+      const uint32_t at = atomicAdd(&n_parts, 1u << bits);
+      for (uint32_t i = 0; i < 1u << bits; ++i) parts[1 + at + i] = (uint32_t)b | i << 16 | (uint32_t)bits << 24;
+    }
   }
+  __syncthreads();
+  if (tid == 0) parts[0] = n_parts;
 }
 
 // Dynamic LDS: uint32 base[nbc] (the tile's first position in every bucket), then the waves'
@@ -556,58 +588,68 @@ __device__ __forceinline__ void vb_small(const uint2 *__restrict__ mine, uint32_
   }
 }
 
-// Buckets above VB_STAGED pairs (hub sources): 32-bit cursors, the pairs are read twice and the
-// results stored as they come.  LDS: cur[VB_WAVES][n_local].
+// Buckets above VB_STAGED pairs (hub sources), or one part of them: local ids [k0, k0 + n_ids).  32-bit cursors, the
+// pairs are read twice and the results stored as they come.  LDS: cur[VB_WAVES][n_ids].
 template <bool WANT_EDGES, int VB_WAVES>
 __device__ __forceinline__ void vb_large(const uint2 *__restrict__ mine, uint32_t n, uint32_t p0, int64_t b,
+                                         uint32_t k0, uint32_t n_ids,
                                          uint32_t *__restrict__ cur, uint32_t *__restrict__ s_wave,
+                                         uint32_t *__restrict__ s_below,
                                          const uint32_t *__restrict__ rows, int64_t *__restrict__ ptrT,
                                          int32_t *__restrict__ rowT, int32_t *__restrict__ edgeT, const VsShape &S) {
   constexpr int VB_THREADS = VB_WAVES * HC_WAVE;
   const int tid = (int)threadIdx.x;
   const int lane = hc_lane();
   const int wave = tid >> 6;
-  const uint32_t n_local = 1u << S.lb;
   const uint32_t share = ((n + VB_WAVES - 1) / VB_WAVES + HC_WAVE - 1) / HC_WAVE * HC_WAVE;
   const uint32_t q_begin = (uint32_t)wave * share < n ? (uint32_t)wave * share : n;
   const uint32_t q_end = q_begin + share < n ? q_begin + share : n;
-  uint32_t *my = cur + (uint32_t)wave * n_local;
-  for (uint32_t i = tid; i < VB_WAVES * n_local; i += VB_THREADS) cur[i] = 0u;
+  uint32_t *my = cur + (uint32_t)wave * n_ids;
+  for (uint32_t i = tid; i < VB_WAVES * n_ids; i += VB_THREADS) cur[i] = 0u;
   __syncthreads();
+  uint32_t below_k0 = 0u;                                // pairs of smaller ids
 #pragma unroll 4
-  for (uint32_t i = q_begin + lane; i < q_end; i += HC_WAVE) atomicAdd(&my[vb_swz32(mine[i].x)], 1u);
+  for (uint32_t i = q_begin + lane; i < q_end; i += HC_WAVE) {
+    const uint32_t id = mine[i].x, k = id - k0;
+    if (id < k0) ++below_k0;
+    else if (k < n_ids) atomicAdd(&my[vb_swz32(k)], 1u);
+  }
+#pragma unroll
+  for (int d = HC_WAVE / 2; d > 0; d >>= 1) below_k0 += (uint32_t)__shfl_xor((int)below_k0, d, HC_WAVE);
+  if (lane == 0) s_below[wave] = below_k0;
   __syncthreads();
   {
-    const uint32_t per = n_local >= (uint32_t)VB_THREADS ? n_local / VB_THREADS : 1u;   // ids per thread
-    const uint32_t k0 = (uint32_t)tid * per;
+    const uint32_t per = n_ids >= (uint32_t)VB_THREADS ? n_ids / VB_THREADS : 1u;   // ids per thread
+    const uint32_t at0 = (uint32_t)tid * per;
     uint32_t sum = 0u;
-    if (k0 < n_local)
-      for (uint32_t k = k0; k < k0 + per; ++k) {
+    if (at0 < n_ids)
+      for (uint32_t k = at0; k < at0 + per; ++k) {
         const uint32_t at = vb_swz32(k);
 #pragma unroll
-        for (int w = 0; w < VB_WAVES; ++w) sum += cur[(uint32_t)w * n_local + at];
+        for (int w = 0; w < VB_WAVES; ++w) sum += cur[(uint32_t)w * n_ids + at];
       }
     const uint32_t incl = vs_wave_incl_scan(sum, lane);
     if (lane == HC_WAVE - 1) s_wave[wave] = incl;
     __syncthreads();
     uint32_t run = incl - sum;
     for (int w = 0; w < wave; ++w) run += s_wave[w];
-    if (k0 < n_local)
-      for (uint32_t k = k0; k < k0 + per; ++k) {
+    for (int w = 0; w < VB_WAVES; ++w) run += s_below[w];
+    if (at0 < n_ids)
+      for (uint32_t k = at0; k < at0 + per; ++k) {
         const uint32_t at = vb_swz32(k);
         uint32_t c[VB_WAVES];
 #pragma unroll
-        for (int w = 0; w < VB_WAVES; ++w) c[w] = cur[(uint32_t)w * n_local + at];
+        for (int w = 0; w < VB_WAVES; ++w) c[w] = cur[(uint32_t)w * n_ids + at];
 #pragma unroll
         for (int w = 0; w < VB_WAVES; ++w) {
-          cur[(uint32_t)w * n_local + at] = run;
+          cur[(uint32_t)w * n_ids + at] = run;
           run += c[w];
         }
       }
   }
   __syncthreads();
-  for (uint32_t k = tid; k < n_local; k += VB_THREADS) {
-    const int64_t id = b * (int64_t)n_local + k;
+  for (uint32_t k = tid; k < n_ids; k += VB_THREADS) {
+    const int64_t id = b * ((int64_t)1 << S.lb) + k0 + k;
     if (id <= S.n_src) ptrT[id] = (int64_t)p0 + cur[vb_swz32(k)];    // wave 0's cursor = the segment's start
   }
   __syncthreads();
@@ -618,13 +660,12 @@ __device__ __forceinline__ void vb_large(const uint2 *__restrict__ mine, uint32_
 #pragma unroll
     for (int d = 0; d < DEPTH; ++d) {
       const uint32_t i = i0 + d * HC_WAVE + lane;
-      pr[d] = i < q_end ? mine[i] : make_uint2(0u, 0u);
+      pr[d] = i < q_end ? mine[i] : make_uint2(0xffffffffu, 0u);     // no local id
     }
 #pragma unroll
     for (int d = 0; d < DEPTH; ++d) {
-      const uint32_t i = i0 + d * HC_WAVE + lane;
-      const bool live = i < q_end;
-      const uint32_t k = pr[d].x;
+      const uint32_t k = pr[d].x - k0;
+      const bool live = pr[d].x != 0xffffffffu && k < n_ids;
       uint32_t before = 0u, same = 0u;
       if (live) {
         uint32_t *c = &my[vb_swz32(k)];
@@ -648,12 +689,25 @@ __device__ __forceinline__ void vb_large(const uint2 *__restrict__ mine, uint32_
 template <bool WANT_EDGES, int VB_WAVES>
 __global__ __launch_bounds__(VB_WAVES * HC_WAVE) void vs_bucket(const uint2 *__restrict__ pairs,
                                                          const uint32_t *__restrict__ bucket_off,
+                                                         const uint32_t *__restrict__ parts,
                                                          const uint32_t *__restrict__ rows,
                                                          int64_t *__restrict__ ptrT, int32_t *__restrict__ rowT,
                                                          int32_t *__restrict__ edgeT, VsShape S) {
   extern __shared__ uint32_t vb_lds[];
-  __shared__ uint32_t s_wave[VB_WAVES];
-  const int64_t b = blockIdx.x;
+  __shared__ uint32_t s_wave[VB_WAVES], s_below[VB_WAVES];
+  if (blockIdx.x < VB_PART_BLOCKS) {                       // parts of the heavy buckets, in front of the others
+    const uint32_t n_parts = parts[0];
+    for (uint32_t i = blockIdx.x; i < n_parts; i += VB_PART_BLOCKS) {
+      const uint32_t item = parts[1 + i], part = (item >> 16) & 0xffu;
+      const int64_t b = item & 0xffffu;
+      const uint32_t p0 = bucket_off[b], n_ids = (1u << S.lb) >> (item >> 24);
+      vb_large<WANT_EDGES, VB_WAVES>(pairs + p0, bucket_off[b + 1] - p0, p0, b, part * n_ids, n_ids, vb_lds, s_wave, s_below,
+                                     rows, ptrT, rowT, edgeT, S);
+      __syncthreads();                                     // the counters are free again
+    }
+    return;
+  }
+  const int64_t b = (int64_t)blockIdx.x - VB_PART_BLOCKS;
   const uint32_t p0 = bucket_off[b];
   const uint32_t n = bucket_off[b + 1] - p0;               // block-uniform
   if constexpr (VB_WAVES > VB_WAVES_FEW) {
@@ -664,11 +718,12 @@ __global__ __launch_bounds__(VB_WAVES * HC_WAVE) void vs_bucket(const uint2 *__r
     }
   }
   if (n <= VB_STAGED) vb_small<WANT_EDGES, VB_WAVES, VB_STAGED>(pairs + p0, n, p0, b, vb_lds, s_wave, rows, ptrT, rowT, edgeT, S);
-  else vb_large<WANT_EDGES, VB_WAVES>(pairs + p0, n, p0, b, vb_lds, s_wave, rows, ptrT, rowT, edgeT, S);
+  else if (n <= vb_heavy_above(bucket_off[S.nb]))
+    vb_large<WANT_EDGES, VB_WAVES>(pairs + p0, n, p0, b, 0u, 1u << S.lb, vb_lds, s_wave, s_below, rows, ptrT, rowT, edgeT, S);
 }
 
 struct VsLayout {
-  size_t key32, tile_count, group_count, bucket_total, bucket_off, pairs, rows, bits, total;
+  size_t key32, tile_count, group_count, bucket_total, bucket_off, parts, pairs, rows, bits, total;
 };
 
 bool vs_shape(int64_t R, int64_t E, int64_t n_src, VsShape *S) {
@@ -719,6 +774,7 @@ VsLayout vs_layout(const VsShape &S) {
   L.group_count = take((size_t)S.ngroups * S.nbp * sizeof(uint32_t));
   L.bucket_total = take((size_t)S.nbp * sizeof(uint32_t));
   L.bucket_off = take((size_t)(S.nbp + 1) * sizeof(uint32_t));
+  L.parts = take((size_t)(VB_MAX_PARTS + 1) * sizeof(uint32_t));
   L.pairs = take((size_t)S.E * sizeof(uint2));
   L.rows = take((size_t)S.E * sizeof(uint32_t));
   L.bits = take((size_t)((S.n_src + 63) / 64) * 8 + 8);
@@ -743,12 +799,12 @@ bool vs_allow_lds(size_t bytes) {
 }
 
 template <bool WANT_EDGES, int VB_WAVES>
-bool vs_launch_bucket(const uint2 *pairs, const uint32_t *bucket_off, const uint32_t *rows, int64_t *ptrT,
-                      int32_t *rowT, int32_t *edgeT, const VsShape &S, hipStream_t st) {
+bool vs_launch_bucket(const uint2 *pairs, const uint32_t *bucket_off, const uint32_t *parts, const uint32_t *rows,
+                      int64_t *ptrT, int32_t *rowT, int32_t *edgeT, const VsShape &S, hipStream_t st) {
   const size_t lds = vs_bucket_lds(S);
   if (!vs_allow_lds<&vs_bucket<WANT_EDGES, VB_WAVES>>(lds)) return false;
-  vs_bucket<WANT_EDGES, VB_WAVES><<<dim3((unsigned)S.nb), dim3(VB_WAVES * HC_WAVE), lds, st>>>(pairs, bucket_off, rows,
-                                                                                             ptrT, rowT, edgeT, S);
+  vs_bucket<WANT_EDGES, VB_WAVES><<<dim3((unsigned)(VB_PART_BLOCKS + S.nb)), dim3(VB_WAVES * HC_WAVE), lds, st>>>(
+      pairs, bucket_off, parts, rows, ptrT, rowT, edgeT, S);
   return true;
 }
 
@@ -777,6 +833,7 @@ int vs_launch(const int64_t *ptr, const int64_t *idx, const int64_t *hmap_row, c
   uint32_t *group_count = reinterpret_cast<uint32_t *>(ws + L.group_count);
   uint32_t *bucket_total = reinterpret_cast<uint32_t *>(ws + L.bucket_total);
   uint32_t *bucket_off = reinterpret_cast<uint32_t *>(ws + L.bucket_off);
+  uint32_t *parts = reinterpret_cast<uint32_t *>(ws + L.parts);
   uint2 *pairs = reinterpret_cast<uint2 *>(ws + L.pairs);
   uint32_t *rows = reinterpret_cast<uint32_t *>(ws + L.rows);
   const uint32_t *src_bits = nullptr;
@@ -799,19 +856,19 @@ int vs_launch(const int64_t *ptr, const int64_t *idx, const int64_t *hmap_row, c
       tile_count, group_count, S);
   vs_bucket_scan<<<dim3((unsigned)((S.nb + HC_WAVES_PER_BLOCK - 1) / HC_WAVES_PER_BLOCK)), dim3(HC_BLOCK), 0, st>>>(
       group_count, bucket_total, S);
-  vs_bucket_offsets<<<dim3(1), dim3(VS_OFF_THREADS), 0, st>>>(bucket_total, bucket_off, S);
+  vs_bucket_offsets<<<dim3(1), dim3(VS_OFF_THREADS), 0, st>>>(bucket_total, bucket_off, parts, S);
   const bool many = vs_bucket_waves(S) == VB_WAVES_MANY;
   bool ok;
   if (edgeT != nullptr) {
     vs_scatter<false><<<tgrid, dim3(VS_THREADS), lds, st>>>(ptr, key32, tile_count, group_count, bucket_off, pairs,
                                                            rows, S);
-    ok = many ? vs_launch_bucket<true, VB_WAVES_MANY>(pairs, bucket_off, rows, ptrT, rowT, edgeT, S, st)
-              : vs_launch_bucket<true, VB_WAVES_FEW>(pairs, bucket_off, rows, ptrT, rowT, edgeT, S, st);
+    ok = many ? vs_launch_bucket<true, VB_WAVES_MANY>(pairs, bucket_off, parts, rows, ptrT, rowT, edgeT, S, st)
+              : vs_launch_bucket<true, VB_WAVES_FEW>(pairs, bucket_off, parts, rows, ptrT, rowT, edgeT, S, st);
   } else {
     vs_scatter<true><<<tgrid, dim3(VS_THREADS), lds, st>>>(ptr, key32, tile_count, group_count, bucket_off, pairs,
                                                           rows, S);
-    ok = many ? vs_launch_bucket<false, VB_WAVES_MANY>(pairs, bucket_off, rows, ptrT, rowT, edgeT, S, st)
-              : vs_launch_bucket<false, VB_WAVES_FEW>(pairs, bucket_off, rows, ptrT, rowT, edgeT, S, st);
+    ok = many ? vs_launch_bucket<false, VB_WAVES_MANY>(pairs, bucket_off, parts, rows, ptrT, rowT, edgeT, S, st)
+              : vs_launch_bucket<false, VB_WAVES_FEW>(pairs, bucket_off, parts, rows, ptrT, rowT, edgeT, S, st);
   }
   if (!ok) return HC_ELAUNCH;
   return hc_launch_status();
