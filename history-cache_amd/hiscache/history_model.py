@@ -36,7 +36,8 @@ _WGRAD_SLAB_ROWS = 1024
 _WGRAD_SPLIT_MIN_ROWS = 8192
 # The library's own kernel (hc_weight_grad: both operands of a SAGE layer in one pair of launches, 41 us at
 # n = 25 800 and F = 128, 77 us at n = 55 000) takes over when the widths fit it; with fewer rows too (1 000 rows,
-# F = 128: 9 us for both operands; two GEMMs 40 to 227, by the kernel chosen) unless something watches the operators.
+# F = 128: 9 us for both operands; two GEMMs 40 to 227, by the kernel chosen) and for any number of outputs, with the
+# bias' gradient (hc_linear_grad), unless something watches the operators.
 _WGRAD_KERNEL_MIN_ROWS = 2048
 
 
@@ -134,19 +135,24 @@ class _SageConvFunction(torch.autograd.Function):
             g_agg = be.linear(g_out, w_l, transposed=True) if own else g_out @ w_l
         if his is not None:
             his.grad = g_agg
-        g_bl = _column_sums(g_out) if has_bias and need[2] else None
-        g_wl = g_wr = None
+        g_bl = g_wl = g_wr = None
         root = None
         if has_root and need[3]:
             root = x[:R] if x.dtype == g_out.dtype else x[:R].to(g_out.dtype)
-        if (need[1] and root is not None and be.weight_grad_supported(g_out, agg)
-                and (R >= _WGRAD_KERNEL_MIN_ROWS or be.plain_operands(g_out, agg, root))):
+        want_bias = has_bias and need[2]
+        if (need[1] and root is not None and agg.shape[1] % 64 == 0 and max(agg.shape[1], g_out.shape[1]) <= 4096
+                and agg.shape == root.shape and be.plain_operands(g_out, agg, root)):
+            g_wl, g_wr, g_bl = be.linear_grad(g_out, agg, root, want_bias)
+        elif (need[1] and root is not None and R >= _WGRAD_KERNEL_MIN_ROWS
+                and be.weight_grad_supported(g_out, agg)):
             g_wl, g_wr = be.weight_grad(g_out, agg, root)          # both products in one pair of launches
         else:
             if need[1]:
                 g_wl = _weight_grad(g_out, agg)
             if root is not None:
                 g_wr = _weight_grad(g_out, root)
+        if want_bias and g_bl is None:
+            g_bl = _column_sums(g_out)
         g_x = None
         if need[0]:
             n_src = x.shape[0]

@@ -131,6 +131,8 @@ _SIGNATURES = {
                                    _c_i64, _c_i64, _c_p]),
     "hc_weight_grad_workspace_bytes": (_c_sz, [_c_i64, _c_i64, _c_i64, _c_int]),
     "hc_weight_grad": (_c_int, [_c_p, _c_p, _c_p, _c_i64, _c_i64, _c_i64, _c_p, _c_p, _c_p, _c_sz, _c_p]),
+    "hc_linear_grad_workspace_bytes": (_c_sz, [_c_i64, _c_i64, _c_i64, _c_int]),
+    "hc_linear_grad": (_c_int, [_c_p, _c_p, _c_p, _c_i64, _c_i64, _c_i64, _c_p, _c_p, _c_p, _c_p, _c_sz, _c_p]),
     "hc_stage_arrays": (_c_int, [_c_p, _c_p, _c_p, _c_p, _c_p, _c_p, _c_int, _c_p, _c_p, _c_int, _c_p]),
     "hc_ring_lookup_dev": (_c_int, [_c_p, _c_i64, _c_p, _c_p, _c_p, _c_p, _c_i64, _c_p, _c_int, _c_i64, _c_i64, _c_p,
                                     _c_p, _c_i64, _c_p]),
@@ -1404,6 +1406,26 @@ def weight_grad(g, x0, x1=None):
                               _c_p(p + 4 * H * F) if x1 is not None else _c_p(None), _ptr(ws), ws.numel(),
                               _stream()), "hc_weight_grad")
     return (dw[0], dw[1]) if x1 is not None else dw[0]
+
+
+def linear_grad(g, x0, x1, want_bias):
+    """``g.t() @ x0``, ``g.t() @ x1`` and (``want_bias``, else None) ``g.sum(0)`` in two launches: what the backward of
+    ``x0 @ w0.t() + x1 @ w1.t() + bias`` owes to its parameters.  g [n, H], x [n, F], fp32; F a multiple of 64, H and F
+    at most 4096, H any."""
+    lib = load_library()
+    for name, t in (("g", g), ("x0", x0), ("x1", x1)):
+        _dev(t, name, torch.float32)
+    if g.dim() != 2 or x0.dim() != 2 or x0.shape[0] != g.shape[0] or x1.shape != x0.shape:
+        raise ValueError("g [n, H], x0 and x1 [n, F] must have the same number of rows")
+    (n, H), F = g.shape, x0.shape[1]
+    ws_bytes = int(lib.hc_linear_grad_workspace_bytes(n, H, F, 2))
+    dw = torch.empty((2, H, F), dtype=torch.float32, device=g.device)
+    db = torch.empty(H, dtype=torch.float32, device=g.device) if want_bias else None
+    ws = _workspace(ws_bytes, g.device)
+    p = dw.data_ptr()
+    _check(lib.hc_linear_grad(_ptr(g), _ptr(x0), _ptr(x1), n, H, F, _c_p(p), _c_p(p + 4 * H * F), _ptr(db), _ptr(ws),
+                              ws_bytes, _stream()), "hc_linear_grad")
+    return dw[0], dw[1], db
 
 
 _PLAIN = (torch.Tensor, torch.nn.Parameter)

@@ -718,6 +718,14 @@ size_t hc_weight_grad_workspace_bytes(int64_t n, int64_t H, int64_t F, int n_ope
 int hc_weight_grad(const float *g, const float *x0, const float *x1, int64_t n, int64_t H, int64_t F,
                    float *dw0, float *dw1, void *workspace, size_t workspace_bytes, void *stream);
 
+/* hc_linear_grad: hc_weight_grad for any H up to 4096 (a last layer's classes),
+ * with the gradient of the bias, dbias[H] = the sums of g's columns (nullable),
+ * in the same two launches.  F % 64 == 0, at most 4096; dw 16-byte aligned.
+ * workspace: hc_linear_grad_workspace_bytes(n, H, F, operands), 16-byte aligned. */
+size_t hc_linear_grad_workspace_bytes(int64_t n, int64_t H, int64_t F, int n_operands);
+int hc_linear_grad(const float *g, const float *x0, const float *x1, int64_t n, int64_t H, int64_t F,
+                   float *dw0, float *dw1, float *dbias, void *workspace, size_t workspace_bytes, void *stream);
+
 /* ---------------------------------------------------------------- recorded iterations
  * Entry points for callers that record the launches of one training iteration
  * once (a HIP graph over arrays of a fixed, padded size) and replay them for

@@ -36,3 +36,25 @@ def test_relational_weight_gradient(n, K, F, H):
         got = hm._rel_weight_grad(agg, g)
     assert tuple(got.shape) == (K, F, H)
     _close(got.view(K * F, H), agg.view(n, K * F), g, n)
+
+
+@pytest.mark.parametrize("n", (1, 5, 33, 64, 1000, 4097))
+@pytest.mark.parametrize("H,F", ((1, 64), (10, 128), (47, 64), (63, 64), (65, 128), (153, 256), (172, 256), (256, 64)))
+def test_linear_grad_for_any_number_of_outputs(n, H, F):
+    gen = torch.Generator(device=DEV).manual_seed(n + H)
+    g, x0, x1 = (torch.randn(n, c, device=DEV, generator=gen) for c in (H, F, F))
+    d0, d1, db = be.linear_grad(g, x0, x1, True)
+    _close(d0, g, x0, n)
+    _close(d1, g, x1, n)
+    assert db.shape == (H,)
+    _close(db.view(H, 1), g, torch.ones(n, 1, device=DEV), n)
+    e0, e1, none = be.linear_grad(torch.empty(n * H + 1, device=DEV)[1:].view(n, H).copy_(g), x0, x1, False)
+    assert none is None and torch.equal(e0, d0) and torch.equal(e1, d1)      # the order depends on nothing else
+
+
+def test_linear_grad_refuses_what_does_not_fit():
+    g, x = torch.randn(9, 10, device=DEV), torch.randn(9, 64, device=DEV)
+    for call in (lambda: be.linear_grad(g, x, x[:8], True), lambda: be.linear_grad(g, x[:8], x[:8], True),
+                 lambda: be.linear_grad(g.half(), x, x, True), lambda: be.linear_grad(g, x[:, :32].contiguous(), x[:, :32].contiguous(), True)):
+        with pytest.raises(ValueError):
+            call()
