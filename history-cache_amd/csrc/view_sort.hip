@@ -62,7 +62,7 @@ constexpr int VB_FEW_LOCAL_BITS = 10;
 // it is the work, not the chain, that one compute unit is too small for.)
 constexpr uint32_t VB_HEAVY_PAIRS = VB_STAGED, VB_PART_PAIRS = 2048;
 constexpr int VB_PARTS_BITS = 5;                         // at most 32 parts
-constexpr int VB_PART_BLOCKS = 512;                      // blocks that work through the parts
+constexpr int VB_PART_BLOCKS = 512;                      // most blocks that work through the parts
 constexpr int VB_MAX_PARTS = 256 << VB_PARTS_BITS;       // fewer than 256 buckets hold more than a 256th of the pairs
 
 __host__ __device__ __forceinline__ uint32_t vb_heavy_above(uint32_t live) {
@@ -195,6 +195,7 @@ struct VsShape {
   int lb;          // bits of a local id
   int nb;          // buckets: ids 0 .. n_src (ptrT has an entry for n_src too)
   int nbp;         // row pitch of the per-tile and per-group count matrices
+  int part_blocks; // blocks that work through the parts of heavy buckets
   int nbc;         // pitch of a wave's 16-bit counters in vs_scatter's LDS (even)
 };
 
@@ -316,7 +317,8 @@ __global__ __launch_bounds__(VS_OFF_THREADS) void vs_bucket_offsets(const uint32
                                                                      uint32_t *__restrict__ bucket_off,
                                                                      uint32_t *__restrict__ parts, VsShape S) {
   __shared__ uint32_t s_wave[VS_OFF_THREADS / HC_WAVE];
-  __shared__ uint32_t n_parts;
+  __shared__ uint32_t n_parts, n_heavy;
+  __shared__ uint2 heavy[256];                           // a heavy bucket with log2 of its parts, and its first part
   constexpr int PER = (VS_MAX_BUCKETS + VS_OFF_THREADS - 1) / VS_OFF_THREADS;
   const int tid = (int)threadIdx.x;
   const int lane = hc_lane();
@@ -330,7 +332,7 @@ __global__ __launch_bounds__(VS_OFF_THREADS) void vs_bucket_offsets(const uint32
   }
   const uint32_t incl = vs_wave_incl_scan(sum, lane);
   if (lane == HC_WAVE - 1) s_wave[wave] = incl;
-  if (tid == 0) n_parts = 0u;
+  if (tid == 0) n_parts = n_heavy = 0u;
   __syncthreads();
   uint32_t run = incl - sum, live = 0u;
   for (int w = 0; w < VS_OFF_THREADS / HC_WAVE; ++w) {
@@ -349,11 +351,15 @@ __global__ __launch_bounds__(VS_OFF_THREADS) void vs_bucket_offsets(const uint32
       int bits = 1;
       while (bits < VB_PARTS_BITS && ((uint32_t)VB_PART_PAIRS << bits) < c[q]) ++bits;
       if (bits > S.lb) bits = S.lb;
-      const uint32_t at = atomicAdd(&n_parts, 1u << bits);
-      for (uint32_t i = 0; i < 1u << bits; ++i) parts[1 + at + i] = (uint32_t)b | i << 16 | (uint32_t)bits << 24;
+      heavy[atomicAdd(&n_heavy, 1u)] = make_uint2((uint32_t)b | (uint32_t)bits << 24, atomicAdd(&n_parts, 1u << bits));
     }
   }
   __syncthreads();
+  for (uint32_t i = tid; i < n_heavy << VB_PARTS_BITS; i += VS_OFF_THREADS) {
+    const uint2 h = heavy[i >> VB_PARTS_BITS];
+    const uint32_t part = i & ((1u << VB_PARTS_BITS) - 1u);
+    if (part < 1u << (h.x >> 24)) parts[1 + h.y + part] = h.x | part << 16;
+  }
   if (tid == 0) parts[0] = n_parts;
 }
 
@@ -695,9 +701,9 @@ __global__ __launch_bounds__(VB_WAVES * HC_WAVE) void vs_bucket(const uint2 *__r
                                                          int32_t *__restrict__ edgeT, VsShape S) {
   extern __shared__ uint32_t vb_lds[];
   __shared__ uint32_t s_wave[VB_WAVES], s_below[VB_WAVES];
-  if (blockIdx.x < VB_PART_BLOCKS) {                       // parts of the heavy buckets, in front of the others
+  if ((int)blockIdx.x < S.part_blocks) {                   // parts of the heavy buckets, in front of the others
     const uint32_t n_parts = parts[0];
-    for (uint32_t i = blockIdx.x; i < n_parts; i += VB_PART_BLOCKS) {
+    for (uint32_t i = blockIdx.x; i < n_parts; i += S.part_blocks) {
       const uint32_t item = parts[1 + i], part = (item >> 16) & 0xffu;
       const int64_t b = item & 0xffffu;
       const uint32_t p0 = bucket_off[b], n_ids = (1u << S.lb) >> (item >> 24);
@@ -707,7 +713,7 @@ __global__ __launch_bounds__(VB_WAVES * HC_WAVE) void vs_bucket(const uint2 *__r
     }
     return;
   }
-  const int64_t b = (int64_t)blockIdx.x - VB_PART_BLOCKS;
+  const int64_t b = (int64_t)blockIdx.x - S.part_blocks;
   const uint32_t p0 = bucket_off[b];
   const uint32_t n = bucket_off[b + 1] - p0;               // block-uniform
   if constexpr (VB_WAVES > VB_WAVES_FEW) {
@@ -744,6 +750,8 @@ bool vs_shape(int64_t R, int64_t E, int64_t n_src, VsShape *S) {
   S->nb = (int)((ids + ((int64_t)1 << lb) - 1) >> lb);
   S->nbp = (S->nb + 63) / 64 * 64;
   S->nbc = (S->nb + 1) / 2 * 2;
+  // (one per VB_HEAVY_PAIRS slots: with few slots the blocks that find no part cost more than they could give)
+  S->part_blocks = (int)(E / VB_HEAVY_PAIRS < VB_PART_BLOCKS ? E / VB_HEAVY_PAIRS : VB_PART_BLOCKS);
   S->ntiles = (E + VS_TILE - 1) / VS_TILE;
   S->ngroups = (S->ntiles + VS_GROUP - 1) / VS_GROUP;
   return true;
@@ -803,7 +811,7 @@ bool vs_launch_bucket(const uint2 *pairs, const uint32_t *bucket_off, const uint
                       int64_t *ptrT, int32_t *rowT, int32_t *edgeT, const VsShape &S, hipStream_t st) {
   const size_t lds = vs_bucket_lds(S);
   if (!vs_allow_lds<&vs_bucket<WANT_EDGES, VB_WAVES>>(lds)) return false;
-  vs_bucket<WANT_EDGES, VB_WAVES><<<dim3((unsigned)(VB_PART_BLOCKS + S.nb)), dim3(VB_WAVES * HC_WAVE), lds, st>>>(
+  vs_bucket<WANT_EDGES, VB_WAVES><<<dim3((unsigned)(S.part_blocks + S.nb)), dim3(VB_WAVES * HC_WAVE), lds, st>>>(
       pairs, bucket_off, parts, rows, ptrT, rowT, edgeT, S);
   return true;
 }
