@@ -34,10 +34,10 @@ class _GradSink:
 # 72 - 131 and 107 - 193 us: linear in n.  Below this many rows the single GEMM is used (21 us at 5 800).
 _WGRAD_SLAB_ROWS = 1024
 _WGRAD_SPLIT_MIN_ROWS = 8192
-# The library's own kernel (hc_weight_grad: both operands of a SAGE layer in one pair of launches, 41 us at
-# n = 25 800 and F = 128, 77 us at n = 55 000) takes over when the widths fit it; with fewer rows too (1 000 rows,
-# F = 128: 9 us for both operands; two GEMMs 40 to 227, by the kernel chosen) and for any number of outputs, with the
-# bias' gradient (hc_linear_grad), unless something watches the operators.
+# The library's own kernel (hc_linear_grad: both operands of a SAGE layer and the bias in one pair of launches, 41 us at
+# n = 25 800 and F = 128, 77 us at n = 55 000) takes over when the inner width fits it; with fewer rows too (1 000 rows,
+# F = 128: 9 us for both operands; two GEMMs 40 to 227, by the kernel chosen), unless something watches the operators or
+# the gradient is not in memory (batched gradients).
 _WGRAD_KERNEL_MIN_ROWS = 2048
 
 
@@ -144,7 +144,7 @@ class _SageConvFunction(torch.autograd.Function):
                 and agg.shape == root.shape and be.plain_operands(g_out, agg, root)):
             g_wl, g_wr, g_bl = be.linear_grad(g_out, agg, root, want_bias)
         elif (need[1] and root is not None and R >= _WGRAD_KERNEL_MIN_ROWS
-                and be.weight_grad_supported(g_out, agg)):
+                and be.weight_grad_supported(g_out, agg) and be.in_memory(g_out, agg, root)):
             g_wl, g_wr = be.weight_grad(g_out, agg, root)          # both products in one pair of launches
         else:
             if need[1]:
@@ -441,7 +441,7 @@ def _rel_weight_grad(agg, g):
     n, K, Fin = agg.shape
     a2 = agg.reshape(n, K * Fin)
     # (4 200 rows, 3 840 x 256: 88 us against 150 for the slabs' batched GEMM and their sum)
-    if hiscache_backend.weight_grad_supported(a2, g) and hiscache_backend.plain_operands(a2, g):
+    if hiscache_backend.weight_grad_supported(a2, g) and hiscache_backend.plain_operands(g, a2):
         return hiscache_backend.weight_grad(a2, g).view(K, Fin, -1)
     S = max(_REL_WGRAD_SLABS, n // _WGRAD_SLAB_ROWS)
     m = n // S * S

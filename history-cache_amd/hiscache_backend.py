@@ -1431,14 +1431,25 @@ def linear_grad(g, x0, x1, want_bias):
 _PLAIN = (torch.Tensor, torch.nn.Parameter)
 
 
+def in_memory(*tensors):
+    """Do the values of these tensors lie where ``data_ptr()`` says?  Batched by a function transform or by
+    ``is_grads_batched`` they have no memory of their own (``data_ptr()`` raises, whatever their type says), zeros that
+    were never written have none either, and a lazily negated first operand (in a backward pass the gradient, the one
+    that comes from outside) lies there with the other sign."""
+    try:
+        return not tensors[0].is_neg() and all(t is None or t.data_ptr() != 0 for t in tensors)
+    except RuntimeError:
+        return False
+
+
 def plain_operands(a, *others):
-    """May a library call stand for torch operators on these tensors: plain, packed fp32 tensors on the current GPU, no
-    autocast, nothing that records or replaces operators?"""
+    """May a library call stand for torch operators on these tensors: plain, packed fp32 tensors in the memory of the
+    current GPU, no autocast, nothing that records or replaces operators?"""
     return (a.is_cuda and a.device.index == torch.cuda.current_device()
             and all(t is None or (type(t) in _PLAIN and t.dtype == torch.float32 and t.device == a.device
                                   and t.is_contiguous() and t.numel() > 0) for t in (a, *others))
             and not torch.is_grad_enabled() and not torch.is_autocast_enabled("cuda")
-            and torch._C._len_torch_dispatch_stack() == 0)
+            and torch._C._len_torch_dispatch_stack() == 0 and in_memory(a, *others))
 
 
 def linear_supported(a, *others):
