@@ -37,7 +37,8 @@ _WGRAD_SPLIT_MIN_ROWS = 8192
 # The library's own kernel (hc_linear_grad: both operands of a SAGE layer and the bias in one pair of launches, 41 us at
 # n = 25 800 and F = 128, 77 us at n = 55 000) takes over when the inner width fits it; with fewer rows too (1 000 rows,
 # F = 128: 9 us for both operands; two GEMMs 40 to 227, by the kernel chosen), unless something watches the operators or
-# the gradient is not in memory (batched gradients).
+# the gradient is not in memory (batched gradients).  Under autocast, which would round the operators' operands to half
+# precision, only from this many rows on.
 _WGRAD_KERNEL_MIN_ROWS = 2048
 
 
@@ -144,7 +145,7 @@ class _SageConvFunction(torch.autograd.Function):
                 and agg.shape == root.shape and be.plain_operands(g_out, agg, root)):
             g_wl, g_wr, g_bl = be.linear_grad(g_out, agg, root, want_bias)
         elif (need[1] and root is not None and R >= _WGRAD_KERNEL_MIN_ROWS
-                and be.weight_grad_supported(g_out, agg) and be.in_memory(g_out, agg, root)):
+                and be.weight_grad_supported(g_out, agg) and be.plain_operands(g_out, agg, root, autocast=True)):
             g_wl, g_wr = be.weight_grad(g_out, agg, root)          # both products in one pair of launches
         else:
             if need[1]:

@@ -1442,13 +1442,13 @@ def in_memory(*tensors):
         return False
 
 
-def plain_operands(a, *others):
+def plain_operands(a, *others, autocast=False):
     """May a library call stand for torch operators on these tensors: plain, packed fp32 tensors in the memory of the
-    current GPU, no autocast, nothing that records or replaces operators?"""
+    current GPU, no autocast (unless ``autocast``), nothing that records or replaces operators?"""
     return (a.is_cuda and a.device.index == torch.cuda.current_device()
             and all(t is None or (type(t) in _PLAIN and t.dtype == torch.float32 and t.device == a.device
                                   and t.is_contiguous() and t.numel() > 0) for t in (a, *others))
-            and not torch.is_grad_enabled() and not torch.is_autocast_enabled("cuda")
+            and not torch.is_grad_enabled() and (autocast or not torch.is_autocast_enabled("cuda"))
             and torch._C._len_torch_dispatch_stack() == 0 and in_memory(a, *others))
 
 

@@ -1,8 +1,10 @@
-"""Weight gradients of a first layer from a gradient that does not lie in memory as it is named, batched or lazily negated; on both
-sides of 2 048 rows, from which on the library's kernel was once taken without a look at it."""
+"""Weight gradients of a first layer where something stands between the operators and the memory: batched gradients, a lazily
+negated one, a recorded backward (``create_graph``), a dispatch mode; on both sides of 2 048 rows, from which on the library's
+kernel was once taken whatever was watching."""
 import numpy as np
 import pytest
 import torch
+from torch.utils._python_dispatch import TorchDispatchMode
 
 from hiscache.history_model import MyRGCNConvHistory2, MySageConvHistory
 
@@ -56,6 +58,35 @@ def test_a_negated_gradient(kind, rows):
     v = torch.randn(rows, H, device=DEV, generator=torch.Generator(device=DEV).manual_seed(1))
     want = torch.autograd.grad(out, params, -v, retain_graph=True)
     close(torch.autograd.grad(out, params, torch._neg_view(v)), want, rows)
+
+
+@pytest.mark.parametrize("rows", ROWS)
+def test_a_recorded_backward(rows):
+    conv, params, run = layer("sage", rows)
+    second = {}
+    for conv.fused in (True, False):                         # one node, and operator by operator
+        first = torch.autograd.grad(run().square().sum(), params, create_graph=True)
+        assert all(t.requires_grad for t in first)
+        second[conv.fused] = torch.autograd.grad(sum(t.square().mean() for t in first), params)
+    close(second[True], second[False], rows)
+
+
+@pytest.mark.parametrize("rows", ROWS)
+@pytest.mark.parametrize("kind", ("sage", "rgcn"))
+def test_a_dispatch_mode_sees_the_products(kind, rows):
+    class Seen(TorchDispatchMode):
+        names = []
+
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            self.names.append(str(func))
+            return func(*args, **(kwargs or {}))
+
+    _, params, run = layer(kind, rows)
+    out = run()
+    Seen.names = []
+    with Seen():
+        torch.autograd.grad(out, params, torch.ones_like(out))
+    assert any("mm" in n for n in Seen.names)
 
 
 def test_what_lies_in_memory():
