@@ -282,6 +282,7 @@ int lin_launch(LinArgs a, bool kn, bool vec, hipStream_t st) {
 // 47 14.4 / 9.3; 6 000, 128, 128 9.9 / 10.4; 36 000, 256, 256 84 / 140.
 constexpr int64_t LIN_SMALL = (int64_t)1 << 19;
 constexpr int64_t LIN_MAX = (int64_t)1 << 20;      // N and K; a tile's rows and W are addressed by 32-bit offsets
+constexpr int LIN_PIECE = 128;                     // longest piece of K
 
 }  // namespace
 
@@ -291,14 +292,15 @@ static int lin_run(const LinArgs &a, bool kn, hipStream_t st) {
   for (const void *p : {(const void *)a.a0, (const void *)a.a1, (const void *)a.w0, (const void *)a.w1, (const void *)a.bias,
                         (const void *)a.add, (const void *)a.out})
     vec = vec && reinterpret_cast<uintptr_t>(p) % 16 == 0;
-  if (a.M <= LIN_SMALL / a.N) return lin_launch<32, 32, 128>(a, kn, vec, st);
+  if (a.M <= LIN_SMALL / a.N) return lin_launch<32, 32, LIN_PIECE>(a, kn, vec, st);
   return lin_launch<64, 64, 32>(a, kn, vec, st);
 }
 
-// N and K as the kernel takes them
+// N and K as the kernel takes them.  W [K, N] is read up to one piece (LIN_PIECE rows at most) behind its last row: their
+// offsets must not come round to W's first rows, and the offset that stands for no element must lie behind its last.
 static int lin_widths(int64_t N, int64_t K) {
   HC_REQUIRE(N >= 1 && K >= 1);
-  return N > LIN_MAX || K > LIN_MAX || N * K >= (int64_t)1 << 30 ? HC_EUNSUPPORTED : HC_OK;
+  return N > LIN_MAX || K > LIN_MAX || (K + LIN_PIECE) * N >= (int64_t)1 << 30 ? HC_EUNSUPPORTED : HC_OK;
 }
 
 extern "C" int hc_linear(const float *a0, const float *w0, const float *a1, const float *w1, int w_is_kn,

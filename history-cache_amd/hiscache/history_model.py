@@ -128,7 +128,7 @@ class _SageConvFunction(torch.autograd.Function):
             return (None,) * 13
         g_out = g_out.contiguous()
         need = ctx.needs_input_grad
-        own = be.linear_supported(g_out, w_l, w_r if has_root else None)
+        own = be.linear_supported(g_out, w_l, w_r if has_root else None, transposed=True)
         # gradient reaching the aggregation output; a feature layer that keeps none has no use for it
         his = sink.target() if sink is not None and sink.target is not None else None
         g_agg = None

@@ -1452,12 +1452,19 @@ def plain_operands(a, *others, autocast=False):
             and torch._C._len_torch_dispatch_stack() == 0 and in_memory(a, *others))
 
 
-def linear_supported(a, *others):
+def linear_limits(M, N, K):
+    """The sizes that ``hc_linear`` takes: N and K, the offsets of W's rows up to one piece behind its last, and the
+    number of tiles."""
+    return max(N, K) <= 1 << 20 and (K + 128) * N < 1 << 30 and -(-M // 64) * -(-N // 64) <= (1 << 24) - 1
+
+
+def linear_supported(a, w, *others, transposed=False):
     """Does :func:`linear` cover a product of these tensors as the torch operators would compute it?  An inner size off a
     multiple of four is read element by element, and the library is the faster one above 256 (2 000 rows of 602 to 64: 23
     against 25 us)."""
     k = a.shape[1]
-    return (k % 4 == 0 or k <= 256) and plain_operands(a, *others)
+    return ((k % 4 == 0 or k <= 256) and linear_limits(a.shape[0], w.shape[1 if transposed else 0], k)
+            and plain_operands(a, w, *others))
 
 
 def linear(a0, w0, a1=None, w1=None, bias=None, transposed=False, out=None, norm=None):

@@ -397,3 +397,19 @@ def test_batch_view_fields_of_saved_and_foreign_views():
     old.__setstate__((None, {k: getattr(view, k) for k in ("ptrT", "rowT", "edgeT", "rows", "n_src", "num_edge")}))
     assert old.max_in_degree is None and old.max_out_degree is None and old.covers(3, 2)
     assert view.row_bound(3, 2) == 1 and view.row_bound(4, 2) is None and view.row_bound(3, 3) is None
+
+
+def test_sizes_beyond_the_dense_kernel_go_to_the_operators():
+    """hc_linear refuses what its 32-bit offsets cannot address, before anything is launched, and the layers do not offer it."""
+    import hiscache_backend as be
+    lib = be.load_library()
+    buf = np.zeros(64, np.float32)
+    p, null = ctypes.c_void_p(buf.ctypes.data), ctypes.c_void_p(None)
+    for M, N, K in ((1, (1 << 20) + 1, 1), (1, 1, (1 << 20) + 1), (1, 1 << 15, 1 << 15), (1, 1 << 20, 1000), (1, 1 << 20, 896),
+                    (1, (1 << 20) - 1, 1000), (1 << 33, 1, 4)):
+        assert not be.linear_limits(M, N, K)
+        for kn in (0, 1):
+            assert lib.hc_linear(p, p, null, null, kn, null, null, p, M, N, K, null) == 5
+        assert lib.hc_linear_bn_relu(p, p, null, null, null, null, null, p, p, 1e-5, p, M, N, K, null) == 5
+    for M, N, K in ((1, 1 << 20, 895), (1, 1, 1 << 20), (1_000_000, 256, 768), ((1 << 30) - 64, 1, 4)):
+        assert be.linear_limits(M, N, K)
