@@ -37,6 +37,11 @@ constexpr int WG_TILE_F = 64;       // columns of dW per block
 constexpr int WG_PIECE = 32;        // rows of g and x per piece
 constexpr int WG_TARGET_BLOCKS = 1024;
 constexpr int WG_MIN_SLAB_ROWS = 64;
+// Rows summed in one chain; a slab's chains are added one after the other, so that the error does not grow with the slab
+// (a wide dW has few slabs: 30 000 rows, 3 840 x 256 are five of 6 000).  Error against 64 bits, one chain per slab / chains of
+// 1 024, 512, 256 rows: 30 000 rows, 1 280 x 256 8.6e-7 / 5.5, 4.0, 3.0e-7; 200 000, 256 x 256, two operands 14.1e-7 / 5.7, 4.1,
+// 3.1e-7 (batched library products over 1 024 rows each: 5.8e-7); the time is the same (200 000, 256 x 256 515 / 526 us).
+constexpr int WG_CHAIN_ROWS = 256;
 
 struct WgShape {
   int tiles_h, tiles_f;
@@ -129,11 +134,21 @@ __global__ __launch_bounds__(HC_BLOCK) void wg_partial(const float *__restrict__
       *reinterpret_cast<wg_quad *>(&sx[s][f / QX * LDX + f % QX * 4]) = rx[i];
     }
   };
-  wg_acc acc[TM][TN];
+  wg_acc acc[TM][TN], sum[TM][TN];
 #pragma unroll
   for (int i = 0; i < TM; ++i)
 #pragma unroll
-    for (int j = 0; j < TN; ++j) acc[i][j] = wg_acc{0.f, 0.f, 0.f, 0.f};
+    for (int j = 0; j < TN; ++j) acc[i][j] = sum[i][j] = wg_acc{0.f, 0.f, 0.f, 0.f};
+  static_assert(WG_CHAIN_ROWS % BK == 0, "whole pieces per chain");
+  const auto end_chain = [&]() {
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j) {
+        sum[i][j] += acc[i][j];
+        acc[i][j] = wg_acc{0.f, 0.f, 0.f, 0.f};
+      }
+  };
   const auto step = [&](int s, int k) {
     float u[TM], v[TN];
 #pragma unroll
@@ -164,6 +179,7 @@ __global__ __launch_bounds__(HC_BLOCK) void wg_partial(const float *__restrict__
     __builtin_amdgcn_sched_barrier(0);
     s ^= 1;
     stage(s);
+    if (((uint32_t)(r - lo) + BK) % WG_CHAIN_ROWS == 0) end_chain();
   }
   __syncthreads();
   for (int k = 0; k < (int)(hi - r); k += 4) step(s, k);           // the last piece: 1 to WG_PIECE rows
@@ -171,13 +187,14 @@ __global__ __launch_bounds__(HC_BLOCK) void wg_partial(const float *__restrict__
     add_columns(s);
     part_sum[(slab * HC_WAVES_PER_BLOCK + wave) * (sh.tiles_h * BM) + h0 + lane] = col_sum;
   }
+  end_chain();
   // partial tile of this block, tiles ordered (operand, tile, slab)
   float *o = part + ((int64_t)in_slab * sh.slabs + slab) * (BM * BN);
 #pragma unroll
   for (int i = 0; i < TM; ++i)
 #pragma unroll
     for (int j = 0; j < TN; ++j)
-      *reinterpret_cast<wg_acc *>(o + (wm + i * 16 + l16) * BN + wn + j * 16 + 4 * k4) = acc[i][j];
+      *reinterpret_cast<wg_acc *>(o + (wm + i * 16 + l16) * BN + wn + j * 16 + 4 * k4) = sum[i][j];
 }
 
 // dW[op][h][f]: a quarter of the slabs per wave, in slab order, then the quarters in order.  Four columns per lane;
@@ -214,8 +231,14 @@ __global__ __launch_bounds__(HC_BLOCK) void wg_reduce(const float *__restrict__ 
     float4 v[FLIGHT];
 #pragma unroll
     for (int j = 0; j < FLIGHT; ++j) v[j] = *reinterpret_cast<const float4 *>(p + (k + j) * TILE);
+    // pairs, pairs of pairs, then the sum so far: an eighth of the additions in one chain
 #pragma unroll
-    for (int j = 0; j < FLIGHT; ++j) plus(v[j]);
+    for (int w = FLIGHT / 2; w > 0; w /= 2)
+#pragma unroll
+      for (int j = 0; j < w; ++j) {
+        v[j].x += v[j + w].x; v[j].y += v[j + w].y; v[j].z += v[j + w].z; v[j].w += v[j + w].w;
+      }
+    plus(v[0]);
   }
   for (; k < end; ++k) plus(*reinterpret_cast<const float4 *>(p + k * TILE));
   if (wave > 0) s_part[wave - 1][lane] = s;

@@ -58,3 +58,37 @@ def test_linear_grad_refuses_what_does_not_fit():
                  lambda: be.linear_grad(g.half(), x, x, True), lambda: be.linear_grad(g, x[:, :32].contiguous(), x[:, :32].contiguous(), True)):
         with pytest.raises(ValueError):
             call()
+
+
+@pytest.mark.parametrize("H,F", ((1024, 1024), (2048, 512)))
+def test_long_slabs_are_summed_in_short_chains(H, F):
+    # 256 tiles of dW leave four slabs of 2 048 rows.  2^27 in the first row: what is added to it four rows at a time is less
+    # than half a unit (16) and lost, which must not be more than the first chain's 256 rows; chains' sums are added exactly
+    n = 8192
+    g, x = torch.ones(n, H, device=DEV), torch.ones(n, F, device=DEV)
+    g[0] = 2.0 ** 27
+    err = (be.weight_grad(g, x).double() - (2.0 ** 27 + n - 1)).abs()
+    assert float(err.max()) <= 256
+
+
+@pytest.mark.parametrize("n", (1, 65, 1000, 4097, 16_390))
+@pytest.mark.parametrize("H,F", ((64, 64), (47, 128), (172, 64)))
+def test_whole_numbers_are_summed_exactly(n, H, F):
+    """Odd numbers up to 4 095, which half-precision types do not hold, and few enough of them that every partial sum is exact:
+    a row left out, taken twice or rounded shows."""
+    gen = torch.Generator(device=DEV).manual_seed(n + H)
+
+    def odd(c):
+        return 2.0 * torch.randint(-2048, 2048, (n, c), device=DEV, generator=gen) + 1.0
+
+    def few(c):
+        share = min(1.0, 2.0 ** 23 / (4095 * n))
+        return torch.randint(0, 2, (n, c), device=DEV, generator=gen).mul(2).sub(1) * (
+            torch.rand(n, c, device=DEV, generator=gen) < share).float()
+
+    for g, x0, x1 in ((odd(H), few(F), few(F)), (few(H), odd(F), odd(F))):
+        d0, d1, db = be.linear_grad(g, x0, x1, True)
+        for got, x in ((d0, x0), (d1, x1), (db.view(H, 1), torch.ones(n, 1, device=DEV))):
+            assert torch.equal(got.double(), g.double().t() @ x.double())
+        if H % 64 == 0:
+            assert torch.equal(be.weight_grad(g, x0), d0)
