@@ -11,6 +11,10 @@
 // and 64 x 128, pieces of 16 and 64 columns, v_mfma_f32_32x32x2_f32 and two or three blocks per compute unit instead of
 // four: 2 to 30% slower where the rows are few, no faster where they are many.
 //
+// Loads of A, loads of W and the way out are 16 bytes wide wherever their own width and alignment allow it: the gradient of
+// 47 classes is read by single elements, W and the result are not.  One product with W as [K, N], inner size 47, everything
+// by single elements / only A: 60 000 rows, N = 256 50 / 26 us; 20 000, 768 53 / 26; 1 000, 256 4.2 / 3.4.
+//
 // A block of four waves stages K in pieces through two LDS buffers: the loads of a piece are issued in front of the
 // matrix instructions of the one before it (kept there by a scheduling barrier: left alone, the compiler moves them
 // behind, and every wave waits for them).  Rows and columns behind the matrices are read
@@ -39,6 +43,7 @@ struct LinArgs {
   float *out;
   int64_t M;
   int N, K, tiles_n;
+  bool whole;                                  // four adjacent columns of the result, `add` and the bias lie on 16 bytes
   const float *mean, *var, *gamma, *beta;      // batch normalisation and ReLU behind the bias (NORM)
   float eps;
 };
@@ -60,7 +65,7 @@ __device__ __forceinline__ lin_quad lin_load(hc_buffer b, uint32_t row, int at, 
   }
 }
 
-template <int BM, int BN, int BK, bool KN, bool VEC, bool TWO, bool NORM>
+template <int BM, int BN, int BK, bool KN, bool VEC_A, bool VEC_W, bool TWO, bool NORM>
 __global__ __launch_bounds__(HC_BLOCK) void lin_tile(LinArgs a) {
   constexpr int WM = BM / 2, WN = BN / 2, TM = WM / 16, TN = WN / 16;
   constexpr int LDA = BK + 2, LDW = KN ? BN + 16 : BK + 2;
@@ -86,13 +91,13 @@ __global__ __launch_bounds__(HC_BLOCK) void lin_tile(LinArgs a) {
 #pragma unroll
     for (int i = 0; i < NA; ++i) {
       const int f = t + i * HC_BLOCK;
-      ra[i] = lin_load<VEC>(ba, (uint32_t)(f / QA) * (uint32_t)a.K * 4u, k0 + f % QA * 4, a.K);
+      ra[i] = lin_load<VEC_A>(ba, (uint32_t)(f / QA) * (uint32_t)a.K * 4u, k0 + f % QA * 4, a.K);
     }
 #pragma unroll
     for (int i = 0; i < NW; ++i) {
       const int f = t + i * HC_BLOCK;
-      if constexpr (KN) rw[i] = lin_load<VEC>(bw, (uint32_t)(k0 + f / QW) * (uint32_t)a.N * 4u, n0 + f % QW * 4, a.N);
-      else rw[i] = lin_load<VEC>(bw, (uint32_t)(f / QW) * (uint32_t)a.K * 4u, k0 + f % QW * 4, a.K);
+      if constexpr (KN) rw[i] = lin_load<VEC_W>(bw, (uint32_t)(k0 + f / QW) * (uint32_t)a.N * 4u, n0 + f % QW * 4, a.N);
+      else rw[i] = lin_load<VEC_W>(bw, (uint32_t)(f / QW) * (uint32_t)a.K * 4u, k0 + f % QW * 4, a.K);
     }
   };
   const auto put = [&](float *at, const lin_quad &v) {
@@ -191,7 +196,6 @@ __global__ __launch_bounds__(HC_BLOCK) void lin_tile(LinArgs a) {
 #pragma unroll
       for (int j = 0; j < TN; ++j) acc[i][j] = sum[i][j];
   }
-  const bool whole = VEC && a.N % 4 == 0;
   const auto plus = [&](const float *__restrict__ add, int64_t row_step) {
     lin_acc v[TM][TN];
 #pragma unroll
@@ -202,7 +206,7 @@ __global__ __launch_bounds__(HC_BLOCK) void lin_tile(LinArgs a) {
       for (int j = 0; j < TN; ++j) {
         const int n = n0 + wn + j * 16 + 4 * g;
         const float *o = add + m * row_step;
-        if (whole) {
+        if (a.whole) {
           v[i][j] = *reinterpret_cast<const lin_acc *>(o + (n < a.N ? n : a.N - 4));
         } else {
 #pragma unroll
@@ -242,7 +246,7 @@ __global__ __launch_bounds__(HC_BLOCK) void lin_tile(LinArgs a) {
     for (int j = 0; j < TN; ++j) {
       const int n = n0 + wn + j * 16 + 4 * g;
       float *o = a.out + m * a.N + n;
-      if (whole) {
+      if (a.whole) {
         if (n < a.N) *reinterpret_cast<lin_acc *>(o) = acc[i][j];
       } else {
 #pragma unroll
@@ -254,25 +258,26 @@ __global__ __launch_bounds__(HC_BLOCK) void lin_tile(LinArgs a) {
 }
 
 template <int BM, int BN, int BK>
-int lin_launch(LinArgs a, bool kn, bool vec, hipStream_t st) {
+int lin_launch(LinArgs a, bool kn, bool vec_a, bool vec_w, hipStream_t st) {
   a.tiles_n = (a.N + BN - 1) / BN;
   const int64_t blocks = (a.M + BM - 1) / BM * a.tiles_n;
   if (!hc_grid_ok(blocks)) return HC_EUNSUPPORTED;
   const dim3 grid((unsigned)blocks), block(HC_BLOCK);
-#define HC_LIN(KN, VEC)                                                                        \
-  {                                                                                            \
-    if (a.a1 != nullptr) lin_tile<BM, BN, BK, KN, VEC, true, NORM><<<grid, block, 0, st>>>(a); \
-    else lin_tile<BM, BN, BK, KN, VEC, false, NORM><<<grid, block, 0, st>>>(a);                \
+#define HC_LIN(KN, VEC_A, VEC_W)                                                                               \
+  {                                                                                                            \
+    if (a.a1 != nullptr) lin_tile<BM, BN, BK, KN, VEC_A, VEC_W, true, NORM><<<grid, block, 0, st>>>(a);        \
+    else lin_tile<BM, BN, BK, KN, VEC_A, VEC_W, false, NORM><<<grid, block, 0, st>>>(a);                       \
   }
   constexpr bool NORM = false;
   if (a.mean != nullptr) {
     constexpr bool NORM = true;
-    if (vec) HC_LIN(false, true)
-    else HC_LIN(false, false)
-  } else if (kn && vec) HC_LIN(true, true)
-  else if (kn) HC_LIN(true, false)
-  else if (vec) HC_LIN(false, true)
-  else HC_LIN(false, false)
+    if (vec_a && vec_w) HC_LIN(false, true, true)
+    else HC_LIN(false, false, false)
+  } else if (kn && vec_a && vec_w) HC_LIN(true, true, true)
+  else if (kn && vec_w) HC_LIN(true, false, true)
+  else if (kn) HC_LIN(true, false, false)
+  else if (vec_a && vec_w) HC_LIN(false, true, true)
+  else HC_LIN(false, false, false)
 #undef HC_LIN
   return hc_launch_status();
 }
@@ -281,19 +286,26 @@ int lin_launch(LinArgs a, bool kn, bool vec, hipStream_t st) {
 // deep pieces (128 columns) take fewer round trips.  64 x 64 / 32 x 32: 1 000 rows, K = 256, N = 172 13.5 / 8.3 us; 4 000, 256,
 // 47 14.4 / 9.3; 6 000, 128, 128 9.9 / 10.4; 36 000, 256, 256 84 / 140.
 constexpr int64_t LIN_SMALL = (int64_t)1 << 19;
+// Up to this many columns tiles of 64 x 64 are half or more padding, and pieces of 64 columns leave room for another block per
+// compute unit.  Two products and the bias, 64 x 64 / 32 x 32 with pieces of 64: 60 000 rows, K = 768, N = 10 108 / 72 us (library
+// GEMMs 80); 200 000, 256, 32 118 / 89 (108); 30 000, 256, 32 22 / 15 (26); 1 000, 64, 10 with pieces of 128 4.4 / 3.5.
+constexpr int LIN_NARROW = 32;
 constexpr int64_t LIN_MAX = (int64_t)1 << 20;      // N and K; a tile's rows and W are addressed by 32-bit offsets
 constexpr int LIN_PIECE = 128;                     // longest piece of K
 
 }  // namespace
 
-static int lin_run(const LinArgs &a, bool kn, hipStream_t st) {
+static int lin_run(LinArgs a, bool kn, hipStream_t st) {
   HC_REQUIRE(a.a0 && a.w0 && a.out && (a.a1 == nullptr) == (a.w1 == nullptr) && a.M >= 1);
-  bool vec = a.K % 4 == 0 && (!kn || a.N % 4 == 0);
-  for (const void *p : {(const void *)a.a0, (const void *)a.a1, (const void *)a.w0, (const void *)a.w1, (const void *)a.bias,
-                        (const void *)a.add, (const void *)a.out})
-    vec = vec && reinterpret_cast<uintptr_t>(p) % 16 == 0;
-  if (a.M <= LIN_SMALL / a.N) return lin_launch<32, 32, LIN_PIECE>(a, kn, vec, st);
-  return lin_launch<64, 64, 32>(a, kn, vec, st);
+  const auto on16 = [](const float *p, const float *q, const float *r) {
+    return (reinterpret_cast<uintptr_t>(p) | reinterpret_cast<uintptr_t>(q) | reinterpret_cast<uintptr_t>(r)) % 16 == 0;
+  };
+  const bool vec_a = a.K % 4 == 0 && on16(a.a0, a.a1, nullptr);
+  const bool vec_w = (kn ? a.N : a.K) % 4 == 0 && on16(a.w0, a.w1, nullptr);
+  a.whole = a.N % 4 == 0 && on16(a.out, a.add, a.bias);
+  if (a.N <= LIN_NARROW) return lin_launch<32, 32, 64>(a, kn, vec_a, vec_w, st);
+  if (a.M <= LIN_SMALL / a.N) return lin_launch<32, 32, LIN_PIECE>(a, kn, vec_a, vec_w, st);
+  return lin_launch<64, 64, 32>(a, kn, vec_a, vec_w, st);
 }
 
 // N and K as the kernel takes them.  W [K, N] is read up to one piece (LIN_PIECE rows at most) behind its last row: their
@@ -307,7 +319,7 @@ extern "C" int hc_linear(const float *a0, const float *w0, const float *a1, cons
                          const float *bias, const float *add, float *out, int64_t M, int64_t N, int64_t K,
                          void *stream) {
   if (const int rc = lin_widths(N, K)) return rc;
-  const LinArgs a{a0, a1, w0, w1, bias, add, out, M, (int)N, (int)K, 0, nullptr, nullptr, nullptr, nullptr, 0.f};
+  const LinArgs a{a0, a1, w0, w1, bias, add, out, M, (int)N, (int)K, 0, false, nullptr, nullptr, nullptr, nullptr, 0.f};
   return lin_run(a, w_is_kn != 0, static_cast<hipStream_t>(stream));
 }
 
@@ -317,6 +329,6 @@ extern "C" int hc_linear_bn_relu(const float *a0, const float *w0, const float *
                                  void *stream) {
   if (const int rc = lin_widths(N, K)) return rc;
   HC_REQUIRE(running_mean && running_var);
-  const LinArgs a{a0, a1, w0, w1, bias, nullptr, out, M, (int)N, (int)K, 0, running_mean, running_var, gamma, beta, eps};
+  const LinArgs a{a0, a1, w0, w1, bias, nullptr, out, M, (int)N, (int)K, 0, false, running_mean, running_var, gamma, beta, eps};
   return lin_run(a, false, static_cast<hipStream_t>(stream));
 }

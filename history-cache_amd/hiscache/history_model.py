@@ -427,6 +427,13 @@ def edge_types_by_node_ranges(ptr, idx, sub_to_full, num_node, type_bounds, pair
 # sum.  Below this inner size one GEMM is the faster spelling.
 _REL_SPLIT_MIN_INNER = 2048
 _REL_WGRAD_SLABS = 8
+# The weight gradient by the library's own kernel (hc_weight_grad), where it was the faster one at every number of rows
+# measured, GEMM or slabs / own, device us: 1 280 x 256, 2 048 rows 36 / 26, 4 200 63 / 42, 30 000 413 / 240; 640 x 64, 2 048 17 / 10;
+# 2 560 x 128, 4 200 58 / 42; 3 840 x 64, 4 200 61 / 32.  Not with fewer rows (1 000, 1 280 x 256 12 / 20), two launches
+# where one has time enough, nor for wide gradients of an inner size that is split (3 840 x 256, 4 200 92 / 95, 30 000 481 / 672;
+# 1 000 rows 32 / 33, and with the larger error, 2.6e-7 against 2.1e-7).
+_REL_WGRAD_KERNEL_MIN_ROWS = 2048
+_REL_WGRAD_KERNEL_AREA = 1280 * 256
 
 
 def _rel_matmul(agg, weight):
@@ -441,8 +448,9 @@ def _rel_weight_grad(agg, g):
     """agg^T @ g in the weight's layout: agg [n, K, F], g [n, H] -> [K, F, H]."""
     n, K, Fin = agg.shape
     a2 = agg.reshape(n, K * Fin)
-    # (4 200 rows, 3 840 x 256: 88 us against 150 for the slabs' batched GEMM and their sum)
-    if hiscache_backend.weight_grad_supported(a2, g) and hiscache_backend.plain_operands(g, a2):
+    area = K * Fin * g.shape[1]
+    if (n >= max(_REL_WGRAD_KERNEL_MIN_ROWS, area // 160) and (K * Fin < _REL_SPLIT_MIN_INNER or area <= _REL_WGRAD_KERNEL_AREA)
+            and hiscache_backend.weight_grad_supported(a2, g) and hiscache_backend.plain_operands(g, a2)):
         return hiscache_backend.weight_grad(a2, g).view(K, Fin, -1)
     S = max(_REL_WGRAD_SLABS, n // _WGRAD_SLAB_ROWS)
     m = n // S * S

@@ -1458,12 +1458,20 @@ def linear_limits(M, N, K):
     return max(N, K) <= 1 << 20 and (K + 128) * N < 1 << 30 and -(-M // 64) * -(-N // 64) <= (1 << 24) - 1
 
 
+# Elements of a matrix whose rows are read one element at a time up to which hc_linear is the faster one, two products forward
+# and one backward, library / own, device us: 20 000 rows, inner size 129, 256 outputs 49 / 45 and 31 / 34, 47 outputs 36 / 21 and
+# 15 / 13; 30 000, 129, 256 68 / 62 and 33 / 50; 100 000, 99, 256 159 / 151 and 74 / 108; 100 000, 255, 10 62 / 93 and 44 / 59.
+_LINEAR_SINGLE_ELEMENTS = 3 << 20
+
+
 def linear_supported(a, w, *others, transposed=False):
-    """Does :func:`linear` cover a product of these tensors as the torch operators would compute it?  An inner size off a
-    multiple of four is read element by element, and the library is the faster one above 256 (2 000 rows of 602 to 64: 23
-    against 25 us)."""
-    k = a.shape[1]
-    return ((k % 4 == 0 or k <= 256) and linear_limits(a.shape[0], w.shape[1 if transposed else 0], k)
+    """Does :func:`linear` cover a product of these tensors as the torch operators would compute it, and is it the faster
+    one?  An inner size off a multiple of four is read element by element, and so is W as [K, N] where N is off one: the
+    library is the faster one with many rows, and above an inner size of 256 (2 000 rows of 602 to 64: 23 against 25 us)."""
+    M, k = a.shape
+    N = w.shape[1 if transposed else 0]
+    single = max(k if k % 4 else 0, N if transposed and N % 4 else 0)
+    return ((k % 4 == 0 or k <= 256) and M * single <= _LINEAR_SINGLE_ELEMENTS and linear_limits(M, N, k)
             and plain_operands(a, w, *others))
 
 

@@ -89,3 +89,41 @@ def test_a_layer_under_autocast_or_a_dispatch_mode_keeps_its_operators(watch):
         with Seen() as seen:
             conv(x, ptr, idx, none, none, 0, 2)
         assert any("mm" in n for n in seen.names)
+
+
+@pytest.mark.parametrize("M,N,K", ((300, 64, 47), (300, 47, 64), (9000, 64, 47), (9000, 68, 64), (700, 32, 65), (17_000, 32, 129),
+                                   (40_001, 4, 63), (65, 1, 64), (2100, 256, 10)))
+@pytest.mark.parametrize("transposed", (False, True))
+def test_every_operand_off_its_boundary_by_itself(M, N, K, transposed):
+    """Loads of either operand and stores are 16 bytes wide or not, each by its own width and address: the same bits."""
+    gen = torch.Generator(device=DEV).manual_seed(M + N + K)
+
+    def rnd(*shape):
+        return torch.randn(*shape, device=DEV, generator=gen)
+
+    def off(t):
+        return torch.empty(t.numel() + 1, device=DEV)[1:].view(t.shape).copy_(t)
+
+    ws = (K, N) if transposed else (N, K)
+    a, w, b, c, bias, base = rnd(M, K), rnd(*ws), rnd(M, K), rnd(*ws), rnd(N), rnd(M, N)
+    kw = dict(transposed=transposed)
+    want, added = be.linear(a, w, b, c, bias, **kw), be.linear(a, w, out=base.clone(), **kw)
+    op = (lambda t: t.double()) if transposed else (lambda t: t.double().t())
+    size = a.double().abs() @ op(w).abs() + b.double().abs() @ op(c).abs() + bias.double().abs()
+    exact = a.double() @ op(w) + b.double() @ op(c) + bias.double()
+    assert bool(((want.double() - exact).abs() <= 1.01 * (K + 2) * 2.0 ** -24 * size).all())
+    for i in range(5):
+        ops = [off(t) if i == k else t for k, t in enumerate((a, w, b, c, bias))]
+        assert torch.equal(be.linear(*ops, **kw), want)
+    assert torch.equal(be.linear(a, w, out=off(base), **kw), added)
+
+
+def test_tall_products_of_odd_widths_stay_with_the_library():
+    def takes(M, N, K, transposed):
+        with torch.no_grad():
+            return be.linear_supported(torch.empty(M, K, device=DEV), torch.empty((K, N) if transposed else (N, K), device=DEV),
+                                       transposed=transposed)
+
+    assert takes(1000, 172, 256, False) and takes(1000, 256, 47, True) and takes(20_000, 256, 129, False)
+    assert not takes(100_000, 256, 99, False) and not takes(100_000, 256, 47, True) and not takes(100_000, 99, 256, True)
+    assert takes(100_000, 99, 256, False) and takes(200_000, 256, 100, True) and not takes(1000, 64, 602 + 1, False)

@@ -38,6 +38,20 @@ def test_relational_weight_gradient(n, K, F, H):
     _close(got.view(K * F, H), agg.view(n, K * F), g, n)
 
 
+@pytest.mark.parametrize("n,KF,H,own", ((1000, 1280, 256, False), (2047, 640, 64, False), (2048, 640, 64, True), (2047, 1280, 256, False),
+                                        (2048, 1280, 256, True), (3000, 1920, 256, False), (4200, 1920, 256, True),
+                                        (4200, 3840, 64, True), (4200, 3840, 256, False), (30_000, 3840, 256, False)))
+def test_relational_weight_gradient_by_the_faster_of_the_two(n, KF, H, own, monkeypatch):
+    calls = []
+    real = be.weight_grad
+    monkeypatch.setattr(be, "weight_grad", lambda *a: (calls.append(1), real(*a))[1])
+    agg, g = torch.randn(n, 5, KF // 5, device=DEV), torch.randn(n, H, device=DEV)
+    with torch.no_grad():
+        got = hm._rel_weight_grad(agg, g)
+    assert bool(calls) == own
+    _close(got.view(KF, H), agg.view(n, KF), g, n)
+
+
 @pytest.mark.parametrize("n", (1, 5, 33, 64, 1000, 4097))
 @pytest.mark.parametrize("H,F", ((1, 64), (10, 128), (47, 64), (63, 64), (65, 128), (153, 256), (172, 256), (256, 64)))
 def test_linear_grad_for_any_number_of_outputs(n, H, F):
