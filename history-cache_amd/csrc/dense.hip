@@ -30,8 +30,12 @@
 // its way through memory less: an evaluation batch of 4 000 seeds, 256 channels, two such layers, 774 us as two launches
 // each, 681 as one.
 //
-// Summation order: every product is summed from zero in ascending k, the second product is added to the first, then
-// `add`, then the bias -- whatever the tile, so a row's result does not depend on how many rows there are.
+// Summation order: a product by itself is two chains, the even and the odd steps of four columns, each summed from zero in
+// ascending k, and added at the end; of two products each is one chain, and the second is added to the first; then `add`, then
+// the bias -- whatever the tile, so a row's result does not depend on how many rows there are.  Two chains because the library
+// has them where the rows are few: error against 64 bits of 1 000 rows, inner size 256, one chain 2.9e-7, two 2.1e-7 (library
+// 2.1); 172 2.4, 1.7 (1.7); 47 1.2, 0.9 (0.9).  With two products the library has one chain as well.  Held to the registers of
+// four waves per SIMD the 64 x 64 tile is a little faster with two than it was with one: 55 000 rows, 256 to 128 36.7 / 36.3 us.
 #include "hc_common.h"
 
 namespace {
@@ -66,7 +70,7 @@ __device__ __forceinline__ lin_quad lin_load(hc_buffer b, uint32_t row, int at, 
 }
 
 template <int BM, int BN, int BK, bool KN, bool VEC_A, bool VEC_W, bool TWO, bool NORM>
-__global__ __launch_bounds__(HC_BLOCK) void lin_tile(LinArgs a) {
+__global__ __launch_bounds__(HC_BLOCK, BM == 64 ? 4 : 1) void lin_tile(LinArgs a) {
   constexpr int WM = BM / 2, WN = BN / 2, TM = WM / 16, TN = WN / 16;
   constexpr int LDA = BK + 2, LDW = KN ? BN + 16 : BK + 2;
   constexpr int QA = BK / 4, QW = KN ? BN / 4 : BK / 4;                  // four-element pieces of a staged row
@@ -118,12 +122,15 @@ __global__ __launch_bounds__(HC_BLOCK) void lin_tile(LinArgs a) {
       else put(&sw[b][f / QW * LDW + f % QW * 4], rw[i]);
     }
   };
-  lin_acc acc[TM][TN], sum[TWO ? TM : 1][TWO ? TN : 1];
+  constexpr int CHAINS = TWO ? 1 : 2;
+  static_assert(BK % 8 == 0, "a piece starts with the first chain");
+  lin_acc chain[CHAINS][TM][TN], sum[TWO ? TM : 1][TWO ? TN : 1];
+  auto &acc = chain[0], &other = chain[CHAINS - 1];
 #pragma unroll
   for (int i = 0; i < TM; ++i)
 #pragma unroll
-    for (int j = 0; j < TN; ++j) acc[i][j] = lin_acc{0.f, 0.f, 0.f, 0.f};
-  const auto step = [&](int b, int k) {
+    for (int j = 0; j < TN; ++j) acc[i][j] = other[i][j] = lin_acc{0.f, 0.f, 0.f, 0.f};
+  const auto step = [&](lin_acc (&to)[TM][TN], int b, int k) {
     float x[TM], y[TN];
 #pragma unroll
     for (int i = 0; i < TM; ++i) x[i] = sa[b][(wm + i * 16 + l16) * LDA + k + g];
@@ -133,7 +140,7 @@ __global__ __launch_bounds__(HC_BLOCK) void lin_tile(LinArgs a) {
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
-      for (int j = 0; j < TN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(y[j], x[i], acc[i][j], 0, 0, 0);
+      for (int j = 0; j < TN; ++j) to[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(y[j], x[i], to[i][j], 0, 0, 0);
   };
   load(0);
   if constexpr (NORM) {
@@ -157,7 +164,10 @@ __global__ __launch_bounds__(HC_BLOCK) void lin_tile(LinArgs a) {
       load(k0 + BK);
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int k = 0; k < BK; k += 4) step(b, k);
+      for (int k = 0; k < BK; k += 8) {
+        step(acc, b, k);
+        step(other, b, k + 4);
+      }
       __builtin_amdgcn_sched_barrier(0);
       b ^= 1;
       stage(b);
@@ -173,13 +183,26 @@ __global__ __launch_bounds__(HC_BLOCK) void lin_tile(LinArgs a) {
     const int left = a.K - k0;
     if (left == BK) {
 #pragma unroll
-      for (int k = 0; k < BK; k += 4) step(b, k);
+      for (int k = 0; k < BK; k += 8) {
+        step(acc, b, k);
+        step(other, b, k + 4);
+      }
     } else {
-      for (int k = 0; k < left; k += 4) step(b, k);
+      int k = 0;
+      for (; k + 4 < left; k += 8) {
+        step(acc, b, k);
+        step(other, b, k + 4);
+      }
+      if (k < left) step(acc, b, k);
     }
     b ^= 1;
     if (TWO && p == 0) stage(b);
-    if constexpr (TWO) {
+    if constexpr (!TWO) {
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) acc[i][j] += other[i][j];
+    } else {
 #pragma unroll
       for (int i = 0; i < TM; ++i)
 #pragma unroll

@@ -686,9 +686,10 @@ int hc_bn_relu_eval(const float *x, const float *bias, const float *gamma, const
  * gradients (hiscache/history_model.py:94-98).  w_is_kn == 0: w [N, K], as
  * torch.nn.Linear keeps a weight, op = transpose; != 0: w [K, N] as it is.
  * a1 and w1, add [M, N] and bias [N] may be NULL; add may be out (the product is
- * added to what is there).  Every product is summed in fp32 from zero in
- * ascending k, then first + second + add + bias: a row's result does not depend
- * on M.  HC_EUNSUPPORTED: N or K above 2^20, (K + 128) * N of 2^30 or more,
+ * added to what is there).  A product by itself is summed in fp32 in two chains,
+ * the even and the odd groups of four k, each from zero in ascending k; of two
+ * products each is one such chain.  Then first + second + add + bias: a row's
+ * result does not depend on M.  HC_EUNSUPPORTED: N or K above 2^20, (K + 128) * N of 2^30 or more,
  * 2^24 tiles or more. */
 int hc_linear(const float *a0, const float *w0, const float *a1, const float *w1, int w_is_kn,
               const float *bias, const float *add, float *out, int64_t M, int64_t N, int64_t K,

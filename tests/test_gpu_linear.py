@@ -127,3 +127,15 @@ def test_tall_products_of_odd_widths_stay_with_the_library():
     assert takes(1000, 172, 256, False) and takes(1000, 256, 47, True) and takes(20_000, 256, 129, False)
     assert not takes(100_000, 256, 99, False) and not takes(100_000, 256, 47, True) and not takes(100_000, 99, 256, True)
     assert takes(100_000, 99, 256, False) and takes(200_000, 256, 100, True) and not takes(1000, 64, 602 + 1, False)
+
+
+@pytest.mark.parametrize("M", (40, 9000))
+@pytest.mark.parametrize("transposed", (False, True))
+def test_a_product_by_itself_is_two_chains(M, transposed):
+    # 2^27 in the first column: what is added to it four columns at a time is less than half a unit (16) and lost, but only
+    # in the chain that holds it, 128 of 256 columns; the other chain is exact
+    K, N = 256, 64
+    a = torch.ones(M, K, device=DEV)
+    a[:, 0] = 2.0 ** 27
+    got = be.linear(a, torch.ones((K, N) if transposed else (N, K), device=DEV), transposed=transposed)
+    assert float((got.double() - (2.0 ** 27 + K - 1)).abs().max()) <= 128
