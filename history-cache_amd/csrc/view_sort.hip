@@ -58,12 +58,27 @@ constexpr int VB_FEW_LOCAL_BITS = 10;
 // ids.  The whole view, rows / rows and slots: 3 M pairs over 1 M sources, popular ones among them, 127 / 284 -> 109 / 141 us;
 // 14 M over 3 M 633 / 1526 -> 399 / 722; 1 M over 200 000 75 / 110 -> 61 / 70; evenly spread ones as before (up to 1 us for the
 // blocks without work).  Parts of 4096 or 8192 pairs: 2 to 15% slower with up to 1 M pairs, 2 to 4% faster or slower above; 128
-// blocks instead of 512: up to 17% slower.  (Ranking several shares of a bucket side by side in a wave changed nothing:
+// blocks: up to 17% slower than with 512.  (Ranking several shares of a bucket side by side in a wave changed nothing:
 // it is the work, not the chain, that one compute unit is too small for.)
+// Parts grow until there is at most one per block, and there are no more blocks for them than compute units: a popular source is
+// one part whatever is done, a chain that is slower where another part reads its pairs on the same compute unit, and with many
+// such sources the others' parts are work done for nothing.  3 M pairs over 1 M sources, 10 sources with half of them, rows, one
+// block per bucket / 512 blocks and 32 parts each / now: 326 / 398 / 324 us; 100 with nine tenths 130 / 277 / 122; 14 M over 3 M,
+// 100 with nine tenths 500 / 1 500 / 440; popular neighbours, as above, 633 / 397 / 396.  Blocks of four waves leave room for a second
+// one: 14 M over 6 M, popular neighbours, rows and slots, 2 150 us with one block per bucket, 256 / 512 blocks 1 670 / 1 540.
 constexpr uint32_t VB_HEAVY_PAIRS = VB_STAGED, VB_PART_PAIRS = 2048;
 constexpr int VB_PARTS_BITS = 5;                         // at most 32 parts
-constexpr int VB_PART_BLOCKS = 512;                      // most blocks that work through the parts
-constexpr int VB_MAX_PARTS = 256 << VB_PARTS_BITS;       // fewer than 256 buckets hold more than a 256th of the pairs
+constexpr int VB_PART_GROWTH = 20;                       // VB_PART_PAIRS << 20: any bucket is one part
+constexpr int VB_PART_BLOCKS = 256, VB_PART_BLOCKS_FEW = 512;   // most blocks for the parts, and most parts (FEW: of four waves each)
+static_assert(VS_MAX_EDGES >> VB_PART_GROWTH <= VB_PART_PAIRS, "a bucket fits the longest part");
+
+// log2 of the parts of a bucket of n pairs with 2^lb local ids, parts of VB_PART_PAIRS << grown pairs.
+__device__ __forceinline__ int vb_part_bits(uint32_t n, int grown, int lb) {
+  const uint32_t x = (n - 1u) / VB_PART_PAIRS >> grown;
+  const int bits = x > 0u ? 32 - __builtin_clz(x) : 0;
+  const int most = lb < VB_PARTS_BITS ? lb : VB_PARTS_BITS;
+  return bits < most ? bits : most;
+}
 
 __host__ __device__ __forceinline__ uint32_t vb_heavy_above(uint32_t live) {
   return live / 256 > VB_HEAVY_PAIRS ? live / 256 : VB_HEAVY_PAIRS;
@@ -318,7 +333,8 @@ __global__ __launch_bounds__(VS_OFF_THREADS) void vs_bucket_offsets(const uint32
                                                                      uint32_t *__restrict__ parts, VsShape S) {
   __shared__ uint32_t s_wave[VS_OFF_THREADS / HC_WAVE];
   __shared__ uint32_t n_parts, n_heavy;
-  __shared__ uint2 heavy[256];                           // a heavy bucket with log2 of its parts, and its first part
+  __shared__ uint32_t with[VB_PART_GROWTH + 1];          // parts of all heavy buckets, of VB_PART_PAIRS << i pairs
+  __shared__ uint2 heavy[256];                           // a heavy bucket with its pairs, then with log2 of its parts and its first part
   constexpr int PER = (VS_MAX_BUCKETS + VS_OFF_THREADS - 1) / VS_OFF_THREADS;
   const int tid = (int)threadIdx.x;
   const int lane = hc_lane();
@@ -333,6 +349,7 @@ __global__ __launch_bounds__(VS_OFF_THREADS) void vs_bucket_offsets(const uint32
   const uint32_t incl = vs_wave_incl_scan(sum, lane);
   if (lane == HC_WAVE - 1) s_wave[wave] = incl;
   if (tid == 0) n_parts = n_heavy = 0u;
+  if (tid <= VB_PART_GROWTH) with[tid] = 0u;
   __syncthreads();
   uint32_t run = incl - sum, live = 0u;
   for (int w = 0; w < VS_OFF_THREADS / HC_WAVE; ++w) {
@@ -348,11 +365,21 @@ __global__ __launch_bounds__(VS_OFF_THREADS) void vs_bucket_offsets(const uint32
     run += c[q];
     if (b == S.nb - 1) bucket_off[S.nb] = run;
     if (c[q] > heavy_above) {                            // parts[1 + i]: bucket, part, log2 of the number of parts
-      int bits = 1;
-      while (bits < VB_PARTS_BITS && ((uint32_t)VB_PART_PAIRS << bits) < c[q]) ++bits;
-      if (bits > S.lb) bits = S.lb;
-      heavy[atomicAdd(&n_heavy, 1u)] = make_uint2((uint32_t)b | (uint32_t)bits << 24, atomicAdd(&n_parts, 1u << bits));
+      heavy[atomicAdd(&n_heavy, 1u)] = make_uint2((uint32_t)b, c[q]);
     }
+  }
+  __syncthreads();
+  for (uint32_t i = tid; i < n_heavy * (VB_PART_GROWTH + 1); i += VS_OFF_THREADS) {
+    const int g = (int)(i % (VB_PART_GROWTH + 1));
+    atomicAdd(&with[g], 1u << vb_part_bits(heavy[i / (VB_PART_GROWTH + 1)].y, g, S.lb));
+  }
+  __syncthreads();
+  int g = 0;
+  while (g < VB_PART_GROWTH && with[g] > (uint32_t)S.part_blocks) ++g;
+  if ((uint32_t)tid < n_heavy) {
+    const uint2 v = heavy[tid];
+    const int bits = vb_part_bits(v.y, g, S.lb);
+    heavy[tid] = make_uint2(v.x | (uint32_t)bits << 24, atomicAdd(&n_parts, 1u << bits));
   }
   __syncthreads();
   for (uint32_t i = tid; i < n_heavy << VB_PARTS_BITS; i += VS_OFF_THREADS) {
@@ -732,6 +759,8 @@ struct VsLayout {
   size_t key32, tile_count, group_count, bucket_total, bucket_off, parts, pairs, rows, bits, total;
 };
 
+int vs_bucket_waves(const VsShape &S) { return S.lb <= VB_MANY_LOCAL_BITS ? VB_WAVES_MANY : VB_WAVES_FEW; }
+
 bool vs_shape(int64_t R, int64_t E, int64_t n_src, VsShape *S) {
   if (E <= 0 || E > VS_MAX_EDGES || n_src < 0 || n_src > 0x7ffffffeLL) return false;
   const int64_t ids = n_src + 1;
@@ -751,7 +780,8 @@ bool vs_shape(int64_t R, int64_t E, int64_t n_src, VsShape *S) {
   S->nbp = (S->nb + 63) / 64 * 64;
   S->nbc = (S->nb + 1) / 2 * 2;
   // (one per VB_HEAVY_PAIRS slots: with few slots the blocks that find no part cost more than they could give)
-  S->part_blocks = (int)(E / VB_HEAVY_PAIRS < VB_PART_BLOCKS ? E / VB_HEAVY_PAIRS : VB_PART_BLOCKS);
+  const int most = vs_bucket_waves(*S) == VB_WAVES_FEW ? VB_PART_BLOCKS_FEW : VB_PART_BLOCKS;
+  S->part_blocks = (int)(E / VB_HEAVY_PAIRS < most ? E / VB_HEAVY_PAIRS : most);
   S->ntiles = (E + VS_TILE - 1) / VS_TILE;
   S->ngroups = (S->ntiles + VS_GROUP - 1) / VS_GROUP;
   return true;
@@ -761,7 +791,6 @@ bool vs_shape(int64_t R, int64_t E, int64_t n_src, VsShape *S) {
 size_t vs_scatter_lds(const VsShape &S) {
   return (size_t)S.nbc * sizeof(uint32_t) + (size_t)VS_WAVES * S.nbc * sizeof(uint16_t);
 }
-int vs_bucket_waves(const VsShape &S) { return S.lb <= VB_MANY_LOCAL_BITS ? VB_WAVES_MANY : VB_WAVES_FEW; }
 size_t vs_bucket_lds(const VsShape &S) {
   const size_t n_local = (size_t)1 << S.lb, waves = (size_t)vs_bucket_waves(S);
   const size_t small = waves * ((n_local + 1) / 2) * sizeof(uint32_t) + (size_t)VB_STAGED * sizeof(uint32_t);
@@ -782,7 +811,7 @@ VsLayout vs_layout(const VsShape &S) {
   L.group_count = take((size_t)S.ngroups * S.nbp * sizeof(uint32_t));
   L.bucket_total = take((size_t)S.nbp * sizeof(uint32_t));
   L.bucket_off = take((size_t)(S.nbp + 1) * sizeof(uint32_t));
-  L.parts = take((size_t)(VB_MAX_PARTS + 1) * sizeof(uint32_t));
+  L.parts = take((size_t)(VB_PART_BLOCKS_FEW + 1) * sizeof(uint32_t));
   L.pairs = take((size_t)S.E * sizeof(uint2));
   L.rows = take((size_t)S.E * sizeof(uint32_t));
   L.bits = take((size_t)((S.n_src + 63) / 64) * 8 + 8);
