@@ -77,7 +77,7 @@ constexpr size_t FWD_HEAD_BYTES = FWD_COUNT_BYTES + 256;
 // like the launch itself.
 constexpr int64_t FWD_STAGE_MIN_EDGES = (int64_t)1 << 18;
 constexpr int64_t FWD_STAGE_BYTES = (int64_t)96 << 20;
-constexpr size_t FWD_STAGE_LIST_BYTES = (SEG_MAX_REGIONS + FWD_STAGED_ROWS) * sizeof(int32_t);
+constexpr size_t FWD_STAGE_LIST_BYTES = (SEG_MAX_REGIONS + 3 * FWD_STAGED_ROWS + 64) * sizeof(int32_t);    // counts, list, order
 size_t fwd_stage_bytes(int mode, int64_t E, int64_t F, int64_t n_head) {
   if (mode != HC_SUBST_ROW || n_head <= 1 || F % FWD_STAGED_COLS != 0 || E < FWD_STAGE_MIN_EDGES || F > 0x3fffffffLL / n_head) return 0;
   const int64_t edge = (F + 1) * n_head * (int64_t)sizeof(float);
@@ -121,7 +121,8 @@ int fwd_prepare_lists(FwdArgs &a, bool src_mode, FwdScratch ws, int64_t n_src, i
     a.staged.count = static_cast<int32_t *>(ws.ptr);
     a.staged.item = a.staged.count + SEG_MAX_REGIONS;
     a.staged.cap = FWD_STAGED_ROWS;
-    a.stage = reinterpret_cast<float *>(a.staged.item + FWD_STAGED_ROWS);
+    a.staged_order = a.staged.item + FWD_STAGED_ROWS;
+    a.stage = reinterpret_cast<float *>(static_cast<char *>(ws.ptr) + FWD_STAGE_LIST_BYTES);
     a.stage_floats = (int64_t)((stage_bytes - FWD_STAGE_LIST_BYTES) / sizeof(float));
     ws.ptr = static_cast<char *>(ws.ptr) + stage_bytes;
     ws.bytes -= stage_bytes;

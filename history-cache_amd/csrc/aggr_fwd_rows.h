@@ -74,6 +74,7 @@ constexpr int W_NONE = 0, W_EDGE = 1, W_EDGE_HEAD = 2;
 // rows of 3 edges of 64 columns from 443 to 526 us.)
 struct FwdPlan {
   int64_t far_above, listed, staged_above;
+  int64_t staged, staged_fit;  // with staged rows, written by fwd_stage: rows in staged_order, and how many of them have copies
 };
 
 // Rows of several heads are never split: the longest of them is one chain of additions, and a wave that follows it
@@ -87,7 +88,11 @@ struct FwdPlan {
 constexpr int FWD_STAGED_COLS = 4;
 constexpr int FWD_STAGED_UNIT = 64;         // edges per read of a slice: a kilobyte
 constexpr int FWD_STAGED_ROWS = 512;        // at most
-constexpr int64_t FWD_STAGED_MIN = 2048;    // edges: below, the copy takes longer than it saves
+// Edges: below, the copy takes longer than it saves (262 000 edges x 128 columns, longest row of 2 190 edges: 48 us, with its
+// copy 56; 2 612 edges: 56 / 50).  Rows of fewer columns have more weights beside them and are summed more slowly, 38 edges a
+// microsecond with 8 heads of 8 columns (524 000 edges, rows of up to 8 400, those above 2 432 / 2 048 copied: 85 / 80 us).
+constexpr int64_t FWD_STAGED_MIN = 2432, FWD_STAGED_MIN_NARROW = 2048;
+constexpr int64_t FWD_STAGED_NARROW = 128;  // columns: fewer are narrow
 
 struct FwdArgs {
   const int64_t *ptr, *idx;
@@ -107,6 +112,7 @@ struct FwdArgs {
   int64_t slice_above;        // rows with more edges belong to the front blocks, when there are any (0: none)
   SegList near, far;          // whole-row and slice-wise tasks of the front blocks
   SegList staged;             // rows that are copied side by side first, ...
+  int32_t *staged_order;      // ... in their order: the rows, from FWD_STAGED_ROWS on the first unit of each copy, ...
   float *stage;               // ... and the room for that (several heads; nullable)
   int64_t stage_floats;
   int n_tiles;                // tiles of the lists; 0: every front block looks the rows through itself
@@ -128,7 +134,8 @@ __device__ __forceinline__ int64_t fwd_far_above(const FwdArgs &a, int64_t total
 __device__ __forceinline__ int64_t fwd_staged_above(const FwdArgs &a, int64_t total) {
   int64_t t = total / 20000 * a.F;
   if (t < total / FWD_STAGED_ROWS) t = total / FWD_STAGED_ROWS;
-  return t < FWD_STAGED_MIN ? FWD_STAGED_MIN : t;
+  const int64_t least = a.F < FWD_STAGED_NARROW ? FWD_STAGED_MIN_NARROW : FWD_STAGED_MIN;
+  return t < least ? least : t;
 }
 
 // The staged rows: row i's copy starts at unit unit[i] (of FWD_STAGED_UNIT edges), F + n_head floats per edge: the row's
@@ -161,34 +168,56 @@ __device__ __forceinline__ void fwd_block_scan(int32_t *sum, int lane, int wave,
 }
 
 // Reads the list of the rows to be staged (all threads of the block).  Returns how many of them have room; they are the
-// first of the list, `*n` rows.  Every block arrives at the same result.
+// first of the list, `*n` rows, the longest first if there is not room for all: what is left takes as long as its longest
+// row.  (1 M edges x 128 columns in two heads, power-law rows of up to 14 900 edges, not room for all of them: 280 us without
+// copies, 208 with the first of the list and the others behind them, now 154.)  Every block of fwd_stage arrives at the
+// same result; the first one writes it down for the front blocks.
 __device__ __forceinline__ int fwd_read_staged(const FwdArgs &a, FwdStaged &s, int lane, int wave, int *n) {
   static_assert(SEG_MAX_REGIONS == 2 * HC_BLOCK && FWD_STAGED_ROWS == 2 * HC_BLOCK, "two tiles and two rows per thread");
-  *n = 0;
-  if (a.plan->listed == 0) return 0;
-  const int64_t above = a.plan->staged_above;
   const int t = (int)threadIdx.x;
   const int c0 = 2 * t < a.n_tiles ? a.staged.count[2 * t] : 0, c1 = 2 * t + 1 < a.n_tiles ? a.staged.count[2 * t + 1] : 0;
+  const int64_t listed = a.plan->listed, above = a.plan->staged_above;
   int x0, x1, rows;
   fwd_block_scan(s.sum, lane, wave, c0, c1, x0, x1, rows);
-  if (rows == 0) return 0;
+  *n = 0;
+  if (listed == 0 || rows == 0) return 0;
   for (int k = 0; k < c0 + c1; ++k) {
     const int64_t part = seg_part(a.ptr, (int64_t)(k < c0 ? 2 * t : 2 * t + 1) * a.tile, above);
     s.row[x0 + k] = a.staged.item[part + (k < c0 ? k : k - c0)];
   }
   __syncthreads();
-  const auto units = [&](int i) -> int {
-    if (i >= rows) return 0;
-    const int64_t r = s.row[i];
-    return (int)((a.ptr[r + 1] - a.ptr[r] + FWD_STAGED_UNIT - 1) / FWD_STAGED_UNIT);
+  const int64_t room = a.stage_floats / (FWD_STAGED_UNIT * (a.F + a.n_head));
+  int u0, u1, all;
+  const auto place = [&]() {
+    const auto units = [&](int i) -> int {
+      if (i >= rows) return 0;
+      const int64_t r = s.row[i];
+      return (int)((a.ptr[r + 1] - a.ptr[r] + FWD_STAGED_UNIT - 1) / FWD_STAGED_UNIT);
+    };
+    u0 = units(2 * t);
+    u1 = units(2 * t + 1);
+    fwd_block_scan(s.sum, lane, wave, u0, u1, x0, x1, all);
   };
-  const int u0 = units(2 * t), u1 = units(2 * t + 1);
-  int all;
-  fwd_block_scan(s.sum, lane, wave, u0, u1, x0, x1, all);
+  place();
+  if (all > room) {
+    s.unit[2 * t] = u0;
+    s.unit[2 * t + 1] = u1;
+    const int r0 = 2 * t < rows ? s.row[2 * t] : 0, r1 = 2 * t + 1 < rows ? s.row[2 * t + 1] : 0;
+    __syncthreads();
+    int p0 = 0, p1 = 0;
+    for (int i = 0; i < rows; ++i) {
+      const int u = s.unit[i];
+      p0 += u > u0 || (u == u0 && i < 2 * t);
+      p1 += u > u1 || (u == u1 && i < 2 * t + 1);
+    }
+    if (2 * t < rows) s.row[p0] = r0;
+    if (2 * t + 1 < rows) s.row[p1] = r1;
+    __syncthreads();
+    place();
+  }
   s.unit[2 * t] = x0;
   s.unit[2 * t + 1] = x1;
   if (t == HC_BLOCK - 1) s.unit[FWD_STAGED_ROWS] = all;
-  const int64_t room = a.stage_floats / (FWD_STAGED_UNIT * (a.F + a.n_head));
   const int fit = __syncthreads_count(2 * t < rows && x0 + u0 <= room) + __syncthreads_count(2 * t + 1 < rows && x1 + u1 <= room);
   *n = rows;
   return fit;
@@ -201,6 +230,14 @@ __global__ __launch_bounds__(HC_BLOCK) void fwd_stage(FwdArgs a) {
   const int lane = hc_lane(), wave = hc_wave_in_block();
   int n;
   const int fit = fwd_read_staged(a, s, lane, wave, &n);
+  if (blockIdx.x == 0) {                               // for the launch that sums
+    for (int i = (int)threadIdx.x; i < n; i += HC_BLOCK) a.staged_order[i] = s.row[i];
+    for (int i = (int)threadIdx.x; i <= fit && n > 0; i += HC_BLOCK) a.staged_order[FWD_STAGED_ROWS + i] = s.unit[i];
+    if (threadIdx.x == 0) {
+      a.plan->staged = n;
+      a.plan->staged_fit = fit;
+    }
+  }
   if (fit == 0) return;
   const int units = s.unit[fit];
   for (int u = (int)blockIdx.x * HC_WAVES_PER_BLOCK + wave; u < units; u += (int)gridDim.x * HC_WAVES_PER_BLOCK) {
@@ -256,13 +293,14 @@ struct FwdSlice {
 
 // Columns 4 slice .. 4 slice + 3 of staged row i, summed in edge order by one wave: every lane reads 16 bytes of a unit
 // (four units ahead, into registers) and passes them through the LDS; lane l then adds up column l % 4.
-__device__ __forceinline__ void fwd_sum_staged(const FwdArgs &a, const FwdStaged &s, FwdSlice &b, int i, int slice, int lane) {
+__device__ __forceinline__ void fwd_sum_staged(const FwdArgs &a, FwdSlice &b, int i, int slice, int lane) {
   constexpr int AHEAD = 4;
   typedef float quad __attribute__((ext_vector_type(4)));
-  const int64_t row = s.row[i], deg = a.ptr[row + 1] - a.ptr[row];
-  const int units = s.unit[i + 1] - s.unit[i];
+  const int32_t *unit = a.staged_order + FWD_STAGED_ROWS + i;
+  const int64_t row = a.staged_order[i], deg = a.ptr[row + 1] - a.ptr[row];
+  const int units = unit[1] - unit[0];
   const int64_t len = (int64_t)units * FWD_STAGED_UNIT;
-  const float *from = a.stage + (int64_t)s.unit[i] * FWD_STAGED_UNIT * (a.F + a.n_head);
+  const float *from = a.stage + (int64_t)unit[0] * FWD_STAGED_UNIT * (a.F + a.n_head);
   const int h = (int)((int64_t)slice * FWD_STAGED_COLS / (a.F / a.n_head));
   const quad *x = reinterpret_cast<const quad *>(from + (int64_t)slice * len * FWD_STAGED_COLS) + lane;
   const float *w = from + len * a.F + h * len + lane;
@@ -714,7 +752,7 @@ constexpr int FWD_SELF_ITEMS = 512;
 template <typename T, typename TH, int VEC, int CHUNKS, int UNROLL, bool SRC, int WMODE>
 __device__ __forceinline__ void fwd_front(const FwdArgs &a, int64_t far_above, int lane, int wave,
                                           float (*part)[HC_WAVE * VEC * CHUNKS], int *self_rows, int *self_n,
-                                          FwdStaged *staged, FwdSlice *slice) {
+                                          FwdSlice *slice) {
   constexpr int SV = sizeof(T) == 2 && VEC > 1 ? 2 : 1;
   constexpr int SL = FWD_SLICE_LANES * SV;
   const int ns = (int)((a.F + SL - 1) / SL);
@@ -784,18 +822,20 @@ __device__ __forceinline__ void fwd_front(const FwdArgs &a, int64_t far_above, i
       for (int i = 0; i < SV; ++i)
         if (on) a.vout[row * a.F + c + i] = s[i];
     };
-    if (a.stage != nullptr && seg_index(a.staged.count, a.n_tiles, lane).total > 0) {
-      int rows;
-      const int fit = fwd_read_staged(a, *staged, lane, wave, &rows);
+    // wave 0 of every block has the copied rows; those without room begin with wave 1 then, the other listed ones with wave 2
+    int turn = wave;
+    if (a.stage != nullptr && a.plan->staged > 0) {
+      const int rows = (int)a.plan->staged, fit = (int)a.plan->staged_fit;
       const int pieces = (int)(a.F / FWD_STAGED_COLS);
       if (wave == 0)
         for (int64_t t = blockIdx.x; t < (int64_t)fit * pieces; t += a.front)
-          fwd_sum_staged(a, *staged, *slice, (int)(t / pieces), (int)(t % pieces), lane);
-      // rows that found no room are summed like the other long ones
-      for (int64_t t = (int64_t)wave * a.front + blockIdx.x; t < (int64_t)(rows - fit) * ns; t += (int64_t)HC_WAVES_PER_BLOCK * a.front)
-        slice_of((int64_t)staged->row[fit + (int)(t / ns)], (int)(t % ns));
+          fwd_sum_staged(a, *slice, (int)(t / pieces), (int)(t % pieces), lane);
+      const int next = (wave + 3) % HC_WAVES_PER_BLOCK;
+      for (int64_t t = (int64_t)next * a.front + blockIdx.x; t < (int64_t)(rows - fit) * ns; t += (int64_t)HC_WAVES_PER_BLOCK * a.front)
+        slice_of((int64_t)a.staged_order[fit + (int)(t / ns)], (int)(t % ns));
+      if (fit > 0) turn = (wave + 2) % HC_WAVES_PER_BLOCK;
     }
-    for (int64_t t = (int64_t)wave * a.front + blockIdx.x; t < tasks; t += (int64_t)HC_WAVES_PER_BLOCK * a.front)
+    for (int64_t t = (int64_t)turn * a.front + blockIdx.x; t < tasks; t += (int64_t)HC_WAVES_PER_BLOCK * a.front)
       slice_of(far_row((int)(t / ns)), (int)(t % ns));
     return;
   } else {
@@ -848,12 +888,9 @@ __device__ __forceinline__ void fwd_block(const FwdArgs &a) {
   __shared__ float part[HC_WAVES_PER_BLOCK - 1][HC_WAVE * VEC * CHUNKS];
   __shared__ int self_rows[FWD_SELF_ITEMS];
   __shared__ int long_rows[FWD_ROWS_PER_BLOCK];    // (front blocks: the waves' counts)
-  FwdStaged *staged = nullptr;
   FwdSlice *slice = nullptr;
   if constexpr (WMODE == W_EDGE_HEAD) {
-    __shared__ FwdStaged staged_s;
     __shared__ __attribute__((aligned(16))) FwdSlice slice_s;
-    staged = &staged_s;
     slice = &slice_s;
   }
   __shared__ int n_long_s;
@@ -874,8 +911,7 @@ __device__ __forceinline__ void fwd_block(const FwdArgs &a) {
     if constexpr (PART != FWD_BODY) {
       if ((int)blockIdx.x < a.front) {
         if (listed)
-          fwd_front<T, TH, VEC, CHUNKS, UNROLL, SRC, WMODE>(a, far_above, lane, wave, part, self_rows, long_rows, staged,
-                                                               slice);
+          fwd_front<T, TH, VEC, CHUNKS, UNROLL, SRC, WMODE>(a, far_above, lane, wave, part, self_rows, long_rows, slice);
         return;
       }
     }

@@ -9,8 +9,10 @@ from test_gpu_long_rows import DEV, T, block
 
 pytestmark = pytest.mark.gpu
 
-# (at 300 000 edges and 128 columns rows above 2 048 edges are copied; the first two lie at the block's ends)
+# (at 300 000 edges rows above 2 048 edges are copied, above 2 432 with 128 columns and more, 64 edges at a time; the first two
+# lie at the block's ends)
 LENGTHS = [2049, 40_000, 2048, 2047, 2080, 2081, 2303, 2304, 2305, 100_001, 119_999, 5000, 3000, 129]
+EDGE_LENGTHS = [2433, 40_000, 2432, 2431, 2495, 2496, 2497, 2559, 2560, 2561, 100_001, 119_999, 5000, 3000, 129]
 
 
 @pytest.fixture(scope="module")
@@ -42,17 +44,19 @@ def check(be, orc, F, H, lengths, dtype=torch.float32, history=False, shift=0, R
 
 @pytest.mark.parametrize("F,H,dtype,shift", [(32, 4, torch.float32, 0), (8, 2, torch.float32, 0), (40, 3, torch.float32, 1),
                                              (32, 4, torch.float16, 0), (24, 2, torch.bfloat16, 3), (12, 4, torch.float32, 0)])
-def test_staged_rows(be, orc, F, H, dtype, shift):
-    check(be, orc, F, H, LENGTHS, dtype, shift=shift)
+@pytest.mark.parametrize("lengths", (LENGTHS, EDGE_LENGTHS))
+def test_staged_rows(be, orc, F, H, dtype, shift, lengths):
+    check(be, orc, F, H, lengths, dtype, shift=shift)
 
 
 def test_staged_rows_beside_history_rows(be, orc):
     check(be, orc, 32, 4, LENGTHS, history=True)
 
 
-@pytest.mark.parametrize("lengths", ([9000, 40_000, 120_000, 100_001, 30_000, 9001], [120_000, 9000, 40_000, 100_001]))
+@pytest.mark.parametrize("lengths", ([9000, 40_000, 120_000, 100_001, 30_000, 9001], [120_000, 9000, 40_000, 100_001],
+                                     [8100 + 137 * (i * 7 % 29) for i in range(30)]))      # (the four longest of 30; two are equal)
 def test_copies_without_room(be, orc, lengths):
-    """512 columns: 96 MB hold 48 000 edges, so that some of these rows, or all, are summed from the matrix."""
+    """512 columns: 96 MB hold 48 000 edges, so that some of these rows, or all but the longest, are summed from the matrix."""
     check(be, orc, 64, 8, lengths)
 
 
