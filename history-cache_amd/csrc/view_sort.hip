@@ -369,13 +369,13 @@ __global__ __launch_bounds__(VS_OFF_THREADS) void vs_bucket_offsets(const uint32
     }
   }
   __syncthreads();
-  for (uint32_t i = tid; i < n_heavy * (VB_PART_GROWTH + 1); i += VS_OFF_THREADS) {
-    const int g = (int)(i % (VB_PART_GROWTH + 1));
-    atomicAdd(&with[g], 1u << vb_part_bits(heavy[i / (VB_PART_GROWTH + 1)].y, g, S.lb));
-  }
-  __syncthreads();
   int g = 0;
-  while (g < VB_PART_GROWTH && with[g] > (uint32_t)S.part_blocks) ++g;
+  if (n_heavy << VB_PARTS_BITS > (uint32_t)S.part_blocks) {
+    for (uint32_t i = tid; i < n_heavy * (VB_PART_GROWTH + 1); i += VS_OFF_THREADS)
+      atomicAdd(&with[i % (VB_PART_GROWTH + 1)], 1u << vb_part_bits(heavy[i / (VB_PART_GROWTH + 1)].y, i % (VB_PART_GROWTH + 1), S.lb));
+    __syncthreads();
+    while (g < VB_PART_GROWTH && with[g] > (uint32_t)S.part_blocks) ++g;
+  }
   if ((uint32_t)tid < n_heavy) {
     const uint2 v = heavy[tid];
     const int bits = vb_part_bits(v.y, g, S.lb);
