@@ -1437,7 +1437,10 @@ def in_memory(*tensors):
     were never written have none either, and a lazily negated first operand (in a backward pass the gradient, the one
     that comes from outside) lies there with the other sign."""
     try:
-        return not tensors[0].is_neg() and all(t is None or t.data_ptr() != 0 for t in tensors)
+        for t in tensors:
+            if t is not None and t.data_ptr() == 0:
+                return False
+        return not tensors[0].is_neg()
     except RuntimeError:
         return False
 
@@ -1445,11 +1448,15 @@ def in_memory(*tensors):
 def plain_operands(a, *others, autocast=False):
     """May a library call stand for torch operators on these tensors: plain, packed fp32 tensors in the memory of the
     current GPU, no autocast (unless ``autocast``), nothing that records or replaces operators?"""
-    return (a.is_cuda and a.device.index == torch.cuda.current_device()
-            and all(t is None or (type(t) in _PLAIN and t.dtype == torch.float32 and t.device == a.device
-                                  and t.is_contiguous() and t.numel() > 0) for t in (a, *others))
-            and not torch.is_grad_enabled() and (autocast or not torch.is_autocast_enabled("cuda"))
-            and torch._C._len_torch_dispatch_stack() == 0 and in_memory(a, *others))
+    device = a.device
+    if (device.type != "cuda" or device.index != torch.cuda.current_device() or torch.is_grad_enabled()
+            or torch._C._len_torch_dispatch_stack() != 0 or (not autocast and torch.is_autocast_enabled("cuda"))):
+        return False
+    for t in (a, *others):
+        if t is not None and (type(t) not in _PLAIN or t.dtype is not torch.float32 or t.device != device
+                              or not t.is_contiguous() or t.numel() == 0):
+            return False
+    return in_memory(a, *others)
 
 
 def linear_limits(M, N, K):
@@ -1464,15 +1471,25 @@ def linear_limits(M, N, K):
 _LINEAR_SINGLE_ELEMENTS = 3 << 20
 
 
+# Longest inner size with up to 64 columns (tiles of 64 x 64, a few of them per compute unit) up to which hc_linear is the faster
+# one with more results than the small tiles take (hc_linear's LIN_SMALL), two products and the bias, library / own: 19 877 rows, 768
+# to 47 44 / 59 us, 768 to 36 45 / 58, 640 to 48 44 / 49, 1 024 to 64 70 / 77, 512 to 47 43 / 43; 114 689, 768 to 47 190 / 217.
+_LINEAR_NARROW_INNER = 512
+
+
 def linear_supported(a, w, *others, transposed=False):
     """Does :func:`linear` cover a product of these tensors as the torch operators would compute it, and is it the faster
     one?  An inner size off a multiple of four is read element by element, and so is W as [K, N] where N is off one: the
-    library is the faster one with many rows, and above an inner size of 256 (2 000 rows of 602 to 64: 23 against 25 us)."""
+    library is the faster one with many rows, above an inner size of 256 (2 000 rows of 602 to 64: 23 against 25 us), and where
+    both are long (the gradient of 602 columns from 2 111 rows of 512: 25 against 34, of 256: 20 against 21, of 172: 20
+    against 17; from 1 003 rows of 512: 19 against 23, of 384: 19 each, of 256: 19 against 14)."""
     M, k = a.shape
     N = w.shape[1 if transposed else 0]
     single = max(k if k % 4 else 0, N if transposed and N % 4 else 0)
-    return ((k % 4 == 0 or k <= 256) and M * single <= _LINEAR_SINGLE_ELEMENTS and linear_limits(M, N, k)
-            and plain_operands(a, w, *others))
+    long = k > 256 if k % 4 else transposed and N % 4 != 0 and N > 256 and k >= 256 and M * k > 400_000
+    narrow = k > _LINEAR_NARROW_INNER and 32 < N <= 64 and M * N > 1 << 19
+    return (not long and M * single <= _LINEAR_SINGLE_ELEMENTS and not narrow
+            and (max(M, N * k) <= 1 << 20 or linear_limits(M, N, k)) and plain_operands(a, w, *others))
 
 
 def linear(a0, w0, a1=None, w1=None, bias=None, transposed=False, out=None, norm=None):

@@ -127,6 +127,11 @@ def test_tall_products_of_odd_widths_stay_with_the_library():
     assert takes(1000, 172, 256, False) and takes(1000, 256, 47, True) and takes(20_000, 256, 129, False)
     assert not takes(100_000, 256, 99, False) and not takes(100_000, 256, 47, True) and not takes(100_000, 99, 256, True)
     assert takes(100_000, 99, 256, False) and takes(200_000, 256, 100, True) and not takes(1000, 64, 602 + 1, False)
+    # W [K, N] of an odd N and a long inner size, and few columns of a long inner size
+    assert takes(300, 255, 512, True) and takes(2000, 602, 252, True) and not takes(2000, 602, 256, True)
+    assert takes(1000, 602, 256, True) and not takes(1000, 602, 512, True) and takes(2000, 602, 256, False)
+    assert takes(5000, 47, 768, False) and not takes(20_000, 47, 768, False) and not takes(20_000, 64, 516, False)
+    assert takes(20_000, 32, 768, False) and takes(20_000, 65, 768, False) and takes(20_000, 47, 512, False)
 
 
 @pytest.mark.parametrize("M", (40, 9000))
@@ -139,3 +144,17 @@ def test_a_product_by_itself_is_two_chains(M, transposed):
     a[:, 0] = 2.0 ** 27
     got = be.linear(a, torch.ones((K, N) if transposed else (N, K), device=DEV), transposed=transposed)
     assert float((got.double() - (2.0 ** 27 + K - 1)).abs().max()) <= 128
+
+
+@pytest.mark.parametrize("N", (4, 64))
+@pytest.mark.parametrize("transposed", (False, True))
+def test_rows_behind_2_to_the_31_elements(N, transposed):
+    """Both operands' rows and, with 64 columns, the result's: the bits of the same rows by themselves."""
+    K, M = 64, (1 << 25) + 70
+    a = torch.randn(M, K, device=DEV)
+    w, c = (torch.randn(*((K, N) if transposed else (N, K)), device=DEV) for _ in range(2))
+    one, two = be.linear(a, w, transposed=transposed), be.linear(a, w, a, c, transposed=transposed)
+    for rows in (slice(0, 200), slice((1 << 25) - 130, M)):
+        part = a[rows].contiguous()
+        assert torch.equal(one[rows], be.linear(part, w, transposed=transposed))
+        assert torch.equal(two[rows], be.linear(part, w, part, c, transposed=transposed))
