@@ -42,8 +42,8 @@ __device__ __forceinline__ void tier_copy_row(const TS *__restrict__ s, TD *__re
 }
 
 // A wave serves HOT_ROWS consecutive requested rows: one lane per row reads the row's mask byte, id and slot (three
-// dependent reads for all rows at once instead of once per row), then the wave copies the rows HOT_INFLIGHT at a
-// time, every row's load issued before the first store.  With a wave per row the launch is a chain of four round
+// dependent reads for all rows at once instead of once per row), then the wave copies hot_loads(RPL) loads' rows at
+// a time, every load issued before the first store.  With a wave per row the launch is a chain of four round
 // trips per 512-byte row and runs at a fraction of the memory rate.  Rows of at most 32 (16) steps of TV elements are
 // copied two (four) at a time by one load, so that no lane is idle and all 16 rows are on their way at once.
 // 300 000 rows out of 2 M, all / half of them asked for, one row per load and then: 512 bytes 66 / 54 us, 63 / 42 (4.9 / 5.5

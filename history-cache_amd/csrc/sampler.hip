@@ -31,6 +31,10 @@ constexpr int32_t SP_PROV = 0x40000000;  // map values at or above this are edge
 // Lanes that share one row in the pick kernel: the fanout where two rows or more fit the wave so, else 16.  The kernel is
 // bound by the arithmetic of the permutation (64-bit multiplications, walked until every lane of the wave is done), so
 // what counts is how many lanes have a pick: three hops of 15, 10 and 5 from 1 000 seeds 55 us with groups of 16, now 42.
+// Between 17 and 32 (three or two rows per wave instead of four that take two rounds each), groups of 16 / of the fanout, us:
+// hops of 20 and 20 from 1 000 seeds, power-law degrees of 7 on average 55 / 49, of 15 64 / 55, every degree 100 84 / 76; from
+// 20 000 seeds, power-law 7 101 / 93, every degree 7 (no row needs the permutation) 104 / 107; one hop of 25 or 32 from 20 000, power-law
+// 15 46 / 42 and 45 / 43, every degree 7 35 / 35, 100 59 / 59 and 65 / 67.
 constexpr int SP_GROUP = 16;
 __host__ __device__ __forceinline__ int sp_group(int64_t fanout) { return fanout <= HC_WAVE / 2 ? (int)fanout : SP_GROUP; }
 constexpr int SP_BLOCK = HC_BLOCK;       // threads of the kernels that own a tile
