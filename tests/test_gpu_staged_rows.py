@@ -54,7 +54,8 @@ def test_staged_rows_beside_history_rows(be, orc):
 
 
 @pytest.mark.parametrize("lengths", ([9000, 40_000, 120_000, 100_001, 30_000, 9001], [120_000, 9000, 40_000, 100_001],
-                                     [8100 + 137 * (i * 7 % 29) for i in range(30)]))      # (the four longest of 30; two are equal)
+                                     [8100 + 137 * (i * 7 % 29) for i in range(30)],      # the four longest
+                                     [8100 + 60 * (i * 7 % 27) for i in range(26)] + [13_000, 10_000, 12_500, 12_000]))      # the longest again
 def test_copies_without_room(be, orc, lengths):
     """512 columns: 96 MB hold 48 000 edges, so that some of these rows, or all but the longest, are summed from the matrix."""
     check(be, orc, 64, 8, lengths)
